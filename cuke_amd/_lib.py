@@ -10,6 +10,7 @@ import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libkge_mi355.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
 
 MODELS = {"TransE": 0, "TransH": 1, "TransR": 2, "DistMult": 3, "ComplEx": 4, "RotatE": 5,
           "TransF": 6, "RESCAL": 7}
@@ -123,7 +124,12 @@ EXPORTS = {
                                               C.c_float, C.c_float, C.c_void_p]),
     "kge_train_step_staged": (C.c_int, [C.POINTER(Tables), C.POINTER(StepBatch), C.POINTER(StepBatch), C.POINTER(StepBuffers),
                                         C.c_void_p, C.c_void_p]),
+    "kge_train_step": (C.c_int, [C.POINTER(Tables), C.POINTER(StepBatch), C.POINTER(StepBuffers), C.c_int, C.c_void_p, C.c_void_p]),
     "kge_sample_negatives": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, C.c_uint64, C.c_uint64, C.c_void_p]),
+    "kge_sample_batch": (C.c_int, [C.c_void_p] * 4 + [C.c_int64] + [C.c_void_p] * 4 +
+                         [C.c_int64, C.c_int64, C.c_uint64, C.c_uint64, C.c_void_p]),
+    "kge_widen_ids": (C.c_int, [C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.POINTER(C.c_int64), C.c_int, C.c_void_p]),
+    "kge_publish_counts": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "kge_check_indices": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),
 }
 
@@ -149,6 +155,23 @@ def lib() -> C.CDLL:
                            f"{ABI_VERSION}: rebuild it with `python -m cuke_amd.build`")
         _lib = handle
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/host.cpp), loaded beside the library it calls into."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise KgeError(f"{HOST_PATH} is missing: build it with `python -m cuke_amd.build`")
+        import torch  # noqa: F401  (its libraries have to be in the process first)
+        from . import _host as module
+        module.set_error(KgeError)
+        _host = module
+    return _host
 
 
 def check(rc: int, what: str) -> None:

@@ -61,6 +61,42 @@ __global__ void sample_negatives_kernel(int64_t *out, int64_t count, uint64_t n_
     }
 }
 
+// One batch of a training loop in one launch: the triples order[0 .. B) of a resident triple list (three columns) and
+// the negatives of sample_negatives_kernel.  A few kilobytes either way: what it replaces is three synchronous host
+// copies per batch.
+__global__ void sample_batch_kernel(const int64_t *ch, const int64_t *cr, const int64_t *ct, const int64_t *order, int64_t B,
+                                    int64_t *h, int64_t *r, int64_t *t, int64_t *neg, int64_t count, uint64_t n_ent,
+                                    uint64_t seed, uint64_t step)
+{
+    const uint64_t base = seed ^ splitmix64(step);
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < B + count; i += (int64_t)gridDim.x * blockDim.x) {
+        if (i < B) {
+            const int64_t q = order[i];
+            h[i] = ch[q], r[i] = cr[q], t[i] = ct[q];
+        } else {
+            const int64_t k = i - B;
+            neg[k] = (int64_t)__umul64hi(splitmix64(base ^ ((uint64_t)k * 0x9E3779B97F4A7C15ull)), n_ent);
+        }
+    }
+}
+
+struct WidenArgs {
+    const int32_t *src[4];
+    int64_t *dst[4];
+    int64_t len[4];
+};
+__global__ void widen_ids_kernel(WidenArgs a)
+{
+    const int q = blockIdx.y;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.len[q]; i += (int64_t)gridDim.x * blockDim.x)
+        a.dst[q][i] = a.src[q][i];
+}
+
+__global__ void publish_counts_kernel(const int32_t *a, const int32_t *b, uint64_t *word)
+{
+    __hip_atomic_store(word, (uint64_t)(uint32_t)a[0] | (uint64_t)(uint32_t)b[0] << 32, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 static int validate_tables(const kge_tables *tab)
 {
     if (!tab || !tab->ent) return KGE_EINVAL;
@@ -298,6 +334,46 @@ int kge_sample_negatives(int64_t *out, int64_t count, int64_t n_ent, uint64_t se
     const int64_t blocks = ceil_div(count, 256);
     hipLaunchKernelGGL(sample_negatives_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0,
                        as_stream(stream), out, count, (uint64_t)n_ent, seed, step);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+int kge_sample_batch(const int64_t *col_h, const int64_t *col_r, const int64_t *col_t, const int64_t *order, int64_t batch,
+                     int64_t *h, int64_t *r, int64_t *t, int64_t *neg, int64_t count, int64_t n_ent, uint64_t seed, uint64_t step,
+                     void *stream)
+{
+    if (batch < 0 || count < 0 || n_ent <= 0) return KGE_ESHAPE;
+    if (batch + count == 0) return KGE_OK;
+    if ((batch > 0 && (!col_h || !col_r || !col_t || !order || !h || !r || !t)) || (count > 0 && !neg)) return KGE_EINVAL;
+    const int64_t blocks = ceil_div(batch + count, 256);
+    hipLaunchKernelGGL(sample_batch_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, as_stream(stream),
+                       col_h, col_r, col_t, order, batch, h, r, t, neg, count, (uint64_t)n_ent, seed, step);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+int kge_widen_ids(const int32_t *const *src, int64_t *const *dst, const int64_t *len, int n_parts, void *stream)
+{
+    if (!src || !dst || !len || n_parts < 1 || n_parts > 4) return KGE_EINVAL;
+    WidenArgs a{};
+    int64_t most = 0;
+    for (int q = 0; q < n_parts; ++q) {
+        if (len[q] < 0 || (len[q] > 0 && (!src[q] || !dst[q]))) return KGE_EINVAL;
+        a.src[q] = src[q], a.dst[q] = dst[q], a.len[q] = len[q];
+        most = len[q] > most ? len[q] : most;
+    }
+    if (most == 0) return KGE_OK;
+    const int64_t blocks = ceil_div(most, 256);
+    hipLaunchKernelGGL(widen_ids_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024), (unsigned)n_parts), dim3(256), 0,
+                       as_stream(stream), a);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+int kge_publish_counts(const int32_t *first, const int32_t *second, uint64_t *host_word, void *stream)
+{
+    if (!first || !second || !host_word) return KGE_EINVAL;
+    hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(1), 0, as_stream(stream), first, second, host_word);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

@@ -12,6 +12,51 @@ using namespace kge;
 
 static hipEvent_t as_event(void *e) { return reinterpret_cast<hipEvent_t>(e); }
 
+// Forward, loss and backward of one batch on `stream`.
+static int step_body(const kge_tables *tab, kge_batch *bat, const kge_step_buffers *buf, void *fws, size_t fws_bytes, void *stream)
+{
+    int rc = kge_score_fwd(tab, bat, buf->pos, buf->neg, buf->side_pos, buf->side_neg, buf->residual, fws, fws_bytes, stream);
+    if (rc) return rc;
+    if (buf->loss) {
+        if ((rc = kge_margin_loss(buf->pos, buf->neg, bat->batch, bat->n_neg, buf->margin, buf->sign, buf->loss, buf->dpos, buf->dneg,
+                                  buf->loss_workspace, buf->loss_workspace_bytes, stream)))
+            return rc;
+    }
+    kge_saved saved{buf->pos, buf->neg, buf->side_pos, buf->side_neg, buf->residual, nullptr, 0, bat->back_rows};
+    if (tab->model == KGE_TRANSR || tab->model == KGE_RESCAL) saved.fwd_workspace = fws, saved.fwd_workspace_bytes = fws_bytes;
+    return kge_score_bwd(tab, bat, &saved, buf->dpos, buf->dneg, &buf->grads, buf->bwd_workspace, buf->bwd_workspace_bytes, stream);
+}
+
+extern "C" int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const kge_step_buffers *buf, int fused, void *stream,
+                              void *side_stream)
+{
+    if (!tab || !cur || !buf || !cur->bat.insp_jobs) return KGE_EINVAL;
+    const bool projection = tab->model == KGE_TRANSR || tab->model == KGE_RESCAL;
+    kge_batch *bat = &cur->bat;
+    const kge_inspect_job *jobs = bat->insp_jobs;
+    void *fws = cur->fwd_workspace ? cur->fwd_workspace : buf->fwd_workspace;
+    const size_t fws_bytes = cur->fwd_workspace ? cur->fwd_workspace_bytes : buf->fwd_workspace_bytes;
+    bat->plans_ready = 0, bat->insp_ready = nullptr, bat->fuse_inspection = 0;
+    int rc;
+    if (projection && (rc = kge_inspect_batch(&jobs[1], 1, stream))) return rc;  // the forward pass is planned from the relation groups
+    if (fused) {
+        bat->fuse_inspection = 1;
+        rc = step_body(tab, bat, buf, fws, fws_bytes, stream);
+        bat->fuse_inspection = 0;
+        return rc;
+    }
+    if (!side_stream || !cur->inspected || !cur->planned) return KGE_EINVAL;
+    hipStream_t st = as_stream(stream), side = as_stream(side_stream);
+    if (hipEventRecord(as_event(cur->planned), st) != hipSuccess || hipStreamWaitEvent(side, as_event(cur->planned), 0) != hipSuccess)
+        return KGE_ELAUNCH;
+    if ((rc = kge_inspect_batch(jobs, projection ? 1 : 2, side_stream))) return rc;
+    if (hipEventRecord(as_event(cur->inspected), side) != hipSuccess) return KGE_ELAUNCH;
+    bat->insp_ready = cur->inspected;  // backward waits for it right before its segmented reduction
+    rc = step_body(tab, bat, buf, fws, fws_bytes, stream);
+    bat->insp_ready = nullptr;
+    return rc;
+}
+
 extern "C" int kge_train_step_staged(const kge_tables *tab, kge_step_batch *cur, kge_step_batch *next, const kge_step_buffers *buf,
                                      void *stream, void *side_stream)
 {
@@ -58,17 +103,7 @@ extern "C" int kge_train_step_staged(const kge_tables *tab, kge_step_batch *cur,
         const int rc = kge_inspect_batch(&bat->insp_jobs[1], 1, stream);
         if (rc) return rc;
     }
-    int rc = kge_score_fwd(tab, bat, buf->pos, buf->neg, buf->side_pos, buf->side_neg, buf->residual, fws, fws_bytes, stream);
-    if (rc) return rc;
-    if (buf->loss) {
-        if ((rc = kge_margin_loss(buf->pos, buf->neg, bat->batch, bat->n_neg, buf->margin, buf->sign, buf->loss, buf->dpos, buf->dneg,
-                                  buf->loss_workspace, buf->loss_workspace_bytes, stream)))
-            return rc;
-    }
-    kge_saved saved{buf->pos, buf->neg, buf->side_pos, buf->side_neg, buf->residual, nullptr, 0, bat->back_rows};
-    if (projection) saved.fwd_workspace = fws, saved.fwd_workspace_bytes = fws_bytes;
-    if ((rc = kge_score_bwd(tab, bat, &saved, buf->dpos, buf->dneg, &buf->grads, buf->bwd_workspace, buf->bwd_workspace_bytes, stream)))
-        return rc;
+    if (const int rc = step_body(tab, bat, buf, fws, fws_bytes, stream)) return rc;
     if (hipEventRecord(as_event(cur->released), st) != hipSuccess) return KGE_ELAUNCH;
     cur->released_valid = 1;
     return KGE_OK;

@@ -89,6 +89,11 @@ class TrainSampler:
         self.dev = torch.device(device)
         self.step = 0
         self._order, self._pos, self._epoch = None, 0, 0
+        # The triples (24 bytes each) and the epoch's order (8) stay on the device, so that a batch is one gather
+        # launch instead of a numpy gather and three host-to-device copies that each wait for the stream.  Lists of
+        # more than a gigabyte are batched on the host.
+        self._resident = self.dev.type == "cuda" and 32 * len(self.h) <= 1 << 30
+        self._triples = self._order_dev = None
 
     def _next_ids(self):
         if self._order is None or self._pos + self.batch > len(self._order):
@@ -96,23 +101,39 @@ class TrainSampler:
             self._order = np.random.default_rng([self.seed, self._epoch]).permutation(n) if self.shuffle \
                 else np.arange(n)
             self._pos, self._epoch = 0, self._epoch + 1
-        ids = self._order[self._pos:self._pos + self.batch]
+            if self._order_dev is not None:
+                torch.cuda.synchronize(self.dev)  # once per epoch: batches may have been taken on other streams too
+                self._order_dev = None
+        at = self._pos
         self._pos += self.batch
-        return ids
+        return at
 
     def __iter__(self):
         return self
 
     def __next__(self):
-        ids = self._next_ids()
-        h, r, t = (torch.from_numpy(x[ids]).to(self.dev) for x in (self.h, self.r, self.t))
+        at = self._next_ids()
         count = (self.batch // self.chunk) * self.n_neg
+        got = None
+        if self._resident:
+            if self._triples is None:
+                self._triples = torch.from_numpy(np.stack((self.h, self.r, self.t))).to(self.dev)
+            if self._order_dev is None:
+                self._order_dev = torch.from_numpy(self._order.astype(np.int64, copy=False)).to(self.dev)
+            got = _lib.host().sample_batch(self._triples, self._order_dev, at, self.batch, count, self.n_entities, self.seed, self.step)
+        if got is None:
+            got = self._host_batch(at, count)
+        if self.mode == "both":
+            self.neg_mode = "head" if self.step % 2 else "tail"
+        self.step += 1
+        return got
+
+    def _host_batch(self, at, count):
+        ids = self._order[at:at + self.batch]
+        h, r, t = (torch.from_numpy(x[ids]).to(self.dev) for x in (self.h, self.r, self.t))
         neg = torch.empty(count, dtype=torch.int64, device=self.dev)
         _lib.check(_lib.lib().kge_sample_negatives(C.c_void_p(neg.data_ptr()), count, self.n_entities,
                                                    self.seed, self.step,
                                                    C.c_void_p(torch.cuda.current_stream().cuda_stream)),
                    "kge_sample_negatives")
-        if self.mode == "both":
-            self.neg_mode = "head" if self.step % 2 else "tail"
-        self.step += 1
         return h, r, t, neg

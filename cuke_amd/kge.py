@@ -9,7 +9,9 @@ that :class:`KGEModel` offers what a training step needs and the reference does
 not have: scalar scores, shared negatives, and sparse row gradients.
 
 torch is used for device memory and streams only; every computation is a kernel
-of libkge_mi355.so reached through the C ABI.
+of libkge_mi355.so reached through the C ABI.  The eager calls go through csrc/host.cpp, the same
+sequence in native code; what it does not take (other dtypes, devices, layouts, wrong shapes) falls
+through to the code here, which converts or raises.
 """
 from __future__ import annotations
 
@@ -107,10 +109,43 @@ class Inspection:
         return self.seg_offsets[: self.num_unique + 1]
 
 
+def _up256(x: int) -> int:
+    return (x + 255) & ~255
+
+
+class _PackedInspection(Inspection):
+    """An inspection made by the native host path: the ids in one tensor, everything else in one block
+    ([num_unique][seg_offsets][perm][inverse][sorted_seg], each on a 256-byte boundary).  The views are made
+    when they are asked for; most callers never look."""
+
+    def __init__(self, ids, block, struct: bytes):
+        self._c = _lib.Inspection.from_buffer_copy(struct)
+        self.n, self.n_rows = self._c.n, self._c.n_rows
+        self.unique_ids, self._block, self._u = ids, block, None
+
+    def __getattr__(self, name):  # (only what is not there yet)
+        n, i4 = self.n, _up256(4 * max(self.n, 1))
+        after_seg = 256 + _up256(4 * (n + 1))
+        at = {"num_unique_dev": (0, 1), "seg_offsets": (256, n + 1), "perm": (after_seg, max(n, 1)),
+              "inverse": (after_seg + i4, max(n, 1)), "sorted_seg": (after_seg + 2 * i4, max(n, 1))}.get(name)
+        if at is None:
+            raise AttributeError(name)
+        view = self._block[at[0]:at[0] + 4 * at[1]].view(torch.int32)
+        setattr(self, name, view)
+        return view
+
+
+def _insp_address(ins) -> int:
+    return 0 if ins is None else C.addressof(ins._c)
+
+
 def inspect(parts, n_rows: int) -> Inspection:
     """Radix-sort and dedup the concatenation of up to four int64 index tensors."""
     if isinstance(parts, torch.Tensor):
         parts = [parts]
+    packed = _lib.host().inspect(parts, n_rows)
+    if packed is not None:
+        return _PackedInspection(*packed)
     if not 1 <= len(parts) <= 4:
         raise ValueError("inspect takes one to four index tensors")
     dev = parts[0].device
@@ -218,6 +253,7 @@ class KGEModel:
                                 int(self.E.shape[0]), self.n_rel, self.E.data_ptr(),
                                 self.R.data_ptr() if (self.R is not None and self.rel_dim) else None,
                                 self.A.data_ptr() if self.A is not None else None)
+        self._tab_address = C.addressof(self._tab)
 
     @property
     def pair_sums(self) -> str:
@@ -284,6 +320,14 @@ class KGEModel:
         ``neg_mode='tail'``: neg[b, k] scores (h_b, r_b, neg_k), the reference's shared-negative layout
         (apps/examples/examples.py:1404-1444); ``'head'``: (neg_k, r_b, t_b), the head-corrupted batches of
         the reference's sampler (apps/kge/data/sampler.py:287-353)."""
+        if neg_mode in NEG_MODES:
+            got = _lib.host().score(self._tab_address, self.E, h, r, t, neg, chunk, NEG_MODES[neg_mode], _insp_address(ent_insp),
+                                    _insp_address(rel_insp), for_backward)
+            if got is not None:
+                pos, negs, side_pos, side_neg, residual, fwd_ws, back_rows, batch, own_rel = got
+                if own_rel is not None:
+                    rel_insp = _PackedInspection(*own_rel)
+                return Forward(pos, negs, side_pos, side_neg, residual, None, fwd_ws, back_rows, batch, neg_mode, ent_insp, rel_insp)
         if neg is not None and self.model == "RESCAL":
             # a dot-product tile over B projected rows: (E[h] Proj[r]) . E[t'] for replaced tails,
             # E[h'] . (Proj[r] E[t]) for replaced heads; shapes outside the grouped kernels: the pairs as
@@ -367,6 +411,22 @@ class KGEModel:
                            rel_insp=fw.rel_insp, fwd_ws=fw.fwd_ws)
             return self.backward(flat, g)
         h, r, t, neg, C_, N = fw.batch
+        if factor_max and (self.model not in ("TransR", "RESCAL") or neg is not None):
+            raise ValueError("factor_max applies to TransR / RESCAL without shared negatives")
+        ei, ri = fw.ent_insp, fw.rel_insp
+        got = _lib.host().backward(self._tab_address, self.E, fw.batch, NEG_MODES[fw.neg_mode], _insp_address(ei), _insp_address(ri),
+                                   (-1 if ei is None or ei._u is None else ei._u, -1 if ri is None or ri._u is None else ri._u),
+                                   (fw.pos, fw.neg, fw.side_pos, fw.side_neg, fw.residual, fw.fwd_ws, fw.back_rows), dpos, dneg,
+                                   int(factor_max))
+        if got is not None:
+            own_ent, own_rel, ue, ur, ent_rows, rel_rows, aux_rows, aux_x, aux_q, struct = got
+            if own_ent is not None:
+                ei = fw.ent_insp = _PackedInspection(*own_ent)
+            if own_rel is not None:
+                ri = fw.rel_insp = _PackedInspection(*own_rel)
+            ei._u, ri._u = ue, ur
+            return SparseGrads(ei.unique_ids[:ue], ent_rows, ri.unique_ids[:ur], rel_rows, aux_rows, aux_x, aux_q, int(factor_max),
+                               ri.offsets() if factor_max else None, _lib.Grads.from_buffer_copy(struct), ri)
         if fw.ent_insp is None or fw.rel_insp is None:
             e_insp, r_insp = self.inspect_batch(h, r, t, neg)
             fw.ent_insp = fw.ent_insp if fw.ent_insp is not None else e_insp
@@ -393,8 +453,6 @@ class KGEModel:
             aux_rows = torch.empty((min(B, self.n_rel), self.dim * self.dim), **f32)
         aux_x = aux_q = None
         if factor_max:
-            if self.model not in ("TransR", "RESCAL") or neg is not None:
-                raise ValueError("factor_max applies to TransR / RESCAL without shared negatives")
             aux_x, aux_q = torch.empty((B, self.dim), **f32), torch.empty((B, self.dim), **f32)
         grads = _lib.Grads(_ptr(ent_rows), _ptr(rel_rows), _ptr(aux_rows), _ptr(aux_x), _ptr(aux_q), int(factor_max), 0)
         L = _lib.lib()
@@ -413,6 +471,9 @@ class KGEModel:
 
 def margin_loss(pos: torch.Tensor, neg: torch.Tensor, margin: float, sign: float = 1.0):
     """mean_{b,k} max(0, margin - sign * (pos[b] - neg[b, k])) and its gradients (loss, dpos, dneg)."""
+    got = _lib.host().margin_loss(pos, neg, margin, sign)
+    if got is not None:
+        return got
     B, N = neg.shape
     L = _lib.lib()
     loss = torch.empty(1, dtype=torch.float32, device=pos.device)
@@ -435,6 +496,8 @@ def _inplace_table(table):
 
 def sparse_sgd(table: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: float) -> None:
     """table[id] -= lr * rows[u] for the inspection's unique ids (in place, no host sync)."""
+    if _lib.host().sparse_step(table, None, _insp_address(insp), rows, lr, 0.0):
+        return
     t = _inplace_table(table)
     _lib.check(_lib.lib().kge_sparse_sgd(_ptr(t), int(rows.shape[1]), _ptr(insp.unique_ids), _ptr(insp.num_unique_dev),
                                          int(rows.shape[0]), _ptr(rows), float(lr), _stream()), "kge_sparse_sgd")
@@ -443,6 +506,8 @@ def sparse_sgd(table: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: fl
 def sparse_adagrad(table: torch.Tensor, state: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: float,
                    eps: float = 1e-10) -> None:
     """Row-wise Adagrad: state[id] += mean(g^2); table[id] -= lr * g / (sqrt(state[id]) + eps)."""
+    if _lib.host().sparse_step(table, state, _insp_address(insp), rows, lr, eps):
+        return
     t = _inplace_table(table)
     if not state.is_contiguous():
         raise ValueError("state must be contiguous: it is updated in place")
@@ -483,12 +548,18 @@ def _sizes_ok(batch_size, dim, Eemb, h):
 
 def transE(batch_size, dim, nnodes, Eemb, h, t, nedges, Remb, r, *reuse):
     """apps/kge/test_cuke.py:54 -> [batch, dim] = (Eemb[h] - Eemb[t]) + Remb[r]."""
+    out = _lib.host().call(0, Eemb, Remb, None, h, r, t, batch_size, dim, True)
+    if out is not None:
+        return out
     _sizes_ok(batch_size, dim, Eemb, h)
     return KGEModel("TransE", Eemb, Remb).residual(h, r, t)
 
 
 def transH(batch_size, dim, nnodes, Eemb, h, t, nedges, Remb, r, *rest):
     """apps/kge/test_cuke.py:104: (..., rel_ids, uniq, buf, cnt, projection_emb)."""
+    out = _lib.host().call(1, Eemb, Remb, rest[-1] if rest else None, h, r, t, batch_size, dim, True)
+    if out is not None:
+        return out
     _sizes_ok(batch_size, dim, Eemb, h)
     Pemb = rest[-1]
     return KGEModel("TransH", Eemb, Remb, Pemb).residual(h, r, t)
@@ -496,6 +567,9 @@ def transH(batch_size, dim, nnodes, Eemb, h, t, nedges, Remb, r, *rest):
 
 def transR(batch_size, dim, nnodes, Eemb, h, t, nedges, Proj, r, *rest):
     """apps/kge/test_cuke.py:153: (batch, dim, 0, E, h, t, 0, Proj, r, uniq, buf, cnt, Remb)."""
+    out = _lib.host().call(2, Eemb, rest[-1] if rest else None, Proj, h, r, t, batch_size, dim, True)
+    if out is not None:
+        return out
     _sizes_ok(batch_size, dim, Eemb, h)
     Remb = rest[-1]
     m = KGEModel("TransR", Eemb, Remb, Proj)
@@ -504,6 +578,9 @@ def transR(batch_size, dim, nnodes, Eemb, h, t, nedges, Proj, r, *rest):
 
 def transF(batch_size, dim, nnodes, Eemb, h, nedges, Remb, r, *rest):
     """apps/kge/test_cuke.py:198: (batch, dim, nnodes, E, h, nedges, R, r, uniq, buf, cnt, t) -> [batch]."""
+    out = _lib.host().call(6, Eemb, Remb, None, h, r, rest[-1] if rest else None, batch_size, dim, False)
+    if out is not None:
+        return out
     _sizes_ok(batch_size, dim, Eemb, h)
     t = rest[-1]
     return KGEModel("TransF", Eemb, Remb).score(h, r, t).pos
@@ -511,6 +588,9 @@ def transF(batch_size, dim, nnodes, Eemb, h, nedges, Remb, r, *rest):
 
 def RESCAL(batch_size, dim, nnodes, Eemb, h, nedges, Proj, r, *rest):
     """apps/kge/test_cuke.py:244: (batch, dim, nnodes, E, h, nedges, Proj, r, uniq, buf, cnt, t) -> [batch]."""
+    out = _lib.host().call(7, Eemb, None, Proj, h, r, rest[-1] if rest else None, batch_size, dim, False)
+    if out is not None:
+        return out
     _sizes_ok(batch_size, dim, Eemb, h)
     t = rest[-1]
     m = KGEModel("RESCAL", Eemb, None, Proj)
@@ -572,6 +652,7 @@ class TrainStep:
         self._staged, self._stage_at = collections.deque(), 0
         self._pipelined = False   # the ring of run(pipeline=True) has been set up
         self._timeline = None     # set by kernel_times()
+        self._native = None       # structures of the one-call steps, see _native_state()
         self.side = torch.cuda.Stream(device=dev)  # default priority
         self._dev_index = dev.index if dev.index is not None else torch.cuda.current_device()
         self.pos = torch.empty(B, **f32)
@@ -890,6 +971,17 @@ class TrainStep:
         st = C.c_void_p(main.cuda_stream)
         for s_ in self._sets:  # cached unique counts belong to the batches of earlier steps
             s_.ent_insp._u = s_.rel_insp._u = None
+        if backward and overlap and not pipeline and not self._staged and self._timeline is None and self.bat.timeline is None and \
+                self.B > 0 and (not fused or self.fusable) and self._native_ready():
+            # the ordinary step as one library call (same launches in the same order as the calls below)
+            batches, buf = self._native_state()
+            buf.margin, buf.sign = self.margin, self.sign
+            if fused is None:
+                fused = self.fusable
+            _lib.check(self.L.kge_train_step(C.byref(self.m._tab), C.byref(batches[self._cur]), C.byref(buf), 1 if fused else 0,
+                                             st, C.c_void_p(self.side.cuda_stream)), "kge_train_step")
+            self._record_done(main)
+            return
         if not pipeline:
             self.bat.plans_ready = 0  # the forward call plans for itself
         if fused is None:
@@ -1043,10 +1135,20 @@ class TrainStep:
         main.wait_stream(side)                                   # join
 
     # ---- the staged issue from native code: one library call per step ----
+    def _native_key(self):
+        """What the cached structures were built from and a caller can change: the batches and the upstream gradients."""
+        return (len(self._sets), None if self.dpos is None else self.dpos.data_ptr(), None if self.dneg is None else self.dneg.data_ptr())
+
+    def _native_ready(self) -> bool:
+        """The structures exist, or may be built now (events cannot be created in the middle of a graph capture)."""
+        return self._native is not None and self._native_for == self._native_key() or not torch.cuda.is_current_stream_capturing()
+
     def _native_state(self):
         """kge_step_batch per batch (events created once) and the kge_step_buffers of this TrainStep."""
-        if getattr(self, "_native", None) is not None:
+        key = self._native_key()
+        if self._native is not None and self._native_for == key:
             return self._native
+        self._native_for = key
         main = torch.cuda.current_stream()
 
         def event():
@@ -1064,7 +1166,8 @@ class TrainStep:
                 if getattr(s_, "ws_f", None) is None:
                     s_.ws_f = torch.empty(max(self._ws_f_bytes, 1), dtype=torch.uint8, device=self.m.dev)
                 sb.fwd_workspace, sb.fwd_workspace_bytes = s_.ws_f.data_ptr(), self._ws_f_bytes
-            s_.native_events = [event() for _ in range(3)]
+            if getattr(s_, "native_events", None) is None:
+                s_.native_events = [event() for _ in range(3)]
             sb.inspected, sb.planned, sb.released = (e.cuda_event for e in s_.native_events)
             sb.released_valid = 0
             batches.append(sb)

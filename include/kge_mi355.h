@@ -432,6 +432,23 @@ int kge_sparse_adagrad_factored(float *proj, float *state, int64_t dim, const kg
 int kge_sample_negatives(int64_t *out, int64_t count, int64_t n_ent, uint64_t seed, uint64_t step, void *stream);
 
 /*
+ * The same with the batch's positives: row i < batch is triple order[i] of a resident triple list
+ * (col_h / col_r / col_t), and neg[count] are the ids kge_sample_negatives draws.  One launch per batch
+ * in place of three host-to-device copies and the sampler's own.
+ */
+int kge_sample_batch(const int64_t *col_h, const int64_t *col_r, const int64_t *col_t, const int64_t *order, int64_t batch,
+                     int64_t *h, int64_t *r, int64_t *t, int64_t *neg, int64_t count, int64_t n_ent, uint64_t seed, uint64_t step,
+                     void *stream);
+
+/* 32-bit id arrays widened to the 64-bit ids every other entry point takes: up to four arrays in one launch
+   (src / dst / len: host arrays of n_parts device pointers / lengths). */
+int kge_widen_ids(const int32_t *const *src, int64_t *const *dst, const int64_t *len, int n_parts, void *stream);
+
+/* Writes two device counts (kge_inspection.num_unique) to one 64-bit word of pinned host memory, first in the low
+   half: lets the host wait for an inspection without waiting for what was enqueued behind it. */
+int kge_publish_counts(const int32_t *first, const int32_t *second, uint64_t *host_word, void *stream);
+
+/*
  * One step of a staged training loop in ONE call (host-side sequencing only; no counterpart in the
  * reference, which has no training loop).  It enqueues what a host loop would enqueue with seven to ten
  * calls: on `side_stream` the inspection of the NEXT batch (TransR / RESCAL without negatives: both
@@ -481,6 +498,17 @@ typedef struct kge_step_buffers {
 
 int kge_train_step_staged(const kge_tables *tab, kge_step_batch *cur, kge_step_batch *next, const kge_step_buffers *buf,
                           void *stream, void *side_stream);
+
+/*
+ * One step that inspects its own batch, in one call: what a host loop would issue as inspection, kge_score_fwd,
+ * kge_margin_loss (when buf->loss is set) and kge_score_bwd.  fused != 0: the inspection rides in the score kernels'
+ * launches (kge_fused_inspection_ok must hold for the batch), everything on `stream`.  fused == 0: the inspection
+ * runs on `side_stream` beside the forward pass (TransR / RESCAL: the entity half; the relation half goes first on
+ * `stream`), and kge_score_bwd waits for it before its reduction; cur->planned and cur->inspected are the fork and join events.
+ * cur->fwd_workspace, where set, is used in place of buf->fwd_workspace.
+ */
+int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const kge_step_buffers *buf, int fused, void *stream,
+                   void *side_stream);
 
 /* Sets flag[0] (int32, caller-zeroed) to 1 if any idx[i] is outside [0, n_rows). */
 int kge_check_indices(const int64_t *idx, int64_t n, int64_t n_rows, int32_t *flag, void *stream);

@@ -1,0 +1,68 @@
+"""The native host path: what it takes gives the results of the general path, and what it does not take falls
+through to it (other integer widths, non-contiguous inputs, host-side batches)."""
+import numpy as np
+import pytest
+import torch
+
+from cuke_amd import synth
+from helpers import gpu_model
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("model,kw", [("ComplEx", dict(chunk=32, n_neg=17)), ("TransH", dict(chunk=64, n_neg=8, norm_p=1)),
+                                      ("TransR", dict(chunk=32, n_neg=5)), ("TransR", dict()), ("RESCAL", dict(chunk=128, n_neg=3))])
+def test_narrow_ids_and_strided_inputs_give_the_same_bits(model, kw):
+    w = synth.custom_workload(model, n_ent=200, n_rel=9, dim=24, batch=128, sigma=0.3, seed=4, **kw)
+    m, ix = gpu_model(w)
+    forms = [ix, {k: v.to(torch.int32) for k, v in ix.items()},
+             {k: torch.stack((v, v), 1)[:, 0] for k, v in ix.items()}]  # the last one is not contiguous
+    dpos = torch.randn(w.batch, device="cuda")
+    dneg = torch.randn((w.batch, w.n_neg), device="cuda") if w.chunk else None
+    out = []
+    for f in forms:
+        fw = m.score(f["h"], f["r"], f["t"], f.get("neg"), w.chunk or None)
+        g = m.backward(fw, dpos, dneg)
+        assert g.ent_rows.shape[0] == g.ent_ids.numel() == fw.ent_insp.num_unique == int(fw.ent_insp.num_unique_dev.item())
+        ei = fw.ent_insp
+        assert int(ei.offsets()[-1]) == ei.n and torch.equal(ei.inverse[ei.perm.long()], ei.sorted_seg)
+        out.append([x for x in (fw.pos, fw.neg, g.ent_ids, g.ent_rows, g.rel_ids, g.rel_rows, g.aux_rows) if x is not None])
+    # (the third form goes through the general path where it is not contiguous and through the native one after that)
+    for other in out[1:]:
+        assert len(other) == len(out[0]) and all(torch.equal(x, y) for x, y in zip(out[0], other))
+
+
+def test_resident_sampler_equals_the_host_batches_over_epochs(oracle):
+    from cuke_amd.data import TrainSampler
+    rng = np.random.default_rng(3)
+    triples = tuple(rng.integers(0, n, 103) for n in (50, 7, 50))
+    kw = dict(n_entities=50, batch_size=20, neg_sample_size=3, neg_chunk_size=5, seed=9, mode="both")
+    a, b = TrainSampler(triples, **kw), TrainSampler(triples, **kw)
+    b._resident = False
+    for step in range(13):  # five batches an epoch
+        x, y = next(a), next(b)
+        assert a.neg_mode == b.neg_mode
+        assert all(torch.equal(p, q) and p.dtype == torch.int64 for p, q in zip(x, y)), step
+
+
+def test_train_step_in_one_call_equals_the_call_by_call_issue():
+    from cuke_amd.kge import TrainStep
+    for model, kw in (("DistMult", dict(chunk=64, n_neg=32)), ("TransR", dict()), ("TransR", dict(chunk=32, n_neg=8))):
+        w = synth.custom_workload(model, n_ent=400, n_rel=12, dim=48, batch=256, sigma=0.2, rel_zipf=1.1, seed=20, **kw)
+        m, ix = gpu_model(w)
+        loss = dict(loss="margin") if w.chunk else {}
+        st = TrainStep(m, ix["h"], ix["r"], ix["t"], ix.get("neg"), w.chunk or None, **loss)
+
+        def outputs():
+            g = st.sparse_grads()
+            return [x.clone() for x in (st.pos, st.neg, st.loss, g.ent_ids, g.ent_rows, g.rel_rows, g.aux_rows) if x is not None]
+
+        st.run()
+        one = outputs()
+        st._native_ready = lambda: False  # the Python sequence
+        st.run()
+        assert all(torch.equal(x, y) for x, y in zip(one, outputs())), model
+        del st._native_ready
+        if st.fusable:
+            st.run(fused=False)
+            assert all(torch.equal(x, y) for x, y in zip(one, outputs())), model

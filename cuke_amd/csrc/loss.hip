@@ -9,37 +9,64 @@ namespace kge {
 
 constexpr int kLossWaves = 4;
 
+// Bound by its two passes over the [B, N] scores (read, gradient written), 128 bits per lane where rows allow it.
+// A workgroup strides over the rows and leaves ONE partial loss: with one per row the single workgroup that adds them
+// up walked 16384 to 30000 doubles, 18 to 30 us; over at most kLossBlocks partials it is 2 us.
+constexpr int kLossBlocks = 1024;
+
+template <int V>
 __global__ __launch_bounds__(kLossWaves *kWave) void margin_rows_kernel(
     const float *pos, const float *neg, int64_t B, int64_t N, float margin, float sign, float inv,
-    float *dpos, float *dneg, double *row_loss)
+    float *dpos, float *dneg, double *block_loss)
 {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t b = (int64_t)blockIdx.x * kLossWaves + (threadIdx.x >> 6);
-    if (b >= B) return;
-    const float p = pos[b];
-    float sum = 0.0f;
-    int cnt = 0;
-    for (int64_t k = lane; k < N; k += kWave) {
-        const float v = margin - sign * (p - neg[b * N + k]);
-        const bool on = v > 0.0f;
-        sum += on ? v : 0.0f;
-        cnt += on ? 1 : 0;
-        if (dneg) dneg[b * N + k] = on ? sign * inv : 0.0f;
+    __shared__ double s_part[kLossWaves];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    double total = 0.0;
+    for (int64_t b = (int64_t)blockIdx.x * kLossWaves + wave; b < B; b += (int64_t)gridDim.x * kLossWaves) {
+        const float p = pos[b];
+        float sum = 0.0f;
+        int cnt = 0;
+        for (int64_t k = lane * V; k < N; k += kWave * V) {
+            const Vec<V> s = Vec<V>::load(neg + b * N + k);
+            Vec<V> g;
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                const float v = margin - sign * (p - s.v[e]);
+                const bool on = v > 0.0f;
+                sum += on ? v : 0.0f;
+                cnt += on ? 1 : 0;
+                g.v[e] = on ? sign * inv : 0.0f;
+            }
+            if (dneg) g.store(dneg + b * N + k);
+        }
+        sum = wave_sum(sum);
+        cnt = wave_sum_i(cnt);
+        total += (double)sum;
+        if (lane == 0 && dpos) dpos[b] = -sign * inv * (float)cnt;
     }
-    sum = wave_sum(sum);
-    cnt = wave_sum_i(cnt);
-    if (lane == 0) {
-        row_loss[b] = (double)sum;
-        if (dpos) dpos[b] = -sign * inv * (float)cnt;
+    if (lane == 0) s_part[wave] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < kLossWaves; ++w) t += s_part[w];
+        block_loss[blockIdx.x] = t;
     }
 }
 
-__global__ __launch_bounds__(256) void margin_total_kernel(const double *row_loss, int64_t B, double scale,
+__global__ __launch_bounds__(256) void margin_total_kernel(const double *block_loss, int n, double scale,
                                                            float *loss)
 {
     __shared__ double s[256];
     double acc = 0.0;
-    for (int64_t i = threadIdx.x; i < B; i += 256) acc += row_loss[i];
+    double v[kLossBlocks / 256];  // all loads of a thread in flight together
+#pragma unroll
+    for (int q = 0; q < kLossBlocks / 256; ++q) {
+        const int i = threadIdx.x + 256 * q;
+        v[q] = block_loss[i < n ? i : 0];
+        if (i >= n) v[q] = 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < kLossBlocks / 256; ++q) acc += v[q];
     s[threadIdx.x] = acc;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
@@ -49,7 +76,7 @@ __global__ __launch_bounds__(256) void margin_total_kernel(const double *row_los
     if (threadIdx.x == 0) loss[0] = (float)(s[0] * scale);
 }
 
-// Scratch of kge_margin_loss_static: the per-row partial losses, one double per positive.  Every
+// Scratch of kge_margin_loss_static: the partial losses, at most one double per positive.  Every
 // GPU the library runs on holds its own copy of this array (512 KiB) until the process ends.
 constexpr int64_t kStaticLossRows = KGE_MARGIN_LOSS_STATIC_MAX_BATCH;
 static __device__ __align__(256) double scratch[kStaticLossRows];
@@ -96,12 +123,16 @@ int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n
     const double count = (double)batch * (double)n_neg;
     const float inv = count > 0 ? (float)(1.0 / count) : 0.0f;
     double *rows = static_cast<double *>(workspace);
-    if (batch > 0)
-        hipLaunchKernelGGL(margin_rows_kernel, dim3((unsigned)ceil_div(batch, kLossWaves)),
-                           dim3(kLossWaves * kWave), 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos,
-                           dneg, rows);
-    hipLaunchKernelGGL(margin_total_kernel, dim3(1), dim3(256), 0, st, rows, batch,
-                       count > 0 ? 1.0 / count : 0.0, loss);
+    const int64_t want = ceil_div(batch, kLossWaves);
+    const int blocks = (int)(want < kLossBlocks ? want : kLossBlocks);  // (one partial each: never more than the workspace's `batch`)
+    if (batch > 0) {
+        const dim3 grid((unsigned)blocks), block(kLossWaves * kWave);
+        if (n_neg % 4 == 0 && aligned16(neg) && (!dneg || aligned16(dneg)))
+            hipLaunchKernelGGL(margin_rows_kernel<4>, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
+        else
+            hipLaunchKernelGGL(margin_rows_kernel<1>, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
+    }
+    hipLaunchKernelGGL(margin_total_kernel, dim3(1), dim3(256), 0, st, rows, blocks, count > 0 ? 1.0 / count : 0.0, loss);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }
@@ -113,7 +144,7 @@ int kge_margin_loss_static(const float *pos, const float *neg, int64_t batch, in
     double *rows = nullptr;
     const int rc = static_scratch(&rows);
     if (rc) return rc;
-    // every row slot the total kernel reads is written by the row kernel of the same call first,
+    // every slot the total kernel reads is written by the row kernel of the same call first,
     // so nothing left behind by an earlier call needs clearing
     return kge_margin_loss(pos, neg, batch, n_neg, margin, sign, loss, dpos, dneg, rows,
                            sizeof(double) * (size_t)kStaticLossRows, stream);

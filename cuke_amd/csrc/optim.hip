@@ -38,6 +38,103 @@ __global__ __launch_bounds__(256) void sparse_step_kernel(float *table, float *s
     }
 }
 
+// Rows of thousands of floats (a projection matrix as one row): a workgroup of 1024 threads per row.  One wave per row left
+// 600 rows of 160 KB with 600 waves on the chip, each a serial stream read twice.  Bound by the gradient read
+// once and the table read and written; up to 4096 NQ floats the gradient stays in registers between the norm and
+// the update (NQ quads per thread), wider rows are read twice, the second time mostly from the caches.
+// 588 rows of 40000 floats, Adagrad: 167 -> 53 us (282 MB at 5.3 TB/s).
+constexpr int kWideThreads = 1024;
+
+template <bool ADAGRAD, int NQ>  // NQ = 0: any width
+__global__ __launch_bounds__(kWideThreads) void wide_step_kernel(float *table, float *state, int d, const int64_t *ids,
+                                                                 const int32_t *num_unique, const float *rows, float lr, float eps)
+{
+    __shared__ float s_red[kWideThreads / kWave];
+    const int u = blockIdx.x, tid = threadIdx.x, q4 = d >> 2;
+    if (u >= num_unique[0]) return;
+    const int64_t id = ids[u];
+    const float4 *g = reinterpret_cast<const float4 *>(rows + (int64_t)u * d);
+    float4 *w = reinterpret_cast<float4 *>(table + id * (int64_t)d);
+    auto apply = [](float4 &m, const float4 &v, float scale) {
+        m.x -= scale * v.x, m.y -= scale * v.y, m.z -= scale * v.z, m.w -= scale * v.w;
+    };
+    auto square = [](const float4 &v, float sum) { return fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, sum)))); };
+    float4 gv[NQ ? NQ : 1];
+    if constexpr (NQ > 0) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const int f = tid + kWideThreads * q;
+            gv[q] = g[f < q4 ? f : 0];  // clamped: unconditional loads
+            if (f >= q4) gv[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    float scale = lr;
+    if constexpr (ADAGRAD) {
+        float sq = 0.0f;
+        if constexpr (NQ > 0) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) sq = square(gv[q], sq);
+        } else {
+            float part[4] = {0.f, 0.f, 0.f, 0.f};
+            int f = tid;
+            for (; f + 3 * kWideThreads < q4; f += 4 * kWideThreads) {
+                float4 v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = g[f + kWideThreads * e];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[e] = square(v[e], part[e]);
+            }
+            for (; f < q4; f += kWideThreads) part[0] = square(g[f], part[0]);
+            sq = (part[0] + part[1]) + (part[2] + part[3]);
+        }
+        sq = wave_sum(sq);
+        if ((tid & (kWave - 1)) == 0) s_red[tid >> 6] = sq;
+        __syncthreads();
+        sq = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kWideThreads / kWave; ++i) sq += s_red[i];
+        const float s = state[id] + sq / (float)d;
+        __syncthreads();  // every thread has read the old state
+        if (tid == 0) state[id] = s;
+        scale = lr / (sqrtf(s) + eps);
+    }
+    if constexpr (NQ > 0) {
+        constexpr int kFly = 4;
+#pragma unroll
+        for (int q0 = 0; q0 < NQ; q0 += kFly) {
+            float4 m[kFly];
+#pragma unroll
+            for (int e = 0; e < kFly; ++e) {
+                const int f = tid + kWideThreads * (q0 + e);
+                m[e] = w[f < q4 ? f : 0];
+            }
+#pragma unroll
+            for (int e = 0; e < kFly; ++e) {
+                const int f = tid + kWideThreads * (q0 + e);
+                apply(m[e], gv[q0 + e], scale);
+                if (f < q4) w[f] = m[e];
+            }
+        }
+    } else {
+        int f = tid;
+        for (; f + 3 * kWideThreads < q4; f += 4 * kWideThreads) {
+            float4 v[4], m[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = g[f + kWideThreads * e], m[e] = w[f + kWideThreads * e];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) apply(m[e], v[e], scale), w[f + kWideThreads * e] = m[e];
+        }
+        for (; f < q4; f += kWideThreads) {
+            const float4 v = g[f];
+            float4 m = w[f];
+            apply(m, v, scale);
+            w[f] = m;
+        }
+    }
+}
+
+constexpr int64_t kWideDim = 4096;  // from here a row gives every one of the 1024 threads a quad
+
 template <bool ADAGRAD>
 static int launch_step(float *table, float *state, int64_t dim, const int64_t *ids, const int32_t *num_unique,
                        int64_t capacity, const float *rows, float lr, float eps, hipStream_t st)
@@ -45,6 +142,19 @@ static int launch_step(float *table, float *state, int64_t dim, const int64_t *i
     if (!table || !ids || !num_unique || !rows || (ADAGRAD && !state)) return KGE_EINVAL;
     if (dim <= 0 || dim > (1 << 20) || capacity < 0) return KGE_ESHAPE;
     if (capacity == 0) return KGE_OK;
+    if (dim >= kWideDim && dim % 4 == 0 && aligned16(table) && aligned16(rows)) {
+        const dim3 wgrid((unsigned)capacity), wblock(kWideThreads);
+        const int64_t per = ceil_div(dim / 4, kWideThreads);
+#define WIDE_STEP(NQ) hipLaunchKernelGGL((wide_step_kernel<ADAGRAD, NQ>), wgrid, wblock, 0, st, table, state, (int)dim, ids, num_unique, rows, lr, eps)
+        if (!ADAGRAD || per > 16) WIDE_STEP(0);
+        else if (per <= 4) WIDE_STEP(4);
+        else if (per <= 8) WIDE_STEP(8);
+        else if (per <= 12) WIDE_STEP(12);
+        else WIDE_STEP(16);
+#undef WIDE_STEP
+        KGE_CHECK_LAUNCH();
+        return KGE_OK;
+    }
     const dim3 grid((unsigned)ceil_div(capacity, 4)), block(256);
     if (dim % 4 == 0 && aligned16(table) && aligned16(rows))
         hipLaunchKernelGGL((sparse_step_kernel<ADAGRAD, 4>), grid, block, 0, st, table, state, (int)dim, ids, num_unique,

@@ -66,3 +66,26 @@ def test_train_step_in_one_call_equals_the_call_by_call_issue():
         if st.fusable:
             st.run(fused=False)
             assert all(torch.equal(x, y) for x, y in zip(one, outputs())), model
+
+
+@pytest.mark.parametrize("dim", [4096, 4100, 4 * 1024 * 4 + 4, 40000, 65536, 65540, 100004])
+@pytest.mark.parametrize("opt", ["sgd", "adagrad"])
+def test_optimizer_rows_of_thousands_of_floats(oracle, dim, opt):
+    """A workgroup per row: widths on both sides of the register-resident variants' edges."""
+    from cuke_amd.kge import inspect, sparse_adagrad, sparse_sgd
+    from helpers import assert_close
+    rng = np.random.default_rng(dim)
+    table, state = rng.standard_normal((9, dim)).astype(np.float32), rng.random(9).astype(np.float32)
+    ids = np.array([7, 2, 2, 5, 0, 7], dtype=np.int64)
+    rows = rng.standard_normal((6, dim)).astype(np.float32)
+    ins = inspect(torch.from_numpy(ids).cuda(), 9)
+    t, s, g = torch.from_numpy(table).cuda(), torch.from_numpy(state).cuda(), torch.from_numpy(rows).cuda()
+    u = ins.ids().cpu().numpy()
+    if opt == "sgd":
+        sparse_sgd(t, ins, g, 0.1)
+        assert_close(t.cpu().numpy(), oracle.sparse_sgd(table, u, rows[:len(u)], 0.1), what="table")
+    else:
+        sparse_adagrad(t, s, ins, g, 0.1)
+        wt, ws = oracle.sparse_adagrad(table, state, u, rows[:len(u)], 0.1)
+        assert_close(t.cpu().numpy(), wt, what="table")
+        assert_close(s.cpu().numpy(), ws, what="state")

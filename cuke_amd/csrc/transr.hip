@@ -20,6 +20,7 @@
 namespace kge {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 constexpr int kTM = 32;          // triples per tile
 #ifndef KGE_TR_RING
@@ -75,101 +76,131 @@ struct TilePlan {
 #endif
 constexpr int kDmWgs = KGE_TR_DM_WGS;  // workgroups of a dM launch: three per CU, what its registers allow
 
-// Inclusive scan over the 1024 threads of the block: shuffle scan inside each wave, then the 16
-// wave totals are scanned by every wave for itself (two barriers in all).
-__device__ int block_inclusive_scan_1024(int v, int *s_scan)
+// Inclusive scan of x across the wave, on the DPP lanes (rows of 16, then the rows' totals).
+__device__ __forceinline__ int wave_inclusive_scan(int x)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int u = __shfl_up(v, o, kWave);
-        if (lane >= o) v += u;
-    }
-    __syncthreads();  // s_scan may still be read from the previous call
-    if (lane == 63) s_scan[wave] = v;
-    __syncthreads();
-    int before = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) before += w < wave ? s_scan[w] : 0;
-    return v + before;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr:1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+    return x;
 }
 
-// One workgroup per plan: block 0 builds `plan0` with tiles of `tile0` positions (the GEMM plan), block 1
-// (when launched) `plan1`, the chunked plan of the dM kernel: chunks of `tile1` positions, `nib` row blocks per
-// chunk, groups of at most `small_max` triples as one item.
-__global__ __launch_bounds__(1024) void transr_plan_kernel(const int32_t *num_unique, const int32_t *seg_offsets,
-                                                          const int64_t *unique_ids, TilePlan plan0, int tile0,
-                                                          TilePlan plan1, int tile1, int nib, int small_max)
+// Exclusive scans of N counts over the 1024 threads of the block, with their totals: one barrier for all of them.
+// s_tot: [N][16], not written again before another barrier.
+template <int N>
+__device__ __forceinline__ void block_exclusive_scans(const int (&v)[N], int *s_tot, int (&before)[N], int (&total)[N])
 {
-    const bool chunked = blockIdx.x != 0;
-    const TilePlan &plan = chunked ? plan1 : plan0;
-    const int tile = chunked ? tile1 : tile0;
-    __shared__ int s_scan[1024];
-    __shared__ int s_carry[6];  // tiles, split slots, splits, thin groups, long items, small items
-    const int U = num_unique[0];
-    if (threadIdx.x < 6) s_carry[threadIdx.x] = 0;
-    __syncthreads();
-    for (int base = 0; base < U; base += 1024) {
-        const int g = base + threadIdx.x;
-        int s0 = 0, s1 = 0, cnt = 0, rid = 0, thin = 0, n_long = 0, n_small = 0;
-        if (g < U) {
-            s0 = seg_offsets[g], s1 = seg_offsets[g + 1];
-            rid = (int)unique_ids[g];
-            const int n = s1 - s0;
-            cnt = (n + tile - 1) / tile;
-            if (chunked) {  // groups of at most kThin triples have no tiles: thin work writes those
-                thin = n <= kThin ? 1 : 0;
-                if (thin) cnt = 0;
-                else if (n <= small_max) n_small = 1;
-                else n_long = cnt * nib;
-            }
-        }
-        const int inc_t = block_inclusive_scan_1024(cnt, s_scan);
-        const int start = s_carry[0] + inc_t - cnt;
-        int pstart = -1, inc_p = 0, inc_s = 0, inc_th = 0, inc_l = 0, inc_m = 0;
-        if (chunked) {
-            const int pc = cnt > 1 ? cnt : 0, sg = cnt > 1 ? 1 : 0;
-            inc_p = block_inclusive_scan_1024(pc, s_scan);
-            inc_s = block_inclusive_scan_1024(sg, s_scan);
-            inc_th = block_inclusive_scan_1024(thin, s_scan);
-            inc_l = block_inclusive_scan_1024(n_long, s_scan);
-            inc_m = block_inclusive_scan_1024(n_small, s_scan);
-            if (sg) {
-                pstart = s_carry[1] + inc_p - pc;
-                const int si = s_carry[2] + inc_s - 1;
-                plan.split_seg[si] = g;
-                plan.split_first[si] = pstart;
-                plan.split_cnt[si] = cnt;
-            }
-            if (thin) plan.thin_g[s_carry[3] + inc_th - 1] = g;
-            if (n_small) {  // from the back of the list
-                const int at = plan.max_items - 1 - (s_carry[5] + inc_m - 1);
-                plan.item_tile[at] = start, plan.item_blk[at] = -1;
-            }
-            int at = s_carry[4] + inc_l - n_long;
-            for (int q = 0; q < (n_long ? cnt : 0); ++q)
-                for (int ib = 0; ib < nib; ++ib, ++at) plan.item_tile[at] = start + q, plan.item_blk[at] = ib;
-        }
-        for (int q = 0; q < cnt; ++q) {
-            plan.tile_seg[start + q] = g;
-            plan.tile_p0[start + q] = s0 + q * tile;
-            if (plan.tile_end) plan.tile_end[start + q] = s1, plan.tile_rid[start + q] = rid;
-            if (plan.tile_part) plan.tile_part[start + q] = pstart >= 0 ? pstart + q : -1;
-        }
-        __syncthreads();
-        if (threadIdx.x == 1023) {
-            s_carry[0] += inc_t;
-            s_carry[1] += inc_p, s_carry[2] += inc_s, s_carry[3] += inc_th, s_carry[4] += inc_l, s_carry[5] += inc_m;
-        }
-        __syncthreads();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int inc[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        inc[k] = wave_inclusive_scan(v[k]);
+        if (lane == 63) s_tot[16 * k + wave] = inc[k];
     }
-    if (threadIdx.x == 0) {
-        plan.num_tiles[0] = s_carry[0];
-        if (chunked) {
-            plan.num_split[0] = s_carry[2];
-            plan.num_thin[0] = s_carry[3];
-            plan.num_items[0] = s_carry[4], plan.num_items[1] = s_carry[5];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const int t = wave_inclusive_scan(lane < 16 ? s_tot[16 * k + lane] : 0);
+        total[k] = __builtin_amdgcn_readlane(t, 15);
+        before[k] = inc[k] - v[k] + (wave > 0 ? __builtin_amdgcn_readlane(t, wave > 0 ? wave - 1 : 0) : 0);
+    }
+}
+
+// The plan of one workgroup of 1024 threads: a thread per group, its counts placed by scans.  CHUNKED: the plan of the
+// dM kernel (`nib` row blocks per chunk, groups of at most `small_max` triples as one item).  Groups of more than two
+// entries are written by their whole wave (one thread writing its entries in turn made the kernel as long as the
+// largest group: 190 us for groups of thousands).  What is left is the launch and two round trips to memory.
+template <bool CHUNKED>
+__device__ __forceinline__ void plan_body(const int32_t *num_unique, const int32_t *seg_offsets, const int64_t *unique_ids, const TilePlan &plan,
+                                          int tile, int nib, int small_max, int (*s_tot)[96])
+{
+    constexpr int N = CHUNKED ? 6 : 1;  // tiles; then split slots, splits, thin groups, long items, small items
+    const int U = num_unique[0], tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int per = U < 1024 ? (U + 15) / 16 : 64;  // groups per wave: few groups are spread over all of them
+    const int blk0 = CHUNKED ? lane % nib : 0, q0 = CHUNKED ? lane / nib : 0, dblk = CHUNKED ? 64 % nib : 0, dq = CHUNKED ? 64 / nib : 0;
+    int carry[N] = {};
+    for (int base = 0, turn = 0; base < U; base += 1024, turn ^= 1) {
+        const int g0 = base + wave * per, g = lane < per ? g0 + lane : U, gc = g < U ? g : U - 1;
+        const int s0 = seg_offsets[gc], s1 = seg_offsets[gc + 1], rid = CHUNKED ? 0 : (int)unique_ids[gc];
+        const int n = g < U ? s1 - s0 : 0;
+        int v[N], at[N], total[N];
+        v[0] = (n + tile - 1) / tile;
+        if constexpr (CHUNKED) {  // groups of at most kThin triples have no tiles: thin work writes those
+            const bool thin = n <= kThin;
+            if (thin) v[0] = 0;
+            v[1] = v[0] > 1 ? v[0] : 0;
+            v[2] = v[0] > 1 ? 1 : 0;
+            v[3] = thin && n > 0 ? 1 : 0;
+            v[5] = !thin && n <= small_max ? 1 : 0;
+            v[4] = !thin && n > small_max ? v[0] * nib : 0;
         }
+        block_exclusive_scans<N>(v, s_tot[turn], at, total);
+#pragma unroll
+        for (int k = 0; k < N; ++k) at[k] += carry[k], carry[k] += total[k];
+        int part = -1;
+        if constexpr (CHUNKED) {
+            if (v[2]) {
+                part = at[1];
+                plan.split_seg[at[2]] = g, plan.split_first[at[2]] = part, plan.split_cnt[at[2]] = v[0];
+            }
+            if (v[3]) plan.thin_g[at[3]] = g;
+            if (v[5]) {  // from the back of the list
+                const int i = plan.max_items - 1 - at[5];
+                plan.item_tile[i] = at[0], plan.item_blk[i] = -1;
+            }
+        }
+        auto entry = [&](int e, int q, int g_, int p0, int end, int rid_, int part_) {
+            plan.tile_seg[e] = g_;
+            plan.tile_p0[e] = p0 + q * tile;
+            if constexpr (CHUNKED) plan.tile_part[e] = part_ >= 0 ? part_ + q : -1;
+            else plan.tile_end[e] = end, plan.tile_rid[e] = rid_;
+        };
+        const bool many = v[0] > 2 || (CHUNKED && v[CHUNKED ? 4 : 0] > 0);
+        if (!many) {
+            if (v[0] > 0) entry(at[0], 0, g, s0, s1, rid, part);
+            if (v[0] > 1) entry(at[0] + 1, 1, g, s0, s1, rid, part);
+        }
+        for (uint64_t m = __ballot(many); m; m &= m - 1) {
+            const int l = __ffsll((unsigned long long)m) - 1;  // (uniform: the ballot is)
+            const int cnt = __builtin_amdgcn_readlane(v[0], l), to = __builtin_amdgcn_readlane(at[0], l);
+            const int p0 = __builtin_amdgcn_readlane(s0, l), end = __builtin_amdgcn_readlane(s1, l), r = __builtin_amdgcn_readlane(rid, l);
+            const int pt = __builtin_amdgcn_readlane(part, l), g_ = g0 + l;
+            for (int q = lane; q < cnt; q += 64) entry(to + q, q, g_, p0, end, r, pt);
+            if constexpr (CHUNKED) {
+                const int items = __builtin_amdgcn_readlane(v[4], l), io = __builtin_amdgcn_readlane(at[4], l);
+                for (int e = lane, q = q0, b = blk0; e < items; e += 64) {
+                    plan.item_tile[io + e] = to + q, plan.item_blk[io + e] = b;
+                    q += dq, b += dblk;
+                    if (b >= nib) b -= nib, ++q;
+                }
+            }
+        }
+    }
+    if (tid == 0) {
+        plan.num_tiles[0] = carry[0];
+        if constexpr (CHUNKED) {
+            plan.num_split[0] = carry[2];
+            plan.num_thin[0] = carry[3];
+            plan.num_items[0] = carry[4], plan.num_items[1] = carry[5];
+        }
+    }
+}
+
+// One workgroup per plan: block 0 the dM kernel's `dm` with chunks of `chunk` positions, block 1 `tiles` with tiles of
+// `tile1` positions, block 2 `tall` with tiles of `tile2`; a plan without memory is not wanted.
+__global__ __launch_bounds__(1024) void transr_plan_kernel(const int32_t *num_unique, const int32_t *seg_offsets,
+                                                          const int64_t *unique_ids, TilePlan dm, int chunk, int nib, int small_max,
+                                                          TilePlan tiles, int tile1, TilePlan tall, int tile2)
+{
+    __shared__ int s_tot[2][96];
+    if (blockIdx.x == 0) {
+        plan_body<true>(num_unique, seg_offsets, unique_ids, dm, chunk, nib, small_max, s_tot);
+    } else {
+        const TilePlan &p = blockIdx.x == 1 ? tiles : tall;
+        if (p.num_tiles) plan_body<false>(num_unique, seg_offsets, unique_ids, p, blockIdx.x == 1 ? tile1 : tile2, 0, 0, s_tot);
     }
 }
 
@@ -1472,12 +1503,14 @@ static SumRider dm_finish_rider(const DmArgs &a, int64_t max_split)
     return r;
 }
 
+#include "transr_tall.hpp"
+
 // ---- host side -----------------------------------------------------------------------------
 static size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
 struct RPlan {
-    size_t off_plan, off_dplan, off_occ, off_part_e, off_part_r, off_dpart, total;
-    int64_t tiles, dtiles, dsplit, dslots;
+    size_t off_plans, off_occ, off_part_e, off_part_r, off_dpart, total;
+    int64_t dsplit, dslots;
 };
 
 // (items > 0: a chunked plan with its work lists)
@@ -1489,26 +1522,6 @@ static int dm_nib(int64_t d) { return (int)ceil_div(d, 32); }
 static int dm_small_max(int64_t d) { return dm_small_fits((int)d) ? kDmSmall : kThin; }
 static int64_t dm_item_cap(int64_t dtiles, int64_t d) { return dtiles * ceil_div(d, 32); }
 static size_t dplan_ints(int64_t dtiles, int64_t dsplit, int64_t d) { return plan_ints(dtiles, dsplit, dm_item_cap(dtiles, d)); }
-
-static RPlan make_rplan(const kge_tables *tab, const kge_batch *bat)
-{
-    RPlan p{};
-    const int64_t B = bat->batch, d = tab->dim;
-    const int64_t groups = B < tab->n_rel ? B : tab->n_rel;
-    p.tiles = max_tiles(tab, bat);
-    p.dtiles = groups + B / kDmChunk + 1;
-    p.dsplit = B / kDmChunk + 1;            // a split group has more than kDmChunk triples
-    p.dslots = 2 * (B / kDmChunk) + 2;      // sum over split groups of ceil(n_g / chunk)
-    size_t o = 0;
-    p.off_plan = o, o += up256(sizeof(int32_t) * plan_ints(p.tiles, 0));
-    p.off_dplan = o, o += up256(sizeof(int32_t) * dplan_ints(p.dtiles, p.dsplit, d));
-    p.off_occ = o, o += up256(sizeof(float) * (size_t)(2 * B * d));
-    p.off_part_e = o, o += up256(sizeof(float) * (size_t)seg_partial_floats(2 * B, d));
-    p.off_part_r = o, o += up256(sizeof(float) * (size_t)seg_partial_floats(B, d));
-    p.off_dpart = o, o += up256(sizeof(float) * (size_t)(p.dslots * d * d));
-    p.total = o;
-    return p;
-}
 
 static TilePlan plan_at(void *base, int64_t tiles, int64_t split, int64_t items = 0)
 {
@@ -1532,17 +1545,95 @@ static TilePlan plan_at(void *base, int64_t tiles, int64_t split, int64_t items 
     }
     return p;
 }
-static TilePlan dplan_at(void *base, int64_t dtiles, int64_t dsplit, int64_t d)
+
+// The three plans of a batch: 32-triple tiles (the forward pass with back rows; tiles == 0: not wanted), chunks and
+// work lists of the dM kernel, 64-triple tiles.  A backward pass that is handed the forward pass's workspace
+// (kge_saved.fwd_workspace) finds its plans there and launches no plan kernel of its own.
+struct Plans {
+    TilePlan tiles, dm, tall;
+};
+struct PlanSizes {
+    int64_t tiles, dtiles, dsplit, tall, d;
+};
+
+static size_t plans_bytes(const PlanSizes &z)
 {
-    return plan_at(base, dtiles, dsplit, dm_item_cap(dtiles, d));
+    return (z.tiles ? up256(sizeof(int32_t) * plan_ints(z.tiles, 0)) : 0) + up256(sizeof(int32_t) * dplan_ints(z.dtiles, z.dsplit, z.d)) +
+           (z.tall ? up256(sizeof(int32_t) * plan_ints(z.tall, 0)) : 0);
 }
 
-// The forward workspace holds both tile plans of the batch: the 32-triple tiles of the GEMM kernels
-// and the chunked plan of the dM kernel.  A backward pass that is handed this workspace
-// (kge_saved.fwd_workspace) finds its plans there and launches no plan kernel of its own.
-static size_t fwd_plan_bytes(const kge_tables *tab, const kge_batch *bat)
+static Plans plans_at(void *base, const PlanSizes &z)
 {
-    return up256(sizeof(int32_t) * plan_ints(max_tiles(tab, bat), 0));
+    char *p = static_cast<char *>(base);
+    Plans r{};
+    if (z.tiles) r.tiles = plan_at(p, z.tiles, 0), p += up256(sizeof(int32_t) * plan_ints(z.tiles, 0));
+    r.dm = plan_at(p, z.dtiles, z.dsplit, dm_item_cap(z.dtiles, z.d)), p += up256(sizeof(int32_t) * dplan_ints(z.dtiles, z.dsplit, z.d));
+    if (z.tall) r.tall = plan_at(p, z.tall, 0);
+    return r;
+}
+
+static void launch_plans(const kge_inspection *ri, const int32_t *seg_offsets, const Plans &p, int64_t d, hipStream_t st)
+{
+    hipLaunchKernelGGL(transr_plan_kernel, dim3(3), dim3(1024), 0, st, ri->num_unique, seg_offsets, ri->unique_ids, p.dm, kDmChunk,
+                       dm_nib(d), dm_small_max(d), p.tiles, kTM, p.tall, kTallRows);
+}
+
+static PlanSizes plan_sizes(const kge_tables *tab, const kge_batch *bat)
+{
+    const int64_t B = bat->batch, groups = B < tab->n_rel ? B : tab->n_rel;
+    return PlanSizes{max_tiles(tab, bat), groups + B / kDmChunk + 1, B / kDmChunk + 1 /* a split group has more than kDmChunk triples */,
+                     want_tall(tab->dim, B, tab->n_rel) ? tall_tiles(groups, B) : 0, tab->dim};
+}
+
+static size_t lds_with(const FusedInsp &fi, size_t own)
+{
+    return fi.blocks > 0 && (size_t)fi.lds_bytes > own ? (size_t)fi.lds_bytes : own;
+}
+
+template <int MODE>
+static int launch_short(const GemmArgs &a, const FusedInsp &fi, hipStream_t st)
+{
+    const size_t lds = lds_with(fi, gemm_lds_bytes(a.d));
+    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(&transr_gemm_kernel<MODE>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxGemmLds) != hipSuccess)
+        return KGE_ELAUNCH;
+    hipLaunchKernelGGL(transr_gemm_kernel<MODE>, dim3((unsigned)(a.max_tiles + a.thin_groups + fi.blocks)), dim3(256), lds, st, a, fi);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+// The grouped product of mode `mode` (see transr_gemm_body) over at most `groups` groups: by 64-row tiles if the plans
+// hold them (want_tall), by 32-row tiles and streamed small groups if not.  part: tall_part_floats() where a.pos is set.
+static int launch_product(int mode, GemmArgs a, const Plans &p, const PlanSizes &z, int64_t groups, float *part, int64_t B,
+                          const FusedInsp &fi, hipStream_t st)
+{
+    if (z.tall) {
+        a.plan = p.tall;
+        return launch_tall(mode, a, z.tall, part, B, fi, st);
+    }
+    a.plan = p.tiles, a.max_tiles = (int)z.tiles, a.thin_groups = (int)groups;
+    switch (mode) {
+    case 0: return launch_short<0>(a, fi, st);
+    case 1: return launch_short<1>(a, fi, st);
+    case 2: return launch_short<2>(a, fi, st);
+    default: return launch_short<3>(a, fi, st);
+    }
+}
+
+static RPlan make_rplan(const kge_tables *tab, const kge_batch *bat)
+{
+    RPlan p{};
+    const int64_t B = bat->batch, d = tab->dim;
+    p.dsplit = plan_sizes(tab, bat).dsplit;
+    p.dslots = 2 * (B / kDmChunk) + 2;      // sum over split groups of ceil(n_g / chunk)
+    size_t o = 0;
+    p.off_plans = o, o += plans_bytes(plan_sizes(tab, bat));
+    p.off_occ = o, o += up256(sizeof(float) * (size_t)(2 * B * d));
+    p.off_part_e = o, o += up256(sizeof(float) * (size_t)seg_partial_floats(2 * B, d));
+    p.off_part_r = o, o += up256(sizeof(float) * (size_t)seg_partial_floats(B, d));
+    p.off_dpart = o, o += up256(sizeof(float) * (size_t)(p.dslots * d * d));
+    p.total = o;
+    return p;
 }
 
 static bool pad_path_ok(const kge_tables *, const kge_batch *);
@@ -1553,27 +1644,11 @@ static int launch_transr_plan_padded(const kge_tables *, const kge_batch *, void
 static int launch_transr_bwd_padded(const kge_tables *, const kge_batch *, const kge_saved *, const float *, const kge_grads *, void *,
                                     size_t, hipStream_t);
 
+// forward workspace: the plans, then the column blocks' partial scores of wide rows
 size_t transr_fwd_workspace(const kge_tables *tab, const kge_batch *bat)
 {
     if (pad_path_ok(tab, bat)) return transr_fwd_workspace_padded(tab, bat);  // row width not a multiple of four
-    const RPlan p = make_rplan(tab, bat);
-    return fwd_plan_bytes(tab, bat) + up256(sizeof(int32_t) * dplan_ints(p.dtiles, p.dsplit, tab->dim));
-}
-
-// A launch with more than 64 KB of dynamic LDS has to be allowed per kernel first.
-template <int MODE>
-static int allow_lds(size_t bytes)
-{
-    if (bytes <= 64 * 1024) return KGE_OK;
-    return hipFuncSetAttribute(reinterpret_cast<const void *>(&transr_gemm_kernel<MODE>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxGemmLds) == hipSuccess
-               ? KGE_OK
-               : KGE_ELAUNCH;
-}
-
-static size_t lds_with(const FusedInsp &fi, size_t own)
-{
-    return fi.blocks > 0 && (size_t)fi.lds_bytes > own ? (size_t)fi.lds_bytes : own;
+    return plans_bytes(plan_sizes(tab, bat)) + up256(sizeof(float) * tall_part_floats(tab->dim, bat->batch));
 }
 
 // Whether the forward pass of this batch can also write the rows phi(y_b) Proj^T (kge_batch.back_rows).
@@ -1607,34 +1682,26 @@ int launch_transr_fwd(const kge_tables *tab, const kge_batch *bat, float *pos, f
         return rc;
     }
     const kge_inspection *ri = bat->rel_insp;
-    const int64_t tiles = max_tiles(tab, bat);
-    TilePlan plan = plan_at(workspace, tiles, 0);
-    const RPlan rp = make_rplan(tab, bat);
-    TilePlan dplan = dplan_at(static_cast<char *>(workspace) + fwd_plan_bytes(tab, bat), rp.dtiles, rp.dsplit, tab->dim);
-    if (!bat->plans_ready)
-        hipLaunchKernelGGL(transr_plan_kernel, dim3(2), dim3(1024), 0, st, ri->num_unique, ri->seg_offsets, ri->unique_ids, plan,
-                           kTM, dplan, kDmChunk, dm_nib(tab->dim), dm_small_max(tab->dim));
+    const PlanSizes z = plan_sizes(tab, bat);
+    const Plans plans = plans_at(workspace, z);
+    if (!bat->plans_ready) launch_plans(ri, ri->seg_offsets, plans, tab->dim, st);
     GemmArgs a{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
-               plan, nullptr, nullptr, pos, resid, nullptr, nullptr, (int)tab->dim, tab->norm_p, thin_groups(tab, bat), (int)tiles,
-               BwdSrc{}, bat->back_rows};
-    size_t own = gemm_lds_bytes((int)tab->dim);
-    if (a.back && thin_both_lds_bytes((int)tab->dim) > own) own = thin_both_lds_bytes((int)tab->dim);
-    const size_t lds = lds_with(fi, own);
-    const dim3 grid((unsigned)(tiles + a.thin_groups + fi.blocks));
-    if (a.back) {
-        if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(&transr_fwd_back_kernel),
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxGemmLds) != hipSuccess)
-            return KGE_ELAUNCH;
-        hipLaunchKernelGGL(transr_fwd_back_kernel, grid, dim3(256), lds, st, a, fi);
-    } else {
-        if (const int rc = rescal ? allow_lds<1>(lds) : allow_lds<0>(lds)) return rc;
-        if (rescal)
-            hipLaunchKernelGGL(transr_gemm_kernel<1>, grid, dim3(256), lds, st, a, fi);
-        else
-            hipLaunchKernelGGL(transr_gemm_kernel<0>, grid, dim3(256), lds, st, a, fi);
+               plans.tiles, nullptr, nullptr, pos, resid, nullptr, nullptr, (int)tab->dim, tab->norm_p,
+               thin_groups(tab, bat), (int)z.tiles, BwdSrc{}, bat->back_rows};
+    if (!a.back) {
+        float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + plans_bytes(z));
+        const int rc = launch_product(rescal ? 1 : 0, a, plans, z, a.thin_groups, part, bat->batch, fi, st);
+        timeline_mark(bat->timeline, st, "transr_plan_kernel + transr_gemm_kernel<fwd>");
+        return rc;
     }
-    timeline_mark(bat->timeline, st, a.back ? "transr_plan_kernel + transr_fwd_back_kernel"
-                                            : "transr_plan_kernel + transr_gemm_kernel<fwd>");
+    size_t own = gemm_lds_bytes((int)tab->dim);
+    if (thin_both_lds_bytes((int)tab->dim) > own) own = thin_both_lds_bytes((int)tab->dim);
+    const size_t lds = lds_with(fi, own);
+    if (lds > 64 * 1024 && hipFuncSetAttribute(reinterpret_cast<const void *>(&transr_fwd_back_kernel),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxGemmLds) != hipSuccess)
+        return KGE_ELAUNCH;
+    hipLaunchKernelGGL(transr_fwd_back_kernel, dim3((unsigned)(z.tiles + a.thin_groups + fi.blocks)), dim3(256), lds, st, a, fi);
+    timeline_mark(bat->timeline, st, "transr_plan_kernel + transr_fwd_back_kernel");
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }
@@ -1651,16 +1718,13 @@ int launch_rescal_head_rows(const kge_tables *tab, const kge_batch *bat, float *
     if (!workspace || workspace_bytes < transr_fwd_workspace(tab, bat)) return KGE_EWORKSPACE;
     const kge_inspection *ri = bat->rel_insp;
     const int d = (int)tab->dim;
-    const int64_t tiles = max_tiles(tab, bat);
-    TilePlan plan = plan_at(workspace, tiles, 0);
+    const PlanSizes z = plan_sizes(tab, bat);
     const BwdSrc src{tab->ent, nullptr, nullptr, nullptr, bat->h, bat->t, ri->perm, tab->norm_p, 1, nullptr, 1};
     GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
-                plan, nullptr, nullptr, nullptr, nullptr, u, nullptr, d, tab->norm_p, thin_groups(tab, bat), (int)tiles, src};
-    if (const int rc = allow_lds<2>(gemm_lds_bytes(d))) return rc;
-    hipLaunchKernelGGL(transr_gemm_kernel<2>, dim3((unsigned)(tiles + ga.thin_groups)), dim3(256), gemm_lds_bytes(d), st, ga, FusedInsp{});
+                TilePlan{}, nullptr, nullptr, nullptr, nullptr, u, nullptr, d, tab->norm_p, 0, 0, src};
+    const int rc = launch_product(2, ga, plans_at(workspace, z), z, thin_groups(tab, bat), nullptr, bat->batch, FusedInsp{}, st);
     timeline_mark(bat->timeline, st, "transr_gemm_kernel<head rows>");
-    KGE_CHECK_LAUNCH();
-    return KGE_OK;
+    return rc;
 }
 
 // The tile plans alone (what launch_transr_fwd builds first), for callers that plan a batch ahead.
@@ -1672,11 +1736,7 @@ int launch_transr_plan(const kge_tables *tab, const kge_batch *bat, void *worksp
     if (!mfma_path_ok(tab, bat) || gemm_lds_bytes((int)tab->dim) > kMaxGemmLds) return KGE_EUNSUPPORTED;
     if (!workspace || workspace_bytes < transr_fwd_workspace(tab, bat)) return KGE_EWORKSPACE;
     const kge_inspection *ri = bat->rel_insp;
-    const RPlan rp = make_rplan(tab, bat);
-    TilePlan plan = plan_at(workspace, max_tiles(tab, bat), 0);
-    TilePlan dplan = dplan_at(static_cast<char *>(workspace) + fwd_plan_bytes(tab, bat), rp.dtiles, rp.dsplit, tab->dim);
-    hipLaunchKernelGGL(transr_plan_kernel, dim3(2), dim3(1024), 0, st, ri->num_unique, ri->seg_offsets, ri->unique_ids, plan, kTM,
-                       dplan, kDmChunk, dm_nib(tab->dim), dm_small_max(tab->dim));
+    launch_plans(ri, ri->seg_offsets, plans_at(workspace, plan_sizes(tab, bat)), tab->dim, st);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }
@@ -1691,8 +1751,8 @@ int launch_transr_plan(const kge_tables *tab, const kge_batch *bat, void *worksp
 int launch_rescal_neg_tiles(const kge_tables *, const kge_batch *, const float *, const float *, float *, float *, hipStream_t);
 
 struct RescalNegPlan {
-    size_t off_plan, off_dplan, off_xs, off_qs, off_g0, off_occ, off_part_e, off_dpart, total;
-    int64_t tiles, dtiles, dsplit, dslots, nn;
+    size_t off_plans, off_xs, off_qs, off_g0, off_occ, off_part_e, off_dpart, total;
+    int64_t dsplit, dslots, nn;
 };
 
 static RescalNegPlan make_rescal_neg_plan(const kge_tables *tab, const kge_batch *bat)
@@ -1700,7 +1760,7 @@ static RescalNegPlan make_rescal_neg_plan(const kge_tables *tab, const kge_batch
     RescalNegPlan p{};
     const RPlan r = make_rplan(tab, bat);
     const int64_t B = bat->batch, d = tab->dim;
-    p.tiles = r.tiles, p.dtiles = r.dtiles, p.dsplit = r.dsplit, p.dslots = r.dslots;
+    p.dsplit = r.dsplit, p.dslots = r.dslots;
     p.nn = bat->chunk > 0 ? (B / bat->chunk) * bat->n_neg : 0;
     size_t o = 0;
     auto take = [&](size_t bytes) {
@@ -1708,8 +1768,7 @@ static RescalNegPlan make_rescal_neg_plan(const kge_tables *tab, const kge_batch
         o += up256(bytes > 0 ? bytes : 1);
         return at;
     };
-    p.off_plan = take(sizeof(int32_t) * plan_ints(p.tiles, 0));
-    p.off_dplan = take(sizeof(int32_t) * dplan_ints(p.dtiles, p.dsplit, d));
+    p.off_plans = take(plans_bytes(plan_sizes(tab, bat)));
     p.off_xs = take(sizeof(float) * (size_t)(B * d));
     p.off_qs = take(sizeof(float) * (size_t)(B * d));
     p.off_g0 = take(sizeof(float) * (size_t)(B * d));
@@ -1787,27 +1846,17 @@ int launch_rescal_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     // (occurrence rows: [h of the B positives | t of the B positives | negatives])
     hipLaunchKernelGGL(rescal_neg_prep_kernel, dim3((unsigned)ceil_div(B, 4)), dim3(256), 0, st, tab->ent, bat->h, bat->t, ri->perm, dpos,
                        dneg ? g0 : nullptr, saved->residual, xs, qs, head ? occ : occ + B * d, B, d, head ? 1 : 0);
-    TilePlan plan = plan_at(ws + p.off_plan, p.tiles, 0), dplan = dplan_at(ws + p.off_dplan, p.dtiles, p.dsplit, d);
-    hipLaunchKernelGGL(transr_plan_kernel, dim3(2), dim3(1024), 0, st, ri->num_unique, ri->seg_offsets, ri->unique_ids, plan, kTM, dplan,
-                       kDmChunk, dm_nib(d), dm_small_max(d));
-    if (head) {
-        // the tails' rows: (g E[h] + G) Proj[r], the forward product on rows given as an array, written per triple
-        GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
-                    plan, xs, nullptr, nullptr, occ + B * d, nullptr, nullptr, d, tab->norm_p, thin_groups(tab, bat), (int)p.tiles,
-                    BwdSrc{}};
-        if (const int rc = allow_lds<1>(gemm_lds_bytes(d))) return rc;
-        hipLaunchKernelGGL(transr_gemm_kernel<1>, dim3((unsigned)(p.tiles + ga.thin_groups)), dim3(256), gemm_lds_bytes(d), st, ga,
-                           FusedInsp{});
-    } else {
-        GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
-                    plan, qs, nullptr, nullptr, nullptr, occ, nullptr, d, tab->norm_p, thin_groups(tab, bat), (int)p.tiles, BwdSrc{}};
-        if (const int rc = allow_lds<2>(gemm_lds_bytes(d))) return rc;
-        hipLaunchKernelGGL(transr_gemm_kernel<2>, dim3((unsigned)(p.tiles + ga.thin_groups)), dim3(256), gemm_lds_bytes(d), st, ga,
-                           FusedInsp{});
-    }
+    const PlanSizes z = plan_sizes(tab, bat);
+    const Plans plans = plans_at(ws + p.off_plans, z);
+    launch_plans(ri, ri->seg_offsets, plans, d, st);
+    // head: the tails' rows (g E[h] + G) Proj[r], the forward product on rows given as an array, written per triple
+    GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
+                TilePlan{}, head ? xs : qs, nullptr, nullptr, head ? occ + B * d : nullptr, head ? nullptr : occ, nullptr, d, tab->norm_p, 0, 0,
+                BwdSrc{}};
+    if (const int rc = launch_product(head ? 1 : 2, ga, plans, z, thin_groups(tab, bat), nullptr, B, FusedInsp{}, st)) return rc;
     timeline_mark(bat->timeline, st, "transr_gemm_kernel<dX>");
     // dProj[r][i][j] = sum over the group of xs[i] qs[j] in both modes
-    DmArgs da{xs, qs, ri->seg_offsets, dplan, grads->aux_rows, reinterpret_cast<float *>(ws + p.off_dpart), d, ri->num_unique,
+    DmArgs da{xs, qs, ri->seg_offsets, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + p.off_dpart), d, ri->num_unique,
               BwdSrc{}, nullptr, nullptr, 0};
     hipLaunchKernelGGL(transr_dm_kernel, dim3((unsigned)kDmWgs), dim3(256), dm_lds_bytes(d), st, da, FusedInsp{}, SegL1Rider{});
     timeline_mark(bat->timeline, st, "transr_dm_kernel");
@@ -1845,9 +1894,8 @@ int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_sav
     // the plans: left behind by the forward pass, or built here
     const bool have_plans = saved->fwd_workspace && saved->fwd_workspace_bytes >= transr_fwd_workspace(tab, bat);
     char *pbase = have_plans ? static_cast<char *>(const_cast<void *>(saved->fwd_workspace)) : nullptr;
-    TilePlan plan = have_plans ? plan_at(pbase, p.tiles, 0) : plan_at(ws + p.off_plan, p.tiles, 0);
-    TilePlan dplan = have_plans ? dplan_at(pbase + fwd_plan_bytes(tab, bat), p.dtiles, p.dsplit, d)
-                                : dplan_at(ws + p.off_dplan, p.dtiles, p.dsplit, d);
+    const PlanSizes z = plan_sizes(tab, bat);
+    const Plans plans = plans_at(have_plans ? pbase : ws + p.off_plans, z);
 
     // fused entity inspection (its histogram rode with the forward GEMM): first digit pass in a launch
     // of its own, second with the dX GEMM, dedup with dM
@@ -1861,28 +1909,23 @@ int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_sav
         hipLaunchKernelGGL(transr_insp_step_kernel, dim3((unsigned)f1.blocks), dim3(256), lds_with(f1, 0), st, f1);
         timeline_mark(bat->timeline, st, "inspector step");
     }
-    if (!have_plans)
-        hipLaunchKernelGGL(transr_plan_kernel, dim3(2), dim3(1024), 0, st, ri->num_unique, ri->seg_offsets, ri->unique_ids, plan, kTM,
-                           dplan, kDmChunk, dm_nib(d), dm_small_max(d));
+    if (!have_plans) launch_plans(ri, ri->seg_offsets, plans, d, st);
     // Upstream rows q and left operands x are formed inside the two kernels from the forward pass's rows
     // (BwdSrc); RESCAL's tail occurrence rows g * v come out of the dX kernel's staging.
     const BwdSrc src{tab->ent, saved->residual, dpos, saved->pos, bat->h, bat->t, ri->perm, tab->norm_p, rescal ? 1 : 0,
                      rescal ? occ + B * d : nullptr};
     // dX = Q M^T -> occurrence rows of h (and -dX for t)
     GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
-                plan, nullptr, nullptr, nullptr, nullptr, occ, rescal ? nullptr : occ + B * d, d, tab->norm_p, thin_groups(tab, bat),
-                (int)p.tiles, src};
+                TilePlan{}, nullptr, nullptr, nullptr, nullptr, occ, rescal ? nullptr : occ + B * d, d, tab->norm_p, 0, 0, src};
     // dM = X^T Q per relation group
-    DmArgs da{nullptr, nullptr, ri->seg_offsets, dplan, grads->aux_rows, reinterpret_cast<float *>(ws + p.off_dpart), d,
+    DmArgs da{nullptr, nullptr, ri->seg_offsets, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + p.off_dpart), d,
               ri->num_unique, src, factored ? grads->aux_x : nullptr, factored ? grads->aux_q : nullptr, grads->aux_factor_max};
     // With the forward pass's rows z_b = phi(y_b) Proj^T at hand (kge_saved.back_rows) the entity gradients are
     // +-coef_b z_b and no kernel reads the projections again: the reduction scales the rows as it loads them.
     const bool have_back = saved->back_rows != nullptr;
     if (have_back && (rescal || !aligned16(saved->back_rows))) return KGE_EINVAL;
     if (!have_back) {
-        if (const int rc = allow_lds<2>(lds_with(f2, gemm_lds_bytes(d)))) return rc;
-        hipLaunchKernelGGL(transr_gemm_kernel<2>, dim3((unsigned)(p.tiles + ga.thin_groups + f2.blocks)), dim3(256),
-                           lds_with(f2, gemm_lds_bytes(d)), st, ga, f2);
+        if (const int rc = launch_product(2, ga, plans, z, thin_groups(tab, bat), nullptr, B, f2, st)) return rc;
         timeline_mark(bat->timeline, st, "transr_gemm_kernel<dX>");
     } else if (f2.blocks > 0) {  // the inspector step that would have ridden with dX
         hipLaunchKernelGGL(transr_insp_step_kernel, dim3((unsigned)f2.blocks), dim3(256), lds_with(f2, 0), st, f2);

@@ -1,0 +1,377 @@
+// The grouped product of TransR / RESCAL in tiles of 64 triples x 128 columns, where want_tall says so (below): forward
+// scores, the row list of the shared negatives, and dX; the forward pass with back rows keeps its 32-triple
+// tiles.  This file is included by transr.hip (inside namespace kge).
+//
+// A relation's projection is read once per 64 of its triples instead of once per 32, a wave feeds four row blocks
+// from every 128-byte piece it loads, and the left operand goes through LDS in slices of 64 columns (double buffered), so
+// that two to four workgroups fit a CU whatever the row width is (whole rows in LDS left one at width 1024).
+//   what bounds it: the matrix cores where groups are large (8192 x 1024 over 51 relations), the projections'
+//   bytes where they are small (4096 x 512 over 237).  Measured against the 32-row tiles: 8192 x 1024 over 51
+//   relations (RESCAL) 329 -> 229 us, 81 TFLOP/s; 512 x 1000 over 40 the call 178 -> 69 us; one relation with 24576
+//   rows of 1024 reaches 111 TFLOP/s.
+// Tiles of fewer rows run one to three of the four 16-row blocks, so a tail costs what it holds.
+//
+// A superstep of the projection comes back after about two microseconds when the chip is busy, so what a CU holds in
+// flight (three workgroups x three supersteps x 8 KB) sets the pace of what the matrix cores do not.
+
+constexpr int kTallRows = 64;   // triples per tile
+constexpr int kTallCols = 128;  // columns per workgroup at most: 32 per wave, two 16-column MFMA blocks
+constexpr int kTallKC = 64;     // columns of the left operand staged at a time
+constexpr int kTallPitch = kTallKC + 4;
+constexpr int kTallRing = 4;    // supersteps (16 rows of k) of the projection in flight per wave, one of them in use
+constexpr int kTallWgs = 4096;  // workgroups of a launch at most; they stride over the tiles
+// (global, not generic: a pointer that went through LDS would otherwise be followed with flat loads, which also count as LDS
+// operations and are waited for as such)
+typedef const float __attribute__((address_space(1))) *global_f32;
+
+struct TallRows {  // what a tile knows about its rows (LDS, behind the staging buffers)
+    global_f32 v[kTallRows], w[kTallRows];     // the rows the left operand is formed from
+    int64_t t[kTallRows];                      // MODE 1: tail ids
+    int b[kTallRows];
+    float f[kTallRows], g[kTallRows];          // MODE 3: factor of the relation row, whether there is a t; MODE 2: coefficient, upstream gradient
+    float sum[4][kTallRows];
+};
+constexpr size_t kTallLds = sizeof(float) * 2 * kTallRows * kTallPitch + sizeof(TallRows);
+
+__device__ __forceinline__ float4 load4g(global_f32 p)
+{
+    typedef const floatx4 __attribute__((address_space(1))) *global_f32x4;
+    const floatx4 v = *(global_f32x4)p;
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+__host__ __device__ inline int tall_col_blocks(int d) { return (d + kTallCols - 1) / kTallCols; }
+// columns of a block / of a wave: an even split, multiples of four / two
+__host__ __device__ inline int tall_block_cols(int d) { return ((d + tall_col_blocks(d) - 1) / tall_col_blocks(d) + 3) & ~3; }
+
+struct TallArgs {
+    GemmArgs g;    // plan: tiles of kTallRows
+    float *part;   // [column blocks][B] partial scores where there is more than one column block (pos set), else unused
+    int64_t B;
+};
+
+// One superstep's B operands of a lane as they are loaded: at(e, s) = column e, k = 16 q + 4 kk + s.
+template <int MODE>
+struct TallSlot {
+    floatx2 r[4];
+    __device__ __forceinline__ float at(int e, int s) const { return r[s][e]; }
+};
+template <>
+struct TallSlot<2> {
+    floatx4 r[2];
+    __device__ __forceinline__ float at(int e, int s) const { return r[e][s]; }
+};
+
+// Two B-operand values per k row for this lane: columns n0 + 2 li + {0, 1} of M (MODE 2: of M^T).  Addresses are the
+// uniform base plus a 32-bit byte offset (a projection has at most 2^20 elements: no 64-bit address arithmetic on the
+// vector ALUs, which would take issue slots from the matrix instructions); a k beyond the last row is clamped to
+// it (the staged left operand is zero there).
+template <int MODE>
+struct TallLoader {
+    const char *M;
+    uint32_t off[2], last, d4, k0;  // bytes
+    __device__ __forceinline__ void init(const float *M_, int d_, int n0, int wcols, int li, int kk)
+    {
+        M = reinterpret_cast<const char *>(M_), d4 = 4u * (uint32_t)d_;
+        const uint32_t col = (uint32_t)(n0 + (2 * li < wcols ? 2 * li : 0));
+        if constexpr (MODE != 2) off[0] = 4u * (uint32_t)kk * d4 + 4u * col, last = ((uint32_t)d_ - 1) * d4 + 4u * col;
+        else off[0] = col * d4, off[1] = off[0] + d4, last = d4 - 16, k0 = 16u * (uint32_t)kk;
+    }
+    __device__ __forceinline__ void load(int q, TallSlot<MODE> &dst) const
+    {
+        if constexpr (MODE != 2) {
+            const uint32_t o = off[0] + 16u * (uint32_t)q * d4;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const uint32_t f = o + s * d4;
+                dst.r[s] = *reinterpret_cast<const floatx2 *>(M + (f < last ? f : last));
+            }
+        } else {
+            const uint32_t k = k0 + 64u * (uint32_t)q, kc = k < last ? k : last;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) dst.r[e] = *reinterpret_cast<const floatx4 *>(M + (off[e] + kc));
+        }
+    }
+};
+
+// RB row blocks of one tile against this wave's columns.  The next slice of the left operand is staged while this one
+// is multiplied: fetch(i, c) requests row block i of slice c, put(i, c) writes it to LDS buffer c & 1.  Loads return in
+// order, so the requests go out behind the first superstep's piece of the projection and the writes wait until the
+// end of the slice, when everything in front of them has been used anyway.
+template <int MODE, int RB, typename Fetch, typename Put>
+__device__ __forceinline__ void tall_sweep(const TallLoader<MODE> &bl, int nq, TallSlot<MODE> (&ring)[kTallRing], const float *lds, int li, int kk,
+                                           Fetch fetch, Put put, floatx4 (&acc)[RB][2])
+{
+    static_assert(kTallRing == kTallKC / 16, "ring slot u is superstep u of every slice");
+    const int nc = (nq + kTallRing - 1) / kTallRing;
+#pragma unroll 1
+    for (int c = 0; c < nc; ++c) {
+        const float *sX = lds + (c & 1) * (kTallRows * kTallPitch) + li * kTallPitch + 4 * kk;
+        const int next = c + 1 < nc ? c + 1 : c;  // (past the end: the last slice once more, into the buffer nobody reads; no branch around a load)
+#pragma unroll
+        for (int u = 0; u < kTallRing; ++u) {
+            const int q = kTallRing * c + u;
+            bl.load(q + kTallRing - 1, ring[(u + kTallRing - 1) % kTallRing]);
+            if (u == 0) {
+#pragma unroll
+                for (int i = 0; i < RB; ++i) fetch(i, next);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (q >= nq) continue;  // uniform
+            float4 a[RB];
+#pragma unroll
+            for (int m = 0; m < RB; ++m) a[m] = *reinterpret_cast<const float4 *>(sX + 16 * m * kTallPitch + 16 * u);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int m = 0; m < RB; ++m) {
+                    const float av = s == 0 ? a[m].x : s == 1 ? a[m].y : s == 2 ? a[m].z : a[m].w;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) acc[m][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, ring[u].at(e, s), acc[m][e], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i) put(i, c + 1);
+        __syncthreads();
+    }
+}
+
+// MODE as in transr_gemm_body: 0 forward TransR, 1 forward RESCAL (or rows given as an array), 2 dX, 3 list rows.
+// RB: 16-row blocks the tile runs (a template parameter: the staging and accumulator registers follow it).
+template <int MODE, int RB>
+__device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int tile, int cb)
+{
+    const GemmArgs &a = t.g;
+    const int d = a.d, ncb = tall_col_blocks(d);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kk = lane >> 4;
+    // (uniform, but the compiler cannot know: the kernel also stores)
+    const int p0 = __builtin_amdgcn_readfirstlane(a.plan.tile_p0[tile]), seg_end = __builtin_amdgcn_readfirstlane(a.plan.tile_end[tile]);
+    const int64_t rid = __builtin_amdgcn_readfirstlane(a.plan.tile_rid[tile]);
+    const int rows = seg_end - p0 < kTallRows ? seg_end - p0 : kTallRows;
+    const float *M = a.proj + rid * (int64_t)d * d;
+
+    const int bc = tall_block_cols(d), c0 = cb * bc, span = d - c0 < bc ? d - c0 : bc;
+    const int cw = ((span + 3) / 4 + 1) & ~1;
+    const int n0 = c0 + wave * cw;
+    const int wcols = n0 >= c0 + span ? 0 : (c0 + span - n0 < cw ? c0 + span - n0 : cw);
+    TallLoader<MODE> bl;
+    TallSlot<MODE> ring[kTallRing];
+    bl.init(M, d, wcols > 0 ? n0 : c0, wcols, li, kk);
+    const int nq = (d + 15) / 16;
+#pragma unroll
+    for (int u = 0; u + 1 < kTallRing; ++u) bl.load(u, ring[u]);  // the projection's first pieces fly during the index chain below
+    __builtin_amdgcn_sched_barrier(0);
+
+    TallRows &R = *reinterpret_cast<TallRows *>(lds + 2 * kTallRows * kTallPitch);
+    const bool array = a.xs != nullptr && (MODE == 1 || MODE == 2);
+    const bool derived = MODE == 2 && !array;
+    if (tid < kTallRows) {
+        const int p = p0 + (tid < rows ? tid : 0);
+        int b;
+        if constexpr (MODE == 3) b = p, R.f[tid] = a.rs[p];
+        else b = (MODE == 2 && derived) ? a.src.perm[p] : (a.perm ? a.perm[p] : p);
+        R.b[tid] = b;
+        if constexpr (MODE == 2) {
+            if (derived) {
+                const RowMeta m = bwd_row_meta(a.src, p, d);
+                R.f[tid] = m.coef, R.g[tid] = a.src.dpos ? a.src.dpos[b] : 0.0f;
+                R.v[tid] = (global_f32)(bwd_qbase(a.src) + m.qoff), R.w[tid] = (global_f32)(a.src.resid + (int64_t)b * d);
+            } else {
+                R.v[tid] = (global_f32)(a.xs + (int64_t)p * d);
+            }
+        } else {
+            const int64_t h = a.h[b], t = a.t[b];
+            R.v[tid] = (global_f32)(array ? a.xs + (int64_t)p * d : a.ent + h * d);
+            R.w[tid] = (global_f32)(a.ent + (MODE == 3 && t < 0 ? 0 : t) * d);  // (MODE 3, t = -1: no row; read and, in put(), dropped)
+            if constexpr (MODE == 1) R.t[tid] = t;
+            if constexpr (MODE == 3) R.g[tid] = t >= 0 ? 1.0f : 0.0f;
+        }
+    }
+    __syncthreads();
+
+    // Staging: thread tid takes the quad tid % 16 of row tid / 16 of a row block.
+    const int srow = tid >> 4, scol = (tid & 15) * 4;
+    const bool l1 = derived && !a.src.rescal && a.src.norm_p == 1;
+    const bool occ = derived && a.src.occ_v && cb == 0;
+    constexpr bool kTwo = MODE == 0 || MODE == 3;
+    float4 v[RB], w[RB];
+    auto fetch = [&](int i, int c) {
+        const int k4 = c * kTallKC + scol < d ? c * kTallKC + scol : 0;  // clamped: unconditional loads, masked in put()
+        v[i] = load4g(R.v[16 * i + srow] + k4);
+        if constexpr (kTwo) w[i] = load4g(R.w[16 * i + srow] + k4);
+        else w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (MODE == 2)
+            if (occ) w[i] = load4g(R.w[16 * i + srow] + k4);
+    };
+    auto put = [&](int i, int c) {
+        const int row = 16 * i + srow, col = c * kTallKC + scol;
+        const bool colok = col < d;
+        const float4 vv = v[i], ww = w[i];
+        float4 x = vv;
+        if constexpr (MODE == 0) x = make_float4(vv.x - ww.x, vv.y - ww.y, vv.z - ww.z, vv.w - ww.w);
+        if constexpr (MODE == 3) {
+            const bool keep = R.g[row] != 0.0f;
+            x = make_float4(vv.x - (keep ? ww.x : 0.0f), vv.y - (keep ? ww.y : 0.0f), vv.z - (keep ? ww.z : 0.0f), vv.w - (keep ? ww.w : 0.0f));
+        }
+        if constexpr (MODE == 2) {
+            if (derived) {
+                x = scaled4(R.f[row], l1 ? sgn4(vv) : vv);
+                if (occ && row < rows && colok)  // RESCAL: the tail's occurrence row g * (E[h] Proj[r])
+                    *reinterpret_cast<float4 *>(a.src.occ_v + (int64_t)R.b[row] * d + col) = scaled4(R.g[row], ww);
+            }
+        }
+        const bool ok = row < rows && colok;
+        x = make_float4(ok ? x.x : 0.0f, ok ? x.y : 0.0f, ok ? x.z : 0.0f, ok ? x.w : 0.0f);
+        *reinterpret_cast<float4 *>(&lds[(c & 1) * (kTallRows * kTallPitch) + row * kTallPitch + scol]) = x;
+    };
+
+    const bool colok = 2 * li < wcols;
+    const int col = colok ? n0 + 2 * li : c0;
+    float2 rv = make_float2(0.f, 0.f);  // the relation's row, for the epilogue
+    if constexpr (MODE == 0 || MODE == 3) rv = *reinterpret_cast<const float2 *>(a.rel + rid * (int64_t)d + col);
+    floatx4 acc[RB][2];
+#pragma unroll
+    for (int m = 0; m < RB; ++m) acc[m][0] = acc[m][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < RB; ++i) fetch(i, 0);
+#pragma unroll
+    for (int i = 0; i < RB; ++i) put(i, 0);
+    __syncthreads();
+    tall_sweep<MODE, RB>(bl, nq, ring, lds, li, kk, fetch, put, acc);
+
+    // Lane (li, kk) holds rows 16 m + 4 kk + r, columns n0 + 2 li + {0, 1}.  Everything is read before the first
+    // store: a load between two stores makes the compiler wait for the stores in front of it.
+    const bool want_pos = MODE < 2 && a.pos;
+    int rb[RB][4];
+    float2 y[RB][4];
+#pragma unroll
+    for (int m = 0; m < RB; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * m + 4 * kk + r;
+            rb[m][r] = R.b[row];
+            y[m][r] = make_float2(acc[m][0][r], acc[m][1][r]);
+            if constexpr (MODE == 0) y[m][r].x += rv.x, y[m][r].y += rv.y;
+            if constexpr (MODE == 3) {
+                const float f = R.f[row];  // +-1 or 0: exact products
+                y[m][r].x += f * rv.x, y[m][r].y += f * rv.y;
+            }
+        }
+    if constexpr (MODE < 2) {
+        if (want_pos) {  // uniform
+#pragma unroll
+            for (int m0 = 0; m0 < RB; m0 += 2) {
+            float2 tv[RB][4];
+            if constexpr (MODE == 1) {  // the tails' rows, two blocks in one batch of loads
+#pragma unroll
+                for (int m = m0; m < RB && m < m0 + 2; ++m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int row = 16 * m + 4 * kk + r;
+                        tv[m][r] = *reinterpret_cast<const float2 *>(a.ent + R.t[row < rows ? row : 0] * (int64_t)d + col);
+                    }
+            }
+#pragma unroll
+            for (int m = m0; m < RB && m < m0 + 2; ++m)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float s;
+                    if constexpr (MODE == 1) s = fmaf(y[m][r].x, tv[m][r].x, y[m][r].y * tv[m][r].y);
+                    else s = a.norm_p == 1 ? fabsf(y[m][r].x) + fabsf(y[m][r].y) : fmaf(y[m][r].x, y[m][r].x, y[m][r].y * y[m][r].y);
+                    s = row16_sum(colok ? s : 0.0f);
+                    if (li == 0) R.sum[wave][16 * m + 4 * kk + r] = s;
+                }
+            }
+        }
+    }
+    float *const out = MODE == 2 ? a.occ_h : a.resid;
+    if (out && colok) {
+#pragma unroll
+        for (int m = 0; m < RB; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (16 * m + 4 * kk + r < rows) {
+                    const int64_t o = (int64_t)rb[m][r] * d + col;
+                    *reinterpret_cast<float2 *>(out + o) = y[m][r];
+                    if constexpr (MODE == 2)
+                        if (a.occ_t) *reinterpret_cast<float2 *>(a.occ_t + o) = make_float2(-y[m][r].x, -y[m][r].y);
+                }
+    }
+    if constexpr (MODE < 2) {
+        if (want_pos) {
+            __syncthreads();
+            if (tid < rows) {
+                const float s = (R.sum[0][tid] + R.sum[1][tid]) + (R.sum[2][tid] + R.sum[3][tid]);
+                if (ncb > 1) t.part[(int64_t)cb * t.B + R.b[tid]] = s;
+                else a.pos[R.b[tid]] = (MODE == 0 && a.norm_p == 2) ? sqrtf(s) : s;
+            }
+        }
+    }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256, 3) void transr_tall_kernel(TallArgs t, FusedInsp fi)
+{
+    extern __shared__ __align__(16) float lds[];
+    if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(lds))) return;
+    const int ncb = tall_col_blocks(t.g.d), n = t.g.plan.num_tiles[0] * ncb, step = (int)gridDim.x - fi.blocks;
+    for (int it = (int)blockIdx.x - fi.blocks; it < n; it += step) {
+        const int tile = it / ncb, cb = it % ncb, rows = t.g.plan.tile_end[tile] - t.g.plan.tile_p0[tile];
+        if (rows > 48) tall_tile<MODE, 4>(t, lds, tile, cb);
+        else if (rows > 32) tall_tile<MODE, 3>(t, lds, tile, cb);
+        else if (rows > 16) tall_tile<MODE, 2>(t, lds, tile, cb);
+        else tall_tile<MODE, 1>(t, lds, tile, cb);
+        __syncthreads();  // the next tile reuses the staging buffers
+    }
+}
+
+// Scores from the column blocks' partial sums, in block order.
+__global__ __launch_bounds__(256) void tall_finish_kernel(const float *part, int ncb, int64_t B, int root, float *pos)
+{
+    const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (b >= B) return;
+    float s = 0.0f;
+    for (int q = 0; q < ncb; ++q) s += part[q * B + b];
+    pos[b] = root ? sqrtf(s) : s;
+}
+
+
+// Whether a batch of `rows` rows in at most n_rel groups goes by these tiles rather than by 32-row tiles and streamed
+// small groups (transr_gemm_kernel).  Measured side by side over 64 to 1024 columns and 1 to 500 rows per group:
+//   up to 128 columns   one column block: the 64-row tile reads a projection half as often, 5 to 20 % of the call from
+//                       four rows per group on (16000 rows x 128, 500 groups: 47.5 -> 39.6 us); below, streaming wins
+//   up to 256           two column blocks stage every row twice: only where the 32-row tiles would leave compute units idle
+//   above               a 32-row tile is one workgroup however wide its rows are: few groups leave the chip idle
+//                       (512 x 300, 60 groups: 42 -> 28 us; 8192 x 1024, 51 groups: 355 -> 238 us); many groups of a few
+//                       rows are bound by reading the projections, which streaming does better
+static bool want_tall(int64_t d, int64_t rows, int64_t n_rel)
+{
+    const int64_t groups = rows < n_rel ? rows : n_rel, short_tiles = groups + rows / 32;
+    if (d <= 2 * kTallCols) return short_tiles <= 256 || (d <= kTallCols && rows >= 4 * n_rel);
+    return groups <= 256 || rows >= 16 * n_rel;
+}
+
+static int64_t tall_tiles(int64_t groups, int64_t rows) { return groups + rows / kTallRows + 1; }
+static size_t tall_part_floats(int64_t d, int64_t B) { return tall_col_blocks((int)d) > 1 ? (size_t)tall_col_blocks((int)d) * (size_t)B : 0; }
+
+// max_tiles: upper bound of the plan's tiles (a.plan holds tiles of kTallRows).  part: tall_part_floats() where a.pos is set.
+static int launch_tall(int mode, const GemmArgs &a, int64_t max_tiles, float *part, int64_t B, const FusedInsp &fi, hipStream_t st)
+{
+    const int ncb = tall_col_blocks(a.d);
+    if (a.pos && ncb > 1 && !part) return KGE_EWORKSPACE;
+    const TallArgs t{a, part, B};
+    const int64_t items = max_tiles * ncb;
+    const dim3 grid((unsigned)((items < kTallWgs ? items : kTallWgs) + fi.blocks)), block(256);
+    const size_t lds = fi.blocks > 0 && (size_t)fi.lds_bytes > kTallLds ? (size_t)fi.lds_bytes : kTallLds;
+    switch (mode) {
+    case 0: hipLaunchKernelGGL(transr_tall_kernel<0>, grid, block, lds, st, t, fi); break;
+    case 1: hipLaunchKernelGGL(transr_tall_kernel<1>, grid, block, lds, st, t, fi); break;
+    case 2: hipLaunchKernelGGL(transr_tall_kernel<2>, grid, block, lds, st, t, fi); break;
+    default: hipLaunchKernelGGL(transr_tall_kernel<3>, grid, block, lds, st, t, fi);
+    }
+    if (a.pos && ncb > 1)
+        hipLaunchKernelGGL(tall_finish_kernel, dim3((unsigned)ceil_div(B, 256)), dim3(256), 0, st, part, ncb, B,
+                           mode == 0 && a.norm_p == 2 ? 1 : 0, a.pos);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}

@@ -1,0 +1,51 @@
+"""TransR / RESCAL: the 64-row tiles of the grouped product and the rule between them and the 32-row tiles."""
+import numpy as np
+import pytest
+import torch
+
+from cuke_amd import synth
+from helpers import assert_close, gpu_model
+
+pytestmark = pytest.mark.gpu
+
+EDGES = (1, 4, 5, 15, 16, 17, 31, 33, 48, 49, 63, 64, 65, 129)  # rows of a group around one to four row blocks and one to three tiles
+
+
+@pytest.mark.parametrize("model", ["TransR", "RESCAL"])
+@pytest.mark.parametrize("dim,singles", [(4, 0), (36, 0), (124, 0), (128, 0), (132, 0), (260, 0), (388, 0), (512, 0), (1000, 0),
+                                         # (many groups of one row beside them: the 32-row tiles)
+                                         (4, 900), (36, 900), (132, 300), (260, 600)])
+def test_groups_at_the_edges_of_a_tile(oracle, model, dim, singles):
+    sizes = EDGES + (1,) * singles
+    w = synth.custom_workload(model, n_ent=300, n_rel=len(sizes) + 1, dim=dim, batch=sum(sizes), norm_p=2, sigma=0.2, seed=dim)
+    a = w.arrays
+    a["r"][:] = np.random.default_rng(dim).permutation(np.repeat(np.arange(len(sizes)), sizes))
+    m, ix = gpu_model(w)
+    from cuke_amd.kge import inspect
+    fw = m.score(ix["h"], ix["r"], ix["t"], rel_insp=inspect([ix["r"]], m.n_rel))
+    pos, _ = oracle.score(model, a["E"], a["R"], a["A"], a["h"], a["r"], a["t"], p=2)
+    assert_close(fw.pos.cpu().numpy(), pos, what="scores")
+    dpos = np.random.default_rng(1).standard_normal(w.batch).astype(np.float32)
+    g = m.backward(fw, torch.from_numpy(dpos).to(fw.pos.device))
+    ref = oracle.backward(model, a["E"], a["R"], a["A"], a["h"], a["r"], a["t"], dpos=dpos, p=2)
+    assert_close(g.ent_rows.cpu().numpy(), ref.ent_rows, what="entity rows", rows=True)
+    assert_close(g.aux_rows.cpu().numpy(), ref.aux_rows, what="projection gradients", rows=True)
+
+
+@pytest.mark.parametrize("n_rel,dim", [(3, 36), (3, 132), (3, 260), (60, 36), (200, 12)])
+@pytest.mark.parametrize("model", ["TransR", "RESCAL"])
+def test_shared_negatives_by_both_tiles(oracle, model, n_rel, dim):
+    w = synth.custom_workload(model, n_ent=400, n_rel=n_rel, dim=dim, batch=384, chunk=96, n_neg=21, norm_p=2, sigma=0.2, seed=n_rel)
+    a = w.arrays
+    m, ix = gpu_model(w)
+    fw = m.score(ix["h"], ix["r"], ix["t"], ix["neg"], 96)
+    kw = dict(p=2, neg=a["neg"], chunk=96)
+    pos, neg = oracle.score(model, a["E"], a["R"], a["A"], a["h"], a["r"], a["t"], **kw)
+    assert_close(fw.pos.cpu().numpy(), pos, what="scores")
+    assert_close(fw.neg.cpu().numpy(), neg, what="negatives' scores")
+    rng = np.random.default_rng(2)
+    dpos, dneg = rng.standard_normal(384).astype(np.float32), rng.standard_normal((384, 21)).astype(np.float32)
+    g = m.backward(fw, torch.from_numpy(dpos).cuda(), torch.from_numpy(dneg).cuda())
+    ref = oracle.backward(model, a["E"], a["R"], a["A"], a["h"], a["r"], a["t"], dpos=dpos, dneg=dneg, **kw)
+    assert_close(g.ent_rows.cpu().numpy(), ref.ent_rows, what="entity rows", rows=True)
+    assert_close(g.aux_rows.cpu().numpy(), ref.aux_rows, what="projection gradients", rows=True)

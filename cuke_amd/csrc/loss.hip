@@ -58,15 +58,17 @@ __global__ __launch_bounds__(256) void margin_total_kernel(const double *block_l
 {
     __shared__ double s[256];
     double acc = 0.0;
-    double v[kLossBlocks / 256];  // all loads of a thread in flight together
+    if (n > 0) {  // uniform; an empty batch has no partial, and may have no workspace, to read
+        double v[kLossBlocks / 256];  // all loads of a thread in flight together
 #pragma unroll
-    for (int q = 0; q < kLossBlocks / 256; ++q) {
-        const int i = threadIdx.x + 256 * q;
-        v[q] = block_loss[i < n ? i : 0];
-        if (i >= n) v[q] = 0.0;
+        for (int q = 0; q < kLossBlocks / 256; ++q) {
+            const int i = threadIdx.x + 256 * q;
+            v[q] = block_loss[i < n ? i : 0];
+            if (i >= n) v[q] = 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < kLossBlocks / 256; ++q) acc += v[q];
     }
-#pragma unroll
-    for (int q = 0; q < kLossBlocks / 256; ++q) acc += v[q];
     s[threadIdx.x] = acc;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {

@@ -23,6 +23,18 @@ def test_margin_loss(oracle, B, N, sign):
     assert np.array_equal(dneg.cpu().numpy(), rdn)
 
 
+def test_margin_loss_of_an_empty_batch_is_zero_without_a_workspace():
+    """kge_margin_loss_workspace answers 0 for an empty batch, so the call takes no workspace and reads none."""
+    import ctypes as C
+    from cuke_amd import _lib
+    L = _lib.lib()
+    assert L.kge_margin_loss_workspace(0, 16) == 0
+    loss = torch.full((1,), 7.0, device=DEV)
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert L.kge_margin_loss(None, None, 0, 16, 1.0, 1.0, C.c_void_p(loss.data_ptr()), None, None, None, 0, st) == 0
+    assert loss.item() == 0.0
+
+
 def test_build_index_matches_reference_restatement(oracle):
     from cuke_amd.kge import inspector
     rng = np.random.default_rng(5)

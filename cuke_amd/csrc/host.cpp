@@ -499,25 +499,26 @@ PyObject *py_margin_loss(PyObject *, PyObject *const *args, Py_ssize_t)
     END_HANDLE_TH_ERRORS
 }
 
-// sparse_step(table, state|None, inspection address, rows, lr, eps) -> True, or None; state None: SGD
+// sparse_step(table, state, inspection address, rows, lr, eps, adagrad) -> True, or None; SGD takes no state
 PyObject *py_sparse_step(PyObject *, PyObject *const *args, Py_ssize_t)
 {
     HANDLE_TH_ERRORS
     const int dev = c10::hip::current_device();
     const at::Tensor *table = tensor(args[0]), *state = tensor(args[1]), *rows = tensor(args[3]);
     if (!table || !is_f32(table, table->dim(), dev) || !is_f32(rows, 2, dev)) NOT_HERE;
-    if (args[1] != Py_None && !is_f32(state, 1, dev)) NOT_HERE;
+    const bool adagrad = PyObject_IsTrue(args[6]);
+    if (adagrad && !is_f32(state, 1, dev)) NOT_HERE;
     const auto *ins = static_cast<const kge_inspection *>(PyLong_AsVoidPtr(args[2]));
     const double lr = PyFloat_AsDouble(args[4]), eps = PyFloat_AsDouble(args[5]);
     if (PyErr_Occurred()) return nullptr;
     void *st = stream();
     const int rc = nogil([&] {
-        return state ? kge_sparse_adagrad(table->data_ptr<float>(), state->data_ptr<float>(), rows->size(1), ins->unique_ids, ins->num_unique,
-                                          rows->size(0), rows->data_ptr<float>(), (float)lr, (float)eps, st)
-                     : kge_sparse_sgd(table->data_ptr<float>(), rows->size(1), ins->unique_ids, ins->num_unique, rows->size(0),
-                                      rows->data_ptr<float>(), (float)lr, st);
+        return adagrad ? kge_sparse_adagrad(table->data_ptr<float>(), state->data_ptr<float>(), rows->size(1), ins->unique_ids, ins->num_unique,
+                                            rows->size(0), rows->data_ptr<float>(), (float)lr, (float)eps, st)
+                       : kge_sparse_sgd(table->data_ptr<float>(), rows->size(1), ins->unique_ids, ins->num_unique, rows->size(0),
+                                        rows->data_ptr<float>(), (float)lr, st);
     });
-    if (rc) return fail(rc, state ? "kge_sparse_adagrad" : "kge_sparse_sgd"), nullptr;
+    if (rc) return fail(rc, adagrad ? "kge_sparse_adagrad" : "kge_sparse_sgd"), nullptr;
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }

@@ -518,9 +518,16 @@ def _inplace_table(table):
     return t
 
 
+def _need_state(state):
+    if not isinstance(state, torch.Tensor):
+        raise TypeError(f"state must be a torch.Tensor (got {type(state).__name__})")
+    if not state.is_contiguous():
+        raise ValueError("state must be contiguous: it is updated in place")
+
+
 def sparse_sgd(table: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: float) -> None:
     """table[id] -= lr * rows[u] for the inspection's unique ids (in place, no host sync)."""
-    if _lib.host().sparse_step(table, None, _insp_address(insp), rows, lr, 0.0):
+    if _lib.host().sparse_step(table, None, _insp_address(insp), rows, lr, 0.0, False):
         return
     t = _inplace_table(table)
     _lib.check(_lib.lib().kge_sparse_sgd(_ptr(t), int(rows.shape[1]), _ptr(insp.unique_ids), _ptr(insp.num_unique_dev),
@@ -530,11 +537,10 @@ def sparse_sgd(table: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: fl
 def sparse_adagrad(table: torch.Tensor, state: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: float,
                    eps: float = 1e-10) -> None:
     """Row-wise Adagrad: state[id] += mean(g^2); table[id] -= lr * g / (sqrt(state[id]) + eps)."""
-    if _lib.host().sparse_step(table, state, _insp_address(insp), rows, lr, eps):
+    if _lib.host().sparse_step(table, state, _insp_address(insp), rows, lr, eps, True):
         return
     t = _inplace_table(table)
-    if not state.is_contiguous():
-        raise ValueError("state must be contiguous: it is updated in place")
+    _need_state(state)
     _lib.check(_lib.lib().kge_sparse_adagrad(_ptr(t), _ptr(state), int(rows.shape[1]), _ptr(insp.unique_ids),
                                              _ptr(insp.num_unique_dev), int(rows.shape[0]), _ptr(rows), float(lr),
                                              float(eps), _stream()), "kge_sparse_adagrad")

@@ -89,3 +89,13 @@ def test_optimizer_rows_of_thousands_of_floats(oracle, dim, opt):
         wt, ws = oracle.sparse_adagrad(table, state, u, rows[:len(u)], 0.1)
         assert_close(t.cpu().numpy(), wt, what="table")
         assert_close(s.cpu().numpy(), ws, what="state")
+
+
+def test_adagrad_without_a_state_raises_and_updates_nothing():
+    """(it is not SGD)"""
+    from cuke_amd.kge import inspect, sparse_adagrad
+    table, rows = torch.ones(5, 8, device="cuda"), torch.ones(2, 8, device="cuda")
+    insp = inspect(torch.tensor([3, 1], device="cuda"), 5)
+    with pytest.raises(TypeError):
+        sparse_adagrad(table, None, insp, rows, 0.1)
+    assert torch.equal(table, torch.ones_like(table))

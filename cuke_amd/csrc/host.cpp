@@ -509,6 +509,7 @@ PyObject *py_sparse_step(PyObject *, PyObject *const *args, Py_ssize_t)
     const bool adagrad = PyObject_IsTrue(args[6]);
     if (adagrad && !is_f32(state, 1, dev)) NOT_HERE;
     const auto *ins = static_cast<const kge_inspection *>(PyLong_AsVoidPtr(args[2]));
+    if (!ins) NOT_HERE;  // (no inspection was given)
     const double lr = PyFloat_AsDouble(args[4]), eps = PyFloat_AsDouble(args[5]);
     if (PyErr_Occurred()) return nullptr;
     void *st = stream();

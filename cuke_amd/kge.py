@@ -518,6 +518,11 @@ def _inplace_table(table):
     return t
 
 
+def _need_inspection(insp):
+    if insp is None:
+        raise TypeError("insp is None: KGEModel.backward() fills in Forward.ent_insp / rel_insp")
+
+
 def _need_state(state):
     if not isinstance(state, torch.Tensor):
         raise TypeError(f"state must be a torch.Tensor (got {type(state).__name__})")
@@ -529,6 +534,7 @@ def sparse_sgd(table: torch.Tensor, insp: Inspection, rows: torch.Tensor, lr: fl
     """table[id] -= lr * rows[u] for the inspection's unique ids (in place, no host sync)."""
     if _lib.host().sparse_step(table, None, _insp_address(insp), rows, lr, 0.0, False):
         return
+    _need_inspection(insp)
     t = _inplace_table(table)
     _lib.check(_lib.lib().kge_sparse_sgd(_ptr(t), int(rows.shape[1]), _ptr(insp.unique_ids), _ptr(insp.num_unique_dev),
                                          int(rows.shape[0]), _ptr(rows), float(lr), _stream()), "kge_sparse_sgd")
@@ -539,6 +545,7 @@ def sparse_adagrad(table: torch.Tensor, state: torch.Tensor, insp: Inspection, r
     """Row-wise Adagrad: state[id] += mean(g^2); table[id] -= lr * g / (sqrt(state[id]) + eps)."""
     if _lib.host().sparse_step(table, state, _insp_address(insp), rows, lr, eps, True):
         return
+    _need_inspection(insp)
     t = _inplace_table(table)
     _need_state(state)
     _lib.check(_lib.lib().kge_sparse_adagrad(_ptr(t), _ptr(state), int(rows.shape[1]), _ptr(insp.unique_ids),

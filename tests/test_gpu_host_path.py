@@ -99,3 +99,14 @@ def test_adagrad_without_a_state_raises_and_updates_nothing():
     with pytest.raises(TypeError):
         sparse_adagrad(table, None, insp, rows, 0.1)
     assert torch.equal(table, torch.ones_like(table))
+
+
+def test_optimizer_steps_without_an_inspection_raise_and_update_nothing():
+    """Forward.ent_insp / rel_insp are None until backward() has run: an easy mistake that must not end the process."""
+    from cuke_amd.kge import sparse_adagrad, sparse_sgd
+    table, rows, state = torch.ones(5, 8, device="cuda"), torch.ones(2, 8, device="cuda"), torch.zeros(5, device="cuda")
+    with pytest.raises(TypeError):
+        sparse_adagrad(table, state, None, rows, 0.1)
+    with pytest.raises(TypeError):
+        sparse_sgd(table, None, rows, 0.1)
+    assert torch.equal(table, torch.ones_like(table)) and not state.any()

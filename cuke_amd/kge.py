@@ -123,14 +123,16 @@ class _PackedInspection(Inspection):
         self.n, self.n_rows = self._c.n, self._c.n_rows
         self.unique_ids, self._block, self._u = ids, block, None
 
+    _PARTS = ("num_unique_dev", "seg_offsets", "perm", "inverse", "sorted_seg")
+
     def __getattr__(self, name):  # (only what is not there yet)
+        if name not in self._PARTS:  # (first: an object that is being copied or restored has no fields yet)
+            raise AttributeError(name)
         n, i4 = self.n, _up256(4 * max(self.n, 1))
         after_seg = 256 + _up256(4 * (n + 1))
-        at = {"num_unique_dev": (0, 1), "seg_offsets": (256, n + 1), "perm": (after_seg, max(n, 1)),
-              "inverse": (after_seg + i4, max(n, 1)), "sorted_seg": (after_seg + 2 * i4, max(n, 1))}.get(name)
-        if at is None:
-            raise AttributeError(name)
-        view = self._block[at[0]:at[0] + 4 * at[1]].view(torch.int32)
+        at, count = {"num_unique_dev": (0, 1), "seg_offsets": (256, n + 1), "perm": (after_seg, max(n, 1)),
+                     "inverse": (after_seg + i4, max(n, 1)), "sorted_seg": (after_seg + 2 * i4, max(n, 1))}[name]
+        view = self._block[at:at + 4 * count].view(torch.int32)
         setattr(self, name, view)
         return view
 

@@ -38,6 +38,12 @@ extern "C" int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const 
     const size_t fws_bytes = cur->fwd_workspace ? cur->fwd_workspace_bytes : buf->fwd_workspace_bytes;
     bat->plans_ready = 0, bat->insp_ready = nullptr, bat->fuse_inspection = 0;
     int rc;
+    if (!fused && (!side_stream || !cur->inspected || !cur->planned)) return KGE_EINVAL;
+    hipStream_t st = as_stream(stream), side = as_stream(side_stream);
+    // The fork stands in front of everything this step enqueues: taken behind the relation inspection it would make the
+    // entity inspection wait for that, of which it needs nothing.
+    if (!fused && (hipEventRecord(as_event(cur->planned), st) != hipSuccess || hipStreamWaitEvent(side, as_event(cur->planned), 0) != hipSuccess))
+        return KGE_ELAUNCH;
     if (projection && (rc = kge_inspect_batch(&jobs[1], 1, stream))) return rc;  // the forward pass is planned from the relation groups
     if (fused) {
         bat->fuse_inspection = 1;
@@ -45,10 +51,6 @@ extern "C" int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const 
         bat->fuse_inspection = 0;
         return rc;
     }
-    if (!side_stream || !cur->inspected || !cur->planned) return KGE_EINVAL;
-    hipStream_t st = as_stream(stream), side = as_stream(side_stream);
-    if (hipEventRecord(as_event(cur->planned), st) != hipSuccess || hipStreamWaitEvent(side, as_event(cur->planned), 0) != hipSuccess)
-        return KGE_ELAUNCH;
     if ((rc = kge_inspect_batch(jobs, projection ? 1 : 2, side_stream))) return rc;
     if (hipEventRecord(as_event(cur->inspected), side) != hipSuccess) return KGE_ELAUNCH;
     bat->insp_ready = cur->inspected;  // backward waits for it right before its segmented reduction

@@ -110,3 +110,37 @@ def test_optimizer_steps_without_an_inspection_raise_and_update_nothing():
     with pytest.raises(TypeError):
         sparse_sgd(table, None, rows, 0.1)
     assert torch.equal(table, torch.ones_like(table)) and not state.any()
+
+
+def _hip():
+    """The HIP runtime this process runs on (torch may carry its own copy: never load a second one)."""
+    import ctypes
+    for line in open("/proc/self/maps"):
+        path = line.split()[-1]
+        if "libamdhip64" in path:
+            return ctypes.CDLL(path)
+    raise AssertionError("no HIP runtime in the process")
+
+
+def test_one_call_step_inspects_the_entities_beside_the_relations():
+    """fused == 0, TransR: the entity inspection depends on what came before the step, not on the relation inspection
+    in front of the forward pass.  Captured, the step then starts with two nodes that wait for nothing."""
+    import ctypes as C
+    from cuke_amd.kge import TrainStep
+    w = synth.custom_workload("TransR", n_ent=400, n_rel=12, dim=48, batch=256, chunk=32, n_neg=8, sigma=0.2, seed=20)
+    m, ix = gpu_model(w)
+    st = TrainStep(m, ix["h"], ix["r"], ix["t"], ix["neg"], 32)
+
+    def step():
+        batches, buf = st._native_state()
+        assert st.L.kge_train_step(C.byref(m._tab), C.byref(batches[0]), C.byref(buf), 0,
+                                   C.c_void_p(torch.cuda.current_stream().cuda_stream), C.c_void_p(st.side.cuda_stream)) == 0
+
+    step()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g):
+        step()
+    n = C.c_size_t(0)
+    assert _hip().hipGraphGetRootNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
+    assert n.value == 2

@@ -692,6 +692,7 @@ class TrainStep:
         self._pipelined = False   # the ring of run(pipeline=True) has been set up
         self._timeline = None     # set by kernel_times()
         self._native = None       # structures of the one-call steps, see _native_state()
+        self._form = None         # how the last step was issued, see _order()
         self.side = torch.cuda.Stream(device=dev)  # default priority
         self._dev_index = dev.index if dev.index is not None else torch.cuda.current_device()
         self.pos = torch.empty(B, **f32)
@@ -800,6 +801,7 @@ class TrainStep:
         if int(h.numel()) != self.B or N != self.N or (neg is None) != (self.neg is None):
             raise ValueError("every batch of a TrainStep has the shape of the first one")
         self._sets.append(self._make_set((h, r, t, neg)))
+        self._form = None  # (its index tensors, too, were made on the main stream)
         return len(self._sets) - 1
 
     def select(self, i: int) -> None:
@@ -955,6 +957,7 @@ class TrainStep:
                 raise KgeError(f"batch {batch} does not exist or is already staged")
         if len(self._staged) >= max(len(sets) - 1, 1):
             raise KgeError(f"at most {max(len(sets) - 1, 1)} batches can be staged ahead of run()")
+        self._order("staged")
         s, side = sets[at], self.side
         if s.done_event is not None:
             side.wait_event(s.done_event)  # its inspection may still be read by an earlier step
@@ -1008,6 +1011,8 @@ class TrainStep:
         capturable into one graph: the dependencies cross steps."""
         main = _current_stream(self._dev_index)
         st = C.c_void_p(main.cuda_stream)
+        if backward or self.needs_rel_groups:  # (a plain forward pass touches no inspection)
+            self._order("staged" if pipeline else "run")
         for s_ in self._sets:  # cached unique counts belong to the batches of earlier steps
             s_.ent_insp._u = s_.rel_insp._u = None
         if backward and overlap and not pipeline and not self._staged and self._timeline is None and self.bat.timeline is None and \
@@ -1110,6 +1115,7 @@ class TrainStep:
         return g
 
     def replay(self):
+        self._order("run")
         self.graph.replay()
 
     def capture_staged(self, cur: int, nxt: int, backward=True):
@@ -1141,6 +1147,7 @@ class TrainStep:
     def prime_staged(self, i: int) -> None:
         """Inspect (and, for TransR / RESCAL, plan) batch ``i`` on the current stream: what the side branch of
         the graph before would have done."""
+        self._order("graph")
         self._inspect_ahead(self._sets[i], C.c_void_p(torch.cuda.current_stream().cuda_stream))
 
     def _inspect_ahead(self, s, sst) -> None:
@@ -1174,20 +1181,11 @@ class TrainStep:
         main.wait_stream(side)                                   # join
 
     # ---- the staged issue from native code: one library call per step ----
-    def _native_key(self):
-        """What the cached structures were built from and a caller can change: the batches and the upstream gradients."""
-        return (len(self._sets), None if self.dpos is None else self.dpos.data_ptr(), None if self.dneg is None else self.dneg.data_ptr())
-
     def _native_ready(self) -> bool:
         """The structures exist, or may be built now (events cannot be created in the middle of a graph capture)."""
-        return self._native is not None and self._native_for == self._native_key() or not torch.cuda.is_current_stream_capturing()
+        return self._native is not None and len(self._native[0]) == len(self._sets) or not torch.cuda.is_current_stream_capturing()
 
-    def _native_state(self):
-        """kge_step_batch per batch (events created once) and the kge_step_buffers of this TrainStep."""
-        key = self._native_key()
-        if self._native is not None and self._native_for == key:
-            return self._native
-        self._native_for = key
+    def _native_batch(self, s_):
         main = torch.cuda.current_stream()
 
         def event():
@@ -1195,34 +1193,50 @@ class TrainStep:
             ev.record(main)       # (torch creates the underlying event at its first record)
             return ev
 
-        batches = []
-        for s_ in self._sets:
-            sb = _lib.StepBatch()
-            sb.bat = s_.bat
-            sb.bat.insp_ready, sb.bat.fuse_inspection, sb.bat.plans_ready, sb.bat.timeline = None, 0, 0, None
-            sb.bat.back_rows = self.back_rows.data_ptr() if self.back_rows is not None else None
-            if self._plans_per_set:
-                if getattr(s_, "ws_f", None) is None:
-                    s_.ws_f = torch.empty(max(self._ws_f_bytes, 1), dtype=torch.uint8, device=self.m.dev)
-                sb.fwd_workspace, sb.fwd_workspace_bytes = s_.ws_f.data_ptr(), self._ws_f_bytes
-            if getattr(s_, "native_events", None) is None:
-                s_.native_events = [event() for _ in range(3)]
-            sb.inspected, sb.planned, sb.released = (e.cuda_event for e in s_.native_events)
-            sb.released_valid = 0
-            batches.append(sb)
-        buf = _lib.StepBuffers()
+        sb = _lib.StepBatch()
+        sb.bat = s_.bat
+        sb.bat.insp_ready, sb.bat.fuse_inspection, sb.bat.plans_ready, sb.bat.timeline = None, 0, 0, None
+        sb.bat.back_rows = self.back_rows.data_ptr() if self.back_rows is not None else None
+        if self._plans_per_set:
+            if getattr(s_, "ws_f", None) is None:
+                s_.ws_f = torch.empty(max(self._ws_f_bytes, 1), dtype=torch.uint8, device=self.m.dev)
+            sb.fwd_workspace, sb.fwd_workspace_bytes = s_.ws_f.data_ptr(), self._ws_f_bytes
+        s_.native_events = [event() for _ in range(3)]
+        sb.inspected, sb.planned, sb.released = (e.cuda_event for e in s_.native_events)
+        sb.released_valid = 0
+        return sb
+
+    def _native_state(self):
+        """kge_step_batch per batch, made once (they say which staged inspections and plans are under way), and the
+        kge_step_buffers of this TrainStep, whose pointers are read anew for every step: a loop may bind fresh
+        upstream gradients to ``dpos`` / ``dneg`` each time."""
+        if self._native is None:
+            buf = _lib.StepBuffers()
+            buf.fwd_workspace, buf.fwd_workspace_bytes = self._ws_f.data_ptr(), self._ws_f_bytes
+            buf.bwd_workspace, buf.bwd_workspace_bytes = self._ws_b.data_ptr(), self._ws_b_bytes
+            self._native = ([], buf)
+        batches, buf = self._native
+        for s_ in self._sets[len(batches):]:
+            batches.append(self._native_batch(s_))
         for name in ("pos", "neg", "side_pos", "side_neg", "residual", "dpos", "dneg"):
             t = getattr(self, name)
             setattr(buf, name, t.data_ptr() if t is not None else None)
-        buf.fwd_workspace, buf.fwd_workspace_bytes = self._ws_f.data_ptr(), self._ws_f_bytes
+        buf.loss = None
         if self.loss_kind == "margin":
             buf.loss, buf.margin, buf.sign = self.loss.data_ptr(), self.margin, self.sign
             buf.loss_workspace, buf.loss_workspace_bytes = self._ws_l.data_ptr(), self._ws_l.numel()
         buf.grads = self.grads
-        buf.bwd_workspace, buf.bwd_workspace_bytes = self._ws_b.data_ptr(), self._ws_b_bytes
-        torch.cuda.synchronize()
-        self._native = (batches, buf)
         return self._native
+
+    def _order(self, form: str) -> None:
+        """A step can be issued by run(), by stage() + run(pipeline=True) or by run_native().  Each form orders the work that
+        it puts on the main and on the side stream; going over from one to another (and in front of the first step, whose
+        index tensors were made on the main stream) the two wait for each other once."""
+        if form != self._form and not torch.cuda.is_current_stream_capturing():
+            main = torch.cuda.current_stream()
+            main.wait_stream(self.side)
+            self.side.wait_stream(main)
+            self._form = form
 
     def run_native(self, cur, nxt) -> None:
         """The staged issue in ONE library call (kge_train_step_staged): the step of batch ``cur`` on the current
@@ -1232,6 +1246,7 @@ class TrainStep:
         the same results bit for bit; what it saves is the host's time per step."""
         if self._staged or self._pipelined:
             raise KgeError("run_native() cannot be mixed with the staged pipeline")
+        self._order("native")
         batches, buf = self._native_state()
         st = C.c_void_p(_current_stream(self._dev_index).cuda_stream)
         _lib.check(self.L.kge_train_step_staged(C.byref(self.m._tab), C.byref(batches[cur]) if cur is not None else None,

@@ -144,3 +144,94 @@ def test_one_call_step_inspects_the_entities_beside_the_relations():
     n = C.c_size_t(0)
     assert _hip().hipGraphGetRootNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
     assert n.value == 2
+
+
+def _two_batches(model, **kw):
+    from cuke_amd.kge import TrainStep
+    w = synth.custom_workload(model, n_ent=300, n_rel=9, dim=24, batch=128, sigma=0.3, seed=4, **kw)
+    m, ix = gpu_model(w)
+    b0 = [ix["h"], ix["r"], ix["t"], ix.get("neg")]
+    b1 = [ix["t"].flip(0), ix["r"].flip(0), ix["h"].flip(0), ix["neg"].flip(0) if "neg" in ix else None]
+    return m, (b0, b1), lambda b: TrainStep(m, *b, w.chunk or None)
+
+
+def _step_outputs(st):
+    torch.cuda.synchronize()
+    g = st.sparse_grads()
+    return [x.clone() for x in (st.pos, st.neg, g.ent_ids, g.rel_ids, g.ent_rows, g.rel_rows, g.aux_rows) if x is not None]
+
+
+@pytest.mark.parametrize("model,kw", [("DistMult", dict(chunk=32, n_neg=8)), ("TransR", dict())])
+def test_fresh_upstream_gradients_and_a_new_batch_between_staged_steps(model, kw, monkeypatch):
+    """dpos bound anew for every step, and a batch added when another is staged: the steps follow them, what has been
+    staged stays staged, and nothing waits for the device."""
+    from helpers import assert_close
+    m, batches, make = _two_batches(model, **kw)
+    order, ups = [0, 1, 0, 1], [torch.randn(128, device="cuda") for _ in range(4)]
+    want = []
+    for b, up in zip(order, ups):
+        ref = make(batches[b])
+        ref.dpos = up
+        ref.run()
+        want.append(_step_outputs(ref))
+    st = make(batches[0])
+    sync, waits = torch.cuda.synchronize, []
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: waits.append(1))
+    st.run_native(None, 0)
+    assert st.add_batch(*batches[1]) == 1
+    got = []
+    for k, b in enumerate(order):
+        st.dpos = ups[k].clone()
+        st.run_native(b, order[k + 1] if k + 1 < len(order) else None)
+        assert not waits
+        sync()
+        got.append(_step_outputs(st))
+        waits.clear()
+    for k in range(len(order)):
+        for x, y in zip(got[k], want[k]):
+            assert_close(x.cpu().numpy(), y.cpu().numpy(), what=f"step {k}", rows=x.dim() > 1)
+
+
+@pytest.mark.parametrize("model,kw", [("DistMult", dict(chunk=32, n_neg=8)), ("TransR", dict())])
+def test_forms_of_issue_follow_each_other(model, kw):
+    """A step of one form, then new ids in the same tensors, then a step of another: the second waits for the first on
+    both streams, however far the host is ahead."""
+    m, batches, make = _two_batches(model, **kw)
+    busy = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
+
+    def load(tensors, b):
+        for x, y in zip(tensors, batches[b]):
+            if x is not None:
+                x.copy_(y)
+
+    def native(st):
+        st.run_native(None, 0), st.run_native(0, None)
+
+    def staged(st):
+        st.stage(batch=0), st.run(pipeline=True)
+
+    forms = [lambda st: st.run(), native, staged]
+    want = []
+    for b in (0, 1):
+        st = make(batches[b])
+        st.run()
+        want.append(_step_outputs(st))
+    at = 1 if batches[0][3] is None else 2  # of the entity ids among the outputs
+    n0 = want[0][at].numel()
+    for first in forms:
+        for second in forms:
+            if first is second:
+                continue
+            mine = [x.clone() if x is not None else None for x in batches[0]]
+            st = make(mine)
+            for _ in range(20):  # (milliseconds of work in front of the steps)
+                busy.zero_()
+            first(st)
+            pos, ids, rows = st.pos.clone(), st.ent_insp.unique_ids.clone(), st.ent_rows.clone()
+            load(mine, 1)
+            second(st)
+            got = _step_outputs(st)
+            assert torch.equal(pos, want[0][0]) and torch.equal(ids[:n0], want[0][at])
+            assert torch.allclose(rows[:n0], want[0][at + 2], rtol=1e-4, atol=1e-6)
+            assert torch.equal(got[0], want[1][0]) and torch.equal(got[at], want[1][at]) and torch.equal(got[at + 1], want[1][at + 1])
+            assert torch.allclose(got[at + 2], want[1][at + 2], rtol=1e-4, atol=1e-6)

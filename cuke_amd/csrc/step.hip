@@ -32,11 +32,9 @@ extern "C" int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const 
 {
     if (!tab || !cur || !buf || !cur->bat.insp_jobs) return KGE_EINVAL;
     const bool projection = tab->model == KGE_TRANSR || tab->model == KGE_RESCAL;
-    kge_batch *bat = &cur->bat;
-    const kge_inspect_job *jobs = bat->insp_jobs;
+    const kge_inspect_job *jobs = cur->bat.insp_jobs;
     void *fws = cur->fwd_workspace ? cur->fwd_workspace : buf->fwd_workspace;
     const size_t fws_bytes = cur->fwd_workspace ? cur->fwd_workspace_bytes : buf->fwd_workspace_bytes;
-    bat->plans_ready = 0, bat->insp_ready = nullptr, bat->fuse_inspection = 0;
     int rc;
     if (!fused && (!side_stream || !cur->inspected || !cur->planned)) return KGE_EINVAL;
     hipStream_t st = as_stream(stream), side = as_stream(side_stream);
@@ -45,18 +43,15 @@ extern "C" int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const 
     if (!fused && (hipEventRecord(as_event(cur->planned), st) != hipSuccess || hipStreamWaitEvent(side, as_event(cur->planned), 0) != hipSuccess))
         return KGE_ELAUNCH;
     if (projection && (rc = kge_inspect_batch(&jobs[1], 1, stream))) return rc;  // the forward pass is planned from the relation groups
-    if (fused) {
-        bat->fuse_inspection = 1;
-        rc = step_body(tab, bat, buf, fws, fws_bytes, stream);
-        bat->fuse_inspection = 0;
-        return rc;
+    // (a copy: that this batch was staged, kge_batch.plans_ready, is remembered for the step that uses it)
+    kge_batch own = cur->bat;
+    own.plans_ready = 0, own.insp_ready = nullptr, own.fuse_inspection = fused ? 1 : 0;
+    if (!fused) {
+        if ((rc = kge_inspect_batch(jobs, projection ? 1 : 2, side_stream))) return rc;
+        if (hipEventRecord(as_event(cur->inspected), side) != hipSuccess) return KGE_ELAUNCH;
+        own.insp_ready = cur->inspected;  // backward waits for it right before its segmented reduction
     }
-    if ((rc = kge_inspect_batch(jobs, projection ? 1 : 2, side_stream))) return rc;
-    if (hipEventRecord(as_event(cur->inspected), side) != hipSuccess) return KGE_ELAUNCH;
-    bat->insp_ready = cur->inspected;  // backward waits for it right before its segmented reduction
-    rc = step_body(tab, bat, buf, fws, fws_bytes, stream);
-    bat->insp_ready = nullptr;
-    return rc;
+    return step_body(tab, &own, buf, fws, fws_bytes, stream);
 }
 
 extern "C" int kge_train_step_staged(const kge_tables *tab, kge_step_batch *cur, kge_step_batch *next, const kge_step_buffers *buf,

@@ -122,6 +122,13 @@ def _hip():
     raise AssertionError("no HIP runtime in the process")
 
 
+def _one_call_step(st, fused):
+    import ctypes as C
+    batches, buf = st._native_state()
+    assert st.L.kge_train_step(C.byref(st.m._tab), C.byref(batches[0]), C.byref(buf), fused,
+                               C.c_void_p(torch.cuda.current_stream().cuda_stream), C.c_void_p(st.side.cuda_stream)) == 0
+
+
 def test_one_call_step_inspects_the_entities_beside_the_relations():
     """fused == 0, TransR: the entity inspection depends on what came before the step, not on the relation inspection
     in front of the forward pass.  Captured, the step then starts with two nodes that wait for nothing."""
@@ -131,16 +138,11 @@ def test_one_call_step_inspects_the_entities_beside_the_relations():
     m, ix = gpu_model(w)
     st = TrainStep(m, ix["h"], ix["r"], ix["t"], ix["neg"], 32)
 
-    def step():
-        batches, buf = st._native_state()
-        assert st.L.kge_train_step(C.byref(m._tab), C.byref(batches[0]), C.byref(buf), 0,
-                                   C.c_void_p(torch.cuda.current_stream().cuda_stream), C.c_void_p(st.side.cuda_stream)) == 0
-
-    step()
+    _one_call_step(st, fused=0)
     torch.cuda.synchronize()
     g = torch.cuda.CUDAGraph(keep_graph=True)
     with torch.cuda.graph(g):
-        step()
+        _one_call_step(st, fused=0)
     n = C.c_size_t(0)
     assert _hip().hipGraphGetRootNodes(C.c_void_p(g.raw_cuda_graph()), None, C.byref(n)) == 0
     assert n.value == 2
@@ -235,3 +237,17 @@ def test_forms_of_issue_follow_each_other(model, kw):
             assert torch.allclose(rows[:n0], want[0][at + 2], rtol=1e-4, atol=1e-6)
             assert torch.equal(got[0], want[1][0]) and torch.equal(got[at], want[1][at]) and torch.equal(got[at + 1], want[1][at + 1])
             assert torch.allclose(got[at + 2], want[1][at + 2], rtol=1e-4, atol=1e-6)
+
+
+@pytest.mark.parametrize("fused", [0, 1])
+def test_one_call_step_leaves_a_staged_batch_staged(fused):
+    """TransR without negatives: staging plans the batch; a step that plans for itself in between does not undo that."""
+    m, batches, make = _two_batches("TransR")
+    st = make(batches[0])
+    assert st.fusable
+    st.run_native(None, 0)
+    torch.cuda.synchronize()
+    _one_call_step(st, fused)
+    one = _step_outputs(st)
+    st.run_native(0, None)
+    assert all(torch.equal(x, y) for x, y in zip(one, _step_outputs(st)))

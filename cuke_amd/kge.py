@@ -801,7 +801,8 @@ class TrainStep:
         if int(h.numel()) != self.B or N != self.N or (neg is None) != (self.neg is None):
             raise ValueError("every batch of a TrainStep has the shape of the first one")
         self._sets.append(self._make_set((h, r, t, neg)))
-        self._form = None  # (its index tensors, too, were made on the main stream)
+        if self._form in ("staged", "native"):
+            self.side.wait_stream(torch.cuda.current_stream())  # (its index tensors were made on this one)
         return len(self._sets) - 1
 
     def select(self, i: int) -> None:
@@ -1226,17 +1227,21 @@ class TrainStep:
             buf.loss, buf.margin, buf.sign = self.loss.data_ptr(), self.margin, self.sign
             buf.loss_workspace, buf.loss_workspace_bytes = self._ws_l.data_ptr(), self._ws_l.numel()
         buf.grads = self.grads
-        return self._native
+        return batches, buf
 
     def _order(self, form: str) -> None:
         """A step can be issued by run(), by stage() + run(pipeline=True) or by run_native().  Each form orders the work that
-        it puts on the main and on the side stream; going over from one to another (and in front of the first step, whose
-        index tensors were made on the main stream) the two wait for each other once."""
-        if form != self._form and not torch.cuda.is_current_stream_capturing():
-            main = torch.cuda.current_stream()
-            main.wait_stream(self.side)
+        it puts on the main and on the side stream; going over from one to another, the stream that goes first waits for
+        the other once: the side stream, which inspects ahead in the staged forms, for the steps before (in front
+        of the first step: for the index tensors), the main stream for what has been inspected ahead."""
+        if form == self._form or torch.cuda.is_current_stream_capturing():
+            return
+        last, self._form = self._form, form
+        main = torch.cuda.current_stream()
+        if form in ("staged", "native"):
             self.side.wait_stream(main)
-            self._form = form
+        elif last in ("staged", "native"):
+            main.wait_stream(self.side)
 
     def run_native(self, cur, nxt) -> None:
         """The staged issue in ONE library call (kge_train_step_staged): the step of batch ``cur`` on the current

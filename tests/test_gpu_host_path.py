@@ -251,3 +251,38 @@ def test_one_call_step_leaves_a_staged_batch_staged(fused):
     one = _step_outputs(st)
     st.run_native(0, None)
     assert all(torch.equal(x, y) for x, y in zip(one, _step_outputs(st)))
+
+
+@pytest.mark.parametrize("fused", [0, 1])
+@pytest.mark.parametrize("model,kw", [("DistMult", dict(chunk=32, n_neg=8)), ("RotatE", dict(chunk=64, n_neg=8)), ("TransH", dict(chunk=32, n_neg=8)),
+                                      ("TransR", dict()), ("TransR", dict(chunk=32, n_neg=8)), ("RESCAL", dict(chunk=32, n_neg=8))])
+def test_one_call_step_gives_the_results_of_run(model, kw, fused):
+    m, batches, make = _two_batches(model, **kw)
+    st, ref = make(batches[0]), make(batches[0])
+    ref.run(fused=bool(fused) and ref.fusable)
+    want = _step_outputs(ref)
+    for _ in range(2):
+        for x in (st.pos, st.ent_rows):
+            x.fill_(7.0)
+        _one_call_step(st, fused and st.fusable)
+        assert all(torch.equal(x, y) for x, y in zip(_step_outputs(st), want))
+
+
+def test_a_replaced_stage_is_called():
+    """A loss of one's own, as a subclass or on the object."""
+    from cuke_amd.kge import TrainStep
+    m, batches, make = _two_batches("DistMult", chunk=32, n_neg=8)
+
+    class Own(TrainStep):
+        def loss_grad(self, st):
+            self.dpos = 2.0 * self.pos
+
+    a, b = Own(m, *batches[0], 32), make(batches[0])
+    b.loss_grad = lambda st: setattr(b, "dpos", 2.0 * b.pos)
+    ref = make(batches[0])
+    ref.run()
+    ref.dpos = 2.0 * ref.pos.clone()
+    ref.run()
+    for st in (a, b):
+        st.run()
+        assert all(torch.equal(x, y) for x, y in zip(_step_outputs(st), _step_outputs(ref)))

@@ -370,10 +370,10 @@ int kge_widen_ids(const int32_t *const *src, int64_t *const *dst, const int64_t 
     return KGE_OK;
 }
 
-int kge_publish_counts(const int32_t *first, const int32_t *second, uint64_t *host_word, void *stream)
+int kge_publish_counts(const int32_t *first, const int32_t *second, uint64_t *word, void *stream)
 {
-    if (!first || !second || !host_word) return KGE_EINVAL;
-    hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(1), 0, as_stream(stream), first, second, host_word);
+    if (!first || !second || !word) return KGE_EINVAL;
+    hipLaunchKernelGGL(publish_counts_kernel, dim3(1), dim3(1), 0, as_stream(stream), first, second, word);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

@@ -211,27 +211,43 @@ class SparseGrads:
 
 
 class _StepGrads(SparseGrads):
-    """The gradients of a TrainStep's last run.  How many rows are valid is read from the device when one of the views is
-    first asked for: the factored optimizer steps take the count from the device and need no view, so a training loop
-    that goes on to them does not wait for the step in between (8192 triples of TransR, width 200: about 50 us)."""
+    """The gradients of a TrainStep's last run.  How many rows are valid is written down on the device when the object is
+    made, and read when one of the views is first asked for: the factored optimizer steps take the count from the
+    device and need no view, so a training loop that goes on to them does not wait for the step in between (8192 triples
+    of TransR, width 200: about 50 us).  Every view has the count of its own step, whenever it is asked for; the rows
+    behind it are the TrainStep's buffers, which the next run overwrites."""
 
     def __init__(self, step):
-        self._ent_insp, self._rel_insp, self._c = step.ent_insp, step.rel_insp, step.grads
+        ei, ri = self._ent_insp, self._rel_insp = step.ent_insp, step.rel_insp
+        self._c = step.grads
         self._rows = {"ent_rows": step.ent_rows, "rel_rows": step.rel_rows, "aux_rows": step.aux_rows}
         self.aux_x, self.aux_q, self.factor_max = step.aux_x, step.aux_q, step.factor_max
+        self._counts, self._word = None, None
+        if ei._u is not None and ri._u is not None:
+            self._counts = ei._u, ri._u
+        else:
+            self._word = torch.empty(1, dtype=torch.int64, device=step.m.dev)
+            _lib.check(step.L.kge_publish_counts(_ptr(ei.num_unique_dev), _ptr(ri.num_unique_dev), _ptr(self._word), _stream()),
+                       "kge_publish_counts")
+
+    def _count(self, which: int) -> int:
+        if self._counts is None:
+            word = int(self._word.item())
+            self._counts = word & 0xffffffff, word >> 32
+        return self._counts[which]
 
     def __getattr__(self, name):  # (only what is not there yet)
         if name not in ("ent_ids", "ent_rows", "rel_ids", "rel_rows", "aux_rows"):
             raise AttributeError(name)
-        insp = self._ent_insp if name.startswith("ent") else self._rel_insp
-        all_rows = insp.unique_ids if name.endswith("ids") else self._rows[name]
-        view = all_rows[:insp.num_unique] if all_rows is not None else None
+        ent = name.startswith("ent")
+        all_rows = (self._ent_insp if ent else self._rel_insp).unique_ids if name.endswith("ids") else self._rows[name]
+        view = all_rows[:self._count(0 if ent else 1)] if all_rows is not None else None
         setattr(self, name, view)
         return view
 
     @property
     def rel_seg_offsets(self):
-        return self._rel_insp.offsets() if self.factor_max else None
+        return self._rel_insp.seg_offsets[:self._count(1) + 1] if self.factor_max else None
 
 
 class KGEModel:

@@ -444,9 +444,10 @@ int kge_sample_batch(const int64_t *col_h, const int64_t *col_r, const int64_t *
    (src / dst / len: host arrays of n_parts device pointers / lengths). */
 int kge_widen_ids(const int32_t *const *src, int64_t *const *dst, const int64_t *len, int n_parts, void *stream);
 
-/* Writes two device counts (kge_inspection.num_unique) to one 64-bit word of pinned host memory, first in the low
-   half: lets the host wait for an inspection without waiting for what was enqueued behind it. */
-int kge_publish_counts(const int32_t *first, const int32_t *second, uint64_t *host_word, void *stream);
+/* Writes two device counts (kge_inspection.num_unique) to one 64-bit word, first in the low half.  In pinned host
+   memory the word lets the host wait for an inspection without waiting for what was enqueued behind it; in device
+   memory it keeps the counts of one step past the next. */
+int kge_publish_counts(const int32_t *first, const int32_t *second, uint64_t *word, void *stream);
 
 /*
  * One step of a staged training loop in ONE call (host-side sequencing only; no counterpart in the

@@ -286,3 +286,29 @@ def test_a_replaced_stage_is_called():
     for st in (a, b):
         st.run()
         assert all(torch.equal(x, y) for x, y in zip(_step_outputs(st), _step_outputs(ref)))
+
+
+def test_gradients_of_a_step_keep_their_row_counts_past_the_next_run():
+    """sparse_grads() does not wait, and what is read from it later has the counts of its own step: the views of one
+    object never mix two steps (the rows themselves are overwritten)."""
+    from cuke_amd.kge import sparse_adagrad_factored
+    m, batches, make = _two_batches("TransR")
+    mine = [x.clone() if x is not None else None for x in batches[0]]
+    from cuke_amd.kge import TrainStep
+    st = TrainStep(m, *mine, factor_max=4)
+    state = torch.zeros(m.n_rel, device="cuda")
+    st.run()
+    want = [len(torch.unique(torch.cat((mine[0], mine[2])))), len(torch.unique(mine[1]))]
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        read, later = st.sparse_grads(), st.sparse_grads()
+        sparse_adagrad_factored(m.A, state, later, 0.0)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    assert read.ent_ids.numel() == want[0]
+    mine[0].fill_(3), mine[2].fill_(5), mine[1].fill_(1)  # two entities, one relation
+    st.run()
+    assert st.sparse_grads().ent_ids.tolist() == [3, 5] and st.sparse_grads().rel_rows.shape[0] == 1
+    for g in (read, later):
+        assert [g.ent_ids.numel(), g.rel_ids.numel()] == want == [g.ent_rows.shape[0], g.rel_rows.shape[0]]
+        assert g.aux_rows.shape[0] == want[1] and g.rel_seg_offsets.numel() == want[1] + 1

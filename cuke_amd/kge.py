@@ -1238,14 +1238,18 @@ class TrainStep:
         it puts on the main and on the side stream; going over from one to another, the stream that goes first waits for
         the other once: the side stream, which inspects ahead in the staged forms, for the steps before (in front
         of the first step: for the index tensors), the main stream for what has been inspected ahead."""
-        if form == self._form or torch.cuda.is_current_stream_capturing():
+        if form == self._form:
             return
-        last, self._form = self._form, form
-        main = torch.cuda.current_stream()
-        if form in ("staged", "native"):
-            self.side.wait_stream(main)
-        elif last in ("staged", "native"):
-            main.wait_stream(self.side)
+        ahead = ("staged", "native")
+        if form in ahead or self._form in ahead:  # (others need no wait, and pay for none of this)
+            if torch.cuda.is_current_stream_capturing():
+                return
+            main = torch.cuda.current_stream()
+            if form in ahead:
+                self.side.wait_stream(main)
+            else:
+                main.wait_stream(self.side)
+        self._form = form
 
     def run_native(self, cur, nxt) -> None:
         """The staged issue in ONE library call (kge_train_step_staged): the step of batch ``cur`` on the current

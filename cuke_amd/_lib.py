@@ -128,6 +128,8 @@ EXPORTS = {
     "kge_sample_negatives": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, C.c_uint64, C.c_uint64, C.c_void_p]),
     "kge_sample_batch": (C.c_int, [C.c_void_p] * 4 + [C.c_int64] + [C.c_void_p] * 4 +
                          [C.c_int64, C.c_int64, C.c_uint64, C.c_uint64, C.c_void_p]),
+    "kge_sample_staged_batch": (C.c_int, [C.c_void_p, C.c_int64] + [C.c_void_p] * 4 +
+                                [C.c_int64, C.c_int64, C.c_uint64, C.c_uint64, C.c_void_p, C.c_uint32, C.c_void_p]),
     "kge_widen_ids": (C.c_int, [C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.POINTER(C.c_int64), C.c_int, C.c_void_p]),
     "kge_publish_counts": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "kge_check_indices": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),

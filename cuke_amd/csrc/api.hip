@@ -80,6 +80,29 @@ __global__ void sample_batch_kernel(const int64_t *ch, const int64_t *cr, const 
     }
 }
 
+// The same from ids [3][B] in pinned host memory.  Bound by the launch and one round trip over the host link (a batch of
+// 4096 is 96 KB).  Every workgroup that reads ids says when it has, in a word of its own, so that no event has to be
+// recorded and asked about for the memory to be used again (about 5 us of host time per batch).
+__global__ __launch_bounds__(256) void sample_staged_batch_kernel(const int64_t *ids, int64_t B, int64_t *h, int64_t *r, int64_t *t, int64_t *neg,
+                                                                  int64_t count, uint64_t n_ent, uint64_t seed, uint64_t step,
+                                                                  uint32_t *done, uint32_t mark)
+{
+    const uint64_t base = seed ^ splitmix64(step);
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < B + count; i += (int64_t)gridDim.x * blockDim.x) {
+        if (i < B) {
+            const int64_t a = ids[i], b = ids[B + i], c = ids[2 * B + i];
+            h[i] = a, r[i] = b, t[i] = c;
+        } else {
+            const int64_t k = i - B;
+            neg[k] = (int64_t)__umul64hi(splitmix64(base ^ ((uint64_t)k * 0x9E3779B97F4A7C15ull)), n_ent);
+        }
+    }
+    // (What a thread has stored it has read, so nothing is read behind the barrier.  Relaxed: the word says that the ids have
+    // been read, and orders none of this kernel's own stores, which a release would write back through the L2 first.)
+    __syncthreads();
+    if (threadIdx.x == 0 && (int64_t)blockIdx.x * blockDim.x < B) __hip_atomic_store(done + blockIdx.x, mark, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 struct WidenArgs {
     const int32_t *src[4];
     int64_t *dst[4];
@@ -348,6 +371,19 @@ int kge_sample_batch(const int64_t *col_h, const int64_t *col_r, const int64_t *
     const int64_t blocks = ceil_div(batch + count, 256);
     hipLaunchKernelGGL(sample_batch_kernel, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, as_stream(stream),
                        col_h, col_r, col_t, order, batch, h, r, t, neg, count, (uint64_t)n_ent, seed, step);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+int kge_sample_staged_batch(const int64_t *ids, int64_t batch, int64_t *h, int64_t *r, int64_t *t, int64_t *neg, int64_t count,
+                            int64_t n_ent, uint64_t seed, uint64_t step, uint32_t *done, uint32_t mark, void *stream)
+{
+    if (batch < 0 || count < 0 || n_ent <= 0) return KGE_ESHAPE;
+    if (batch + count == 0) return KGE_OK;
+    if ((batch > 0 && (!ids || !h || !r || !t || !done)) || (count > 0 && !neg)) return KGE_EINVAL;
+    const int64_t blocks = ceil_div(batch + count, 256);
+    hipLaunchKernelGGL(sample_staged_batch_kernel, dim3((unsigned)(blocks < KGE_STAGED_BATCH_WORDS ? blocks : KGE_STAGED_BATCH_WORDS)), dim3(256), 0,
+                       as_stream(stream), ids, batch, h, r, t, neg, count, (uint64_t)n_ent, seed, step, done, mark);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

@@ -19,6 +19,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <mutex>
@@ -524,27 +525,132 @@ PyObject *py_sparse_step(PyObject *, PyObject *const *args, Py_ssize_t)
     END_HANDLE_TH_ERRORS
 }
 
-// sample_batch(triples [3, n], order [n], position, batch, count, n_ent, seed, step) -> (h, r, t, neg)
+// A one-dimensional array of 64-bit ids in host memory (numpy), read where it lies.
+struct HostIds {
+    Py_buffer b{};
+    bool held = false;
+    const char *base = nullptr;
+    int64_t stride = 0;
+    bool take(PyObject *o)
+    {
+        if (PyObject_GetBuffer(o, &b, PyBUF_FORMAT | PyBUF_STRIDES)) return PyErr_Clear(), false;
+        held = true, base = static_cast<const char *>(b.buf), stride = b.ndim == 1 ? b.strides[0] : 0;
+        return b.ndim == 1 && b.itemsize == 8 && b.format && (!std::strcmp(b.format, "l") || !std::strcmp(b.format, "q"));
+    }
+    int64_t size() const { return b.shape[0]; }
+    int64_t at(int64_t i) const { return *reinterpret_cast<const int64_t *>(base + i * stride); }
+    HostIds() = default;
+    HostIds(const HostIds &) = delete;
+    ~HostIds()
+    {
+        if (held) PyBuffer_Release(&b);
+    }
+};
+
+// The pinned memory of one sampler: slots of [KGE_STAGED_BATCH_WORDS done words][3][batch] ids.  A slot is free when the launch
+// that reads it has marked every word; a host that is further ahead gets another, up to 64 slots and 32 MB in all.
+// They are freed with the sampler, behind the launches that still read them.  (Callers hold the GIL.)
+struct Stage {
+    struct Slot {
+        uint32_t *done;
+        int64_t *ids;
+        uint32_t mark;
+        bool idle(int words) const
+        {
+            for (int w = 0; w < words; ++w)
+                if (__atomic_load_n(done + w, __ATOMIC_ACQUIRE) != mark) return false;
+            return true;
+        }
+    };
+    static constexpr size_t kHead = sizeof(uint32_t) * KGE_STAGED_BATCH_WORDS, kMaxSlots = 64, kMaxBytes = size_t(32) << 20;
+    int64_t batch = 0;
+    std::vector<Slot> slots;
+    size_t at = 0;
+
+    int words() const { return (int)std::min<int64_t>(KGE_STAGED_BATCH_WORDS, (batch + 255) / 256); }
+    size_t bytes() const { return kHead + sizeof(int64_t) * 3 * (size_t)batch; }
+    Slot *take()
+    {
+        for (size_t k = 0; k < slots.size(); ++k) {  // oldest first
+            Slot &s = slots[(at + k) % slots.size()];
+            if (s.idle(words())) return at = (at + k + 1) % slots.size(), &s;
+        }
+        if (slots.size() >= kMaxSlots || (slots.size() + 1) * bytes() > kMaxBytes) return nullptr;
+        void *p = nullptr;
+        if (hipHostMalloc(&p, bytes(), hipHostMallocPortable) != hipSuccess) return (void)hipGetLastError(), nullptr;
+        std::memset(p, 0, kHead);
+        slots.push_back(Slot{static_cast<uint32_t *>(p), reinterpret_cast<int64_t *>(static_cast<char *>(p) + kHead), 0});
+        return &slots.back();
+    }
+    ~Stage()
+    {
+        for (const Slot &s : slots) {
+            const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
+            bool idle;
+            while (!(idle = s.idle(words())) && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
+            if (!idle) idle = hipDeviceSynchronize() == hipSuccess;
+            if (idle) (void)hipHostFree(s.done);  // (a device that has failed keeps it)
+        }
+    }
+};
+
+constexpr const char *kStageName = "cuke_amd.sampler_stage";
+
+// sampler_stage(batch): a handle for sample_batch
+PyObject *py_sampler_stage(PyObject *, PyObject *o)
+{
+    HANDLE_TH_ERRORS
+    const int64_t batch = PyLong_AsLongLong(o);
+    if (batch == -1 && PyErr_Occurred()) return nullptr;
+    Stage *s = new Stage;
+    s->batch = batch;
+    return PyCapsule_New(s, kStageName, [](PyObject *c) { delete static_cast<Stage *>(PyCapsule_GetPointer(c, kStageName)); });
+    END_HANDLE_TH_ERRORS
+}
+
+// sample_batch(stage, h, r, t, order: host arrays, position, count, n_ent, seed, step, device) -> (h, r, t, neg) or None.  The triples
+// order[position ..) are gathered into the stage's pinned memory, which one launch reads where it draws the negatives:
+// no copy for the host to wait for, and the arrays are read as they are at this call.
 PyObject *py_sample_batch(PyObject *, PyObject *const *args, Py_ssize_t)
 {
     HANDLE_TH_ERRORS
-    const at::Tensor &tri = THPVariable_Unpack(args[0]), &order = THPVariable_Unpack(args[1]);
-    const int64_t at0 = PyLong_AsLongLong(args[2]), B = PyLong_AsLongLong(args[3]), count = PyLong_AsLongLong(args[4]),
-                  n_ent = PyLong_AsLongLong(args[5]);
-    const uint64_t seed = PyLong_AsUnsignedLongLongMask(args[6]), step = PyLong_AsUnsignedLongLongMask(args[7]);
+    Stage *stage = static_cast<Stage *>(PyCapsule_GetPointer(args[0], kStageName));
+    if (!stage) return nullptr;
+    HostIds col[3], order;
+    for (int k = 0; k < 3; ++k)
+        if (!col[k].take(args[1 + k])) NOT_HERE;
+    if (!order.take(args[4])) NOT_HERE;
+    const int64_t at0 = PyLong_AsLongLong(args[5]), count = PyLong_AsLongLong(args[6]), n_ent = PyLong_AsLongLong(args[7]);
+    const uint64_t seed = PyLong_AsUnsignedLongLongMask(args[8]), step = PyLong_AsUnsignedLongLongMask(args[9]);
+    const int64_t asked = PyLong_AsLongLong(args[10]);  // device index, -1: the current one
     if (PyErr_Occurred()) return nullptr;
-    const int64_t n = tri.size(1);
-    if (tri.device().index() != c10::hip::current_device()) NOT_HERE;
-    if (at0 < 0 || B < 0 || at0 + B > order.numel() || order.numel() > n) return fail(KGE_ESHAPE, "kge_sample_batch"), nullptr;
-    at::Tensor h = at::empty({B}, tri.options()), r = at::empty({B}, tri.options()), t = at::empty({B}, tri.options()),
-               neg = at::empty({count}, tri.options());
-    const int64_t *c = tri.data_ptr<int64_t>();
+    const int dev = c10::hip::current_device();
+    const int64_t B = stage->batch;
+    if ((asked >= 0 && asked != dev) || at0 < 0 || B <= 0 || count < 0 || at0 > order.size() - B) NOT_HERE;
     void *st = stream();
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(st), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
+        NOT_HERE;  // (a replay would read what a later batch has left there)
+    Stage::Slot *slot = stage->take();
+    if (!slot) NOT_HERE;
+    int64_t *ids = slot->ids;
+    const uint64_t rows = (uint64_t)std::min({col[0].size(), col[1].size(), col[2].size()});
+    bool inside = true;
+    for (int64_t i = 0; i < B; ++i) {
+        const uint64_t q = (uint64_t)order.at(at0 + i);
+        if (!(inside = q < rows)) break;
+        ids[i] = col[0].at(q), ids[B + i] = col[1].at(q), ids[2 * B + i] = col[2].at(q);
+    }
+    if (!inside) NOT_HERE;  // (numpy's indexing raises, or counts from the end)
+    const auto i64 = at::TensorOptions().dtype(at::kLong).device(at::kCUDA, (c10::DeviceIndex)dev);
+    at::Tensor h = at::empty({B}, i64), r = at::empty({B}, i64), t = at::empty({B}, i64), neg = at::empty({count}, i64);
+    uint32_t *done = slot->done;
+    const uint32_t mark = ++slot->mark;  // (taken from here on, also for a thread that comes in while the launch is under way)
     const int rc = nogil([&] {
-        return kge_sample_batch(c, c + n, c + 2 * n, order.data_ptr<int64_t>() + at0, B, h.data_ptr<int64_t>(), r.data_ptr<int64_t>(),
-                                t.data_ptr<int64_t>(), neg.data_ptr<int64_t>(), count, n_ent, seed, step, st);
+        return kge_sample_staged_batch(ids, B, h.data_ptr<int64_t>(), r.data_ptr<int64_t>(), t.data_ptr<int64_t>(), neg.data_ptr<int64_t>(), count,
+                                       n_ent, seed, step, done, mark, st);
     });
-    if (rc) return fail(rc, "kge_sample_batch"), nullptr;
+    if (rc) return fail(rc, "kge_sample_staged_batch"), nullptr;
     return Py_BuildValue("(NNNN)", wrap(h), wrap(r), wrap(t), wrap(neg));
     END_HANDLE_TH_ERRORS
 }
@@ -557,6 +663,7 @@ PyMethodDef methods[] = {{"set_error", py_set_error, METH_O, nullptr},
                          FAST(call),
                          FAST(margin_loss),
                          FAST(sparse_step),
+                         {"sampler_stage", py_sampler_stage, METH_O, nullptr},
                          FAST(sample_batch),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

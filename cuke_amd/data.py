@@ -89,11 +89,8 @@ class TrainSampler:
         self.dev = torch.device(device)
         self.step = 0
         self._order, self._pos, self._epoch = None, 0, 0
-        # The triples (24 bytes each) and the epoch's order (8) stay on the device, so that a batch is one gather
-        # launch instead of a numpy gather and three host-to-device copies that each wait for the stream.  Lists of
-        # more than a gigabyte are batched on the host.
-        self._resident = self.dev.type == "cuda" and 32 * len(self.h) <= 1 << 30
-        self._triples = self._order_dev = None
+        self._dev_index = -1 if self.dev.index is None else self.dev.index  # (-1: the current device)
+        self._stage = None  # the native path's pinned memory
 
     def _next_ids(self):
         if self._order is None or self._pos + self.batch > len(self._order):
@@ -101,12 +98,12 @@ class TrainSampler:
             self._order = np.random.default_rng([self.seed, self._epoch]).permutation(n) if self.shuffle \
                 else np.arange(n)
             self._pos, self._epoch = 0, self._epoch + 1
-            if self._order_dev is not None:
-                torch.cuda.synchronize(self.dev)  # once per epoch: batches may have been taken on other streams too
-                self._order_dev = None
         at = self._pos
         self._pos += self.batch
         return at
+
+    def __getstate__(self):  # (a copy has pinned memory of its own)
+        return {**self.__dict__, "_stage": None}
 
     def __iter__(self):
         return self
@@ -115,12 +112,14 @@ class TrainSampler:
         at = self._next_ids()
         count = (self.batch // self.chunk) * self.n_neg
         got = None
-        if self._resident:
-            if self._triples is None:
-                self._triples = torch.from_numpy(np.stack((self.h, self.r, self.t))).to(self.dev)
-            if self._order_dev is None:
-                self._order_dev = torch.from_numpy(self._order.astype(np.int64, copy=False)).to(self.dev)
-            got = _lib.host().sample_batch(self._triples, self._order_dev, at, self.batch, count, self.n_entities, self.seed, self.step)
+        if self.dev.type == "cuda":
+            # the batch's triples gathered from the host arrays into pinned memory and one launch (host.cpp); what that does
+            # not take -- a device that is not the current one, other arrays than int64 -- goes by three copies
+            host = _lib.host()
+            if self._stage is None or self._stage[0] != self.batch:
+                self._stage = self.batch, host.sampler_stage(self.batch)
+            got = host.sample_batch(self._stage[1], self.h, self.r, self.t, self._order, at, count, self.n_entities, self.seed, self.step,
+                                    self._dev_index)
         if got is None:
             got = self._host_batch(at, count)
         if self.mode == "both":

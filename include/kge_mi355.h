@@ -440,6 +440,15 @@ int kge_sample_batch(const int64_t *col_h, const int64_t *col_r, const int64_t *
                      int64_t *h, int64_t *r, int64_t *t, int64_t *neg, int64_t count, int64_t n_ent, uint64_t seed, uint64_t step,
                      void *stream);
 
+/*
+ * The same for a list in host memory: ids [3][batch] are the batch's heads, relations and tails in pinned host memory,
+ * read by the launch.  When they have been read, the first min(KGE_STAGED_BATCH_WORDS, ceil(batch / 256)) words of
+ * `done` (pinned too) all hold `mark`: the caller may write the next batch there then, and needs no event for it.
+ */
+#define KGE_STAGED_BATCH_WORDS 64
+int kge_sample_staged_batch(const int64_t *ids, int64_t batch, int64_t *h, int64_t *r, int64_t *t, int64_t *neg, int64_t count,
+                            int64_t n_ent, uint64_t seed, uint64_t step, uint32_t *done, uint32_t mark, void *stream);
+
 /* 32-bit id arrays widened to the 64-bit ids every other entry point takes: up to four arrays in one launch
    (src / dst / len: host arrays of n_parts device pointers / lengths). */
 int kge_widen_ids(const int32_t *const *src, int64_t *const *dst, const int64_t *len, int n_parts, void *stream);

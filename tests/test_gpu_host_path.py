@@ -312,3 +312,95 @@ def test_gradients_of_a_step_keep_their_row_counts_past_the_next_run():
     for g in (read, later):
         assert [g.ent_ids.numel(), g.rel_ids.numel()] == want == [g.ent_rows.shape[0], g.rel_rows.shape[0]]
         assert g.aux_rows.shape[0] == want[1] and g.rel_seg_offsets.numel() == want[1] + 1
+
+
+def _sampler(n=700, **kw):
+    from cuke_amd.data import TrainSampler
+    rng = np.random.default_rng(3)
+    triples = [rng.integers(0, m, n) for m in (90, 7, 90)]
+    kw = dict(dict(batch_size=128, neg_sample_size=5, neg_chunk_size=32, seed=11, mode="both"), **kw)
+    return triples, TrainSampler(triples, 90, **kw)
+
+
+@pytest.mark.parametrize("device", ["cuda:0", "cuda"])
+@pytest.mark.parametrize("shuffle", [True, False])
+def test_sampler_batches_are_the_host_arrays_in_the_epochs_order(device, shuffle):
+    triples, s = _sampler(device=device, shuffle=shuffle)
+    _, plain = _sampler(device=device, shuffle=shuffle)
+    for step in range(13):  # five batches an epoch
+        got = next(s)
+        want = plain._host_batch(plain._next_ids(), 20)
+        plain.step += 1
+        assert all(torch.equal(x, y) and x.dtype == torch.int64 for x, y in zip(got, want)), step
+        order = np.random.default_rng([11, step // 5]).permutation(700) if shuffle else np.arange(700)
+        ids = order[step % 5 * 128:][:128]
+        assert all(np.array_equal(x.cpu().numpy(), y[ids]) for x, y in zip(got, triples)), step
+
+
+def test_sampler_reads_its_arrays_as_they_are_at_each_batch():
+    """Changed in place, rebound, strided: the next batch has it.  An order that points outside raises."""
+    triples, s = _sampler(shuffle=False)
+    first = next(s)
+    s.h[128:256] = 17
+    assert (next(s)[0] == 17).all()
+    s.t = np.arange(1400)[::2]
+    assert torch.equal(next(s)[2], torch.arange(256, 384, device="cuda") * 2)
+    s.r = np.arange(400)
+    with pytest.raises(IndexError):
+        next(s)
+    assert torch.equal(first[0], torch.from_numpy(triples[0][:128]).cuda())
+
+
+@pytest.mark.parametrize("batch", [1, 255, 256, 257, 64 * 256, 64 * 256 + 1, 50000])
+def test_sampler_batches_of_every_size_reuse_their_pinned_memory(batch):
+    """Around one id per thread, one workgroup, and one and two turns of the whole grid; three epochs of three batches."""
+    import copy
+    triples, s = _sampler(3 * batch, batch_size=batch, neg_chunk_size=batch, neg_sample_size=3)
+    kept = [next(s) for _ in range(5)]
+    again = copy.deepcopy(s)
+    kept += [next(s) for _ in range(4)]
+    for k, got in enumerate(kept):
+        ids = np.random.default_rng([11, k // 3]).permutation(3 * batch)[k % 3 * batch:][:batch]
+        assert all(np.array_equal(x.cpu().numpy(), y[ids]) for x, y in zip(got, triples)), k
+    for k in range(5, 9):
+        assert all(torch.equal(x, y) for x, y in zip(next(again), kept[k])), k
+
+
+def test_batches_of_a_resident_triple_list():
+    """kge_sample_batch, for hosts that keep the triples on the device."""
+    import ctypes as C
+    from cuke_amd import _lib
+    rng = np.random.default_rng(5)
+    cols = [torch.from_numpy(rng.integers(0, 50, 600)).cuda() for _ in range(3)]
+    order = torch.from_numpy(rng.permutation(600)).cuda()
+    h, r, t, neg, neg2 = (torch.empty(n, dtype=torch.int64, device="cuda") for n in (257, 257, 257, 300, 300))
+    p = lambda x: C.c_void_p(x.data_ptr())
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _lib.lib().kge_sample_batch(*map(p, cols), p(order), 257, p(h), p(r), p(t), p(neg), 300, 50, 9, 4, st) == 0
+    assert _lib.lib().kge_sample_negatives(p(neg2), 300, 50, 9, 4, st) == 0
+    assert all(torch.equal(x, c[order[:257]]) for x, c in zip((h, r, t), cols)) and torch.equal(neg, neg2)
+
+
+def test_sampler_keeps_nothing_on_the_device_and_waits_for_nothing():
+    """200 batches from three streams behind a busy device, the host far ahead: every batch is its own, the sampler holds no
+    device memory, and neither a batch nor the end of an epoch (5 batches) synchronises."""
+    triples, s = _sampler(shuffle=False)
+    next(s), torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    busy = torch.empty(1 << 28, dtype=torch.uint8, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    kept = []
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        for k in range(1, 200):
+            with torch.cuda.stream(streams[k % 3]):
+                if k % 40 < 3:
+                    busy.zero_()
+                kept.append(next(s))
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    torch.cuda.synchronize()
+    for k, got in enumerate(kept, 1):
+        assert all(np.array_equal(x.cpu().numpy(), y[k % 5 * 128:][:128]) for x, y in zip(got, triples)), k
+    del kept, got, busy
+    assert torch.cuda.memory_allocated() == before

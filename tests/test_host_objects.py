@@ -28,3 +28,17 @@ def test_packed_inspection_names_its_parts_and_can_be_copied():
         assert x.perm.tolist() == perm and x.inverse.tolist() == inverse and x.sorted_seg.tolist() == sorted_seg
         with pytest.raises(AttributeError):
             x.no_such_part
+
+
+def test_staged_batches_are_validated_on_the_host():
+    import ctypes as C
+    from cuke_amd import _lib
+    f, fake = _lib.lib().kge_sample_staged_batch, C.c_void_p(0x1000)
+    ok = [fake, 8, fake, fake, fake, fake, 4, 10, 1, 0, fake, 1, None]
+
+    def call(**kw):
+        return f(*[kw.get(f"a{i}", x) for i, x in enumerate(ok)])
+    assert call(a1=-1) == call(a6=-1) == call(a7=0) == -2
+    for null in (0, 2, 3, 4, 5, 10):
+        assert call(**{f"a{null}": None}) == -1
+    assert call(a1=0, a6=0) == 0  # empty work: nothing is launched

@@ -134,6 +134,7 @@ __global__ __launch_bounds__(kWideThreads) void wide_step_kernel(float *table, f
 }
 
 constexpr int64_t kWideDim = 4096;  // from here a row gives every one of the 1024 threads a quad
+constexpr int64_t kWideRows = (int64_t(1) << 22) - 1;  // a launch has fewer than 2^32 threads; more rows fill the chip with a wave each
 
 template <bool ADAGRAD>
 static int launch_step(float *table, float *state, int64_t dim, const int64_t *ids, const int32_t *num_unique,
@@ -142,7 +143,7 @@ static int launch_step(float *table, float *state, int64_t dim, const int64_t *i
     if (!table || !ids || !num_unique || !rows || (ADAGRAD && !state)) return KGE_EINVAL;
     if (dim <= 0 || dim > (1 << 20) || capacity < 0) return KGE_ESHAPE;
     if (capacity == 0) return KGE_OK;
-    if (dim >= kWideDim && dim % 4 == 0 && aligned16(table) && aligned16(rows)) {
+    if (dim >= kWideDim && dim % 4 == 0 && capacity <= kWideRows && aligned16(table) && aligned16(rows)) {
         const dim3 wgrid((unsigned)capacity), wblock(kWideThreads);
         const int64_t per = ceil_div(dim / 4, kWideThreads);
 #define WIDE_STEP(NQ) hipLaunchKernelGGL((wide_step_kernel<ADAGRAD, NQ>), wgrid, wblock, 0, st, table, state, (int)dim, ids, num_unique, rows, lr, eps)

@@ -91,6 +91,25 @@ def test_optimizer_rows_of_thousands_of_floats(oracle, dim, opt):
         assert_close(s.cpu().numpy(), ws, what="state")
 
 
+@pytest.mark.parametrize("capacity", [3, (1 << 22) - 1, 1 << 22, 5_000_000])
+def test_optimizer_rows_of_thousands_of_floats_in_arrays_of_millions(capacity):
+    """The row array's capacity (rows past the distinct ids are not read) on both sides of what a workgroup per row can launch."""
+    import ctypes as C
+    from cuke_amd import _lib
+    dim = 4096
+    table, state, rows = torch.ones(5, dim, device="cuda"), torch.zeros(5, device="cuda"), torch.full((3, dim), 2.0, device="cuda")
+    ids, count = torch.tensor([0, 2, 3], device="cuda"), torch.tensor([3], dtype=torch.int32, device="cuda")
+    p = lambda x: C.c_void_p(x.data_ptr())
+    st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _lib.lib().kge_sparse_sgd(p(table), dim, p(ids), p(count), capacity, p(rows), 0.25, st) == 0
+    want = torch.ones(5, dim, device="cuda")
+    want[ids] = 0.5
+    assert torch.equal(table, want)
+    assert _lib.lib().kge_sparse_adagrad(p(table), p(state), dim, p(ids), p(count), capacity, p(rows), 0.25, 0.0, st) == 0
+    want[ids] = 0.25  # state 4, a step of 0.25 * 2 / 2
+    assert torch.equal(state, torch.tensor([4.0, 0, 4, 4, 0], device="cuda")) and torch.equal(table, want)
+
+
 def test_adagrad_without_a_state_raises_and_updates_nothing():
     """(it is not SGD)"""
     from cuke_amd.kge import inspect, sparse_adagrad

@@ -55,17 +55,27 @@ template <int MODE>
 struct TallSlot {
     floatx2 r[4];
     __device__ __forceinline__ float at(int e, int s) const { return r[s][e]; }
+    __device__ __forceinline__ void keep(bool k)
+    {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) r[s] = k ? r[s] : floatx2{0.f, 0.f};
+    }
 };
 template <>
 struct TallSlot<2> {
     floatx4 r[2];
     __device__ __forceinline__ float at(int e, int s) const { return r[e][s]; }
+    __device__ __forceinline__ void keep(bool k)
+    {
+#pragma unroll
+        for (int e = 0; e < 2; ++e) r[e] = k ? r[e] : floatx4{0.f, 0.f, 0.f, 0.f};
+    }
 };
 
 // Two B-operand values per k row for this lane: columns n0 + 2 li + {0, 1} of M (MODE 2: of M^T).  Addresses are the
 // uniform base plus a 32-bit byte offset (a projection has at most 2^20 elements: no 64-bit address arithmetic on the
 // vector ALUs, which would take issue slots from the matrix instructions); a k beyond the last row is clamped to
-// it (the staged left operand is zero there).
+// it (the staged left operand is zero there, and tall_sweep() zeroes the clamped values too).
 template <int MODE>
 struct TallLoader {
     const char *M;
@@ -99,11 +109,11 @@ struct TallLoader {
 // order, so the requests go out behind the first superstep's piece of the projection and the writes wait until the
 // end of the slice, when everything in front of them has been used anyway.
 template <int MODE, int RB, typename Fetch, typename Put>
-__device__ __forceinline__ void tall_sweep(const TallLoader<MODE> &bl, int nq, TallSlot<MODE> (&ring)[kTallRing], const float *lds, int li, int kk,
+__device__ __forceinline__ void tall_sweep(const TallLoader<MODE> &bl, int d, TallSlot<MODE> (&ring)[kTallRing], const float *lds, int li, int kk,
                                            Fetch fetch, Put put, floatx4 (&acc)[RB][2])
 {
     static_assert(kTallRing == kTallKC / 16, "ring slot u is superstep u of every slice");
-    const int nc = (nq + kTallRing - 1) / kTallRing;
+    const int nq = (d + 15) / 16, nc = (nq + kTallRing - 1) / kTallRing;
 #pragma unroll 1
     for (int c = 0; c < nc; ++c) {
         const float *sX = lds + (c & 1) * (kTallRows * kTallPitch) + li * kTallPitch + 4 * kk;
@@ -118,6 +128,7 @@ __device__ __forceinline__ void tall_sweep(const TallLoader<MODE> &bl, int nq, T
             }
             __builtin_amdgcn_sched_barrier(0);
             if (q >= nq) continue;  // uniform
+            if (16 * q + 16 > d) ring[u].keep(16 * q + 4 * kk < d);  // uniform: the last superstep of most widths; keeps 0 * inf out
             float4 a[RB];
 #pragma unroll
             for (int m = 0; m < RB; ++m) a[m] = *reinterpret_cast<const float4 *>(sX + 16 * m * kTallPitch + 16 * u);
@@ -157,7 +168,6 @@ __device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int til
     TallLoader<MODE> bl;
     TallSlot<MODE> ring[kTallRing];
     bl.init(M, d, wcols > 0 ? n0 : c0, wcols, li, kk);
-    const int nq = (d + 15) / 16;
 #pragma unroll
     for (int u = 0; u + 1 < kTallRing; ++u) bl.load(u, ring[u]);  // the projection's first pieces fly during the index chain below
     __builtin_amdgcn_sched_barrier(0);
@@ -237,7 +247,7 @@ __device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int til
 #pragma unroll
     for (int i = 0; i < RB; ++i) put(i, 0);
     __syncthreads();
-    tall_sweep<MODE, RB>(bl, nq, ring, lds, li, kk, fetch, put, acc);
+    tall_sweep<MODE, RB>(bl, d, ring, lds, li, kk, fetch, put, acc);
 
     // Lane (li, kk) holds rows 16 m + 4 kk + r, columns n0 + 2 li + {0, 1}.  Everything is read before the first
     // store: a load between two stores makes the compiler wait for the stores in front of it.

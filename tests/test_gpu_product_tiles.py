@@ -49,3 +49,23 @@ def test_shared_negatives_by_both_tiles(oracle, model, n_rel, dim):
     ref = oracle.backward(model, a["E"], a["R"], a["A"], a["h"], a["r"], a["t"], dpos=dpos, dneg=dneg, **kw)
     assert_close(g.ent_rows.cpu().numpy(), ref.ent_rows, what="entity rows", rows=True)
     assert_close(g.aux_rows.cpu().numpy(), ref.aux_rows, what="projection gradients", rows=True)
+
+
+@pytest.mark.parametrize("model", ["TransR", "RESCAL"])
+@pytest.mark.parametrize("dim", [36, 132, 200, 260, 1000])
+def test_an_infinite_weight_in_the_last_row_stays_in_its_column(model, dim):
+    """Widths that are no multiple of 16: where a tile's last step reaches past the row, the projection's last row is read in its
+    place.  Few groups, so the 64-row tiles take them; one to four rows each, which streaming also kept clean."""
+    w = synth.custom_workload(model, n_ent=50, n_rel=3, dim=dim, batch=8, norm_p=2, sigma=0.2, seed=dim)
+    w.arrays["r"][:] = [0, 0, 0, 0, 1, 1, 2, 2]
+    w.arrays["t"][:] = (w.arrays["h"] + 1) % 50  # (no zero difference: 0 * inf is a NaN of the product itself)
+    w.arrays["A"][1, dim - 1, dim - 2] = np.inf
+    a = {k: torch.from_numpy(v) for k, v in w.arrays.items() if v is not None}
+    m, ix = gpu_model(w)
+    from cuke_amd.kge import inspect
+    got = m.score(ix["h"], ix["r"], ix["t"], rel_insp=inspect([ix["r"]], m.n_rel)).residual.cpu()
+    x = (a["E"][a["h"]] - (a["E"][a["t"]] if model == "TransR" else 0)).double()
+    want = torch.bmm(x[:, None, :], a["A"][a["r"]].double())[:, 0] + (a["R"][a["r"]].double() if model == "TransR" else 0)
+    assert torch.isinf(want).sum() == 2 and not torch.isnan(want).any()
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)].double(), want[torch.isinf(want)])
+    assert not torch.isnan(got).any()

@@ -64,6 +64,14 @@ bool is_ids(const at::Tensor *t, int dev)
            t->is_contiguous();
 }
 
+bool number(PyObject *o, double *out)
+{
+    *out = PyFloat_AsDouble(o);
+    if (!PyErr_Occurred()) return true;
+    PyErr_Clear();  // (the caller converts it, or raises)
+    return false;
+}
+
 PyObject *wrap(const at::Tensor &t)
 {
     if (!t.defined()) Py_RETURN_NONE;
@@ -207,6 +215,7 @@ PyObject *py_inspect(PyObject *, PyObject *const *args, Py_ssize_t)
         if (!is_ids(t, dev) || t->dim() != 1) NOT_HERE;
         ids[q] = *t, n += t->numel();
     }
+    if (!PyLong_Check(args[1])) NOT_HERE;  // (a count of another type: converted by the caller)
     const int64_t n_rows = PyLong_AsLongLong(args[1]);
     if (n_rows == -1 && PyErr_Occurred()) return nullptr;
     void *st = stream();
@@ -483,8 +492,8 @@ PyObject *py_margin_loss(PyObject *, PyObject *const *args, Py_ssize_t)
     const int dev = c10::hip::current_device();
     const at::Tensor *pos = tensor(args[0]), *neg = tensor(args[1]);
     if (!is_f32(pos, 1, dev) || !is_f32(neg, 2, dev) || neg->size(0) != pos->numel()) NOT_HERE;
-    const double margin = PyFloat_AsDouble(args[2]), sign = PyFloat_AsDouble(args[3]);
-    if (PyErr_Occurred()) return nullptr;
+    double margin, sign;
+    if (!number(args[2], &margin) || !number(args[3], &sign)) NOT_HERE;
     const int64_t B = neg->size(0), N = neg->size(1);
     const auto f32 = pos->options().requires_grad(false);
     at::Tensor loss = at::empty({1}, f32), dpos = at::empty({B}, f32), dneg = at::empty({B, N}, f32);
@@ -511,8 +520,8 @@ PyObject *py_sparse_step(PyObject *, PyObject *const *args, Py_ssize_t)
     if (adagrad && !is_f32(state, 1, dev)) NOT_HERE;
     const auto *ins = static_cast<const kge_inspection *>(PyLong_AsVoidPtr(args[2]));
     if (!ins) NOT_HERE;  // (no inspection was given)
-    const double lr = PyFloat_AsDouble(args[4]), eps = PyFloat_AsDouble(args[5]);
-    if (PyErr_Occurred()) return nullptr;
+    double lr, eps;
+    if (!number(args[4], &lr) || !number(args[5], &eps)) NOT_HERE;
     void *st = stream();
     const int rc = nogil([&] {
         return adagrad ? kge_sparse_adagrad(table->data_ptr<float>(), state->data_ptr<float>(), rows->size(1), ins->unique_ids, ins->num_unique,

@@ -423,3 +423,22 @@ def test_sampler_keeps_nothing_on_the_device_and_waits_for_nothing():
         assert all(np.array_equal(x.cpu().numpy(), y[k % 5 * 128:][:128]) for x, y in zip(got, triples)), k
     del kept, got, busy
     assert torch.cuda.memory_allocated() == before
+
+
+def test_numbers_are_converted_as_the_general_path_does():
+    """Whatever int() / float() takes: a row count as a float, a margin or a rate as text or as a tensor."""
+    from cuke_amd.kge import inspect, margin_loss, sparse_sgd
+    ids = torch.tensor([4, 2, 4], device="cuda")
+    ins = inspect(ids, 9.0)
+    assert ins.n_rows == 9 and inspect(ids, np.int64(9)).ids().tolist() == ins.ids().tolist() == [2, 4]
+    with pytest.raises((TypeError, ValueError)):
+        inspect(ids, "many")
+    pos, neg = torch.randn(8, device="cuda"), torch.randn(8, 4, device="cuda")
+    want = margin_loss(pos, neg, 0.5, -1.0)
+    for margin in ("0.5", torch.tensor(0.5), torch.tensor([0.5], device="cuda")):
+        assert all(torch.equal(x, y) for x, y in zip(margin_loss(pos, neg, margin, "-1"), want))
+    with pytest.raises((TypeError, ValueError)):
+        margin_loss(pos, neg, None)
+    table = torch.ones(9, 4, device="cuda")
+    sparse_sgd(table, ins, torch.ones(3, 4, device="cuda"), "0.25")
+    assert table[:, 0].tolist() == [1, 1, 0.75, 1, 0.75, 1, 1, 1, 1]

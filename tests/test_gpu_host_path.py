@@ -442,3 +442,17 @@ def test_numbers_are_converted_as_the_general_path_does():
     table = torch.ones(9, 4, device="cuda")
     sparse_sgd(table, ins, torch.ones(3, 4, device="cuda"), "0.25")
     assert table[:, 0].tolist() == [1, 1, 0.75, 1, 0.75, 1, 1, 1, 1]
+
+
+def test_empty_batches():
+    """Positional calls, scores, losses and inspections of nothing."""
+    from cuke_amd import kge
+    E, R = torch.ones(9, 8, device="cuda"), torch.ones(4, 8, device="cuda")
+    A = torch.ones(4, 8, 8, device="cuda")
+    e = torch.zeros(0, dtype=torch.int64, device="cuda")
+    assert kge.transE(0, 8, 9, E, e, e, 4, R, e).shape == (0, 8)
+    assert kge.transR(0, 8, 0, E, e, e, 0, A, e, R).shape == (0, 8)
+    assert kge.RESCAL(0, 8, 0, E, e, 0, A, e, e).shape == (0,)
+    assert kge.inspect(e, 9).num_unique == 0
+    loss, dpos, dneg = kge.margin_loss(torch.zeros(0, device="cuda"), torch.zeros(0, 5, device="cuda"), 1.0)
+    assert loss.item() == 0.0 and dpos.shape == (0,) and dneg.shape == (0, 5)

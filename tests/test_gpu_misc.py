@@ -23,6 +23,24 @@ def test_margin_loss(oracle, B, N, sign):
     assert np.array_equal(dneg.cpu().numpy(), rdn)
 
 
+@pytest.mark.parametrize("B", [4095, 4096, 4097, 8192 + 5])
+@pytest.mark.parametrize("N,offset", [(8, 0), (8, 1), (8, 4), (7, 0)])
+def test_margin_loss_by_every_workgroup_and_load_width(oracle, B, N, offset):
+    """Around the point from which every one of the 1024 workgroups takes more than one turn, with 128-bit rows, with
+    rows of such a length at an odd address, and with rows of another length."""
+    from cuke_amd.kge import margin_loss
+    rng = np.random.default_rng(B + N)
+    pos, neg = rng.standard_normal(B).astype(np.float32), rng.standard_normal((B, N)).astype(np.float32)
+    dev_neg = torch.zeros(offset + B * N, device=DEV)[offset:].view(B, N)
+    dev_neg.copy_(torch.from_numpy(neg))
+    assert (dev_neg.data_ptr() % 16 == 0) == (offset % 4 == 0)
+    loss, dpos, dneg = margin_loss(torch.from_numpy(pos).to(DEV), dev_neg, 0.7, -1.0)
+    rl, rdp, rdn = oracle.margin_loss(pos, neg, 0.7, -1.0)
+    assert_close(loss.cpu().numpy(), np.array([rl], np.float32), what="loss")
+    assert_close(dpos.cpu().numpy(), rdp, what="dpos")
+    assert np.array_equal(dneg.cpu().numpy(), rdn)
+
+
 def test_margin_loss_of_an_empty_batch_is_zero_without_a_workspace():
     """kge_margin_loss_workspace answers 0 for an empty batch, so the call takes no workspace and reads none."""
     import ctypes as C

@@ -6,9 +6,9 @@
 // from every 128-byte piece it loads, and the left operand goes through LDS in slices of 64 columns (double buffered), so
 // that two to four workgroups fit a CU whatever the row width is (whole rows in LDS left one at width 1024).
 //   what bounds it: the matrix cores where groups are large (8192 x 1024 over 51 relations), the projections'
-//   bytes where they are small (4096 x 512 over 237).  Measured against the 32-row tiles: 8192 x 1024 over 51
-//   relations (RESCAL) 329 -> 229 us, 81 TFLOP/s; 512 x 1000 over 40 the call 178 -> 69 us; one relation with 24576
-//   rows of 1024 reaches 111 TFLOP/s.
+//   bytes where they are small (4096 x 512 over 237).  Whole RESCAL calls, 32-row tiles -> these, on one box: 8192 x 1024
+//   over 51 relations (Zipf) 335 -> 236 us, 73 TFLOP/s; 4096 x 512 over 237 (Zipf) 107 -> 89 us; 512 x 1000 over 40
+//   163 -> 61 us; one relation with 24576 rows of 1024 494 -> 478 us, 108 TFLOP/s.
 // Tiles of fewer rows run one to three of the four 16-row blocks, so a tail costs what it holds.
 //
 // A superstep of the projection comes back after about two microseconds when the chip is busy, so what a CU holds in
@@ -347,17 +347,22 @@ __global__ __launch_bounds__(256) void tall_finish_kernel(const float *part, int
 
 
 // Whether a batch of `rows` rows in at most n_rel groups goes by these tiles rather than by 32-row tiles and streamed
-// small groups (transr_gemm_kernel).  Measured side by side over 64 to 1024 columns and 1 to 500 rows per group:
-//   up to 128 columns   one column block: the 64-row tile reads a projection half as often, 5 to 20 % of the call from
-//                       four rows per group on (16000 rows x 128, 500 groups: 47.5 -> 39.6 us); below, streaming wins
-//   up to 256           two column blocks stage every row twice: only where the 32-row tiles would leave compute units idle
-//   above               a 32-row tile is one workgroup however wide its rows are: few groups leave the chip idle
-//                       (512 x 300, 60 groups: 42 -> 28 us; 8192 x 1024, 51 groups: 355 -> 238 us); many groups of a few
-//                       rows are bound by reading the projections, which streaming does better
+// small groups (transr_gemm_kernel).  The rule sees the counts, not the distribution.  Both sides measured over 64 to
+// 1000 columns, 20 to 1600 groups, 2 to 32 rows per group on average, uniform and Zipf (1.0, 1.2), 64-row time / 32-row
+// time of a TransR score call and of its backward, geometric means (extremes):
+//   up to 128 columns   one column block: a projection is read half as often.  0.86 (0.67 to 1.09) and 0.92 where these
+//                       tiles are taken; at two rows per group and more than 256 tiles 0.92 (0.77 to 1.07)
+//   up to 256           two column blocks stage every row twice: only where the 32-row tiles leave compute units idle.
+//                       Up to 200 tiles 1.00 (0.79 to 1.17) and 0.94; 201 to 256 tiles 1.17 (1.00 to 1.41) and 0.97;
+//                       above 1.17 (0.84 to 1.56) and 0.95
+//   above               a 32-row tile is one workgroup however wide its rows are: few groups leave the chip idle.
+//                       0.76 (0.24 to 1.33) and 0.78; where streaming is taken (many groups of a few rows, bound by
+//                       reading the projections) 0.95 (0.70 to 1.28) and 0.89
 static bool want_tall(int64_t d, int64_t rows, int64_t n_rel)
 {
     const int64_t groups = rows < n_rel ? rows : n_rel, short_tiles = groups + rows / 32;
-    if (d <= 2 * kTallCols) return short_tiles <= 256 || (d <= kTallCols && rows >= 4 * n_rel);
+    if (d <= kTallCols) return short_tiles <= 256 || rows >= 4 * n_rel;
+    if (d <= 2 * kTallCols) return short_tiles <= 200;
     return groups <= 256 || rows >= 16 * n_rel;
 }
 

@@ -1691,7 +1691,7 @@ int launch_transr_fwd(const kge_tables *tab, const kge_batch *bat, float *pos, f
     if (!a.back) {
         float *part = reinterpret_cast<float *>(static_cast<char *>(workspace) + plans_bytes(z));
         const int rc = launch_product(rescal ? 1 : 0, a, plans, z, a.thin_groups, part, bat->batch, fi, st);
-        timeline_mark(bat->timeline, st, "transr_plan_kernel + transr_gemm_kernel<fwd>");
+        timeline_mark(bat->timeline, st, z.tall ? "transr_plan_kernel + transr_tall_kernel<fwd>" : "transr_plan_kernel + transr_gemm_kernel<fwd>");
         return rc;
     }
     size_t own = gemm_lds_bytes((int)tab->dim);
@@ -1723,7 +1723,7 @@ int launch_rescal_head_rows(const kge_tables *tab, const kge_batch *bat, float *
     GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
                 TilePlan{}, nullptr, nullptr, nullptr, nullptr, u, nullptr, d, tab->norm_p, 0, 0, src};
     const int rc = launch_product(2, ga, plans_at(workspace, z), z, thin_groups(tab, bat), nullptr, bat->batch, FusedInsp{}, st);
-    timeline_mark(bat->timeline, st, "transr_gemm_kernel<head rows>");
+    timeline_mark(bat->timeline, st, z.tall ? "transr_tall_kernel<head rows>" : "transr_gemm_kernel<head rows>");
     return rc;
 }
 
@@ -1854,7 +1854,7 @@ int launch_rescal_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
                 TilePlan{}, head ? xs : qs, nullptr, nullptr, head ? occ + B * d : nullptr, head ? nullptr : occ, nullptr, d, tab->norm_p, 0, 0,
                 BwdSrc{}};
     if (const int rc = launch_product(head ? 1 : 2, ga, plans, z, thin_groups(tab, bat), nullptr, B, FusedInsp{}, st)) return rc;
-    timeline_mark(bat->timeline, st, "transr_gemm_kernel<dX>");
+    timeline_mark(bat->timeline, st, z.tall ? "transr_tall_kernel<dX>" : "transr_gemm_kernel<dX>");
     // dProj[r][i][j] = sum over the group of xs[i] qs[j] in both modes
     DmArgs da{xs, qs, ri->seg_offsets, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + p.off_dpart), d, ri->num_unique,
               BwdSrc{}, nullptr, nullptr, 0};
@@ -1926,7 +1926,7 @@ int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_sav
     if (have_back && (rescal || !aligned16(saved->back_rows))) return KGE_EINVAL;
     if (!have_back) {
         if (const int rc = launch_product(2, ga, plans, z, thin_groups(tab, bat), nullptr, B, f2, st)) return rc;
-        timeline_mark(bat->timeline, st, "transr_gemm_kernel<dX>");
+        timeline_mark(bat->timeline, st, z.tall ? "transr_tall_kernel<dX>" : "transr_gemm_kernel<dX>");
     } else if (f2.blocks > 0) {  // the inspector step that would have ridden with dX
         hipLaunchKernelGGL(transr_insp_step_kernel, dim3((unsigned)f2.blocks), dim3(256), lds_with(f2, 0), st, f2);
         timeline_mark(bat->timeline, st, "inspector step");

@@ -682,7 +682,7 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
     GemmArgs ga{tab->ent, tab->rel, tab->aux, x.hl, nullptr, x.tl, nullptr, x.segl, ri->num_unique, ri->unique_ids,
                 TilePlan{}, nullptr, x.rsl, nullptr, y, nullptr, nullptr, d, tab->norm_p, 0, 0, BwdSrc{}};
     if (const int rc = launch_product(3, ga, plans, s.plans, s.U_cap, nullptr, s.B, FusedInsp{}, st)) return rc;
-    timeline_mark(bat->timeline, st, "transr_gemm_kernel<list>");
+    timeline_mark(bat->timeline, st, s.plans.tall ? "transr_tall_kernel<list>" : "transr_gemm_kernel<list>");
 
     NegPairArgs pa{};
     pa.ent = tab->ent, pa.y = y, pa.pos = pos, pa.neg = neg, pa.resid = resid;
@@ -738,7 +738,7 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     GemmArgs ga{tab->ent, tab->rel, tab->aux, x.hl, nullptr, x.tl, nullptr, x.segl, ri->num_unique, ri->unique_ids,
                 TilePlan{}, ql, nullptr, nullptr, nullptr, dxl, nullptr, d, tab->norm_p, 0, 0, BwdSrc{}};
     if (const int rc = launch_product(2, ga, plans, s.plans, s.U_cap, nullptr, s.B, FusedInsp{}, st)) return rc;
-    timeline_mark(bat->timeline, st, "transr_gemm_kernel<dX>");
+    timeline_mark(bat->timeline, st, s.plans.tall ? "transr_tall_kernel<dX>" : "transr_gemm_kernel<dX>");
     DmArgs da{xl, ql, x.segl, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + l.dpart), d, ri->num_unique,
               BwdSrc{}, nullptr, nullptr, 0};
     hipLaunchKernelGGL(transr_dm_kernel, dim3((unsigned)kDmWgs), dim3(256), dm_lds_bytes(d), st, da, FusedInsp{}, SegL1Rider{});

@@ -69,3 +69,15 @@ def test_an_infinite_weight_in_the_last_row_stays_in_its_column(model, dim):
     assert torch.isinf(want).sum() == 2 and not torch.isnan(want).any()
     assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(got)].double(), want[torch.isinf(want)])
     assert not torch.isnan(got).any()
+
+
+@pytest.mark.parametrize("n_rel,dim,kw,form", [(3, 48, {}, "tall"), (900, 144, {}, "gemm"), (3, 48, dict(chunk=32, n_neg=4), "tall"),
+                                               (900, 144, dict(chunk=32, n_neg=4), "gemm")])
+def test_the_timeline_names_the_form_that_ran(n_rel, dim, kw, form):
+    from cuke_amd.kge import TrainStep
+    w = synth.custom_workload("TransR", n_ent=300, n_rel=n_rel, dim=dim, batch=256, sigma=0.2, seed=1, **kw)
+    m, ix = gpu_model(w)
+    st = TrainStep(m, ix["h"], ix["r"], ix["t"], ix.get("neg"), w.chunk or None, back_rows=False)
+    names = [name for name, _ in st.kernel_times(2)]
+    first = "list>" if kw else "fwd>"
+    assert any(n.endswith(f"transr_{form}_kernel<{first}") for n in names) and f"transr_{form}_kernel<dX>" in names, names

@@ -597,8 +597,8 @@ struct Stage {
             const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(100);
             bool idle;
             while (!(idle = s.idle(words())) && std::chrono::steady_clock::now() < until) __builtin_ia32_pause();
-            if (!idle) idle = hipDeviceSynchronize() == hipSuccess;
-            if (idle) (void)hipHostFree(s.done);  // (a device that has failed keeps it)
+            if (!idle && hipDeviceSynchronize() == hipSuccess) idle = s.idle(words());
+            if (idle) (void)hipHostFree(s.done);  // (what a failed launch was to read is kept)
         }
     }
 };

@@ -640,7 +640,9 @@ PyObject *py_sample_batch(PyObject *, PyObject *const *args, Py_ssize_t)
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(static_cast<hipStream_t>(st), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
         NOT_HERE;  // (a replay would read what a later batch has left there)
-    Stage::Slot *slot = stage->take();
+    const auto i64 = at::TensorOptions().dtype(at::kLong).device(at::kCUDA, (c10::DeviceIndex)dev);
+    at::Tensor h = at::empty({B}, i64), r = at::empty({B}, i64), t = at::empty({B}, i64), neg = at::empty({count}, i64);
+    Stage::Slot *slot = stage->take();  // (nothing lets another thread in between here and the new mark below)
     if (!slot) NOT_HERE;
     int64_t *ids = slot->ids;
     const uint64_t rows = (uint64_t)std::min({col[0].size(), col[1].size(), col[2].size()});
@@ -651,8 +653,6 @@ PyObject *py_sample_batch(PyObject *, PyObject *const *args, Py_ssize_t)
         ids[i] = col[0].at(q), ids[B + i] = col[1].at(q), ids[2 * B + i] = col[2].at(q);
     }
     if (!inside) NOT_HERE;  // (numpy's indexing raises, or counts from the end)
-    const auto i64 = at::TensorOptions().dtype(at::kLong).device(at::kCUDA, (c10::DeviceIndex)dev);
-    at::Tensor h = at::empty({B}, i64), r = at::empty({B}, i64), t = at::empty({B}, i64), neg = at::empty({count}, i64);
     uint32_t *done = slot->done;
     const uint32_t mark = ++slot->mark;  // (taken from here on, also for a thread that comes in while the launch is under way)
     const int rc = nogil([&] {

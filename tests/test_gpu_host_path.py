@@ -454,3 +454,36 @@ def test_empty_batches():
     assert kge.inspect(e, 9).num_unique == 0
     loss, dpos, dneg = kge.margin_loss(torch.zeros(0, device="cuda"), torch.zeros(0, 5, device="cuda"), 1.0)
     assert loss.item() == 0.0 and dpos.shape == (0,) and dneg.shape == (0, 5)
+
+
+@pytest.mark.parametrize("model,kw", [("DistMult", dict(chunk=32, n_neg=8)), ("TransR", dict())])
+def test_a_staged_set_is_not_rewritten_before_what_follows_its_step(model, kw):
+    """The ring of next_inputs(): index tensors refilled on a stream of their own, the next batches staged while the device is
+    still busy behind a step; what the caller has put there (an optimizer step, say) reads that step's inspection."""
+    m, batches, make = _two_batches(model, **kw)
+    batches = batches[0], [x // 2 if x is not None and i != 1 else x for i, x in enumerate(batches[0])]  # (other entities)
+    st, copies = make(batches[0]), torch.cuda.Stream()
+    busy = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    want = [torch.unique(torch.cat([x for x in (b[0], b[2], b[3]) if x is not None])) for b in batches]
+    read = []
+
+    def stage(k):
+        tensors = st.next_inputs(copies)
+        with torch.cuda.stream(copies):
+            for x, y in zip(tensors, batches[k % 2]):
+                if x is not None:
+                    x.copy_(y)
+            ready = copies.record_event()
+        st.stage(ready)
+
+    stage(0)
+    for k in range(6):
+        stage(k + 1)
+        st.run(pipeline=True)
+        for _ in range(10):  # (milliseconds)
+            busy.zero_()
+        read.append((st.ent_insp.unique_ids.clone(), st.ent_insp.num_unique_dev.clone()))
+    torch.cuda.synchronize()
+    for k, (ids, n) in enumerate(read):
+        assert torch.equal(ids[:int(n)], want[k % 2]), k

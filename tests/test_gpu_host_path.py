@@ -1,5 +1,7 @@
 """The native host path: what it takes gives the results of the general path, and what it does not take falls
 through to it (other integer widths, non-contiguous inputs, host-side batches)."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -403,6 +405,7 @@ def test_sampler_keeps_nothing_on_the_device_and_waits_for_nothing():
     device memory, and neither a batch nor the end of an epoch (5 batches) synchronises."""
     triples, s = _sampler(shuffle=False)
     next(s), torch.cuda.synchronize()
+    gc.collect()  # (tensors that an earlier test's frames hold in a cycle would otherwise go while the batches are drawn)
     before = torch.cuda.memory_allocated()
     busy = torch.empty(1 << 28, dtype=torch.uint8, device="cuda")
     streams = [torch.cuda.Stream() for _ in range(3)]

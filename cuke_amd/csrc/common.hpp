@@ -36,6 +36,16 @@ __device__ __forceinline__ int wave_sum_i(int v)
     return v;
 }
 
+// Four floats at any 4-byte address.  global_load / store_dwordx4 take dword-aligned addresses, so rows of every width
+// (a row of 150 floats starts 8 bytes off a quad boundary every second time) move 128 bits at a time.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 load_quad(const float *p)
+{
+    const f4u v = *reinterpret_cast<const f4u *>(p);
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ void store_quad(float *p, float4 v) { *reinterpret_cast<f4u *>(p) = f4u{v.x, v.y, v.z, v.w}; }
+
 // V consecutive floats moved with one instruction when V == 4 (global_load_dwordx4).
 template <int V>
 struct Vec;
@@ -44,12 +54,17 @@ struct Vec<4> {
     float v[4];
     __device__ __forceinline__ static Vec load(const float *p)
     {
-        const float4 q = *reinterpret_cast<const float4 *>(p);
+        const float4 q = load_quad(p);
         return Vec{{q.x, q.y, q.z, q.w}};
     }
-    __device__ __forceinline__ void store(float *p) const
+    __device__ __forceinline__ void store(float *p) const { store_quad(p, make_float4(v[0], v[1], v[2], v[3])); }
+    // the elements from `skip` on
+    __device__ __forceinline__ void store_from(float *p, int skip) const
     {
-        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+        if (skip == 0) return store(p);
+#pragma unroll
+        for (int e = 1; e < 4; ++e)
+            if (e >= skip) p[e] = v[e];
     }
 };
 template <>
@@ -57,7 +72,19 @@ struct Vec<1> {
     float v[1];
     __device__ __forceinline__ static Vec load(const float *p) { return Vec{{*p}}; }
     __device__ __forceinline__ void store(float *p) const { *p = v[0]; }
+    __device__ __forceinline__ void store_from(float *p, int) const { *p = v[0]; }
 };
+
+// A row of n floats walked V at a time by lanes that start at column j.  With V == 4 the row has at least four floats
+// and its last piece is moved back to end with the row: it starts at `at`, and the first `skip` of its elements belong to
+// the piece before it as well.  An element-wise result may be stored twice (same bits); a sum leaves them out.
+template <int V>
+struct RowPiece {
+    int at, skip;
+    __device__ __forceinline__ RowPiece(int j, int n) : at(V == 4 && j > n - V ? n - V : j), skip(j - at) {}
+};
+// whether rows (row segments) of n floats can be walked four floats at a time
+__host__ __device__ inline bool quad_row(int64_t n) { return n >= 4; }
 
 __device__ __forceinline__ float sgn(float x) { return x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f); }
 

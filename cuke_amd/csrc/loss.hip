@@ -9,7 +9,7 @@ namespace kge {
 
 constexpr int kLossWaves = 4;
 
-// Bound by its two passes over the [B, N] scores (read, gradient written), 128 bits per lane where rows allow it.
+// Bound by its two passes over the [B, N] scores (read, gradient written), 128 bits per lane from four scores a row on.
 // A workgroup strides over the rows and leaves ONE partial loss: with one per row the single workgroup that adds them
 // up walked 16384 to 30000 doubles, 18 to 30 us; over at most kLossBlocks partials it is 2 us.
 constexpr int kLossBlocks = 1024;
@@ -26,18 +26,21 @@ __global__ __launch_bounds__(kLossWaves *kWave) void margin_rows_kernel(
         const float p = pos[b];
         float sum = 0.0f;
         int cnt = 0;
-        for (int64_t k = lane * V; k < N; k += kWave * V) {
+        for (int64_t k0 = lane * V; k0 < N; k0 += kWave * V) {
+            const int64_t k = V == 4 && k0 > N - V ? N - V : k0;  // the row's last piece ends with it
+            const int skip = (int)(k0 - k);
             const Vec<V> s = Vec<V>::load(neg + b * N + k);
             Vec<V> g;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 const float v = margin - sign * (p - s.v[e]);
                 const bool on = v > 0.0f;
-                sum += on ? v : 0.0f;
-                cnt += on ? 1 : 0;
+                const bool count = on && e >= skip;
+                sum += count ? v : 0.0f;
+                cnt += count ? 1 : 0;
                 g.v[e] = on ? sign * inv : 0.0f;
             }
-            if (dneg) g.store(dneg + b * N + k);
+            if (dneg) g.store_from(dneg + b * N + k, skip);
         }
         sum = wave_sum(sum);
         cnt = wave_sum_i(cnt);
@@ -129,7 +132,7 @@ int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n
     const int blocks = (int)(want < kLossBlocks ? want : kLossBlocks);  // (one partial each: never more than the workspace's `batch`)
     if (batch > 0) {
         const dim3 grid((unsigned)blocks), block(kLossWaves * kWave);
-        if (n_neg % 4 == 0 && aligned16(neg) && (!dneg || aligned16(dneg)))
+        if (quad_row(n_neg))
             hipLaunchKernelGGL(margin_rows_kernel<4>, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
         else
             hipLaunchKernelGGL(margin_rows_kernel<1>, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);

@@ -20,9 +20,10 @@ __global__ __launch_bounds__(256) void sparse_step_kernel(float *table, float *s
     if constexpr (ADAGRAD) {
         float sq = 0.0f;
         for (int j = lane * V; j < d; j += kWave * V) {
-            const Vec<V> gv = Vec<V>::load(g + j);
+            const RowPiece<V> at(j, d);
+            const Vec<V> gv = Vec<V>::load(g + at.at);
 #pragma unroll
-            for (int e = 0; e < V; ++e) sq += gv.v[e] * gv.v[e];
+            for (int e = 0; e < V; ++e) sq += e >= at.skip ? gv.v[e] * gv.v[e] : 0.0f;
         }
         sq = wave_sum(sq);
         const float s = state[id] + sq / (float)d;
@@ -30,11 +31,12 @@ __global__ __launch_bounds__(256) void sparse_step_kernel(float *table, float *s
         scale = lr / (sqrtf(s) + eps);
     }
     for (int j = lane * V; j < d; j += kWave * V) {
-        const Vec<V> gv = Vec<V>::load(g + j);
-        Vec<V> wv = Vec<V>::load(w + j);
+        const RowPiece<V> at(j, d);
+        const Vec<V> gv = Vec<V>::load(g + at.at);
+        Vec<V> wv = Vec<V>::load(w + at.at);
 #pragma unroll
         for (int e = 0; e < V; ++e) wv.v[e] -= scale * gv.v[e];
-        wv.store(w + j);
+        wv.store_from(w + at.at, at.skip);  // (in place: the skipped elements may have been updated already)
     }
 }
 
@@ -157,7 +159,7 @@ static int launch_step(float *table, float *state, int64_t dim, const int64_t *i
         return KGE_OK;
     }
     const dim3 grid((unsigned)ceil_div(capacity, 4)), block(256);
-    if (dim % 4 == 0 && aligned16(table) && aligned16(rows))
+    if (quad_row(dim))
         hipLaunchKernelGGL((sparse_step_kernel<ADAGRAD, 4>), grid, block, 0, st, table, state, (int)dim, ids, num_unique,
                            rows, lr, eps);
     else

@@ -117,7 +117,7 @@ __host__ __device__ inline int narrow_cols(int klen)
 // over the 64-column tiles.  A 64-column tile there would keep 12 of its 16 column lanes idle;
 // instead the column lanes are regrouped as 4 column groups x 4 owner sub-tiles and every thread
 // owns one row (RO_ = 1) of its sub-tile, so all 256 threads work on the 64 owners x 16 columns.
-template <int MODEL, int P, bool OWNER_POS, int RO, bool MF, bool NARROW = false>
+template <int MODEL, int P, bool OWNER_POS, int RO, bool MF, bool VEC, bool VECN, bool NARROW = false>
 __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float *smem, int col_base = 0)
 {
     static_assert(!(NARROW && MF), "the matrix-core loop has no narrow form");
@@ -156,30 +156,42 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     // imaginary ones, [32 x, 32 x + 32) and half + [32 x, 32 x + 32), so that one workgroup holds both parts of
     // every complex element it owns (the positive chain in the epilogue needs them together, and a staging
     // step asks for half as many distinct row pieces of h and r)
-    const bool pair = MODEL == KGE_COMPLEX && MF && !NARROW && a.vec != 0;
+    constexpr bool pair = MODEL == KGE_COMPLEX && MF && !NARROW && VEC;
     const int wide_tiles_x = pair ? (half + 31) / 32
                                   : ((kHasNarrow && narrow_cols(klen)) ? klen / kTI : (klen + kTI - 1) / kTI);
     if (!xcd_tile(lid, NARROW ? 1 : wide_tiles_x, (n_own + TO - 1) / TO, a.n_chunks, c, tile_y, tile_x)) return;
-    // local column lc (a multiple of 4 in 0..63) of the tile -> column of the row; and `lim` where the tile has
-    // that column, else 0 (a paired tile's last columns may lie beyond the half row)
-    auto gcol = [&](int lc) { return pair ? (lc < 32 ? tile_x * 32 + lc : half + tile_x * 32 + (lc - 32)) : (NARROW ? col_base : tile_x * kTI) + lc; };
-    auto climit = [&](int lc, int lim) { return (pair && tile_x * 32 + (lc & 31) >= half) ? 0 : lim; };
+    // The quad of columns that local column lc (a multiple of 4 in 0..63) of the tile stands for starts at gcol(lc): a quad that
+    // would run past its segment's end (a half of a paired tile, else the row) is moved back to end with it.  Its first
+    // gskip(lc) elements belong to another quad, which stores them (4 or more: all of them).
+    const int end = pair ? half : klen;
+    auto lcol = [&](int lc) { return pair ? tile_x * 32 + (lc & 31) : (NARROW ? col_base : tile_x * kTI) + lc; };
+    auto gcol = [&](int lc) {
+        const int j = VEC ? min(lcol(lc), end - 4) : lcol(lc);
+        return pair && lc >= 32 ? half + j : j;
+    };
+    auto gskip = [&](int lc) { return VEC ? lcol(lc) - min(lcol(lc), end - 4) : 0; };
+    auto put = [&](float *row, int lc, float4 v) {
+        const int j = gcol(lc), skip = gskip(lc);
+        if (VEC && skip == 0) return store_quad(row + j, v);
+        const int lim = VEC ? j + 4 : klen;
+        if (skip <= 0 && j + 0 < lim) row[j + 0] = v.x;
+        if (skip <= 1 && j + 1 < lim) row[j + 1] = v.y;
+        if (skip <= 2 && j + 2 < lim) row[j + 2] = v.z;
+        if (skip <= 3 && j + 3 < lim) row[j + 3] = v.w;
+    };
     const int scol = gcol(tx * 4);                                           // columns this thread stages
     const int ctx = NARROW ? (tx & 3) : tx;                                  // column lane it computes
     const int col = gcol(ctx * 4);                                           // columns it owns
     const int ot0 = tile_y * TO;
     auto orow = [&](int o) { return NARROW ? (tx >> 2) * 16 + ty : ty * RO_ + o; };  // owner row inside the tile
-    const bool vec = a.vec != 0;
 
     // ---- owners: registers -----------------------------------------------------------
     float4 own[NPO][RO_];
     float alo[RO_];
-    auto load_owners = [&](auto vtag) {
-    constexpr bool VEC = decltype(vtag)::value;
 #pragma unroll
     for (int o = 0; o < RO_; ++o) {
         const int ol = ot0 + orow(o);
-        const int lim = climit(ctx * 4, ol < n_own ? klen : 0);
+        const int lim = ol < n_own ? klen : 0;
         const int oc = ol < n_own ? ol : n_own - 1;
         alo[o] = 0.0f;
         if constexpr (OWNER_POS) {
@@ -189,8 +201,8 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             float4 q0 = zero4(), q1 = zero4();
             if constexpr (!kDot)
                 load_query<MODEL, VEC>(a.ent + a.h[b] * (int64_t)d, a.rel + rid * (int64_t)a.rel_dim,
-                                  kTH ? a.aux + rid * (int64_t)d : nullptr, alo[o], col, lim, half, q0,
-                                  q1, kRot ? a.query + b * (int64_t)d : nullptr, a.rsign);
+                                       kTH ? a.aux + rid * (int64_t)d : nullptr, kRot ? a.query + b * (int64_t)d : nullptr, alo[o],
+                                       col, lim, half, a.rsign, q0, q1);
             own[0][o] = q0;
             if constexpr (NPO == 2) own[1][o] = q1;
         } else {
@@ -203,9 +215,6 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             for (int q = 0; q < NPO; ++q) own[q][o] = scale4(own[q][o], kSgnScale);
         }
     }
-    };
-    if (vec) load_owners(std::true_type{});
-    else load_owners(std::false_type{});
 
     float4 acc[NOUT][RO_];
 #pragma unroll
@@ -219,11 +228,10 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     // receives D[i = 4 (l / 16) + v][j].  Inside 16 loopers the MFMA step s pairs lane group
     // g = l / 16 with looper 4 g + s; a lane's 128-bit read of four consecutive columns of that
     // looper's row feeds four MFMAs, so MFMA e owns the columns 4 j + e.  A wave owns 16 owners and
-    // all 64 columns (64-owner tiles), or 16 owners and the columns 4 j + {0,1} / {2,3} (32-owner tiles).
-    constexpr int OB = TO / 16, EW = OB;  // owner blocks; MFMAs (columns per lane) per wave
-    static_assert(!kMf || OB == 4 || OB == 2, "MFMA tiling written for 32- and 64-owner tiles");
-    const int mlane = tid & 63, mwave = tid >> 6, fj = mlane & 15, fg = mlane >> 4;
-    const int ob = mwave % OB, e0 = (mwave / OB) * EW;
+    // all 64 columns.
+    constexpr int EW = 4;  // MFMAs (columns per lane) per wave
+    static_assert(!kMf || TO == 64, "a wave per 16 of 64 owners");
+    const int mlane = tid & 63, ob = tid >> 6, fj = mlane & 15, fg = mlane >> 4;
     v4f macc[EW];
 #pragma unroll
     for (int e = 0; e < EW; ++e) macc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -258,13 +266,15 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
         }
     };
 
-    auto load_rows_v = [&](auto vtag, auto ntag, int l0) {
-        constexpr bool VEC = decltype(vtag)::value, VECN = decltype(ntag)::value;
+    // kShift: a quad of coefficients may straddle the end of its row of N and is then read where it ends with the row and moved
+    // into place.  (The whole step twice: a branch between its loads would make the first of them waited for.)
+    auto load_step = [&](auto stag, int l0) {
+        constexpr bool kShift = decltype(stag)::value;
         // looper rows: thread stages rows ty + 16*s, columns col..col+3
 #pragma unroll
         for (int s = 0; s < SL; ++s) {
             const int ll = l0 + ty + 16 * s;
-            const int lim = climit(tx * 4, ll < n_loop ? klen : 0);
+            const int lim = ll < n_loop ? klen : 0;
             if constexpr (OWNER_POS) {
                 const float *pt = a.ent + li0[s] * (int64_t)d;
                 rraw[s][0] = ld4_raw<VEC>(pt, scol, lim);
@@ -277,11 +287,15 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                 if constexpr (kDefer) {
                     load_query_raw<MODEL, VEC>(ph, pr, pw, pq, scol, lim, half, rraw[s]);
                 } else {
-                    load_query<MODEL, VEC>(ph, pr, pw, lal[s], scol, lim, half, rraw[s][0], rraw[s][NRAW - 1], pq, a.rsign);
+                    load_query<MODEL, VEC>(ph, pr, pw, pq, lal[s], scol, lim, half, a.rsign, rraw[s][0], rraw[s][NRAW - 1]);
                 }
             }
         }
         // coefficients of the (TO owners x kKL loopers) block, read along k (contiguous)
+        auto ld = [](const float *p, int kl, int lim) {
+            if constexpr (kShift) return shift_quad(ld4_raw<true>(p, kl, lim), kl + 4 - lim);
+            else return ld4_whole<VECN>(p, kl, lim);
+        };
 #pragma unroll
         for (int s = 0; s < CPT; ++s) {
             const int f = tid + 256 * s;  // float4 index inside the block
@@ -298,13 +312,13 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             }
             const int lim = inside ? a.N : 0;
             const int64_t off = ((int64_t)c * a.C + (inside ? bl : 0)) * a.N;
-            craw[0][s] = ld4<VECN>(a.dneg + off, kl, lim);
-            if constexpr (kL2 && !kTH) craw[1][s] = ld4<VECN>(a.sneg + off, kl, lim);
+            craw[0][s] = ld(a.dneg + off, kl, lim);
+            if constexpr (kL2 && !kTH) craw[1][s] = ld(a.sneg + off, kl, lim);
             if constexpr (kTH) {
-                craw[1][s] = ld4<VECN>(a.side_neg + off, kl, lim);
-                craw[2][s] = ld4<VECN>(a.side_neg + a.plane + off, kl, lim);
+                craw[1][s] = ld(a.side_neg + off, kl, lim);
+                craw[2][s] = ld(a.side_neg + a.plane + off, kl, lim);
                 if constexpr (kL2) {  // fold the norm in now (TransH does not defer)
-                    const float4 sc = ld4<VECN>(a.sneg + off, kl, lim);
+                    const float4 sc = ld(a.sneg + off, kl, lim);
                     float4 &g = craw[0][s];
                     craw[2][s] = mul4(g, craw[2][s]);
                     g.x = sc.x > 0.0f ? g.x / sc.x : 0.0f;
@@ -317,19 +331,14 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             }
         }
     };
-
-    auto load_rows = [&](int l0) {  // one uniform dispatch per step, no branch per load
-        if (vec) {
-            if (a.vecn) load_rows_v(std::true_type{}, std::true_type{}, l0);
-            else load_rows_v(std::true_type{}, std::false_type{}, l0);
-        } else {
-            if (a.vecn) load_rows_v(std::false_type{}, std::true_type{}, l0);
-            else load_rows_v(std::false_type{}, std::false_type{}, l0);
+    auto load_rows = [&](int l0) {
+        if constexpr (VECN) {
+            if ((a.N & 3) && (OWNER_POS ? l0 + kKL : ot0 + TO) > a.N) return load_step(std::true_type{}, l0);
         }
+        load_step(std::false_type{}, l0);
     };
 
-    auto store_step_v = [&](auto vtag, int l0) {
-        constexpr bool VEC = decltype(vtag)::value;
+    auto store_step = [&](int l0) {
 #pragma unroll
         for (int s = 0; s < SL; ++s) {
             float4 q0, q1 = zero4();
@@ -338,7 +347,7 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                 if constexpr (NPL == 2) q1 = rraw[s][NRAW - 1];
             } else {
                 const int ll = l0 + ty + 16 * s;
-                combine_query<MODEL, VEC>(rraw[s], 0.0f, scol, climit(tx * 4, ll < n_loop ? klen : 0), half, a.rsign, q0, q1);
+                combine_query<MODEL, VEC>(rraw[s], 0.0f, scol, ll < n_loop ? klen : 0, half, a.rsign, q0, q1);
             }
             if constexpr (kSc) q0 = scale4(q0, kSgnScale), q1 = scale4(q1, kSgnScale);
             *reinterpret_cast<float4 *>(&sL[0][ty + 16 * s][tx * 4]) = q0;
@@ -375,10 +384,6 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             }
         }
     };
-    auto store_step = [&](int l0) {
-        if (vec) store_step_v(std::true_type{}, l0);
-        else store_step_v(std::false_type{}, l0);
-    };
 
     const int nstep = (n_loop + kKL - 1) / kKL;
     load_idx(0);
@@ -402,14 +407,8 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                 for (int ms = 0; ms < 4; ++ms) {
                     const int l = 16 * q + 4 * fg + ms;
                     const float av = sG[0][l][ob * 16 + fj];
-                    float bv[EW];
-                    if constexpr (EW == 4) {
-                        const float4 b4 = *reinterpret_cast<const float4 *>(&sL[0][l][4 * fj]);
-                        bv[0] = b4.x, bv[1] = b4.y, bv[2] = b4.z, bv[3] = b4.w;
-                    } else {
-                        const float2 b2 = *reinterpret_cast<const float2 *>(&sL[0][l][4 * fj + e0]);
-                        bv[0] = b2.x, bv[1] = b2.y;
-                    }
+                    const float4 b4 = *reinterpret_cast<const float4 *>(&sL[0][l][4 * fj]);
+                    const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
                     for (int e = 0; e < EW; ++e)
                         macc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], macc[e], 0, 0, 0);
@@ -490,12 +489,11 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     }
 
     if constexpr (kMf) {
-        if constexpr (OWNER_POS && EW == 4 && (MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX)) {
+        if constexpr (OWNER_POS && (MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX)) {
             if (a.chain) {  // uniform: the positive chain right here, from the sums in the accumulators
                 const int lc = 4 * fj;
                 const int c0 = gcol(lc);
-                const bool colok = climit(lc, klen) != 0 && c0 + 4 <= d;
-                const int cc = colok ? c0 : 0;  // clamped: unconditional loads
+                auto put4 = [&](float *row, const float (&v)[4]) { put(row, lc, make_float4(v[0], v[1], v[2], v[3])); };
                 int64_t idk[4], ido[4], idr[4];
                 float gp[4];
                 bool rowok[4];
@@ -511,9 +509,9 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                     float4 xk[4], xo[4], xr[4];
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
-                        xk[v] = *reinterpret_cast<const float4 *>(a.ent + idk[v] * (int64_t)d + cc);
-                        xo[v] = *reinterpret_cast<const float4 *>(a.ent + ido[v] * (int64_t)d + cc);
-                        xr[v] = *reinterpret_cast<const float4 *>(a.rel + idr[v] * (int64_t)a.rel_dim + cc);
+                        xk[v] = load_quad(a.ent + idk[v] * (int64_t)d + c0);
+                        xo[v] = load_quad(a.ent + ido[v] * (int64_t)d + c0);
+                        xr[v] = load_quad(a.rel + idr[v] * (int64_t)a.rel_dim + c0);
                     }
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
@@ -522,29 +520,28 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                         float dk[4], dr[4], dother[4];
 #pragma unroll
                         for (int e = 0; e < 4; ++e) distmult_chain(gp[v], k4[e], o4[e], r4[e], macc[e][v], dk[e], dr[e], dother[e]);
-                        if (rowok[v] && colok) {
+                        if (rowok[v]) {
                             const int64_t b = (int64_t)c * a.C + ot0 + ob * 16 + 4 * fg + v;
-                            *reinterpret_cast<float4 *>(a.occ_k + b * (int64_t)d + c0) = make_float4(dk[0], dk[1], dk[2], dk[3]);
-                            *reinterpret_cast<float4 *>(a.occ_r + b * (int64_t)a.rel_dim + c0) = make_float4(dr[0], dr[1], dr[2], dr[3]);
-                            *reinterpret_cast<float4 *>(a.occ_o + b * (int64_t)d + c0) = make_float4(dother[0], dother[1], dother[2], dother[3]);
+                            put4(a.occ_k + b * (int64_t)d, dk);
+                            put4(a.occ_r + b * (int64_t)a.rel_dim, dr);
+                            put4(a.occ_o + b * (int64_t)d, dother);
                         }
                     }
                 } else {
                     // lanes fj < 8 hold the real parts of complex elements idx .. idx + 3, lanes fj + 8 the imaginary
                     // parts of the same elements: each takes the other part from its partner and writes its own side
                     const bool is_re = fj < 8;
-                    const int idx = tile_x * 32 + 4 * (fj & 7);
-                    const int ci = colok ? idx : 0;
+                    const int idx = is_re ? c0 : c0 - half;
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         float Gm[4], Gp[4];
 #pragma unroll
                         for (int e = 0; e < 4; ++e) Gm[e] = macc[e][v], Gp[e] = __shfl_xor(macc[e][v], 8, kWave);
-                        const float *pk = a.ent + idk[v] * (int64_t)d + ci, *po = a.ent + ido[v] * (int64_t)d + ci;
-                        const float *pr = a.rel + idr[v] * (int64_t)a.rel_dim + ci;
-                        const float4 kr4 = *reinterpret_cast<const float4 *>(pk), ki4 = *reinterpret_cast<const float4 *>(pk + half);
-                        const float4 or4 = *reinterpret_cast<const float4 *>(po), oi4 = *reinterpret_cast<const float4 *>(po + half);
-                        const float4 qr4 = *reinterpret_cast<const float4 *>(pr), qi4 = *reinterpret_cast<const float4 *>(pr + half);
+                        const float *pk = a.ent + idk[v] * (int64_t)d, *po = a.ent + ido[v] * (int64_t)d;
+                        const float *pr = a.rel + idr[v] * (int64_t)a.rel_dim;
+                        const float4 kr4 = load_quad(pk + idx), ki4 = load_quad(pk + half + idx);
+                        const float4 or4 = load_quad(po + idx), oi4 = load_quad(po + half + idx);
+                        const float4 qr4 = load_quad(pr + idx), qi4 = load_quad(pr + half + idx);
                         const float kr[4] = {kr4.x, kr4.y, kr4.z, kr4.w}, ki[4] = {ki4.x, ki4.y, ki4.z, ki4.w};
                         const float orr[4] = {or4.x, or4.y, or4.z, or4.w}, oi[4] = {oi4.x, oi4.y, oi4.z, oi4.w};
                         const float qr[4] = {qr4.x, qr4.y, qr4.z, qr4.w}, qi[4] = {qi4.x, qi4.y, qi4.z, qi4.w};
@@ -557,11 +554,11 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                             else complex_chain<false>(gp[v], kr[e], ki[e], orr[e], oi[e], qr[e], qi[e], Gr, Gi, dkr, dki, drr, dri, dor, doi);
                             dk[e] = is_re ? dkr : dki, dr[e] = is_re ? drr : dri, dother[e] = is_re ? dor : doi;
                         }
-                        if (rowok[v] && colok) {
+                        if (rowok[v]) {
                             const int64_t b = (int64_t)c * a.C + ot0 + ob * 16 + 4 * fg + v;
-                            *reinterpret_cast<float4 *>(a.occ_k + b * (int64_t)d + c0) = make_float4(dk[0], dk[1], dk[2], dk[3]);
-                            *reinterpret_cast<float4 *>(a.occ_r + b * (int64_t)a.rel_dim + c0) = make_float4(dr[0], dr[1], dr[2], dr[3]);
-                            *reinterpret_cast<float4 *>(a.occ_o + b * (int64_t)d + c0) = make_float4(dother[0], dother[1], dother[2], dother[3]);
+                            put4(a.occ_k + b * (int64_t)d, dk);
+                            put4(a.occ_r + b * (int64_t)a.rel_dim, dr);
+                            put4(a.occ_o + b * (int64_t)d, dother);
                         }
                     }
                 }
@@ -574,18 +571,7 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             if (ol >= n_own) continue;
             const int64_t row = OWNER_POS ? (int64_t)c * a.C + ol : (int64_t)c * a.N + ol;
             float *dst = a.out0 + row * (int64_t)d;
-            const int c0 = gcol(4 * fj + e0);
-            if (pair && climit(4 * fj + e0, klen) == 0) continue;
-            if (vec && c0 + EW <= klen) {  // rows 16-byte aligned and d % 4 == 0: whole group inside
-                if constexpr (EW == 4)
-                    *reinterpret_cast<float4 *>(dst + c0) = make_float4(macc[0][v], macc[1][v], macc[2][v], macc[3][v]);
-                else
-                    *reinterpret_cast<float2 *>(dst + c0) = make_float2(macc[0][v], macc[1][v]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < EW; ++e)
-                    if (c0 + e < klen) dst[c0 + e] = macc[e][v];
-            }
+            put(dst, 4 * fj, make_float4(macc[0][v], macc[1][v], macc[2][v], macc[3][v]));
         }
         return;
     }
@@ -595,9 +581,9 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
         if (ol >= n_own) continue;
         const int64_t row = OWNER_POS ? (int64_t)c * a.C + ol : (int64_t)c * a.N + ol;
         float *dst = a.out0 + row * (int64_t)d;
-        st4(dst, col, klen, vec, acc[0][o]);
-        if constexpr (kRot) st4(dst + half, col, klen, vec, acc[1][o]);
-        if constexpr (kTH && OWNER_POS) st4(a.out1 + row * (int64_t)d, col, klen, vec, acc[1][o]);
+        put(dst, ctx * 4, acc[0][o]);
+        if constexpr (kRot) put(dst + half, ctx * 4, acc[1][o]);
+        if constexpr (kTH && OWNER_POS) put(a.out1 + row * (int64_t)d, ctx * 4, acc[1][o]);
     }
 }
 
@@ -611,7 +597,10 @@ struct TileGrid {
     int head, neg, narrow_head, narrow_neg;
 };
 
-template <int MODEL, int P, int RO, bool MF>
+// VEC / VECN: rows / coefficient rows by quads, compile-time (as run-time switches their combinations sat side by side in one
+// kernel; taking them apart paid for the overlapping last quads: 4096 x 256 DistMult step 76.5 -> 74.4 us, 1024 x 1000 RotatE
+// 138.9 -> 136.6).  30000 x 150 TransE, 200 negatives: 222 us by single floats, 204 by quads.
+template <int MODEL, int P, int RO, bool MF, bool VEC, bool VECN>
 __global__ __launch_bounds__(256, KGE_TILE_OCC) void bwd_tile_kernel(TileArgs a, float *g0, float *g1, float *occ_neg,
                                                                      TileGrid grid, FusedInsp fi)
 {
@@ -621,13 +610,13 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void bwd_tile_kernel(TileArgs a,
     int lid = (int)blockIdx.x - fi.blocks;
     if (lid < grid.head) {
         a.out0 = g0, a.out1 = g1;
-        bwd_tile_body<MODEL, P, true, RO, MF>(a, lid, smem);
+        bwd_tile_body<MODEL, P, true, RO, MF, VEC, VECN>(a, lid, smem);
         return;
     }
     lid -= grid.head;
     if (lid < grid.neg) {
         a.out0 = occ_neg, a.out1 = nullptr;
-        bwd_tile_body<MODEL, P, false, RO, MF>(a, lid, smem);
+        bwd_tile_body<MODEL, P, false, RO, MF, VEC, VECN>(a, lid, smem);
         return;
     }
     if constexpr (RO == 4 && !MF) {
@@ -636,10 +625,10 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void bwd_tile_kernel(TileArgs a,
         const int col_base = (klen / kTI) * kTI;
         if (lid < grid.narrow_head) {
             a.out0 = g0, a.out1 = g1;
-            bwd_tile_body<MODEL, P, true, RO, MF, true>(a, lid, smem, col_base);
+            bwd_tile_body<MODEL, P, true, RO, MF, VEC, VECN, true>(a, lid, smem, col_base);
         } else {
             a.out0 = occ_neg, a.out1 = nullptr;
-            bwd_tile_body<MODEL, P, false, RO, MF, true>(a, lid - grid.narrow_head, smem, col_base);
+            bwd_tile_body<MODEL, P, false, RO, MF, VEC, VECN, true>(a, lid - grid.narrow_head, smem, col_base);
         }
     }
 }
@@ -653,6 +642,17 @@ static size_t tile_lds_bytes(const FusedInsp &fi)
     const size_t own = sizeof(float) * kFloats;
     return fi.blocks > 0 && (size_t)fi.lds_bytes > own ? (size_t)fi.lds_bytes : own;
 }
+
+// the form of the kernel that the widths allow
+#define LAUNCH_TILE(RO_, MF_, GRID, ...)                                                                                         \
+    do {                                                                                                                         \
+        if (a.vec && a.vecn)                                                                                                     \
+            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, true, true>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi);   \
+        else if (a.vec)                                                                                                          \
+            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, true, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi);  \
+        else                                                                                                                     \
+            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, false, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi); \
+    } while (0)
 
 template <int MODEL, int P>
 static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_t n_chunks, bool dot_valu,
@@ -669,12 +669,12 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
         // matrix-core inner loop (KGE_PAIR_SUMS_VALU keeps the vector-ALU loop): a wave gets all 64
         // columns of its 16 owners with 64-owner tiles, which win at every size
         if (!dot_valu) {
-            // (ComplEx with 128-bit rows: column tiles pair 32 real with the matching 32 imaginary columns)
+            // (ComplEx by quads: column tiles pair 32 real with the matching 32 imaginary columns)
             const int64_t gxm = (MODEL == KGE_COMPLEX && a.vec) ? ceil_div(a.d / 2, 32) : gx;
             const unsigned gh = xcd_grid(gxm, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxm, ceil_div(a.N, 64), n_chunks);
             const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
-            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, 4, true>), dim3(gh + gn + fi.blocks), dim3(256), lds, st, a,
-                               g0, g1, occ_neg, TileGrid{(int)gh, (int)gn, 0, 0}, fi);
+            const TileGrid tg{(int)gh, (int)gn, 0, 0};
+            LAUNCH_TILE(4, true, dim3(gh + gn + fi.blocks), tg);
             KGE_CHECK_LAUNCH();
             return KGE_OK;
         }
@@ -684,20 +684,20 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
         const unsigned nh = narrow ? xcd_grid(1, ceil_div(a.C, 64), n_chunks) : 0;
         const unsigned nn = narrow ? xcd_grid(1, ceil_div(a.N, 64), n_chunks) : 0;
         const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
-        hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, 4, false>), dim3(gh + gn + nh + nn + fi.blocks), dim3(256), lds, st,
-                           a, g0, g1, occ_neg, TileGrid{(int)gh, (int)gn, (int)nh, (int)nn}, fi);
+        const TileGrid tg{(int)gh, (int)gn, (int)nh, (int)nn};
+        LAUNCH_TILE(4, false, dim3(gh + gn + nh + nn + fi.blocks), tg);
     } else if (big >= 512) {
         const unsigned gh = xcd_grid(gx, ceil_div(a.C, 32), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 32), n_chunks);
         const size_t lds = tile_lds_bytes<MODEL, 2>(fi);
-        hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, 2, false>), dim3(gh + gn + fi.blocks), dim3(256), lds, st, a, g0, g1,
-                           occ_neg, TileGrid{(int)gh, (int)gn, 0, 0}, fi);
+        const TileGrid tg{(int)gh, (int)gn, 0, 0};
+        LAUNCH_TILE(2, false, dim3(gh + gn + fi.blocks), tg);
     } else {
         // a batch this small leaves one or two 32-owner workgroups per CU: 16-owner tiles double the
         // waves that hide each other's latency
         const unsigned gh = xcd_grid(gx, ceil_div(a.C, 16), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 16), n_chunks);
         const size_t lds = tile_lds_bytes<MODEL, 1>(fi);
-        hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, 1, false>), dim3(gh + gn + fi.blocks), dim3(256), lds, st, a, g0, g1,
-                           occ_neg, TileGrid{(int)gh, (int)gn, 0, 0}, fi);
+        const TileGrid tg{(int)gh, (int)gn, 0, 0};
+        LAUNCH_TILE(1, false, dim3(gh + gn + fi.blocks), tg);
     }
     KGE_CHECK_LAUNCH();
     return KGE_OK;
@@ -758,7 +758,8 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
     }
 
     if constexpr (MODEL == KGE_TRANSE) {
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const int j = RowPiece<V>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
             const Vec<V> G = ldz<V>(g0, j);
             Vec<V> dh, dt;
@@ -780,7 +781,8 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             dh.store(oh + j), dt.store(ot + j);
         }
     } else if constexpr (MODEL == KGE_DISTMULT) {
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const int j = RowPiece<V>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
             const Vec<V> G = ldz<V>(g0, j);
             Vec<V> dh, dr, dt;
@@ -800,7 +802,8 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             for (int64_t k = lane; k < a.N; k += kWave) S += a.dneg[b * a.N + k];
             S = wave_sum(S);
         }
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const int j = RowPiece<V>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
             const Vec<V> G = ldz<V>(g0, j);
             Vec<V> dh, dr, dt;
@@ -820,7 +823,8 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             dh.store(oh + j), dr.store(orr + j), dt.store(ot + j);
         }
     } else if constexpr (MODEL == KGE_COMPLEX) {
-        for (int j = lane * V; j < half; j += kWave * V) {
+        for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
+            const int j = RowPiece<V>(j0, half).at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> qr = Vec<V>::load(rr + j), qi = Vec<V>::load(rr + half + j);
@@ -840,7 +844,8 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             dtr.store(ot + j), dti.store(ot + half + j);
         }
     } else if constexpr (MODEL == KGE_ROTATE) {
-        for (int j = lane * V; j < half; j += kWave * V) {
+        for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
+            const int j = RowPiece<V>(j0, half).at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> th = Vec<V>::load(rr + j);
@@ -880,14 +885,18 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         const float *w = a.aux + rid * (int64_t)d;
         float *ow = a.occ_w + b * (int64_t)d;
         float sd = 0.0f;
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vw = Vec<V>::load(w + j);
 #pragma unroll
-            for (int e = 0; e < V; ++e) sd += vw.v[e] * (vh.v[e] - vt.v[e]);
+            for (int e = 0; e < V; ++e) sd += e >= at.skip ? vw.v[e] * (vh.v[e] - vt.v[e]) : 0.0f;
         }
         sd = wave_sum(sd);
         float qw = 0.0f, gw = 0.0f;  // q_pos . w and G_q . w
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j),
                          vw = Vec<V>::load(w + j);
             const Vec<V> G = ldz<V>(g0, j);
@@ -895,13 +904,14 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             for (int e = 0; e < V; ++e) {
                 const float u = ((vh.v[e] - vt.v[e]) + vr.v[e]) - sd * vw.v[e];
                 const float q = gs * (P == 1 ? sgn(u) : u);
-                qw += q * vw.v[e];
-                gw += G.v[e] * vw.v[e];
+                qw += e >= at.skip ? q * vw.v[e] : 0.0f;
+                gw += e >= at.skip ? G.v[e] * vw.v[e] : 0.0f;
             }
         }
         qw = wave_sum(qw);
         gw = wave_sum(gw);
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const int j = RowPiece<V>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j),
                          vw = Vec<V>::load(w + j);
             const Vec<V> G = ldz<V>(g0, j), Gw = ldz<V>(g1, j);
@@ -991,7 +1001,7 @@ int launch_rescal_neg_tiles(const kge_tables *tab, const kge_batch *bat, const f
 {
     const int64_t B = bat->batch, d = tab->dim, n_chunks = B / bat->chunk;
     if (n_chunks >= (1 << 24)) return KGE_ESHAPE;
-    const bool vec = rows_vectorizable(tab), vecn = bat->n_neg % 4 == 0 && aligned16(dneg);
+    const bool vec = rows_by_quads(tab), vecn = quad_row(bat->n_neg);
     TileArgs a{tab->ent, nullptr, nullptr, bat->h, bat->r, bat->neg, dneg, nullptr, nullptr, nullptr, query, nullptr, nullptr,
                B * bat->n_neg, (int)bat->chunk, (int)bat->n_neg, (int)d, 0, vec ? 1 : 0, vecn ? 1 : 0, (int)n_chunks, 1.0f,
                0, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -1065,7 +1075,7 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
     float *occ_w = reinterpret_cast<float *>(ws + p.off_occ_w);
     float *g0 = have_neg ? reinterpret_cast<float *>(ws + p.off_g0) : nullptr;
     float *g1 = have_neg && model == KGE_TRANSH ? reinterpret_cast<float *>(ws + p.off_g1) : nullptr;
-    const bool vec = rows_vectorizable(tab);
+    const bool vec = rows_by_quads(tab);
     bool chained = false;  // the gradient tile kernel wrote the positives' occurrence rows itself
     int rc = KGE_OK;
     // inspection fused into the score kernels' launches: the histogram and the first digit pass
@@ -1081,14 +1091,15 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
     if (have_neg) {
         const int64_t n_chunks = B / bat->chunk;
         if (n_chunks >= (1 << 24)) return KGE_ESHAPE;
-        const bool vecn = bat->n_neg % 4 == 0 && aligned16(dneg) && (!saved->neg || aligned16(saved->neg)) &&
-                          (!saved->side_neg || aligned16(saved->side_neg));
+        const bool vecn = quad_row(bat->n_neg);
         const bool dv = pair_sums_valu(tab);
+        // (the vector-ALU tiles of ComplEx walk the row in one piece: a quad must not straddle its halves)
+        const bool tvec = vec && !(model == KGE_COMPLEX && dv && d % 8 != 0);
         // the positive chain in the tile kernel's epilogue: see TileArgs::chain
         chained = (model == KGE_DISTMULT || model == KGE_COMPLEX) && !dv && vec && !bat->fuse_inspection;
         TileArgs a{tab->ent, tab->rel, tab->aux, head ? bat->t : bat->h, bat->r, bat->neg, dneg, saved->neg,
                    saved->side_pos, saved->side_neg, model == KGE_ROTATE ? saved->residual : nullptr, nullptr, nullptr,
-                   B * bat->n_neg, (int)bat->chunk, (int)bat->n_neg, (int)d, (int)tab->rel_dim, vec ? 1 : 0,
+                   B * bat->n_neg, (int)bat->chunk, (int)bat->n_neg, (int)d, (int)tab->rel_dim, tvec ? 1 : 0,
                    vecn ? 1 : 0, (int)n_chunks, head ? -1.0f : 1.0f,
                    chained ? 1 : 0, head ? bat->h : bat->t, dpos, head ? occ_e + B * d : occ_e, head ? occ_e : occ_e + B * d, occ_r};
         float *occ_neg = occ_e + 2 * B * d;

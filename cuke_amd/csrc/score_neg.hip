@@ -109,18 +109,20 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
     const int bt0 = tile_y * TB, kt0 = tile_x * TN;
     const int d = a.d, half = d >> 1;
     const int klen = MODEL == KGE_ROTATE ? half : d;
+    // the reduction axis: the row's columns, for ComplEx those of its padded halves (split_col)
+    constexpr bool kSplit = MODEL == KGE_COMPLEX && VEC4;
+    const int kvirt = kSplit ? 2 * ((half + 3) & ~3) : klen;
+    auto rcol = [&](int jv) { return kSplit ? split_col(jv, half) : jv; };
     // (VEC4, 128-bit row loads, is a compile-time choice: as a run-time one the compiler merges the two
     // forms of the raw loads into the scalar one)
 
-    // rows this thread stages
+    // rows this thread stages (past the tile's edge: its last row again; scores of such rows are not stored)
     const float *ph[SB], *pr[SB], *pw[SB], *pq[SB];
     float pa[SB];
-    bool okb[SB];
 #pragma unroll
     for (int s = 0; s < SB; ++s) {
         const int bl = bt0 + srow + 32 * s;
-        okb[s] = bl < a.C;
-        const int64_t b = (int64_t)c * a.C + (okb[s] ? bl : a.C - 1);
+        const int64_t b = (int64_t)c * a.C + (bl < a.C ? bl : a.C - 1);
         const int64_t rid = a.r[b];
         ph[s] = a.ent + a.h[b] * (int64_t)d;
         pr[s] = a.rel + rid * (int64_t)a.rel_dim;
@@ -129,12 +131,10 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
         pq[s] = (MODEL == KGE_ROTATE || MODEL == KGE_RESCAL) ? a.query + b * (int64_t)d : nullptr;
     }
     const float *pt[SN];
-    bool okk[SN];
 #pragma unroll
     for (int s = 0; s < SN; ++s) {
         const int kl = kt0 + srow + 32 * s;
-        okk[s] = kl < a.N;
-        pt[s] = a.ent + a.neg[(int64_t)c * a.N + (okk[s] ? kl : a.N - 1)] * (int64_t)d;
+        pt[s] = a.ent + a.neg[(int64_t)c * a.N + (kl < a.N ? kl : a.N - 1)] * (int64_t)d;
     }
 
     // The rows of the next slice are requested as raw operands -- clamped addresses, no select, no
@@ -147,15 +147,14 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
 
     auto load_slice_v = [&](auto vtag, int j0) {
         constexpr bool VEC = decltype(vtag)::value;
-        const int j = j0 + scol;
+        const int j = rcol(j0 + scol);
 #pragma unroll
         for (int s = 0; s < SB; ++s)
-            load_query_raw<MODEL, VEC>(ph[s], pr[s], pw[s], pq[s], j, okb[s] ? klen : 0, half, qraw[s]);
+            load_query_raw<MODEL, VEC>(ph[s], pr[s], pw[s], pq[s], j, klen, half, qraw[s]);
 #pragma unroll
         for (int s = 0; s < SN; ++s) {
-            const int lim = okk[s] ? klen : 0;
-            rt[0][s] = ld4_raw<VEC>(pt[s], j, lim);
-            if constexpr (MODEL == KGE_ROTATE) rt[1][s] = ld4_raw<VEC>(pt[s] + half, j, lim);
+            rt[0][s] = ld4_row_raw<MODEL, VEC>(pt[s], j, klen, half);
+            if constexpr (MODEL == KGE_ROTATE) rt[1][s] = ld4_raw<VEC>(pt[s] + half, j, klen);
         }
     };
 
@@ -166,11 +165,11 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
     // the slice that load_slice(j0) requested: query rows formed, tails masked, written to LDS
     auto stage_slice_v = [&](auto vtag, int j0) {
         constexpr bool VEC = decltype(vtag)::value;
-        const int j = j0 + scol;
+        const int j = rcol(j0 + scol);
 #pragma unroll
         for (int q = 0; q < SB; ++q) {
             float4 q0, q1;
-            combine_query<MODEL, VEC>(qraw[q], pa[q], j, okb[q] ? klen : 0, half, a.rsign, q0, q1);
+            combine_query<MODEL, VEC>(qraw[q], pa[q], j, klen, half, a.rsign, q0, q1);
             *reinterpret_cast<float4 *>(&sA[0][srow + 32 * q][scol]) = kScaled ? scale4(q0, kSgnScale) : q0;
             if constexpr (NPA == 2)
                 *reinterpret_cast<float4 *>(&sA[1][srow + 32 * q][scol]) = kScaled ? scale4(q1, kSgnScale) : q1;
@@ -179,7 +178,7 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
         for (int q = 0; q < SN; ++q)
 #pragma unroll
             for (int pl = 0; pl < NPT; ++pl) {
-                const float4 v = mask4<VEC>(rt[pl][q], j, okk[q] ? klen : 0);
+                const float4 v = mask4_row<MODEL, VEC>(rt[pl][q], j, klen, half);
                 *reinterpret_cast<float4 *>(&sT[pl][srow + 32 * q][scol]) = kScaled ? scale4(v, kSgnScale) : v;
             }
     };
@@ -193,7 +192,7 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
 #pragma unroll
         for (int k = 0; k < RK; ++k) acc[i][k] = 0.0f, cdot[i][k] = 0.0f, acc2[i][k] = 0.0f;
 
-    const int nslice = (klen + kKD - 1) / kKD;
+    const int nslice = (kvirt + kKD - 1) / kKD;
     int slice0 = 0, slice1 = nslice;  // this workgroup's share of the reduction axis
     if (a.ksplit > 1) {
         const int per = (nslice + a.ksplit - 1) / a.ksplit;
@@ -271,22 +270,16 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
         auto load_w = [&](int j0) {  // one uniform branch per slice, none per load
             const int j = j0 + scol;
 #pragma unroll
-            for (int q = 0; q < SB; ++q) rw[q] = ld4_raw<VEC4>(pw[q], j, okb[q] ? d : 0);
+            for (int q = 0; q < SB; ++q) rw[q] = ld4_raw<VEC4>(pw[q], j, d);
 #pragma unroll
-            for (int q = 0; q < SN; ++q) rt[0][q] = ld4_raw<VEC4>(pt[q], j, okk[q] ? d : 0);
+            for (int q = 0; q < SN; ++q) rt[0][q] = ld4_raw<VEC4>(pt[q], j, d);
         };
         auto stage_w = [&](int j0) {  // (raw loads, masked when written: see load_slice_v)
             const int j = j0 + scol;
 #pragma unroll
-            for (int q = 0; q < SB; ++q) {
-                const int lim = okb[q] ? d : 0;
-                *reinterpret_cast<float4 *>(&sA[1][srow + 32 * q][scol]) = mask4<VEC4>(rw[q], j, lim);
-            }
+            for (int q = 0; q < SB; ++q) *reinterpret_cast<float4 *>(&sA[1][srow + 32 * q][scol]) = mask4<VEC4>(rw[q], j, d);
 #pragma unroll
-            for (int q = 0; q < SN; ++q) {
-                const int lim = okk[q] ? d : 0;
-                *reinterpret_cast<float4 *>(&sT[0][srow + 32 * q][scol]) = mask4<VEC4>(rt[0][q], j, lim);
-            }
+            for (int q = 0; q < SN; ++q) *reinterpret_cast<float4 *>(&sT[0][srow + 32 * q][scol]) = mask4<VEC4>(rt[0][q], j, d);
         };
         load_w(0);
 #pragma unroll 1
@@ -403,27 +396,24 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_mfma_kernel(NegAr
     if (!xcd_tile(blockIdx.x - fi.blocks, (a.N + TN - 1) / TN, (a.C + TB - 1) / TB, a.n_chunks, c, tile_y, tile_x)) return;
     const int bt0 = tile_y * TB, kt0 = tile_x * TN;
     const int d = a.d, half = d >> 1;
-    // (VEC4, 128-bit row loads, is a compile-time choice: as a run-time one the compiler merges the two
-    // forms of the raw loads into the scalar one)
+    constexpr bool kSplit = MODEL == KGE_COMPLEX && VEC4;  // (the reduction axis: see score_neg_kernel)
+    const int kvirt = kSplit ? 2 * ((half + 3) & ~3) : d;
+    auto rcol = [&](int jv) { return kSplit ? split_col(jv, half) : jv; };
 
     const float *ph[SB], *pr[SB], *pq[SB];
-    bool okb[SB];
 #pragma unroll
     for (int s = 0; s < SB; ++s) {
         const int bl = bt0 + srow + 32 * s;
-        okb[s] = bl < a.C;
-        const int64_t b = (int64_t)c * a.C + (okb[s] ? bl : a.C - 1);
+        const int64_t b = (int64_t)c * a.C + (bl < a.C ? bl : a.C - 1);
         ph[s] = a.ent + a.h[b] * (int64_t)d;
         pr[s] = a.rel + a.r[b] * (int64_t)a.rel_dim;
         pq[s] = MODEL == KGE_RESCAL ? a.query + b * (int64_t)d : nullptr;
     }
     const float *pt[SN];
-    bool okk[SN];
 #pragma unroll
     for (int s = 0; s < SN; ++s) {
         const int kl = kt0 + srow + 32 * s;
-        okk[s] = kl < a.N;
-        pt[s] = a.ent + a.neg[(int64_t)c * a.N + (okk[s] ? kl : a.N - 1)] * (int64_t)d;
+        pt[s] = a.ent + a.neg[(int64_t)c * a.N + (kl < a.N ? kl : a.N - 1)] * (int64_t)d;
     }
 
     // Raw operands of the next slice are in flight during the matrix-core work of this one; they are
@@ -433,23 +423,23 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_mfma_kernel(NegAr
     constexpr int NRAW = query_raw_count<MODEL>();
     float4 qraw[SB][NRAW], rt[SN];
     auto load_slice = [&](int j0, float4 (&qr)[SB][NRAW], float4 (&tr)[SN]) {
-        const int j = j0 + scol;
+        const int j = rcol(j0 + scol);
 #pragma unroll
-        for (int s = 0; s < SB; ++s) load_query_raw<MODEL, VEC4>(ph[s], pr[s], nullptr, pq[s], j, okb[s] ? d : 0, half, qr[s]);
+        for (int s = 0; s < SB; ++s) load_query_raw<MODEL, VEC4>(ph[s], pr[s], nullptr, pq[s], j, d, half, qr[s]);
 #pragma unroll
-        for (int s = 0; s < SN; ++s) tr[s] = ld4_raw<VEC4>(pt[s], j, okk[s] ? d : 0);
+        for (int s = 0; s < SN; ++s) tr[s] = ld4_row_raw<MODEL, VEC4>(pt[s], j, d, half);
     };
     auto stage_slice = [&](int j0, const float4 (&qr)[SB][NRAW], const float4 (&tr)[SN]) {
-        const int j = j0 + scol;
+        const int j = rcol(j0 + scol);
 #pragma unroll
         for (int q = 0; q < SB; ++q) {
             float4 q0, q1;
-            combine_query<MODEL, VEC4>(qr[q], 0.0f, j, okb[q] ? d : 0, half, a.rsign, q0, q1);
+            combine_query<MODEL, VEC4>(qr[q], 0.0f, j, d, half, a.rsign, q0, q1);
             *reinterpret_cast<float4 *>(&sA[srow + 32 * q][scol]) = q0;
         }
 #pragma unroll
         for (int q = 0; q < SN; ++q)
-            *reinterpret_cast<float4 *>(&sT[srow + 32 * q][scol]) = mask4<VEC4>(tr[q], j, okk[q] ? d : 0);
+            *reinterpret_cast<float4 *>(&sT[srow + 32 * q][scol]) = mask4_row<MODEL, VEC4>(tr[q], j, d, half);
     };
 
     // two accumulators per block (one per half of the slice) keep consecutive MFMAs independent
@@ -461,7 +451,7 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_mfma_kernel(NegAr
 #pragma unroll
             for (int n = 0; n < NB; ++n) acc[g][m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int nslice = (d + kKD - 1) / kKD;
+    const int nslice = (kvirt + kKD - 1) / kKD;
     load_slice(0, qraw, rt);
 #pragma unroll 1
     for (int s = 0; s < nslice; ++s) {
@@ -576,8 +566,8 @@ static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, c
     // launches are bound by the rows its workgroups pull from L2, does best with 32x64).  The
     // inspector workgroups that share the machine with these launches raise their wave priority.
     constexpr bool kDotModel = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL;
-    // Rows without 128-bit loads (dim % 4 != 0, unaligned tables) take the 32x32 tile whatever the size:
-    // only that tile is compiled in the scalar-load form.
+    // Rows of fewer than four floats take the 32x32 tile whatever the size: only that tile is compiled in
+    // the scalar-load form.
     const int tile = !a.vec ? 2 : big_tiles >= 1024 ? 4 : (kDotModel && !dot_valu ? 3 : 2);  // 2: 32x32, 3: 32x64, 4: 64x64
     const int TB = tile == 4 ? 64 : 32, TN = tile == 2 ? 32 : 64;
     // (workgroups that score the positives, if the launch carries them, follow the tiles')
@@ -627,7 +617,7 @@ static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, c
 bool score_neg_carries_positives(const kge_tables *tab, const kge_batch *bat)
 {
     const bool dot = (tab->model == KGE_DISTMULT || tab->model == KGE_COMPLEX) && !pair_sums_valu(tab);
-    return (dot || tab->model == KGE_TRANSE) && bat->neg && bat->batch > 0 && !bat->fuse_inspection && rows_vectorizable(tab) &&
+    return (dot || tab->model == KGE_TRANSE) && bat->neg && bat->batch > 0 && !bat->fuse_inspection && rows_by_quads(tab) &&
            ceil_div(bat->batch, kPosWaves) < (1 << 30);
 }
 
@@ -640,7 +630,7 @@ int launch_score_neg(const kge_tables *tab, const kge_batch *bat, const float *s
     if (carry_pos && (fused || !score_neg_carries_positives(tab, bat))) return KGE_EINVAL;
     const int64_t n_chunks = bat->batch / bat->chunk;
     if (n_chunks >= (1 << 24) || bat->chunk >= (1 << 30) || bat->n_neg >= (1 << 30)) return KGE_ESHAPE;
-    const bool vec = rows_vectorizable(tab);
+    const bool vec = rows_by_quads(tab);
     const bool head = bat->neg_mode == KGE_NEG_HEAD;
     NegArgs a{tab->ent, tab->rel, tab->aux, head ? bat->t : bat->h, bat->r, bat->neg, side_pos, query, out, side_neg,
               bat->batch * bat->n_neg, (int)bat->chunk, (int)bat->n_neg, (int)tab->dim, (int)tab->rel_dim, tab->gamma,

@@ -47,40 +47,46 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
     float acc = 0.0f;
 
     if constexpr (MODEL == KGE_TRANSE) {
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j);
             Vec<V> u;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 u.v[e] = (vh.v[e] - vt.v[e]) + vr.v[e];  // same order as the generated loop
-                acc += norm_term<P>(u.v[e]);
+                acc += e >= at.skip ? norm_term<P>(u.v[e]) : 0.0f;
             }
             if (out && valid) u.store(out + j);
         }
     } else if constexpr (MODEL == KGE_TRANSH) {
         const float *w = a.aux + rid * (int64_t)d;
         float sd = 0.0f, wh = 0.0f;
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vw = Vec<V>::load(w + j);
 #pragma unroll
             for (int e = 0; e < V; ++e) {
-                sd += vw.v[e] * (vh.v[e] - vt.v[e]);
-                wh += vw.v[e] * (a.head ? vt.v[e] : vh.v[e]);
+                sd += e >= at.skip ? vw.v[e] * (vh.v[e] - vt.v[e]) : 0.0f;
+                wh += e >= at.skip ? vw.v[e] * (a.head ? vt.v[e] : vh.v[e]) : 0.0f;
             }
         }
         sd = wave_sum(sd);
         wh = wave_sum(wh);
         if (a.side_pos && valid && lane == 0) a.side_pos[b] = wh;
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j), vw = Vec<V>::load(w + j);
             Vec<V> u;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 u.v[e] = ((vh.v[e] - vt.v[e]) + vr.v[e]) - sd * vw.v[e];
-                acc += norm_term<P>(u.v[e]);
+                acc += e >= at.skip ? norm_term<P>(u.v[e]) : 0.0f;
             }
             if (out && valid) u.store(out + j);
         }
@@ -92,7 +98,9 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
         float *x = lds + wave * d;
         for (int i = lane; i < d; i += kWave) x[i] = MODEL == KGE_TRANSR ? eh[i] - et[i] : eh[i];
         __syncthreads();
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             Vec<V> s;
 #pragma unroll
             for (int e = 0; e < V; ++e) s.v[e] = 0.0f;
@@ -107,30 +115,35 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
 #pragma unroll
                 for (int e = 0; e < V; ++e) {
                     s.v[e] += vr.v[e];
-                    acc += norm_term<P>(s.v[e]);
+                    acc += e >= at.skip ? norm_term<P>(s.v[e]) : 0.0f;
                 }
                 if (out && valid) s.store(out + j);
             } else {
                 const Vec<V> vt = Vec<V>::load(et + j);
 #pragma unroll
-                for (int e = 0; e < V; ++e) acc += s.v[e] * vt.v[e];
+                for (int e = 0; e < V; ++e) acc += e >= at.skip ? s.v[e] * vt.v[e] : 0.0f;
                 if (out && valid) s.store(out + j);  // E[h] Proj[r], consumed by the backward pass
             }
         }
     } else if constexpr (MODEL == KGE_DISTMULT) {
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j);
 #pragma unroll
-            for (int e = 0; e < V; ++e) acc += (vh.v[e] * vr.v[e]) * vt.v[e];
+            for (int e = 0; e < V; ++e) acc += e >= at.skip ? (vh.v[e] * vr.v[e]) * vt.v[e] : 0.0f;
         }
     } else if constexpr (MODEL == KGE_TRANSF) {
         float rx = 0.0f;  // r . (the side the shared negatives keep)
-        for (int j = lane * V; j < d; j += kWave * V) {
+        for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
+            const RowPiece<V> at(j0, d);
+            const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j);
 #pragma unroll
             for (int e = 0; e < V; ++e) {
+                if (e < at.skip) continue;
                 acc += (vh.v[e] + vr.v[e]) * vt.v[e] + (vt.v[e] - vr.v[e]) * vh.v[e];
                 rx += vr.v[e] * (a.head ? vt.v[e] : vh.v[e]);
             }
@@ -141,7 +154,9 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
         }
     } else if constexpr (MODEL == KGE_COMPLEX) {
         const int half = d / 2;
-        for (int j = lane * V; j < half; j += kWave * V) {
+        for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
+            const RowPiece<V> at(j0, half);
+            const int j = at.at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> qr = Vec<V>::load(rr + j), qi = Vec<V>::load(rr + half + j);
@@ -149,12 +164,14 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
             for (int e = 0; e < V; ++e) {
                 const float ar = hr.v[e] * qr.v[e] - hi.v[e] * qi.v[e];
                 const float ai = hr.v[e] * qi.v[e] + hi.v[e] * qr.v[e];
-                acc += ar * tr.v[e] + ai * ti.v[e];
+                acc += e >= at.skip ? ar * tr.v[e] + ai * ti.v[e] : 0.0f;
             }
         }
     } else if constexpr (MODEL == KGE_ROTATE) {
         const int half = d / 2;
-        for (int j = lane * V; j < half; j += kWave * V) {
+        for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
+            const RowPiece<V> at(j0, half);
+            const int j = at.at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> th = Vec<V>::load(rr + j);
@@ -166,7 +183,7 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
                 ar.v[e] = hr.v[e] * c - hi.v[e] * sn;
                 ai.v[e] = hr.v[e] * sn + hi.v[e] * c;
                 const float ur = ar.v[e] - tr.v[e], ui = ai.v[e] - ti.v[e];
-                acc += sqrtf(ur * ur + ui * ui);
+                acc += e >= at.skip ? sqrtf(ur * ur + ui * ui) : 0.0f;
                 if (a.head) {  // the kept side is the tail: t e^{-i theta}
                     ar.v[e] = tr.v[e] * c + ti.v[e] * sn;
                     ai.v[e] = ti.v[e] * c - tr.v[e] * sn;

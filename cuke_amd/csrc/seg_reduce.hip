@@ -74,6 +74,7 @@ __global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, Sum
     {
         const int colv = c0 + lane * V;
         const bool active = colv < d;
+        const int cc = active ? RowPiece<V>(colv, d).at : 0;
         Vec<V> acc;
 #pragma unroll
         for (int e = 0; e < V; ++e) acc.v[e] = 0.0f;
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, Sum
 #pragma unroll
             for (int u = 0; u < kFly; ++u) {
                 const int64_t jb = jj + 4 * u;
-                t[u] = Vec<V>::load(a.partial + ((jb <= je ? jb : je) * 2) * (int64_t)d + (active ? colv : 0));
+                t[u] = Vec<V>::load(a.partial + ((jb <= je ? jb : je) * 2) * (int64_t)d + cc);
             }
 #pragma unroll
             for (int u = 0; u < kFly; ++u)
@@ -100,12 +101,12 @@ __global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, Sum
         for (int e = 0; e < V; ++e) s_part[wave][lane * V + e] = acc.v[e];
         __syncthreads();
         if (wave == 0 && active) {
-            Vec<V> r = Vec<V>::load(a.partial + (j * 2 + 1) * (int64_t)d + colv);
+            Vec<V> r = Vec<V>::load(a.partial + (j * 2 + 1) * (int64_t)d + cc);
 #pragma unroll
             for (int e = 0; e < V; ++e)
                 r.v[e] += (s_part[0][lane * V + e] + s_part[1][lane * V + e]) +
                           (s_part[2][lane * V + e] + s_part[3][lane * V + e]);
-            r.store(a.out + (int64_t)sg * d + colv);
+            r.store(a.out + (int64_t)sg * d + cc);
         }
     }
 }
@@ -124,7 +125,7 @@ static int plan_jobs(const SegJob *jobs, int n_jobs, SegL1Rider *out, int64_t *m
         r.jobs.j[m] = SegArgs{jb.occ, jb.identity_perm ? nullptr : jb.ins->perm, jb.ins->sorted_seg,
                               jb.ins->seg_offsets, jb.ins->n, jb.d, jb.out, jb.partial,
                               jb.scale_num, jb.scale_den, (jb.scaled ? 1 : 0) | (jb.sign_rows ? 2 : 0), (int)jb.wrap};
-        v4 = v4 && jb.d % 4 == 0 && aligned16(jb.occ) && aligned16(jb.out) && aligned16(jb.partial);
+        v4 = v4 && quad_row(jb.d);
         ++m;
     }
     for (int q = 0; q < m; ++q) {

@@ -110,7 +110,7 @@ __device__ __forceinline__ void seg_l1_wave(const SegArgs &a, int64_t w)
         wsign[q] = second ? -1.0f : 1.0f;
         src[q] = second ? src[q] - a.wrap : src[q];
     }
-    const int cc = active ? colv : 0;
+    const int cc = active ? RowPiece<V>(colv, d).at : 0;  // (a last piece moved back: the same sums twice)
     Vec<V> v[kSegL];
 #pragma unroll
     for (int q = 0; q < kSegL; ++q) v[q] = Vec<V>::load(a.occ + (int64_t)src[q] * d + cc);
@@ -150,7 +150,7 @@ __device__ __forceinline__ void seg_l1_wave(const SegArgs &a, int64_t w)
         if (sg == prev_id) dst = a.partial + (j * 2 + 0) * (int64_t)d;       // began in an earlier block
         else if (sg == next_id) dst = a.partial + (j * 2 + 1) * (int64_t)d;  // continues in a later block
         else dst = a.out + (int64_t)sg * d;                                   // wholly inside: final
-        if (active) acc.store(dst + colv);
+        if (active) acc.store(dst + cc);
     };
 #pragma unroll
     for (int q = 0; q < kSegL; ++q) {

@@ -11,16 +11,36 @@
 
 namespace kge {
 
-// Four consecutive floats p[j .. j+3], zero where j + e >= lim.  Branch-free: an out-of-range
-// request reads p[0] (always a valid row start here) and discards it, so the callers' loads sit
-// in one basic block and the compiler can issue them back to back.
+// ---- quads of a row -----------------------------------------------------------------------------
+// Rows (segments) of at least four floats are read 128 bits at a time whatever their width and alignment: the quad that
+// would run past the end of the segment is moved back to end with it, so no address lies outside the row.  Its first
+// elements belong to the quad before it as well: a sum over columns leaves them out (mask4), a result per column is
+// formed twice and stored once.  `lim` is the segment's length, or 0 for a row outside the tile.
+//   16-byte rows only (the rule before), everything else by single floats in 32 x 32 tiles: ComplEx, 512 queries
+//   against 14951 candidates, 394 us at width 396 and 384 us at 402 beside 105 us at 400; one TransE step of 30000 x 150 x 200
+//   negatives 466 us beside 374 us at width 152.
+// v moved down by s elements, zeros from above (s <= 0: v; s >= 4: zeros)
+__device__ __forceinline__ float4 shift_quad(float4 v, int s)
+{
+    const bool one = s == 1 || s == 3, two = s == 2 || s == 3, all = s >= 4;
+    v = make_float4(one ? v.y : v.x, one ? v.z : v.y, one ? v.w : v.z, one ? 0.0f : v.w);
+    v = make_float4(two ? v.z : v.x, two ? v.w : v.y, two ? 0.0f : v.z, two ? 0.0f : v.w);
+    return make_float4(all ? 0.0f : v.x, all ? 0.0f : v.y, all ? 0.0f : v.z, all ? 0.0f : v.w);
+}
+
+// Four consecutive floats p[j .. j+3] (VEC: moved back to end with the row), zero where the element
+// is not the quad's own.  Branch-free: an out-of-range request reads a valid address of the row and discards it, so the
+// callers' loads sit in one basic block and the compiler can issue them back to back.
+template <bool VEC>
+__device__ __forceinline__ float4 ld4_raw(const float *p, int j, int lim);
+template <bool VEC>
+__device__ __forceinline__ float4 mask4(float4 v, int j, int lim);
+
 template <bool VEC>
 __device__ __forceinline__ float4 ld4(const float *p, int j, int lim)
 {
-    if constexpr (VEC) {  // rows are 16-byte aligned and lim % 4 == 0
-        const bool ok = j < lim;
-        const float4 v = *reinterpret_cast<const float4 *>(p + (ok ? j : 0));
-        return ok ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (VEC) {
+        return mask4<true>(ld4_raw<true>(p, j, lim), j, lim);
     } else {
         float4 q;
         const bool k0 = j + 0 < lim, k1 = j + 1 < lim, k2 = j + 2 < lim, k3 = j + 3 < lim;
@@ -33,16 +53,18 @@ __device__ __forceinline__ float4 ld4(const float *p, int j, int lim)
     }
 }
 
-__device__ __forceinline__ void st4(float *p, int j, int lim, bool vec, float4 v)
+// The same where a quad lies inside its row or outside it as a whole: lanes outside keep a zero and load nothing, so nothing
+// touches the loaded register (a select on it would be waited for where it stands).
+template <bool VEC>
+__device__ __forceinline__ float4 ld4_whole(const float *p, int j, int lim)
 {
-    if (vec) {
-        if (j < lim) *reinterpret_cast<float4 *>(p + j) = v;
-        return;
+    if constexpr (VEC) {
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (j < lim) v = load_quad(p + j);
+        return v;
+    } else {
+        return ld4<false>(p, j, lim);
     }
-    if (j + 0 < lim) p[j + 0] = v.x;
-    if (j + 1 < lim) p[j + 1] = v.y;
-    if (j + 2 < lim) p[j + 2] = v.z;
-    if (j + 3 < lim) p[j + 3] = v.w;
 }
 
 __device__ __forceinline__ float4 zero4() { return make_float4(0.f, 0.f, 0.f, 0.f); }
@@ -97,66 +119,8 @@ __device__ __forceinline__ int pair_len(int d)
 // (RotatE, already applied in pq) or r (DistMult).  The caller passes the tail row as `ph` and
 // rs = -1; rs multiplies r (its imaginary half for ComplEx), which is exact, so rs = +1
 // reproduces the tail-mode arithmetic bit for bit.
-template <int MODEL, bool VEC>
-__device__ __forceinline__ void load_query(const float *ph, const float *pr, const float *pw, float al,
-                                           int j, int lim, int half, float4 &q0, float4 &q1,
-                                           const float *pq = nullptr, float rs = 1.0f)
-{
-    q1 = zero4();
-    if constexpr (MODEL == KGE_DISTMULT) {
-        q0 = mul4(ld4<VEC>(ph, j, lim), ld4<VEC>(pr, j, lim));
-    } else if constexpr (MODEL == KGE_TRANSE) {
-        const float4 vh = ld4<VEC>(ph, j, lim), vr = ld4<VEC>(pr, j, lim);
-        q0 = make_float4(fmaf(rs, vr.x, vh.x), fmaf(rs, vr.y, vh.y), fmaf(rs, vr.z, vh.z), fmaf(rs, vr.w, vh.w));
-    } else if constexpr (MODEL == KGE_TRANSF) {
-        const float4 vh = ld4<VEC>(ph, j, lim), vr = ld4<VEC>(pr, j, lim);
-        q0 = make_float4(fmaf(rs, vr.x, 2.0f * vh.x), fmaf(rs, vr.y, 2.0f * vh.y), fmaf(rs, vr.z, 2.0f * vh.z),
-                         fmaf(rs, vr.w, 2.0f * vh.w));
-    } else if constexpr (MODEL == KGE_COMPLEX) {
-        float q[4];
-        if constexpr (VEC) {  // half % 4 == 0: the four elements sit on one side of the re|im split
-            const bool re = j < half;
-            const int i = re ? j : j - half;
-            const int l2 = lim ? half : 0;
-            const float4 hr = ld4<true>(ph, i, l2), hi = ld4<true>(ph + half, i, l2);
-            const float4 rr = ld4<true>(pr, i, l2);
-            float4 ri = ld4<true>(pr + half, i, l2);
-            ri = make_float4(rs * ri.x, rs * ri.y, rs * ri.z, rs * ri.w);
-            q[0] = re ? hr.x * rr.x - hi.x * ri.x : hr.x * ri.x + hi.x * rr.x;
-            q[1] = re ? hr.y * rr.y - hi.y * ri.y : hr.y * ri.y + hi.y * rr.y;
-            q[2] = re ? hr.z * rr.z - hi.z * ri.z : hr.z * ri.z + hi.z * rr.z;
-            q[3] = re ? hr.w * rr.w - hi.w * ri.w : hr.w * ri.w + hi.w * rr.w;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int jj = j + e;
-                const bool ok = jj < lim;
-                const int i = ok ? (jj < half ? jj : jj - half) : 0;
-                const float hr = ph[i], hi = ph[i + half], rr = pr[i], ri = rs * pr[i + half];
-                q[e] = ok ? (jj < half ? hr * rr - hi * ri : hr * ri + hi * rr) : 0.0f;
-            }
-        }
-        q0 = make_float4(q[0], q[1], q[2], q[3]);
-    } else if constexpr (MODEL == KGE_RESCAL) {
-        q0 = ld4<VEC>(pq, j, lim);
-    } else if constexpr (MODEL == KGE_ROTATE) {
-        // the rotated head h e^{i theta} was written by the positive kernel ([re | im] row pq):
-        // a plain load here instead of a sincos per element in every tile that needs the row
-        q0 = ld4<VEC>(pq, j, lim);
-        q1 = ld4<VEC>(pq + half, j, lim);
-    } else if constexpr (MODEL == KGE_TRANSH) {
-        const float4 vw = ld4<VEC>(pw, j, lim);
-        const float4 vh = ld4<VEC>(ph, j, lim), vr = ld4<VEC>(pr, j, lim);
-        q1 = vw;
-        q0 = make_float4(fmaf(rs, vr.x, vh.x) - al * vw.x, fmaf(rs, vr.y, vh.y) - al * vw.y,
-                         fmaf(rs, vr.z, vh.z) - al * vw.z, fmaf(rs, vr.w, vh.w) - al * vw.w);
-    } else {
-        q0 = zero4();
-    }
-}
-
-// ---- the same in two steps ---------------------------------------------------------------------
-// A tile kernel that prefetches the next block of rows while it computes on the current one only
+//
+// Loading and forming are two steps.  A tile kernel that prefetches the next block of rows while it computes on the current one only
 // overlaps the two if nothing touches the loaded registers before the compute: any arithmetic
 // on them (h * r, the zero fill of a tail) makes the compiler wait for the loads where they are
 // issued.  load_query_raw() therefore only loads -- clamped to a valid address, no select, no
@@ -164,19 +128,22 @@ __device__ __forceinline__ void load_query(const float *ph, const float *pr, con
 template <bool VEC>
 __device__ __forceinline__ float4 ld4_raw(const float *p, int j, int lim)
 {
-    if constexpr (VEC) {  // rows are 16-byte aligned and lim % 4 == 0
-        return *reinterpret_cast<const float4 *>(p + (j < lim ? j : 0));
+    if constexpr (VEC) {
+        return load_quad(p + max(min(j, lim - 4), 0));
     } else {
         return make_float4(p[j + 0 < lim ? j + 0 : 0], p[j + 1 < lim ? j + 1 : 0], p[j + 2 < lim ? j + 2 : 0],
                            p[j + 3 < lim ? j + 3 : 0]);
     }
 }
 
-// zero the elements at or beyond lim (the whole quad when VEC)
+// the quad that ld4_raw(p, j, lim) loaded, zero where the element is not its own
 template <bool VEC>
 __device__ __forceinline__ float4 mask4(float4 v, int j, int lim)
 {
-    if constexpr (VEC) return j < lim ? v : make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (VEC) {
+        const int skip = j + 4 - lim;  // elements that the quad before it has
+        return make_float4(skip <= 0 ? v.x : 0.0f, skip <= 1 ? v.y : 0.0f, skip <= 2 ? v.z : 0.0f, skip <= 3 ? v.w : 0.0f);
+    }
     return make_float4(j + 0 < lim ? v.x : 0.0f, j + 1 < lim ? v.y : 0.0f, j + 2 < lim ? v.z : 0.0f,
                        j + 3 < lim ? v.w : 0.0f);
 }
@@ -196,7 +163,7 @@ __device__ __forceinline__ void load_query_raw(const float *ph, const float *pr,
         raw[0] = ld4_raw<VEC>(ph, j, lim);
         raw[1] = ld4_raw<VEC>(pr, j, lim);
     } else if constexpr (MODEL == KGE_COMPLEX) {
-        if constexpr (VEC) {  // half % 4 == 0: the four elements sit on one side of the re|im split
+        if constexpr (VEC) {  // (a quad starts at a multiple of four of its half, see split_col)
             const int i = j < half ? j : j - half;
             const int l2 = lim ? half : 0;
             raw[0] = ld4_raw<true>(ph, i, l2), raw[1] = ld4_raw<true>(ph + half, i, l2);
@@ -225,7 +192,7 @@ __device__ __forceinline__ void load_query_raw(const float *ph, const float *pr,
     }
 }
 
-// The query row from its raw operands (same j, lim, half, rs as load_query; same arithmetic).
+// The query row from its raw operands (same j, lim, half as load_query_raw).
 template <int MODEL, bool VEC, int N>
 __device__ __forceinline__ void combine_query(const float4 (&raw)[N], float al, int j, int lim, int half, float rs,
                                               float4 &q0, float4 &q1)
@@ -251,9 +218,10 @@ __device__ __forceinline__ void combine_query(const float4 (&raw)[N], float al, 
         for (int e = 0; e < 4; ++e) {
             const int jj = VEC ? j : j + e;  // VEC: one side of the split for the whole quad
             const float v = jj < half ? hr[e] * rr[e] - hi[e] * ri[e] : hr[e] * ri[e] + hi[e] * rr[e];
-            q[e] = jj < lim ? v : 0.0f;
+            q[e] = VEC || jj < lim ? v : 0.0f;
         }
         q0 = make_float4(q[0], q[1], q[2], q[3]);
+        if constexpr (VEC) q0 = mask4<true>(q0, j < half ? j : j - half, lim ? half : 0);
     } else if constexpr (MODEL == KGE_RESCAL) {
         q0 = mask4<VEC>(raw[0], j, lim);
     } else if constexpr (MODEL == KGE_ROTATE) {
@@ -268,6 +236,38 @@ __device__ __forceinline__ void combine_query(const float4 (&raw)[N], float al, 
     } else {
         q0 = zero4();
     }
+}
+
+// Both steps at once.
+template <int MODEL, bool VEC>
+__device__ __forceinline__ void load_query(const float *ph, const float *pr, const float *pw, const float *pq, float al, int j, int lim,
+                                           int half, float rs, float4 &q0, float4 &q1)
+{
+    float4 raw[query_raw_count<MODEL>()];
+    load_query_raw<MODEL, VEC>(ph, pr, pw, pq, j, lim, half, raw);
+    combine_query<MODEL, VEC>(raw, al, j, lim, half, rs, q0, q1);
+}
+
+// ComplEx rows are two segments of half floats, each walked in quads of its own: column jv of the padded row
+// [re, padded to a multiple of four | im, padded] is column split_col(jv) of the row, and a quad that starts there belongs
+// to one half.
+__device__ __forceinline__ int split_col(int jv, int half)
+{
+    const int hp = (half + 3) & ~3;
+    return jv < hp ? jv : jv - hp + half;
+}
+// a quad of a plain row, or of one half of a ComplEx row (VEC: j as split_col gives it)
+template <int MODEL, bool VEC>
+__device__ __forceinline__ float4 ld4_row_raw(const float *p, int j, int lim, int half)
+{
+    if constexpr (MODEL == KGE_COMPLEX && VEC) return ld4_raw<true>(p + (j < half ? 0 : half), j < half ? j : j - half, lim ? half : 0);
+    else return ld4_raw<VEC>(p, j, lim);
+}
+template <int MODEL, bool VEC>
+__device__ __forceinline__ float4 mask4_row(float4 v, int j, int lim, int half)
+{
+    if constexpr (MODEL == KGE_COMPLEX && VEC) return mask4<true>(v, j < half ? j : j - half, lim ? half : 0);
+    else return mask4<VEC>(v, j, lim);
 }
 
 // XCD-aware tile placement.  The 256 CUs sit in 8 XCDs with one L2 each, and consecutive
@@ -297,11 +297,11 @@ inline unsigned xcd_grid(int64_t tiles_x, int64_t tiles_y, int64_t n_chunks)
     return (unsigned)(kXcds * ceil_div(n_chunks * split, kXcds) * ceil_div(per, split));
 }
 
-inline bool rows_vectorizable(const kge_tables *tab)
+// 128-bit row loads: every row segment (ComplEx, RotatE: each half) has at least four floats
+inline bool rows_by_quads(const kge_tables *tab)
 {
     const bool complex_rows = tab->model == KGE_COMPLEX || tab->model == KGE_ROTATE;
-    return tab->dim % (complex_rows ? 8 : 4) == 0 && aligned16(tab->ent) &&
-           (!tab->rel || aligned16(tab->rel)) && (!tab->aux || aligned16(tab->aux));
+    return quad_row(complex_rows ? tab->dim / 2 : tab->dim);
 }
 
 }  // namespace kge

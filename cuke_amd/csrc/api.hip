@@ -6,7 +6,8 @@
 namespace kge {
 int launch_score_pos(const kge_tables *, const kge_batch *, float *, float *, float *, hipStream_t);
 int launch_score_pos_fused(const kge_tables *, const kge_batch *, float *, float *, float *, const FusedInsp *,
-                           hipStream_t);
+                           hipStream_t, float *query = nullptr);
+size_t split_query_bytes(const kge_tables *, const kge_batch *);
 int launch_score_neg(const kge_tables *, const kge_batch *, const float *, const float *, float *, float *,
                      const FusedInsp *, void *, size_t, hipStream_t, float *carry_pos);
 bool score_neg_carries_positives(const kge_tables *, const kge_batch *);
@@ -247,7 +248,7 @@ size_t kge_score_fwd_workspace(const kge_tables *tab, const kge_batch *bat)
     }
     if ((tab->model == KGE_TRANSR || tab->model == KGE_RESCAL) && bat->rel_insp) return transr_fwd_workspace(tab, bat);
     if (tab->model == KGE_TRANSE || tab->model == KGE_ROTATE) return neg_split_workspace(tab, bat);  // small batches only
-    return 0;
+    return split_query_bytes(tab, bat);  // large batches of dot products only
 }
 
 int kge_transr_plan(const kge_tables *tab, const kge_batch *bat, void *workspace, size_t workspace_bytes, void *stream)
@@ -307,8 +308,11 @@ int kge_score_fwd(const kge_tables *tab, const kge_batch *bat, float *pos, float
     // nothing else does (score_neg_carries_positives; also with the reduction axis of small TransE
     // batches split, where their workgroups follow tile_blocks * ksplit tile workgroups).  `pos` is then
     // written by the negatives' launch, and its timeline entry "score_neg_kernel" includes the positives.
-    const bool carry = want_neg && pos && !side_pos && !residual && !fuse && score_neg_carries_positives(tab, bat);
-    if (!carry && (pos || side_pos || residual)) {
+    // Large batches of dot-product scores: the per-positive kernel leaves the query rows in the workspace for the split tiles.
+    const size_t query_bytes = want_neg ? split_query_bytes(tab, bat) : 0;
+    float *query = query_bytes > 0 && workspace && workspace_bytes >= query_bytes ? static_cast<float *>(workspace) : nullptr;
+    const bool carry = want_neg && pos && !side_pos && !residual && !fuse && !query && score_neg_carries_positives(tab, bat);
+    if (!carry && (pos || side_pos || residual || query)) {
         if (rescal_head) {
             // corrupted heads: the positives' scores from the usual pass, then `residual` takes the rows
             // u_b = Proj[r_b] E[t_b] that the pair scores E[h'] . u_b (and the backward pass) are formed from
@@ -318,13 +322,13 @@ int kge_score_fwd(const kge_tables *tab, const kge_batch *bat, float *pos, float
         } else if ((tab->model == KGE_TRANSR || tab->model == KGE_RESCAL) && bat->rel_insp)
             rc = launch_transr_fwd(tab, bat, pos, residual, workspace, workspace_bytes, st);
         else {
-            rc = launch_score_pos_fused(tab, bat, pos, residual, side_pos, fuse ? &fi0 : nullptr, st);
+            rc = launch_score_pos_fused(tab, bat, pos, residual, side_pos, fuse ? &fi0 : nullptr, st, query);
             timeline_mark(bat->timeline, st, "score_pos_kernel");
         }
         if (rc) return rc;
     }
     if (want_neg) {
-        rc = launch_score_neg(tab, bat, side_pos, (tab->model == KGE_ROTATE || tab->model == KGE_RESCAL) ? residual : nullptr, neg, side_neg,
+        rc = launch_score_neg(tab, bat, side_pos, (tab->model == KGE_ROTATE || tab->model == KGE_RESCAL) ? residual : query, neg, side_neg,
                               fuse ? &fi1 : nullptr, workspace, workspace_bytes, st, carry ? pos : nullptr);
         timeline_mark(bat->timeline, st, "score_neg_kernel");
         return rc;

@@ -14,7 +14,7 @@ constexpr int kLossWaves = 4;
 // up walked 16384 to 30000 doubles, 18 to 30 us; over at most kLossBlocks partials it is 2 us.
 constexpr int kLossBlocks = 1024;
 
-template <int V>
+template <int V, bool RAG>
 __global__ __launch_bounds__(kLossWaves *kWave) void margin_rows_kernel(
     const float *pos, const float *neg, int64_t B, int64_t N, float margin, float sign, float inv,
     float *dpos, float *dneg, double *block_loss)
@@ -27,8 +27,8 @@ __global__ __launch_bounds__(kLossWaves *kWave) void margin_rows_kernel(
         float sum = 0.0f;
         int cnt = 0;
         for (int64_t k0 = lane * V; k0 < N; k0 += kWave * V) {
-            const int64_t k = V == 4 && k0 > N - V ? N - V : k0;  // the row's last piece ends with it
-            const int skip = (int)(k0 - k);
+            const int64_t k = RAG && k0 > N - V ? N - V : k0;  // the row's last piece ends with it
+            const int skip = RAG ? (int)(k0 - k) : 0;
             const Vec<V> s = Vec<V>::load(neg + b * N + k);
             Vec<V> g;
 #pragma unroll
@@ -132,10 +132,8 @@ int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n
     const int blocks = (int)(want < kLossBlocks ? want : kLossBlocks);  // (one partial each: never more than the workspace's `batch`)
     if (batch > 0) {
         const dim3 grid((unsigned)blocks), block(kLossWaves * kWave);
-        if (quad_row(n_neg))
-            hipLaunchKernelGGL(margin_rows_kernel<4>, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
-        else
-            hipLaunchKernelGGL(margin_rows_kernel<1>, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
+        const auto kernel = n_neg % 4 == 0 ? margin_rows_kernel<4, false> : (quad_row(n_neg) ? margin_rows_kernel<4, true> : margin_rows_kernel<1, false>);
+        hipLaunchKernelGGL(kernel, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
     }
     hipLaunchKernelGGL(margin_total_kernel, dim3(1), dim3(256), 0, st, rows, blocks, count > 0 ? 1.0 / count : 0.0, loss);
     KGE_CHECK_LAUNCH();

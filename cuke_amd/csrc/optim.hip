@@ -5,7 +5,7 @@
 
 namespace kge {
 
-template <bool ADAGRAD, int V>
+template <bool ADAGRAD, int V, bool RAG>
 __global__ __launch_bounds__(256) void sparse_step_kernel(float *table, float *state, int d, const int64_t *ids,
                                                           const int32_t *num_unique, const float *rows, float lr,
                                                           float eps)
@@ -20,7 +20,7 @@ __global__ __launch_bounds__(256) void sparse_step_kernel(float *table, float *s
     if constexpr (ADAGRAD) {
         float sq = 0.0f;
         for (int j = lane * V; j < d; j += kWave * V) {
-            const RowPiece<V> at(j, d);
+            const RowPiece<V, RAG> at(j, d);
             const Vec<V> gv = Vec<V>::load(g + at.at);
 #pragma unroll
             for (int e = 0; e < V; ++e) sq += e >= at.skip ? gv.v[e] * gv.v[e] : 0.0f;
@@ -31,7 +31,7 @@ __global__ __launch_bounds__(256) void sparse_step_kernel(float *table, float *s
         scale = lr / (sqrtf(s) + eps);
     }
     for (int j = lane * V; j < d; j += kWave * V) {
-        const RowPiece<V> at(j, d);
+        const RowPiece<V, RAG> at(j, d);
         const Vec<V> gv = Vec<V>::load(g + at.at);
         Vec<V> wv = Vec<V>::load(w + at.at);
 #pragma unroll
@@ -159,12 +159,9 @@ static int launch_step(float *table, float *state, int64_t dim, const int64_t *i
         return KGE_OK;
     }
     const dim3 grid((unsigned)ceil_div(capacity, 4)), block(256);
-    if (quad_row(dim))
-        hipLaunchKernelGGL((sparse_step_kernel<ADAGRAD, 4>), grid, block, 0, st, table, state, (int)dim, ids, num_unique,
-                           rows, lr, eps);
-    else
-        hipLaunchKernelGGL((sparse_step_kernel<ADAGRAD, 1>), grid, block, 0, st, table, state, (int)dim, ids, num_unique,
-                           rows, lr, eps);
+    const auto kernel = dim % 4 == 0 ? sparse_step_kernel<ADAGRAD, 4, false>
+                                     : (quad_row(dim) ? sparse_step_kernel<ADAGRAD, 4, true> : sparse_step_kernel<ADAGRAD, 1, false>);
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, table, state, (int)dim, ids, num_unique, rows, lr, eps);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

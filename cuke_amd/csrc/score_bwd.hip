@@ -734,13 +734,16 @@ __device__ __forceinline__ Vec<V> ldz(const float *p, int j)
 // With negatives that replace the tail the query is built from (h, r); with HEAD it is built from
 // (x, rho) = (t, -r) [TransE, TransH], (t, conj r) [ComplEx], (t, -theta) [RotatE], (t, r) [DistMult],
 // so G chains into the t and r rows instead and the positive triple's own term is kept apart.
-template <int MODEL, int P, int V, bool HEAD>
+// RIDE: inspector workgroups may be aboard (see score_pos_kernel)
+template <int MODEL, int P, int V, bool HEAD, bool RAG, bool RIDE>
 __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi)
 {
     extern __shared__ __align__(16) char dyn_smem[];  // inspector workgroups only
-    if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
+    if constexpr (RIDE) {
+        if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
+    }
     const int lane = threadIdx.x & (kWave - 1);
-    const int64_t b = (int64_t)((int)blockIdx.x - fi.blocks) * 4 + (threadIdx.x >> 6);
+    const int64_t b = (int64_t)((int)blockIdx.x - (RIDE ? fi.blocks : 0)) * 4 + (threadIdx.x >> 6);
     if (b >= a.B) return;  // whole waves leave together; no block-level sync below
     const int d = a.d, half = d >> 1;
     const int64_t rid = a.r[b];
@@ -759,7 +762,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
 
     if constexpr (MODEL == KGE_TRANSE) {
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const int j = RowPiece<V>(j0, d).at;
+            const int j = RowPiece<V, RAG>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
             const Vec<V> G = ldz<V>(g0, j);
             Vec<V> dh, dt;
@@ -782,7 +785,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         }
     } else if constexpr (MODEL == KGE_DISTMULT) {
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const int j = RowPiece<V>(j0, d).at;
+            const int j = RowPiece<V, RAG>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
             const Vec<V> G = ldz<V>(g0, j);
             Vec<V> dh, dr, dt;
@@ -803,7 +806,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             S = wave_sum(S);
         }
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const int j = RowPiece<V>(j0, d).at;
+            const int j = RowPiece<V, RAG>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
             const Vec<V> G = ldz<V>(g0, j);
             Vec<V> dh, dr, dt;
@@ -824,7 +827,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         }
     } else if constexpr (MODEL == KGE_COMPLEX) {
         for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
-            const int j = RowPiece<V>(j0, half).at;
+            const int j = RowPiece<V, RAG>(j0, half).at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> qr = Vec<V>::load(rr + j), qi = Vec<V>::load(rr + half + j);
@@ -845,7 +848,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         }
     } else if constexpr (MODEL == KGE_ROTATE) {
         for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
-            const int j = RowPiece<V>(j0, half).at;
+            const int j = RowPiece<V, RAG>(j0, half).at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> th = Vec<V>::load(rr + j);
@@ -886,7 +889,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         float *ow = a.occ_w + b * (int64_t)d;
         float sd = 0.0f;
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vw = Vec<V>::load(w + j);
 #pragma unroll
@@ -895,7 +898,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         sd = wave_sum(sd);
         float qw = 0.0f, gw = 0.0f;  // q_pos . w and G_q . w
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j),
                          vw = Vec<V>::load(w + j);
@@ -911,7 +914,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         qw = wave_sum(qw);
         gw = wave_sum(gw);
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const int j = RowPiece<V>(j0, d).at;
+            const int j = RowPiece<V, RAG>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j),
                          vw = Vec<V>::load(w + j);
             const Vec<V> G = ldz<V>(g0, j), Gw = ldz<V>(g1, j);
@@ -944,13 +947,15 @@ static int launch_pos_bwd(const PosBwdArgs &a, bool vec4, bool head, const Fused
 {
     const dim3 grid((unsigned)ceil_div(a.B, 4) + (unsigned)fi.blocks), block(256);
     const size_t lds = fi.blocks > 0 ? (size_t)fi.lds_bytes : 0;
-    if (head) {
-        if (vec4) hipLaunchKernelGGL((bwd_pos_kernel<MODEL, P, 4, true>), grid, block, lds, st, a, fi);
-        else hipLaunchKernelGGL((bwd_pos_kernel<MODEL, P, 1, true>), grid, block, lds, st, a, fi);
-    } else {
-        if (vec4) hipLaunchKernelGGL((bwd_pos_kernel<MODEL, P, 4, false>), grid, block, lds, st, a, fi);
-        else hipLaunchKernelGGL((bwd_pos_kernel<MODEL, P, 1, false>), grid, block, lds, st, a, fi);
-    }
+    auto launch = [&](auto htag, auto ride) {
+        constexpr bool HEAD = decltype(htag)::value, RIDE = decltype(ride)::value;
+        const auto kernel = vec4 ? (whole_quads<MODEL>(a.d) ? bwd_pos_kernel<MODEL, P, 4, HEAD, false, RIDE> : bwd_pos_kernel<MODEL, P, 4, HEAD, true, RIDE>)
+                                 : bwd_pos_kernel<MODEL, P, 1, HEAD, false, RIDE>;
+        hipLaunchKernelGGL(kernel, grid, block, lds, st, a, fi);
+    };
+    auto by_rider = [&](auto htag) { fi.blocks > 0 ? launch(htag, std::true_type{}) : launch(htag, std::false_type{}); };
+    if (head) by_rider(std::true_type{});
+    else by_rider(std::false_type{});
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

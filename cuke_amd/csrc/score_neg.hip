@@ -13,6 +13,7 @@
 #include <type_traits>
 
 #include "inspector_mid.hpp"
+#include "mfma_split.hpp"
 #include "score_pos_body.hpp"
 #include "tile_common.hpp"
 
@@ -50,6 +51,13 @@ constexpr int kKD = 32;        // floats of each row staged per step
 constexpr int kLDW = kKD + 4;  // LDS row pitch: +4 floats keeps 128-bit reads of
                                // 8 consecutive rows on distinct banks
 
+template <int MODEL, int P>
+__device__ __forceinline__ void carried_positives(const PosArgs &a, int64_t blk)
+{
+    if (whole_quads<MODEL>(a.d)) score_pos_body<MODEL, P, 4, false, false>(a, nullptr, blk);
+    else score_pos_body<MODEL, P, 4, true, false>(a, nullptr, blk);
+}
+
 // One element of the pair update, per model.
 template <int MODEL, int P, bool SAVE>
 __device__ __forceinline__ void pair_elem(float &acc, float &acc2, float a0, float a1, float t0, float t1,
@@ -74,14 +82,16 @@ __device__ __forceinline__ void pair_elem(float &acc, float &acc2, float a0, flo
     }
 }
 
-template <int MODEL, int P, int RB, int RK, bool SAVE, bool VEC4>
+// RIDE: inspector workgroups may be aboard (and no positives are carried); their code costs the tiles registers and instruction cache
+template <int MODEL, int P, int RB, int RK, bool SAVE, bool VEC4, bool RIDE>
 __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a, FusedInsp fi)
 {
     extern __shared__ __align__(16) char dyn_smem[];
-    if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
-    if constexpr (MODEL == KGE_TRANSE) {  // the positives carried along (NegArgs::pos)
-        if (a.pos_blocks > 0 && (int)blockIdx.x - fi.blocks >= a.tile_blocks) {
-            score_pos_body<MODEL, P, 4>(a.pos, nullptr, (int64_t)((int)blockIdx.x - fi.blocks - a.tile_blocks));
+    if constexpr (RIDE) {
+        if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
+    } else if constexpr (MODEL == KGE_TRANSE) {  // the positives carried along (NegArgs::pos)
+        if (a.pos_blocks > 0 && (int)blockIdx.x >= a.tile_blocks) {
+            carried_positives<MODEL, P>(a.pos, (int64_t)((int)blockIdx.x - a.tile_blocks));
             return;
         }
     }
@@ -100,7 +110,7 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     const int srow = tid >> 3, scol = (tid & 7) * 4;
     int c, tile_y, tile_x;
-    int lid = blockIdx.x - fi.blocks, split = 0;
+    int lid = (int)blockIdx.x - (RIDE ? fi.blocks : 0), split = 0;
     if (a.ksplit > 1) {  // (never TransH: its w . t' sweep needs the whole row)
         const int tiles = a.tile_blocks / a.ksplit;  // a multiple of 8: the tile keeps its XCD
         split = lid / tiles, lid -= split * tiles;
@@ -367,17 +377,19 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
 // s pairs lane group g = l / 16 with k = 4 g + s (any pairing works as long as both operands use
 // it), so a lane's values for four steps are one 128-bit LDS read of its row.
 
-template <int MODEL, int RB, int RK, bool VEC4>
+template <int MODEL, int RB, int RK, bool VEC4, bool RIDE>
 __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_mfma_kernel(NegArgs a, FusedInsp fi)
 {
     extern __shared__ __align__(16) char dyn_smem[];
-    if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
     static_assert(MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL,
                   "dot-product scores only");
-    if (a.pos_blocks > 0 && (int)blockIdx.x - fi.blocks >= a.tile_blocks) {  // the positives carried along
-        if constexpr (MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX)
-            score_pos_body<MODEL, 2, 4>(a.pos, nullptr, (int64_t)((int)blockIdx.x - fi.blocks - a.tile_blocks));
-        return;
+    if constexpr (RIDE) {
+        if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
+    } else if constexpr (MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX) {  // the positives carried along
+        if (a.pos_blocks > 0 && (int)blockIdx.x >= a.tile_blocks) {
+            carried_positives<MODEL, 2>(a.pos, (int64_t)((int)blockIdx.x - a.tile_blocks));
+            return;
+        }
     }
     constexpr int TB = 16 * RB, TN = 16 * RK;
     constexpr int SB = TB / 32, SN = TN / 32;
@@ -393,7 +405,7 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_mfma_kernel(NegAr
     const int fr = lane & 15, fg = lane >> 4;
     const int wrow = (wave >> 1) * (TB / 2), wcol = (wave & 1) * (TN / 2);
     int c, tile_y, tile_x;
-    if (!xcd_tile(blockIdx.x - fi.blocks, (a.N + TN - 1) / TN, (a.C + TB - 1) / TB, a.n_chunks, c, tile_y, tile_x)) return;
+    if (!xcd_tile((int)blockIdx.x - (RIDE ? fi.blocks : 0), (a.N + TN - 1) / TN, (a.C + TB - 1) / TB, a.n_chunks, c, tile_y, tile_x)) return;
     const int bt0 = tile_y * TB, kt0 = tile_x * TN;
     const int d = a.d, half = d >> 1;
     constexpr bool kSplit = MODEL == KGE_COMPLEX && VEC4;  // (the reduction axis: see score_neg_kernel)
@@ -499,6 +511,169 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_mfma_kernel(NegAr
         }
 }
 
+// Large batches of dot-product scores (one chunk against a whole table, chunks of hundreds): 64 MB positives x 128 negatives per
+// workgroup on the bf16 matrix cores (mfma_split.hpp).  The query rows come as an array: the per-positive kernel writes them (RESCAL: the
+// projected rows), since a tile that formed them again from two to four table rows pulled twice the bytes out of L2.
+// A 64 x 64 quarter per wave (a 32 x 64 one reads half as much again out of LDS); two workgroups per CU, one of which stages and
+// splits while the other multiplies.
+//   512 queries x 14951 candidates, width 400: 100 -> 50 us (v_mfma_f32_16x16x4_f32 in 64 x 64 tiles, same box), 122 TFLOP/s; per slice
+//   of 32 columns 2.9 us = 171 TFLOP/s, 1.03 PFLOP/s of bf16, where a large bf16 library product reaches 1.23 on this card: the
+//   matrix cores bound it, and 18 us are the launches, the index chains and the first rows.  16384 x 1024 x 400: 150 -> 110 us.
+//   Built and no faster: eight waves around two LDS buffers with one barrier per slice (54 -> 59 us), the same with fragment reads and
+//   splitting scheduled between the products (60 us), rows touched two slices ahead (54 us).
+template <int MB>
+constexpr size_t split_lds() { return sizeof(__bf16) * kSplitPitch * (64 * MB + 128); }
+
+// Tiles of one column block follow each other on one XCD: the negatives' rows are the large side (a whole table), and one L2 then reads
+// each of them once; the queries fit every L2.
+__device__ __forceinline__ bool xcd_tile_by_cols(int lid, int tiles_x, int tiles_y, int n_chunks, int &c, int &ty, int &tx)
+{
+    const int split = xcd_split(n_chunks), per_v = (tiles_x + split - 1) / split * tiles_y;
+    const int xcd = lid % kXcds, k = lid / kXcds, vc = (k / per_v) * kXcds + xcd;
+    c = vc / split;
+    const int t = k % per_v;
+    ty = t % tiles_y;
+    tx = (t / tiles_y) * split + vc % split;
+    return c < n_chunks && tx < tiles_x;
+}
+static unsigned xcd_grid_by_cols(int64_t tiles_x, int64_t tiles_y, int64_t n_chunks)
+{
+    const int64_t split = xcd_split((int)n_chunks);
+    return (unsigned)(kXcds * ceil_div(n_chunks * split, kXcds) * ceil_div(tiles_x, split) * tiles_y);
+}
+
+struct SplitArgs {
+    const float *query, *ent;   // query rows [B, d]
+    const int64_t *neg;
+    const float *shift;         // TransF: r_b . (kept side), or null
+    float *out;                 // [B, N]
+    int C, N, d, n_chunks;
+    float rsign;
+};
+
+template <int MB>
+__global__ __launch_bounds__(256, 2) void score_neg_split_kernel(SplitArgs a, FusedInsp fi)
+{
+    extern __shared__ __align__(16) char dyn_smem[];
+    if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
+    constexpr int TB = 64 * MB, TN = 128, NB = 2, SB = TB / 32, SN = TN / 32;
+    __bf16(*sA)[kSplitPitch] = reinterpret_cast<__bf16(*)[kSplitPitch]>(dyn_smem);
+    __bf16(*sT)[kSplitPitch] = sA + TB;
+    const int tid = threadIdx.x, srow = tid >> 3, scol = (tid & 7) * 4;
+    const int lane = tid & 63, wave = tid >> 6, fr = lane & 31, fg = lane >> 5;
+    const int wrow = (wave >> 1) * (TB / 2), wcol = (wave & 1) * (TN / 2);
+    const int d = a.d;
+    int c, tile_y, tile_x;
+    if (!xcd_tile_by_cols((int)blockIdx.x - fi.blocks, (a.N + TN - 1) / TN, (a.C + TB - 1) / TB, a.n_chunks, c, tile_y, tile_x)) return;
+    const int bt0 = tile_y * TB, kt0 = tile_x * TN;
+
+    // rows this thread stages (past the tile's edge: its last row again; scores of such rows are not stored)
+    const float *pa[SB], *pt[SN];
+#pragma unroll
+    for (int s = 0; s < SB; ++s) pa[s] = a.query + ((int64_t)c * a.C + min(bt0 + srow + 32 * s, a.C - 1)) * d;
+#pragma unroll
+    for (int s = 0; s < SN; ++s) pt[s] = a.ent + a.neg[(int64_t)c * a.N + min(kt0 + srow + 32 * s, a.N - 1)] * (int64_t)d;
+    float4 ra[SB], rt[SN];
+    auto load_slice = [&](int j0) {
+#pragma unroll
+        for (int s = 0; s < SB; ++s) ra[s] = ld4_raw<true>(pa[s], j0 + scol, d);
+#pragma unroll
+        for (int s = 0; s < SN; ++s) rt[s] = ld4_raw<true>(pt[s], j0 + scol, d);
+    };
+    auto put = [&](__bf16 *row, float4 v) {
+        bf16x4 p[kSplitParts];
+        split_quad(v, p);
+#pragma unroll
+        for (int q = 0; q < kSplitParts; ++q) *reinterpret_cast<bf16x4 *>(row + q * kSplitK + scol) = p[q];
+    };
+
+    floatx16 lead[MB][NB], rest[MB][NB];  // sums of the leading products / of the corrections
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) lead[m][n][v] = 0.0f, rest[m][n][v] = 0.0f;
+
+    load_slice(0);
+#pragma unroll 1
+    for (int j0 = 0; j0 < d; j0 += kSplitK) {
+        if (j0 + kSplitK > d) {  // uniform: the last slice of most widths
+#pragma unroll
+            for (int s = 0; s < SB; ++s) ra[s] = mask4<true>(ra[s], j0 + scol, d);
+#pragma unroll
+            for (int s = 0; s < SN; ++s) rt[s] = mask4<true>(rt[s], j0 + scol, d);
+        }
+#pragma unroll
+        for (int s = 0; s < SB; ++s) put(sA[srow + 32 * s], ra[s]);
+#pragma unroll
+        for (int s = 0; s < SN; ++s) put(sT[srow + 32 * s], rt[s]);
+        __syncthreads();
+        if (j0 + kSplitK < d) load_slice(j0 + kSplitK);
+        __builtin_amdgcn_sched_barrier(0);  // (the requests go out before the products, not after them)
+#pragma unroll
+        for (int u = 0; u < kSplitK / 16; ++u) {
+            bf16x8 av[MB][kSplitParts], tv[NB][kSplitParts];
+#pragma unroll
+            for (int q = 0; q < kSplitParts; ++q) {
+#pragma unroll
+                for (int m = 0; m < MB; ++m) av[m][q] = *reinterpret_cast<const bf16x8 *>(&sA[wrow + 32 * m + fr][q * kSplitK + 16 * u + 8 * fg]);
+#pragma unroll
+                for (int n = 0; n < NB; ++n) tv[n][q] = *reinterpret_cast<const bf16x8 *>(&sT[wcol + 32 * n + fr][q * kSplitK + 16 * u + 8 * fg]);
+            }
+#pragma unroll
+            for (int t = 0; t < kSplitTerms; ++t)
+#pragma unroll
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int n = 0; n < NB; ++n) {
+                        floatx16 &acc = t + 1 < kSplitTerms ? rest[m][n] : lead[m][n];
+                        acc = mfma_bf16(av[m][kTermA[t]], tv[n][kTermB[t]], acc);
+                    }
+        }
+        __syncthreads();
+    }
+
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int bl = bt0 + wrow + 32 * m + 8 * (v >> 2) + 4 * fg + (v & 3);
+            if (bl >= a.C) continue;
+            const int64_t b = (int64_t)c * a.C + bl;
+            const float shift = a.shift ? -a.rsign * a.shift[b] : 0.0f;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const int kl = kt0 + wcol + 32 * n + fr;
+                if (kl >= a.N) continue;
+                float s = lead[m][n][v] + rest[m][n][v];
+                if (s != s) s = pair_dot(a.query + b * d, a.ent + a.neg[(int64_t)c * a.N + kl] * (int64_t)d, d);
+                a.out[b * a.N + kl] = s + shift;
+            }
+        }
+}
+
+// Whether the dot-product scores of this batch go by the split tiles: both sides of the line measured against the fp32 tiles (time
+// of a whole score call, DistMult / ComplEx / TransF).
+//   128 x 128 tiles, two per CU at a time: 468 tiles at width 400 1.6 / 1.8 / 1.5 times faster, 512 at 200 1.1 / 1.3 / 1.1; 256 tiles,
+//   one per CU and nothing to take turns with, 0.81 / 0.88 / 0.85 at width 256.  Short rows are all launch: 512 tiles at width 64
+//   0.9 to 1.0, 3128 at 48 0.95 to 1.2.
+//   Chunks of at most 64 (64 x 128 tiles): 16 x 1024 at width 128 1.1 / 1.3 / 1.1, 16 x 512 at 200 1.1 / 1.2 / 1.1; 32 x 256 at 200
+//   0.94 / 1.07 / 0.99.
+static bool dot_model(int model) { return model == KGE_DISTMULT || model == KGE_COMPLEX || model == KGE_TRANSF || model == KGE_RESCAL; }
+static bool want_split(const kge_tables *tab, const kge_batch *bat)
+{
+    if (!dot_model(tab->model) || pair_sums_valu(tab) || !bat->neg || bat->chunk <= 0 || tab->dim < 96) return false;
+    const int64_t n_chunks = bat->batch / bat->chunk, cols = ceil_div(bat->n_neg, 128);
+    if (bat->chunk <= 64) return cols >= 4 && cols * n_chunks >= 1024;
+    return ceil_div(bat->chunk, 128) * cols * n_chunks >= 384;
+}
+// floats of query rows that the per-positive kernel writes for them (RESCAL brings its own)
+size_t split_query_bytes(const kge_tables *tab, const kge_batch *bat)
+{
+    return want_split(tab, bat) && tab->model != KGE_RESCAL ? sizeof(float) * (size_t)(bat->batch * tab->dim) : 0;
+}
+
 // LDS bytes of a launch: the tile's staging buffers, or what the inspector workgroups need if more
 static size_t neg_lds(int planes, int TB, int TN, int planes_t, const FusedInsp &fi)
 {
@@ -550,10 +725,13 @@ static void launch_neg_k(K kernel, dim3 grid, size_t lds, hipStream_t st, const 
 {
     hipLaunchKernelGGL(kernel, grid, dim3(256), lds, st, a, fi);
 }
-#define NEG_LAUNCH(KERNEL, ...)                                                    \
-    (a.vec ? launch_neg_k(KERNEL<__VA_ARGS__, true>, grid, lds, st, a, fi)         \
-           : launch_neg_k(KERNEL<__VA_ARGS__, false>, grid, lds, st, a, fi))
-#define NEG_LAUNCH_VEC(KERNEL, ...) launch_neg_k(KERNEL<__VA_ARGS__, true>, grid, lds, st, a, fi)
+#define NEG_LAUNCH_VEC(KERNEL, ...)                                                    \
+    (fi.blocks > 0 ? launch_neg_k(KERNEL<__VA_ARGS__, true, true>, grid, lds, st, a, fi) \
+                   : launch_neg_k(KERNEL<__VA_ARGS__, true, false>, grid, lds, st, a, fi))
+#define NEG_LAUNCH(KERNEL, ...)                                                             \
+    (a.vec              ? NEG_LAUNCH_VEC(KERNEL, __VA_ARGS__)                                \
+     : (fi.blocks > 0) ? launch_neg_k(KERNEL<__VA_ARGS__, false, true>, grid, lds, st, a, fi) \
+                        : launch_neg_k(KERNEL<__VA_ARGS__, false, false>, grid, lds, st, a, fi))
 
 template <int MODEL, int P>
 static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, const FusedInsp &fi, hipStream_t st)
@@ -637,8 +815,20 @@ int launch_score_neg(const kge_tables *tab, const kge_batch *bat, const float *s
               vec ? 1 : 0, (int)n_chunks, head ? -1.0f : 1.0f, 1, nullptr, PosArgs{}, 0, 0};
     if (carry_pos) {
         a.pos = PosArgs{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, bat->batch, (int)tab->dim, (int)tab->rel_dim,
-                        tab->gamma, carry_pos, nullptr, nullptr, 0};
+                        tab->gamma, carry_pos, nullptr, nullptr, nullptr, 0};
         a.pos_blocks = (int)ceil_div(bat->batch, kPosWaves);
+    }
+    if (query && want_split(tab, bat)) {
+        const SplitArgs s{query, tab->ent, bat->neg, tab->model == KGE_TRANSF ? side_pos : nullptr, out, (int)bat->chunk, (int)bat->n_neg,
+                          (int)tab->dim, (int)n_chunks, a.rsign};
+        const bool tall = bat->chunk > 64;
+        const unsigned grid = xcd_grid_by_cols(ceil_div(bat->n_neg, 128), ceil_div(bat->chunk, tall ? 128 : 64), n_chunks) + (unsigned)fi.blocks;
+        size_t lds = tall ? split_lds<2>() : split_lds<1>();
+        if (fi.blocks > 0 && (size_t)fi.lds_bytes > lds) lds = (size_t)fi.lds_bytes;
+        if (tall) hipLaunchKernelGGL(score_neg_split_kernel<2>, dim3(grid), dim3(256), lds, st, s, fi);
+        else hipLaunchKernelGGL(score_neg_split_kernel<1>, dim3(grid), dim3(256), lds, st, s, fi);
+        KGE_CHECK_LAUNCH();
+        return KGE_OK;
     }
     // the reduction axis is split when the caller's workspace has room for the partial planes
     const int ksplit = neg_ksplit(tab, bat);

@@ -17,6 +17,7 @@ struct PosArgs {
     float *resid;     // [B, d] or nullptr: residual rows (TransE / TransH / TransR), the projected heads
                       // E[h] Proj[r] (RESCAL) or, for RotatE, the rotated heads h e^{i theta} laid out [re | im]
     float *side_pos;  // [B] TransH: w.h; TransF: r.h (used by the shared-negative kernels)
+    float *query;     // [B, d] or nullptr, DistMult / ComplEx / TransF: the query rows of the shared negatives (tile_common.hpp)
     int head;         // negatives replace the head: side_pos = w.t / r.t, RotatE resid = t e^{-i theta}
 };
 
@@ -30,7 +31,8 @@ __device__ __forceinline__ float norm_term(float u)
 
 // The work of one workgroup of kPosWaves positives: block `blk` takes the positives
 // blk * kPosWaves .. + kPosWaves - 1.  `lds`: kPosWaves * d floats for TransR / RESCAL, else unused.
-template <int MODEL, int P, int V>
+// QUERY: PosArgs::query may be set
+template <int MODEL, int P, int V, bool RAG, bool QUERY>
 __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int64_t blk)
 {
     const int lane = threadIdx.x & (kWave - 1);
@@ -48,7 +50,7 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
 
     if constexpr (MODEL == KGE_TRANSE) {
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j);
@@ -64,7 +66,7 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
         const float *w = a.aux + rid * (int64_t)d;
         float sd = 0.0f, wh = 0.0f;
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vw = Vec<V>::load(w + j);
@@ -78,7 +80,7 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
         wh = wave_sum(wh);
         if (a.side_pos && valid && lane == 0) a.side_pos[b] = wh;
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j), vw = Vec<V>::load(w + j);
@@ -99,7 +101,7 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
         for (int i = lane; i < d; i += kWave) x[i] = MODEL == KGE_TRANSR ? eh[i] - et[i] : eh[i];
         __syncthreads();
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             Vec<V> s;
 #pragma unroll
@@ -127,17 +129,23 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
         }
     } else if constexpr (MODEL == KGE_DISTMULT) {
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j);
 #pragma unroll
             for (int e = 0; e < V; ++e) acc += e >= at.skip ? (vh.v[e] * vr.v[e]) * vt.v[e] : 0.0f;
+            if (QUERY && a.query && valid) {
+                Vec<V> q;
+#pragma unroll
+                for (int e = 0; e < V; ++e) q.v[e] = (a.head ? vt.v[e] : vh.v[e]) * vr.v[e];
+                q.store(a.query + bb * (int64_t)d + j);
+            }
         }
     } else if constexpr (MODEL == KGE_TRANSF) {
         float rx = 0.0f;  // r . (the side the shared negatives keep)
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
-            const RowPiece<V> at(j0, d);
+            const RowPiece<V, RAG> at(j0, d);
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j),
                          vr = Vec<V>::load(rr + j);
@@ -147,6 +155,12 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
                 acc += (vh.v[e] + vr.v[e]) * vt.v[e] + (vt.v[e] - vr.v[e]) * vh.v[e];
                 rx += vr.v[e] * (a.head ? vt.v[e] : vh.v[e]);
             }
+            if (QUERY && a.query && valid) {
+                Vec<V> q;
+#pragma unroll
+                for (int e = 0; e < V; ++e) q.v[e] = fmaf(a.head ? -1.0f : 1.0f, vr.v[e], 2.0f * (a.head ? vt.v[e] : vh.v[e]));
+                q.store(a.query + bb * (int64_t)d + j);
+            }
         }
         if (a.side_pos) {  // uniform
             rx = wave_sum(rx);
@@ -155,7 +169,7 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
     } else if constexpr (MODEL == KGE_COMPLEX) {
         const int half = d / 2;
         for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
-            const RowPiece<V> at(j0, half);
+            const RowPiece<V, RAG> at(j0, half);
             const int j = at.at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
@@ -166,11 +180,21 @@ __device__ __forceinline__ void score_pos_body(const PosArgs &a, float *lds, int
                 const float ai = hr.v[e] * qi.v[e] + hi.v[e] * qr.v[e];
                 acc += e >= at.skip ? ar * tr.v[e] + ai * ti.v[e] : 0.0f;
             }
+            if (QUERY && a.query && valid) {
+                Vec<V> qre, qim;
+                const float rs = a.head ? -1.0f : 1.0f;
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    const float kr = a.head ? tr.v[e] : hr.v[e], ki = a.head ? ti.v[e] : hi.v[e], ri = rs * qi.v[e];
+                    qre.v[e] = kr * qr.v[e] - ki * ri, qim.v[e] = kr * ri + ki * qr.v[e];
+                }
+                qre.store(a.query + bb * (int64_t)d + j), qim.store(a.query + bb * (int64_t)d + half + j);
+            }
         }
     } else if constexpr (MODEL == KGE_ROTATE) {
         const int half = d / 2;
         for (int j0 = lane * V; j0 < half; j0 += kWave * V) {
-            const RowPiece<V> at(j0, half);
+            const RowPiece<V, RAG> at(j0, half);
             const int j = at.at;
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, Sum
     {
         const int colv = c0 + lane * V;
         const bool active = colv < d;
-        const int cc = active ? RowPiece<V>(colv, d).at : 0;
+        const int cc = active ? RowPiece<V, V == 4>(colv, d).at : 0;
         Vec<V> acc;
 #pragma unroll
         for (int e = 0; e < V; ++e) acc.v[e] = 0.0f;

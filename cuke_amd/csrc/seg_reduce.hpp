@@ -110,7 +110,7 @@ __device__ __forceinline__ void seg_l1_wave(const SegArgs &a, int64_t w)
         wsign[q] = second ? -1.0f : 1.0f;
         src[q] = second ? src[q] - a.wrap : src[q];
     }
-    const int cc = active ? RowPiece<V>(colv, d).at : 0;  // (a last piece moved back: the same sums twice)
+    const int cc = active ? RowPiece<V, V == 4>(colv, d).at : 0;  // (a last piece moved back: the same sums twice)
     Vec<V> v[kSegL];
 #pragma unroll
     for (int q = 0; q < kSegL; ++q) v[q] = Vec<V>::load(a.occ + (int64_t)src[q] * d + cc);

@@ -297,6 +297,12 @@ inline unsigned xcd_grid(int64_t tiles_x, int64_t tiles_y, int64_t n_chunks)
     return (unsigned)(kXcds * ceil_div(n_chunks * split, kXcds) * ceil_div(per, split));
 }
 
+// every row segment is a whole number of quads
+template <int MODEL>
+__host__ __device__ inline bool whole_quads(int d)
+{
+    return d % (MODEL == KGE_COMPLEX || MODEL == KGE_ROTATE ? 8 : 4) == 0;
+}
 // 128-bit row loads: every row segment (ComplEx, RotatE: each half) has at least four floats
 inline bool rows_by_quads(const kge_tables *tab)
 {

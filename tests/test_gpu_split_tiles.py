@@ -1,0 +1,71 @@
+"""Dot-product scores on the bf16 matrix cores (three-part splits): tile edges, widths, shapes on both sides of the rule, no worse than
+fp32 against 64 bits, infinities and NaNs as fp32 gives them."""
+import numpy as np
+import pytest
+import torch
+
+from cuke_amd.kge import KGEModel
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(model, n_ent, dim, batch, n_neg, chunks, seed, scale=0.05):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    E, R = (torch.randn(n, dim, generator=g, device="cuda") * scale for n in (n_ent, 7))
+    ids = lambda n, k: torch.randint(0, n, (k,), generator=g, device="cuda")
+    return E, R, ids(n_ent, batch), ids(7, batch), ids(n_ent, batch), ids(n_ent, chunks * n_neg)
+
+
+def _exact(model, E, R, h, r, t, neg, chunk, head):
+    """64-bit scores and, per pair, the sum of the products' magnitudes (the scale of fp32 rounding)."""
+    x, r = (E[t] if head else E[h]).double(), R[r].double()
+    n = E[neg].double().view(-1, neg.numel() // (x.shape[0] // chunk), E.shape[1])
+    s = -1.0 if head else 1.0
+    if model == "DistMult":
+        q, shift = x * r, 0
+    elif model == "TransF":
+        q, shift = 2 * x + s * r, -s * (r * x).sum(1, keepdim=True)
+    else:
+        a, b = torch.complex(*x.chunk(2, 1)), torch.complex(r.chunk(2, 1)[0], s * r.chunk(2, 1)[1])
+        q = torch.view_as_real(a * b)
+        q, shift = torch.cat((q[..., 0], q[..., 1]), 1), 0
+    q3 = q.view(-1, chunk, E.shape[1])
+    return (torch.bmm(q3, n.transpose(1, 2).contiguous()).view(x.shape[0], -1) + shift,
+            torch.bmm(q3.abs(), n.abs().transpose(1, 2).contiguous()).view(x.shape[0], -1) + (shift.abs() if torch.is_tensor(shift) else 0))
+
+
+# (dim, chunk, negatives, chunks): 128 x 128 tiles with ragged edges, one chunk against many, 64 x 128 tiles; then below the rule
+SHAPES = [(96, 130, 129, 96), (101, 65, 384, 128), (400, 257, 20481, 1), (131, 128, 127, 384), (200, 33, 513, 205), (98, 64, 512, 256),
+          (95, 130, 129, 96), (128, 130, 129, 32), (200, 33, 300, 205)]
+
+
+@pytest.mark.parametrize("head", [False, True], ids=["tail", "head"])
+@pytest.mark.parametrize("model", ["DistMult", "ComplEx", "TransF"])
+@pytest.mark.parametrize("dim,chunk,n_neg,chunks", SHAPES)
+def test_scores_against_64_bits(model, dim, chunk, n_neg, chunks, head):
+    if model == "ComplEx":
+        dim += dim % 2
+    E, R, h, r, t, neg = _case(model, 3000, dim, chunk * chunks, n_neg, chunks, dim + n_neg)
+    fw = KGEModel(model, E, R).score(h, r, t, neg, chunk, neg_mode="head" if head else "tail")
+    want, size = _exact(model, E, R, h, r, t, neg, chunk, head)
+    # fp32: the query's own rounding (up to 3 roundings) and the sum's, sqrt(dim) half ulps of the terms' total at most
+    err = (fw.neg.double() - want).abs()
+    assert bool((err <= 2.0 ** -24 * (4 + dim ** 0.5) * size).all()), float((err / size).max() * 2 ** 24)
+
+
+def test_infinities_and_nans_as_fp32_has_them():
+    E, R, h, r, t, neg = _case("DistMult", 3000, 128, 512, 12288, 1, 3, scale=1.0)
+    R.fill_(1.0), E.abs_()
+    E[5, 7], E[6, 8], E[9, 3], E[11, 100], E[12, 127] = float("inf"), float("nan"), 3.4e38, -float("inf"), 1e-30
+    E[13].zero_()
+    h[:6] = torch.tensor([5, 6, 9, 11, 12, 13], device="cuda")
+    neg[:6] = h[:6]
+    fw = KGEModel("DistMult", E, R).score(h, r, t, neg, 512)
+    q, n = E[h].cpu(), E[neg].cpu()
+    want = torch.stack([(q[i] * n[:200]).sum(1) for i in range(200)])
+    got = fw.neg[:200, :200].cpu()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    fine = want.isfinite()
+    assert torch.equal(got[~fine].nan_to_num(nan=0.0), want[~fine].nan_to_num(nan=0.0))
+    assert torch.allclose(got[fine], want[fine], rtol=1e-5)

@@ -53,3 +53,14 @@ def test_inspect_multi_part_ragged(oracle):
     rng = np.random.default_rng(3)
     parts = [rng.integers(0, 777, k, dtype=np.int64) for k in (5, 0, 2047, 1)]
     check(oracle, parts, 777)
+
+
+@pytest.mark.parametrize("n_rows", [1, 2, 128, 512, 513, 129 << 7, 1 << 21, 1 << 32])
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 2047, 2048, 2049, 3071, 4095, 4096, 4097])
+def test_inspect_in_one_workgroup_and_past_it(oracle, n, n_rows):
+    """Edges of the one-workgroup kernel: keys per thread, digits of one to five passes, what goes to the launches behind it."""
+    rng = np.random.default_rng(n * 7 + n_rows)
+    ids = rng.integers(0, n_rows, n, dtype=np.int64)
+    check(oracle, [ids], n_rows)
+    check(oracle, [ids[:n // 3], np.minimum(ids[n // 3:], n_rows // 5)], n_rows)
+    check(oracle, [np.full(n, n_rows - 1, np.int64)], n_rows)

@@ -126,7 +126,13 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     constexpr bool kRot = MODEL == KGE_ROTATE, kTH = MODEL == KGE_TRANSH;
     constexpr bool kDot = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF ||
                           MODEL == KGE_RESCAL;  // score = query . t' (+ const)
-    constexpr bool kMf = kDot && MF;  // the sum over loopers on the matrix cores (else on the vector ALUs)
+    // TransE, L2: sum_l g_l (o - x_l) = o sum_l g_l - sum_l g_l x_l, the owner's row times its coefficients' sum and the dot models'
+    // product, folded once per step like the differences' sum it replaces.  2-norm of the entity rows' error against 64 bits,
+    // differences -> product: margin loss 8.2e-8 -> 7.3e-8 (3000 x 600 x 200 negatives x 150), 9.5e-8 -> 8.5e-8 (1024 x 1024 x 400), gradients of
+    // both signs 1.63e-7 -> 1.54e-7 and 2.17e-7 -> 2.09e-7; unfolded 9.9e-8 / 1.3e-7 / 3.2e-7 / 4.8e-7.
+    // The two orientations at 30000 x 200 x 150: 204 -> 113 us.
+    constexpr bool kDiff = MODEL == KGE_TRANSE && P == 2 && MF;
+    constexpr bool kMf = (kDot || kDiff) && MF;  // the sum over loopers on the matrix cores (else on the vector ALUs)
     constexpr bool kL2 = (MODEL == KGE_TRANSE || kTH) && P == 2;
     // L1 translation models: owner and looper rows carry the factor 2^100, so the sign of a residual
     // element is a single clamp (sgn_of_scaled, tile_common.hpp); the coefficient that multiplies a
@@ -199,7 +205,7 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             const int64_t rid = a.r[b];
             if constexpr (kTH) alo[o] = a.side_pos[b];
             float4 q0 = zero4(), q1 = zero4();
-            if constexpr (!kDot)
+            if constexpr (!kDot && !kDiff)
                 load_query<MODEL, VEC>(a.ent + a.h[b] * (int64_t)d, a.rel + rid * (int64_t)a.rel_dim,
                                        kTH ? a.aux + rid * (int64_t)d : nullptr, kRot ? a.query + b * (int64_t)d : nullptr, alo[o],
                                        col, lim, half, a.rsign, q0, q1);
@@ -207,7 +213,7 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             if constexpr (NPO == 2) own[1][o] = q1;
         } else {
             const float *pt = a.ent + a.neg[(int64_t)c * a.N + oc] * (int64_t)d;
-            own[0][o] = kDot ? zero4() : ld4<VEC>(pt, col, lim);
+            own[0][o] = kDot || kDiff ? zero4() : ld4<VEC>(pt, col, lim);
             if constexpr (NPO == 2) own[1][o] = ld4<VEC>(pt + half, col, lim);
         }
         if constexpr (kSc) {
@@ -232,6 +238,7 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     constexpr int EW = 4;  // MFMAs (columns per lane) per wave
     static_assert(!kMf || TO == 64, "a wave per 16 of 64 owners");
     const int mlane = tid & 63, ob = tid >> 6, fj = mlane & 15, fg = mlane >> 4;
+    float csum = 0.0f;  // kDiff: this lane's share of the coefficients of owner 16 ob + fj
     v4f macc[EW];
 #pragma unroll
     for (int e = 0; e < EW; ++e) macc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
@@ -401,18 +408,32 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
         // into the running one per step, so rounding grows with sqrt(steps) of the large partial
         // sums instead of sqrt(loopers)
         if constexpr (kMf) {
+            v4f mstep[EW];
+            float cstep = 0.0f;
+            if constexpr (kDiff) {
+#pragma unroll
+                for (int e = 0; e < EW; ++e) mstep[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            }
 #pragma unroll
             for (int q = 0; q < kKL / 16; ++q)
 #pragma unroll
                 for (int ms = 0; ms < 4; ++ms) {
                     const int l = 16 * q + 4 * fg + ms;
                     const float av = sG[0][l][ob * 16 + fj];
+                    if constexpr (kDiff) cstep += av;
                     const float4 b4 = *reinterpret_cast<const float4 *>(&sL[0][l][4 * fj]);
                     const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
-                    for (int e = 0; e < EW; ++e)
-                        macc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], macc[e], 0, 0, 0);
+                    for (int e = 0; e < EW; ++e) {
+                        v4f &acc = kDiff ? mstep[e] : macc[e];
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], acc, 0, 0, 0);
+                    }
                 }
+            if constexpr (kDiff) {
+                csum += cstep;
+#pragma unroll
+                for (int e = 0; e < EW; ++e) macc[e] += mstep[e];
+            }
         }
         float4 sacc[NOUT][RO_];
 #pragma unroll
@@ -565,6 +586,30 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                 return;
             }
         }
+        if constexpr (kDiff) {
+            csum += __shfl_xor(csum, 16, kWave);
+            csum += __shfl_xor(csum, 32, kWave);
+            const int c0 = gcol(4 * fj);
+            float4 mine[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {  // (rows past the tile's edge: its last row again, not stored)
+                const int oc = min(ot0 + ob * 16 + 4 * fg + v, n_own - 1);
+                if constexpr (OWNER_POS) {
+                    const int64_t b = (int64_t)c * a.C + oc;
+                    float4 none;
+                    load_query<MODEL, VEC>(a.ent + a.h[b] * (int64_t)d, a.rel + a.r[b] * (int64_t)a.rel_dim, nullptr, nullptr, 0.0f, c0, klen, half,
+                                           a.rsign, mine[v], none);
+                } else {
+                    mine[v] = ld4<VEC>(a.ent + a.neg[(int64_t)c * a.N + oc] * (int64_t)d, c0, klen);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float cs = __shfl(csum, 4 * fg + v, kWave);
+                macc[0][v] = fmaf(mine[v].x, cs, -macc[0][v]), macc[1][v] = fmaf(mine[v].y, cs, -macc[1][v]);
+                macc[2][v] = fmaf(mine[v].z, cs, -macc[2][v]), macc[3][v] = fmaf(mine[v].w, cs, -macc[3][v]);
+            }
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int ol = ot0 + ob * 16 + 4 * fg + v;
@@ -665,7 +710,7 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
     const int64_t big = gx * (ceil_div(a.C, 64) + ceil_div(a.N, 64)) * n_chunks;
     // the size rule follows launch_neg_mp (see there)
     constexpr bool kDotModel = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL;
-    if constexpr (kDotModel) {
+    if constexpr (kDotModel || (MODEL == KGE_TRANSE && P == 2)) {
         // matrix-core inner loop (KGE_PAIR_SUMS_VALU keeps the vector-ALU loop): a wave gets all 64
         // columns of its 16 owners with 64-owner tiles, which win at every size
         if (!dot_valu) {

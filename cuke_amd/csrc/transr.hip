@@ -15,6 +15,7 @@
 //   * j: a lane's float4 of four consecutive matrix columns feeds four MFMAs (one per element),
 //     so MFMA e owns columns n0 + 4 (l % 16) + e.
 #include "inspector_mid.hpp"
+#include "mfma_split.hpp"
 #include "seg_reduce.hpp"
 
 namespace kge {

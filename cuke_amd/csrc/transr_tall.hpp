@@ -19,6 +19,8 @@ constexpr int kTallCols = 128;  // columns per workgroup at most: 32 per wave, t
 constexpr int kTallKC = 64;     // columns of the left operand staged at a time
 constexpr int kTallPitch = kTallKC + 4;
 constexpr int kTallRing = 4;    // supersteps (16 rows of k) of the projection in flight per wave, one of them in use
+constexpr int kSplitRows = 16;    // tiles of more rows go by the bf16 matrix cores ...
+constexpr int kSplitItems = 256;  // ... where a launch has more items than that
 constexpr int kTallWgs = 4096;  // workgroups of a launch at most; they stride over the tiles
 // (global, not generic: a pointer that went through LDS would otherwise be followed with flat loads, which also count as LDS
 // operations and are waited for as such)
@@ -29,9 +31,12 @@ struct TallRows {  // what a tile knows about its rows (LDS, behind the staging 
     int64_t t[kTallRows];                      // MODE 1: tail ids
     int b[kTallRows];
     float f[kTallRows], g[kTallRows];          // MODE 3: factor of the relation row, whether there is a t; MODE 2: coefficient, upstream gradient
-    float sum[4][kTallRows];
+    float sum[8][kTallRows];
 };
-constexpr size_t kTallLds = sizeof(float) * 2 * kTallRows * kTallPitch + sizeof(TallRows);
+// staging: two slices of the left operand, or (split tiles) one slice of both operands in three parts
+constexpr size_t kTallStage = sizeof(__bf16) * kSplitPitch * (kTallRows + kTallCols);
+static_assert(kTallStage >= sizeof(float) * 2 * kTallRows * kTallPitch && kTallStage % 16 == 0, "the row table stands behind both forms");
+constexpr size_t kTallLds = kTallStage + sizeof(TallRows);
 
 __device__ __forceinline__ float4 load4g(global_f32 p)
 {
@@ -147,6 +152,35 @@ __device__ __forceinline__ void tall_sweep(const TallLoader<MODE> &bl, int d, Ta
     }
 }
 
+// fills the row table of the tile's `rows` rows from position p0 on (one thread per row; later rows repeat the first)
+template <int MODE>
+__device__ __forceinline__ void tall_rows(const GemmArgs &a, TallRows &R, int p0, int rows, bool array, bool derived)
+{
+    const int tid = threadIdx.x, d = a.d;
+    if (tid < kTallRows) {
+        const int p = p0 + (tid < rows ? tid : 0);
+        int b;
+        if constexpr (MODE == 3) b = p, R.f[tid] = a.rs[p];
+        else b = (MODE == 2 && derived) ? a.src.perm[p] : (a.perm ? a.perm[p] : p);
+        R.b[tid] = b;
+        if constexpr (MODE == 2) {
+            if (derived) {
+                const RowMeta m = bwd_row_meta(a.src, p, d);
+                R.f[tid] = m.coef, R.g[tid] = a.src.dpos ? a.src.dpos[b] : 0.0f;
+                R.v[tid] = (global_f32)(bwd_qbase(a.src) + m.qoff), R.w[tid] = (global_f32)(a.src.resid + (int64_t)b * d);
+            } else {
+                R.v[tid] = (global_f32)(a.xs + (int64_t)p * d);
+            }
+        } else {
+            const int64_t h = a.h[b], t = a.t[b];
+            R.v[tid] = (global_f32)(array ? a.xs + (int64_t)p * d : a.ent + h * d);
+            R.w[tid] = (global_f32)(a.ent + (MODE == 3 && t < 0 ? 0 : t) * d);  // (MODE 3, t = -1: no row; read and, in put(), dropped)
+            if constexpr (MODE == 1) R.t[tid] = t;
+            if constexpr (MODE == 3) R.g[tid] = t >= 0 ? 1.0f : 0.0f;
+        }
+    }
+}
+
 // MODE as in transr_gemm_body: 0 forward TransR, 1 forward RESCAL (or rows given as an array), 2 dX, 3 list rows.
 // RB: 16-row blocks the tile runs (a template parameter: the staging and accumulator registers follow it).
 template <int MODE, int RB>
@@ -172,31 +206,10 @@ __device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int til
     for (int u = 0; u + 1 < kTallRing; ++u) bl.load(u, ring[u]);  // the projection's first pieces fly during the index chain below
     __builtin_amdgcn_sched_barrier(0);
 
-    TallRows &R = *reinterpret_cast<TallRows *>(lds + 2 * kTallRows * kTallPitch);
+    TallRows &R = *reinterpret_cast<TallRows *>(reinterpret_cast<char *>(lds) + kTallStage);
     const bool array = a.xs != nullptr && (MODE == 1 || MODE == 2);
     const bool derived = MODE == 2 && !array;
-    if (tid < kTallRows) {
-        const int p = p0 + (tid < rows ? tid : 0);
-        int b;
-        if constexpr (MODE == 3) b = p, R.f[tid] = a.rs[p];
-        else b = (MODE == 2 && derived) ? a.src.perm[p] : (a.perm ? a.perm[p] : p);
-        R.b[tid] = b;
-        if constexpr (MODE == 2) {
-            if (derived) {
-                const RowMeta m = bwd_row_meta(a.src, p, d);
-                R.f[tid] = m.coef, R.g[tid] = a.src.dpos ? a.src.dpos[b] : 0.0f;
-                R.v[tid] = (global_f32)(bwd_qbase(a.src) + m.qoff), R.w[tid] = (global_f32)(a.src.resid + (int64_t)b * d);
-            } else {
-                R.v[tid] = (global_f32)(a.xs + (int64_t)p * d);
-            }
-        } else {
-            const int64_t h = a.h[b], t = a.t[b];
-            R.v[tid] = (global_f32)(array ? a.xs + (int64_t)p * d : a.ent + h * d);
-            R.w[tid] = (global_f32)(a.ent + (MODE == 3 && t < 0 ? 0 : t) * d);  // (MODE 3, t = -1: no row; read and, in put(), dropped)
-            if constexpr (MODE == 1) R.t[tid] = t;
-            if constexpr (MODE == 3) R.g[tid] = t >= 0 ? 1.0f : 0.0f;
-        }
-    }
+    tall_rows<MODE>(a, R, p0, rows, array, derived);
     __syncthreads();
 
     // Staging: thread tid takes the quad tid % 16 of row tid / 16 of a row block.
@@ -319,19 +332,242 @@ __device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int til
     }
 }
 
+// The same tile on the bf16 matrix cores (mfma_split.hpp), for tiles of more than kSplitRows rows: RB blocks of 32 rows, a wave takes all of them
+// and 32 columns.  Both operands go through LDS in slices of 32, split once per slice; the projection's pieces are transposed on the way
+// (a thread takes 4 x 4 elements: four rows of it are loaded, four columns written, 64 bytes of a row and 16 banks apart per two lanes).
+//   What bounds it: the matrix cores and the slices' barriers where groups are large, else the projections' bytes.  Whole calls, fp32 tiles
+//   -> these: RESCAL 8192 x 1024 over 51 relations (Zipf) 230 -> 184 us, 8192 x 512 over 11 82 -> 64; TransR 4096 x 512 over 60 64 -> 50,
+//   over 237 91 -> 88 (bytes); the row list and dX of TransR against shared negatives, 4096 x 200 over 1345, 126 + 145 -> 122 + 107 us.
+//   A launch of at most one item per CU runs every slice at its full latency and keeps the fp32 tiles' four supersteps in flight
+//   (4096 x 128 over 20: 25 against 27 us); tiles of at most 16 rows do half of the matrix work in fp32's 16-row blocks.
+template <int MODE, int RB>
+__device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int tile, int cb)
+{
+    const GemmArgs &a = t.g;
+    const int d = a.d, ncb = tall_col_blocks(d);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 31, fg = lane >> 5;
+    const int p0 = __builtin_amdgcn_readfirstlane(a.plan.tile_p0[tile]), seg_end = __builtin_amdgcn_readfirstlane(a.plan.tile_end[tile]);
+    const int64_t rid = __builtin_amdgcn_readfirstlane(a.plan.tile_rid[tile]);
+    const int rows = seg_end - p0 < kTallRows ? seg_end - p0 : kTallRows;
+    const float *M = a.proj + rid * (int64_t)d * d;
+    const int bc = tall_block_cols(d), c0 = cb * bc, span = d - c0 < bc ? d - c0 : bc;
+
+    __bf16(*sX)[kSplitPitch] = reinterpret_cast<__bf16(*)[kSplitPitch]>(lds);
+    __bf16(*sM)[kSplitPitch] = sX + kTallRows;  // by column of the product
+    TallRows &R = *reinterpret_cast<TallRows *>(reinterpret_cast<char *>(lds) + kTallStage);
+    auto put3 = [](__bf16 *at, float4 v) {
+        bf16x4 p[kSplitParts];
+        split_quad(v, p);
+#pragma unroll
+        for (int q = 0; q < kSplitParts; ++q) *reinterpret_cast<bf16x4 *>(at + q * kSplitK) = p[q];
+    };
+
+    // The projection: d % 4 == 0, so a quad lies inside a row or outside it; what lies outside is read from the last quad or row,
+    // meets a left operand that is zero there (k) or is stored nowhere (columns).
+    float4 m[4];
+    const int kb = tid & 7, nb = tid >> 3;
+    const char *base = reinterpret_cast<const char *>(M);
+    const uint32_t d4 = 4u * (uint32_t)d;
+    const uint32_t mcol = 4u * (uint32_t)min(c0 + 4 * nb, d - 4);  // bytes
+    auto load_m = [&](int j0) {
+        if constexpr (MODE != 2) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = load_quad(reinterpret_cast<const float *>(base + ((uint32_t)min(j0 + 4 * kb + i, d - 1) * d4 + mcol)));
+        } else {
+            const uint32_t k = 4u * (uint32_t)min(j0 + 4 * kb, d - 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = load_quad(reinterpret_cast<const float *>(base + ((uint32_t)min(c0 + nb + 32 * i, d - 1) * d4 + k)));
+        }
+    };
+    auto put_m = [&] {
+        if constexpr (MODE != 2) {
+            put3(&sM[4 * nb + 0][4 * kb], make_float4(m[0].x, m[1].x, m[2].x, m[3].x));
+            put3(&sM[4 * nb + 1][4 * kb], make_float4(m[0].y, m[1].y, m[2].y, m[3].y));
+            put3(&sM[4 * nb + 2][4 * kb], make_float4(m[0].z, m[1].z, m[2].z, m[3].z));
+            put3(&sM[4 * nb + 3][4 * kb], make_float4(m[0].w, m[1].w, m[2].w, m[3].w));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) put3(&sM[nb + 32 * i][4 * kb], m[i]);
+        }
+    };
+    load_m(0);  // (flies during the index chain below)
+    __builtin_amdgcn_sched_barrier(0);
+    const bool array = a.xs != nullptr && (MODE == 1 || MODE == 2);
+    const bool derived = MODE == 2 && !array;
+    tall_rows<MODE>(a, R, p0, rows, array, derived);
+    __syncthreads();
+
+    // the left operand: thread tid stages the quad tid % 8 of row tid / 8 of a row block (as tall_tile's fetch and put)
+    const bool l1 = derived && !a.src.rescal && a.src.norm_p == 1;
+    const bool occ = derived && a.src.occ_v && cb == 0;
+    constexpr bool kTwo = MODE == 0 || MODE == 3;
+    float4 v[RB], w[RB];
+    auto load_x = [&](int j0) {
+        const int k4 = min(j0 + 4 * kb, d - 4);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            v[i] = load4g(R.v[32 * i + nb] + k4);
+            if constexpr (kTwo) w[i] = load4g(R.w[32 * i + nb] + k4);
+            else w[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if constexpr (MODE == 2)
+                if (occ) w[i] = load4g(R.w[32 * i + nb] + k4);
+        }
+    };
+    auto form_x = [&](int row, float4 vv, float4 ww) {
+        float4 x = vv;
+        if constexpr (MODE == 0) x = make_float4(vv.x - ww.x, vv.y - ww.y, vv.z - ww.z, vv.w - ww.w);
+        if constexpr (MODE == 3) {
+            const bool keep = R.g[row] != 0.0f;
+            x = make_float4(vv.x - (keep ? ww.x : 0.0f), vv.y - (keep ? ww.y : 0.0f), vv.z - (keep ? ww.z : 0.0f), vv.w - (keep ? ww.w : 0.0f));
+        }
+        if constexpr (MODE == 2)
+            if (derived) x = scaled4(R.f[row], l1 ? sgn4(vv) : vv);
+        return x;
+    };
+    auto put_x = [&](int j0) {
+        const int col = j0 + 4 * kb;
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const int row = 32 * i + nb;
+            const bool ok = row < rows && col < d;
+            const float4 x = form_x(row, v[i], w[i]);
+            if constexpr (MODE == 2)
+                if (occ && ok)  // RESCAL: the tail's occurrence row g * (E[h] Proj[r])
+                    *reinterpret_cast<float4 *>(a.src.occ_v + (int64_t)R.b[row] * d + col) = scaled4(R.g[row], w[i]);
+            put3(&sX[row][4 * kb], make_float4(ok ? x.x : 0.0f, ok ? x.y : 0.0f, ok ? x.z : 0.0f, ok ? x.w : 0.0f));
+        }
+    };
+
+    floatx16 lead[RB], rest[RB];  // sums of the leading products / of the corrections
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lead[i][e] = 0.0f, rest[i][e] = 0.0f;
+    const bool active = 32 * wave < span;  // (uniform per wave)
+    load_x(0);
+#pragma unroll 1
+    for (int j0 = 0; j0 < d; j0 += kSplitK) {
+        put_x(j0);
+        put_m();
+        __syncthreads();
+        if (j0 + kSplitK < d) load_x(j0 + kSplitK), load_m(j0 + kSplitK);
+        __builtin_amdgcn_sched_barrier(0);  // (the requests go out before the products, not after them)
+        if (active) {
+#pragma unroll
+            for (int u = 0; u < kSplitK / 16; ++u) {
+                bf16x8 xv[RB][kSplitParts], mv[kSplitParts];
+#pragma unroll
+                for (int q = 0; q < kSplitParts; ++q) {
+                    mv[q] = *reinterpret_cast<const bf16x8 *>(&sM[32 * wave + fr][q * kSplitK + 16 * u + 8 * fg]);
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) xv[i][q] = *reinterpret_cast<const bf16x8 *>(&sX[32 * i + fr][q * kSplitK + 16 * u + 8 * fg]);
+                }
+#pragma unroll
+                for (int q = 0; q < kSplitTerms; ++q)
+#pragma unroll
+                    for (int i = 0; i < RB; ++i) {
+                        floatx16 &acc = q + 1 < kSplitTerms ? rest[i] : lead[i];
+                        acc = mfma_bf16(xv[i][kTermA[q]], mv[kTermB[q]], acc);
+                    }
+            }
+        }
+        __syncthreads();
+    }
+
+    // A sum that came out NaN (mfma_split.hpp): the caller forms the tile again in fp32.
+    const bool colok = 32 * wave + fr < span;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lead[i][e] += rest[i][e], bad = bad || (colok && lead[i][e] != lead[i][e]);
+    if (__syncthreads_or(bad)) return true;
+
+    // Lane (fr, fg) holds rows 32 i + 8 (e / 4) + 4 fg + e % 4, column c0 + 32 wave + fr.
+    const bool want_pos = MODE < 2 && a.pos;
+    const int col = colok ? c0 + 32 * wave + fr : c0;
+    float rv = 0.0f;  // the relation's row
+    if constexpr (MODE == 0 || MODE == 3) rv = a.rel[rid * (int64_t)d + col];
+    float *const out = MODE == 2 ? a.occ_h : a.resid;
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int e0 = 0; e0 < 16; e0 += 4) {
+            const int row0 = 32 * i + 2 * e0 + 4 * fg;
+            float y[4], tv[4];
+            int rb[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = row0 + e;
+                y[e] = lead[i][e0 + e], rb[e] = R.b[row];
+                if constexpr (MODE == 0) y[e] += rv;
+                if constexpr (MODE == 3) y[e] += R.f[row] * rv;  // +-1 or 0: exact products
+                tv[e] = 0.0f;
+                if constexpr (MODE == 1)
+                    if (want_pos) tv[e] = a.ent[R.t[row < rows ? row : 0] * (int64_t)d + col];
+            }
+            if constexpr (MODE < 2) {
+                if (want_pos) {  // uniform
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float s;
+                        if constexpr (MODE == 1) s = y[e] * tv[e];
+                        else s = a.norm_p == 1 ? fabsf(y[e]) : y[e] * y[e];
+                        s = row16_sum(colok ? s : 0.0f);
+                        if ((fr & 15) == 0) R.sum[2 * wave + (fr >> 4)][row0 + e] = s;
+                    }
+                }
+            }
+            if (out && colok) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (row0 + e < rows) {
+                        const int64_t o = (int64_t)rb[e] * d + col;
+                        out[o] = y[e];
+                        if constexpr (MODE == 2)
+                            if (a.occ_t) a.occ_t[o] = -y[e];
+                    }
+            }
+        }
+    if constexpr (MODE < 2) {
+        if (want_pos) {
+            __syncthreads();
+            if (tid < rows) {
+                float s = 0.0f;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) s += R.sum[q][tid];
+                if (ncb > 1) t.part[(int64_t)cb * t.B + R.b[tid]] = s;
+                else a.pos[R.b[tid]] = (MODE == 0 && a.norm_p == 2) ? sqrtf(s) : s;
+            }
+        }
+    }
+    return false;
+}
+
+// Two loops over the workgroup's items, not two branches in one: side by side in a loop the two forms' invariants are held at once and 17 to 80
+// registers per lane spill.
 template <int MODE>
 __global__ __launch_bounds__(256, 3) void transr_tall_kernel(TallArgs t, FusedInsp fi)
 {
     extern __shared__ __align__(16) float lds[];
     if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(lds))) return;
-    const int ncb = tall_col_blocks(t.g.d), n = t.g.plan.num_tiles[0] * ncb, step = (int)gridDim.x - fi.blocks;
-    for (int it = (int)blockIdx.x - fi.blocks; it < n; it += step) {
-        const int tile = it / ncb, cb = it % ncb, rows = t.g.plan.tile_end[tile] - t.g.plan.tile_p0[tile];
+    const int ncb = tall_col_blocks(t.g.d), n = t.g.plan.num_tiles[0] * ncb, step = (int)gridDim.x - fi.blocks, first = (int)blockIdx.x - fi.blocks;
+    const int split_rows = n > kSplitItems ? kSplitRows : kTallRows;  // tiles of more rows are split
+    uint64_t again = 0;  // items (by turn; launch_tall gives a workgroup at most 64) whose sums were not all numbers
+    auto rows_of = [&](int it) { return t.g.plan.tile_end[it / ncb] - t.g.plan.tile_p0[it / ncb]; };
+    for (int it = first, turn = 0; it < n; it += step, ++turn)
+        if (rows_of(it) > split_rows) {
+            if (split_tile<MODE, 2>(t, lds, it / ncb, it % ncb)) again |= uint64_t(1) << turn;
+            __syncthreads();  // the next tile reuses the staging buffers
+        }
+    for (int it = first, turn = 0; it < n; it += step, ++turn) {
+        const int tile = it / ncb, cb = it % ncb, rows = rows_of(it);
+        if (rows > split_rows && !((again >> turn) & 1)) continue;
         if (rows > 48) tall_tile<MODE, 4>(t, lds, tile, cb);
         else if (rows > 32) tall_tile<MODE, 3>(t, lds, tile, cb);
         else if (rows > 16) tall_tile<MODE, 2>(t, lds, tile, cb);
         else tall_tile<MODE, 1>(t, lds, tile, cb);
-        __syncthreads();  // the next tile reuses the staging buffers
+        __syncthreads();
     }
 }
 
@@ -354,7 +590,10 @@ __global__ __launch_bounds__(256) void tall_finish_kernel(const float *part, int
 //                       tiles are taken; at two rows per group and more than 256 tiles 0.92 (0.77 to 1.07)
 //   up to 256           two column blocks stage every row twice: only where the 32-row tiles leave compute units idle.
 //                       Up to 200 tiles 1.00 (0.79 to 1.17) and 0.94; 201 to 256 tiles 1.17 (1.00 to 1.41) and 0.97;
-//                       above 1.17 (0.84 to 1.56) and 0.95
+//                       above 1.17 (0.84 to 1.56) and 0.95.  Groups that fill their tiles' 64 rows on average (from 32 rows per
+//                       relation on) go by the bf16 matrix cores there: score calls 0.79 to 0.96 (8192 triples over 20 to 237
+//                       relations, width 132 / 200 / 256), TransR's row list of 90000 rows over 588 relations below; at 8 rows
+//                       per relation 0.95 to 1.14, at 2 1.1 to 1.3
 //   above               a 32-row tile is one workgroup however wide its rows are: few groups leave the chip idle.
 //                       0.76 (0.24 to 1.33) and 0.78; where streaming is taken (many groups of a few rows, bound by
 //                       reading the projections) 0.95 (0.70 to 1.28) and 0.89
@@ -362,7 +601,7 @@ static bool want_tall(int64_t d, int64_t rows, int64_t n_rel)
 {
     const int64_t groups = rows < n_rel ? rows : n_rel, short_tiles = groups + rows / 32;
     if (d <= kTallCols) return short_tiles <= 256 || rows >= 4 * n_rel;
-    if (d <= 2 * kTallCols) return short_tiles <= 200;
+    if (d <= 2 * kTallCols) return short_tiles <= 200 || rows >= 32 * n_rel;
     return groups <= 256 || rows >= 16 * n_rel;
 }
 
@@ -376,7 +615,8 @@ static int launch_tall(int mode, const GemmArgs &a, int64_t max_tiles, float *pa
     if (a.pos && ncb > 1 && !part) return KGE_EWORKSPACE;
     const TallArgs t{a, part, B};
     const int64_t items = max_tiles * ncb;
-    const dim3 grid((unsigned)((items < kTallWgs ? items : kTallWgs) + fi.blocks)), block(256);
+    const int64_t wgs = items / 64 + 1 > kTallWgs ? items / 64 + 1 : kTallWgs;  // (at most 64 items each: transr_tall_kernel)
+    const dim3 grid((unsigned)((items < wgs ? items : wgs) + fi.blocks)), block(256);
     const size_t lds = fi.blocks > 0 && (size_t)fi.lds_bytes > kTallLds ? (size_t)fi.lds_bytes : kTallLds;
     switch (mode) {
     case 0: hipLaunchKernelGGL(transr_tall_kernel<0>, grid, block, lds, st, t, fi); break;

@@ -69,3 +69,64 @@ def test_infinities_and_nans_as_fp32_has_them():
     fine = want.isfinite()
     assert torch.equal(got[~fine].nan_to_num(nan=0.0), want[~fine].nan_to_num(nan=0.0))
     assert torch.allclose(got[fine], want[fine], rtol=1e-5)
+
+
+def _grouped(sizes, dim, seed, scale=0.05):
+    """Triples in groups of the given sizes (one relation each), shuffled."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    r = torch.repeat_interleave(torch.arange(len(sizes), device="cuda"), torch.tensor(sizes, device="cuda"))
+    r = r[torch.randperm(r.numel(), generator=g, device="cuda")]
+    E, R = (torch.randn(n, dim, generator=g, device="cuda") * scale for n in (700, len(sizes)))
+    A = torch.randn(len(sizes), dim, dim, generator=g, device="cuda") * scale
+    h, t = (torch.randint(0, 700, (r.numel(),), generator=g, device="cuda") for _ in range(2))
+    return E, R, A, h, r, t
+
+
+# groups on both sides of a tile's 64 rows and of its row blocks; more items than one per CU (and one launch of fewer, in fp32)
+@pytest.mark.parametrize("dim,copies", [(128, 30), (132, 20), (200, 20), (256, 20), (260, 12), (388, 12), (128, 3)])
+def test_grouped_products_against_64_bits(dim, copies):
+    from cuke_amd import kge
+    sizes = [1, 15, 16, 17, 31, 32, 33, 47, 63, 64, 65, 100, 129] * copies
+    E, R, A, h, r, t = _grouped(sizes, dim, dim)
+    B, bound = r.numel(), 2.0 ** -24 * (4 + dim ** 0.5)
+    x = (E[h] - E[t]).double()
+    want, size = torch.empty_like(x), torch.empty_like(x)
+    head, tail = E[h].double(), E[t].double()
+    proj, psize = torch.empty_like(x), torch.empty_like(x)
+    back = torch.empty_like(x)
+    for u in range(len(sizes)):
+        m = r == u
+        M = A[u].double()
+        want[m], size[m] = x[m] @ M + R[u].double(), x[m].abs() @ M.abs() + R[u].abs().double()
+        proj[m], psize[m] = head[m] @ M, head[m].abs() @ M.abs()
+        back[m] = tail[m] @ M.t().contiguous()
+    score = kge.transR(B, dim, 700, E, h, t, len(sizes), A, r, R)
+    err = (score.double() - want).abs() / size
+    assert bool((err <= bound).all()), float(err.max() / bound)
+    m = KGEModel("RESCAL", E, None, A)
+    fw = m.score(h, r, t)
+    err = (fw.pos.double() - (proj * tail).sum(1)).abs() / (psize * tail.abs()).sum(1)
+    assert bool((err <= 2 * bound).all()), float(err.max() / bound)  # (two sums of dim terms, one after the other)
+    g = m.backward(fw, torch.ones(B, device="cuda"))
+    rows = torch.zeros(700, dim, dtype=torch.float64, device="cuda").index_add_(0, h, back).index_add_(0, t, proj)
+    rows = rows[g.ent_ids]
+    assert bool(((g.ent_rows.double() - rows).norm(dim=1) <= 1e-6 * rows.norm(dim=1)).all())
+
+
+def test_grouped_infinities_and_nans_as_fp32_has_them():
+    from cuke_amd import kge
+    E, R, A, h, r, t = _grouped([70, 33, 40] * 100, 128, 1, scale=1.0)
+    E[3, 5], E[4, 6], A[0, 9, 17], A[1, 100, 3], A[200, 127, 127], E[8, 0] = float("inf"), float("nan"), -float("inf"), float("inf"), 3.4e38, 0.0
+    h[:4], t[:4] = 3, torch.tensor([4, 5, 3, 6], device="cuda")
+    got = kge.transR(r.numel(), 128, 700, E, h, t, 300, A, r, R).cpu()
+    x, want, size = (E[h] - E[t]).cpu(), torch.empty(r.numel(), 128), torch.empty(r.numel(), 128, dtype=torch.float64)
+    for u in range(300):
+        m = (r == u).cpu()
+        want[m] = (x[m][:, :, None] * A[u].cpu()).sum(1) + R[u].cpu()
+        size[m] = (x[m][:, :, None].double() * A[u].cpu().double()).abs().sum(1) + R[u].cpu().abs().double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    assert torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    # both sides round: 2 (4 + sqrt(128)) half ulps of the terms' total
+    assert bool(((got.double() - want.double()).abs() <= 2.0 ** -23 * (4 + 128 ** 0.5) * size)[fine].all())

@@ -250,20 +250,6 @@ __device__ __forceinline__ float neg_norm_partial(const NegRow<NQ> &a, const Neg
     return s;
 }
 
-// acc += coef * phi(a - p), phi = sign (L1) or identity (L2: coef already carries 1 / norm)
-template <int P, int NQ>
-__device__ __forceinline__ void neg_accumulate(NegRow<NQ> &acc, const NegRow<NQ> &a, const NegRow<NQ> &p, float coef)
-{
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        const float u0 = a.v[q].x - p.v[q].x, u1 = a.v[q].y - p.v[q].y, u2 = a.v[q].z - p.v[q].z, u3 = a.v[q].w - p.v[q].w;
-        acc.v[q].x = fmaf(coef, P == 1 ? sgn(u0) : u0, acc.v[q].x);
-        acc.v[q].y = fmaf(coef, P == 1 ? sgn(u1) : u1, acc.v[q].y);
-        acc.v[q].z = fmaf(coef, P == 1 ? sgn(u2) : u2, acc.v[q].z);
-        acc.v[q].w = fmaf(coef, P == 1 ? sgn(u3) : u3, acc.v[q].w);
-    }
-}
-
 struct NegPairArgs {
     const float *ent;
     const float *y;         // projected list rows [L, d]
@@ -311,140 +297,120 @@ __global__ __launch_bounds__(256) void tneg_pair_fwd_kernel(NegIdx x, NegPairArg
     }
 }
 
-// Backward, one wave per positive: upstream rows of its two list rows (the positive's own residual
-// row and its a row), their left operands, and the row that goes to the relation table.
-template <int P, int NQ>
-__global__ __launch_bounds__(256) void tneg_pair_bwd_a_kernel(NegIdx x, NegPairArgs a)
+// Backward of the pairs, one pass.  A workgroup owns kNegSeg consecutive positions of the key order, in which the positives of a group sit
+// next to each other, and 256 columns of the rows, a lane one of them.  It holds the group's P rows (KN negatives) in registers beside their
+// sums and walks its positives: a pair element is formed once and goes into both
+//   the a row's upstream gradient   ga_b = sum over k of c_bk phi(a_b - P_k)       (whole in one lane: no sum across lanes), and
+//   the P row's                     Q_k  = - sum over the group's b of the same.
+// A group that lies wholly inside the block leaves its Q rows final, one that began in an earlier block goes to partial slot 0 of the
+// block, one that continues past it to slot 1 (the scheme of seg_reduce.hip); tneg_pair_bwd_p2_kernel adds those up.  The order of
+// every sum is fixed by the sorted order.  The positives' own rows (upstream rows of both list rows, left operands, the row that goes
+// to the relation table) are finished here as well.
+//   Bound by the rows it reads (P rows once per block and group, 90 MB at 4096 x 64 x 200) and the stores behind them.  As two kernels, a wave
+//   per positive over its group's P rows and a wave per (eight positions, negative) over both rows of every pair, it was 600 MB out of the
+//   L2 and 144 us; now 55 us (4096 positives x 64 negatives x 200, 1270 groups).
+template <int P, int KN>
+__global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArgs a, const int32_t *k_sseg, float *partial)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (b >= x.B) return;
-    const int d = x.d;
-    const int N = (int)x.N;
-    const int ra = x.rowa[b], rp = x.rowpos[b];
-    const NegRow<NQ> ya = neg_load_row<NQ>(a.y + (int64_t)ra * d, d, lane);
-    const float *pg = a.y + (int64_t)x.rowp[x.k_inv[b]] * d;
-    NegRow<NQ> ga, z;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) ga.v[q] = make_float4(0.f, 0.f, 0.f, 0.f), z.v[q] = ga.v[q];
-    if (a.dneg) {
-        for (int k0 = 0; k0 < N; k0 += 4) {
-            NegRow<NQ> p[4];
-            float coef[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int k = k0 + u < N ? k0 + u : N - 1;
-                p[u] = neg_load_row<NQ>(pg + (int64_t)k * d, d, lane);
-                const float g = a.dneg[b * (int64_t)N + k];
-                float c = g;
-                if constexpr (P == 2) {
-                    const float s = a.sneg[b * (int64_t)N + k];
-                    c = s > 0.0f ? g / s : 0.0f;
-                }
-                coef[u] = k0 + u < N ? c : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) neg_accumulate<P, NQ>(ga, ya, p[u], coef[u]);
-        }
-    }
-    // the positive's own residual row
-    const NegRow<NQ> yp = neg_load_row<NQ>(a.y + (int64_t)rp * d, d, lane);
-    float gs = a.dpos ? a.dpos[b] : 0.0f;
-    if constexpr (P == 2) {
-        const float s = a.spos[b];
-        gs = s > 0.0f ? gs / s : 0.0f;
-    }
-    NegRow<NQ> qp;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) qp.v[q] = make_float4(0.f, 0.f, 0.f, 0.f);
-    neg_accumulate<P, NQ>(qp, yp, z, gs);
-    const NegRow<NQ> eh = neg_load_row<NQ>(a.ent + x.h[b] * (int64_t)d, d, lane), et = neg_load_row<NQ>(a.ent + x.t[b] * (int64_t)d, d, lane);
-    NegRow<NQ> xp, qr;
-    const float sg = x.head ? -1.0f : 1.0f;
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-        xp.v[q] = make_float4(eh.v[q].x - et.v[q].x, eh.v[q].y - et.v[q].y, eh.v[q].z - et.v[q].z, eh.v[q].w - et.v[q].w);
-        qr.v[q] = make_float4(fmaf(sg, ga.v[q].x, qp.v[q].x), fmaf(sg, ga.v[q].y, qp.v[q].y), fmaf(sg, ga.v[q].z, qp.v[q].z),
-                              fmaf(sg, ga.v[q].w, qp.v[q].w));
-    }
-    neg_store_row(a.ql + (int64_t)rp * d, d, lane, qp);
-    neg_store_row(a.xl + (int64_t)rp * d, d, lane, xp);
-    neg_store_row(a.ql + (int64_t)ra * d, d, lane, ga);
-    neg_store_row(a.xl + (int64_t)ra * d, d, lane, x.head ? et : eh);
-    neg_store_row(a.qr + b * (int64_t)d, d, lane, qr);
-}
-
-// Backward, upstream rows of the P rows: Q_(g,k) = - sum over the positives b of group g of their pair
-// gradients.  The positives sit next to each other in the key order, so this is a segmented sum
-// over the sorted positions whose terms are formed on the fly.  Level 1: a wave owns kNegSeg
-// consecutive sorted positions and one negative k and walks them in order; a group that lies
-// wholly inside the block is final, one that began in an earlier block goes to partial slot 0 of
-// the block, one that continues past it to slot 1 (the scheme of seg_reduce.hip).  Level 2: the
-// block in which a long group starts adds its slot-1 partial and the slot-0 partials of the
-// following blocks.  Work is spread over B N / kNegSeg waves whatever the group sizes are (a hot
-// relation's group has hundreds of positives); the order of the sum is fixed by the sorted order.
-template <int P, int NQ>
-__global__ __launch_bounds__(256) void tneg_pair_bwd_p1_kernel(NegIdx x, NegPairArgs a, const int32_t *k_sseg, float *partial)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int N = (int)x.N, d = x.d;
-    const int64_t j = w / N;
-    const int k = (int)(w % N);
-    const int64_t p0 = j * kNegSeg;
-    if (p0 >= x.B) return;
+    __shared__ float s_c[kNegSeg][kWave];   // the pairs' coefficients, KN negatives at a time
+    __shared__ float s_ga[kNegSeg][256];
+    __shared__ int s_b[kNegSeg], s_g[kNegSeg], s_pa[kNegSeg], s_pp[kNegSeg];
+    const int tid = threadIdx.x, lane = tid & 63, d = x.d, N = (int)x.N;
+    const int64_t j = blockIdx.x, p0 = j * kNegSeg;
     const int cnt = (int)(x.B - p0 < kNegSeg ? x.B - p0 : kNegSeg);
-    int bb[kNegSeg], gg[kNegSeg];
-#pragma unroll
-    for (int q = 0; q < kNegSeg; ++q) {
-        const int64_t pc = p0 + (q < cnt ? q : cnt - 1);  // clamped: unconditional loads, masked at their use
-        bb[q] = x.k_perm[pc], gg[q] = k_sseg[pc];
+    const int col = (int)blockIdx.y * 256 + tid;
+    const bool colok = col < d;
+    const int cc = colok ? col : d - 1;  // clamped: unconditional loads
+    if (tid < kNegSeg) {
+        const int64_t pc = p0 + (tid < cnt ? tid : cnt - 1);
+        const int b = x.k_perm[pc], g = k_sseg[pc];
+        s_b[tid] = b, s_g[tid] = g, s_pa[tid] = x.rowa[b], s_pp[tid] = x.rowp[g];
     }
     const int g_before = p0 > 0 ? k_sseg[p0 - 1] : -1, g_after = p0 + cnt < x.B ? k_sseg[p0 + cnt] : -1;
-    NegRow<NQ> acc;
 #pragma unroll
-    for (int e = 0; e < NQ; ++e) acc.v[e] = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto flush = [&](int g) {
-        float *dst;
-        if (g == g_before) dst = partial + ((j * N + k) * 2 + 0) * (int64_t)d;
-        else if (g == g_after) dst = partial + ((j * N + k) * 2 + 1) * (int64_t)d;
-        else dst = a.ql + (int64_t)(x.rowp[g] + k) * d;
-        neg_store_row(dst, d, lane, acc);
-    };
-    constexpr int kFly = NQ == 1 ? 8 : (NQ == 2 ? 4 : 2);  // positions whose rows are in flight together
-#pragma unroll
-    for (int q0 = 0; q0 < kNegSeg; q0 += kFly) {
-        NegRow<NQ> ya[kFly], pr[kFly];
-        float coef[kFly];
-#pragma unroll
-        for (int u = 0; u < kFly; ++u) {
-            const int q = q0 + u;
-            ya[u] = neg_load_row<NQ>(a.y + (int64_t)x.rowa[bb[q]] * d, d, lane);
-            pr[u] = neg_load_row<NQ>(a.y + (int64_t)(x.rowp[gg[q]] + k) * d, d, lane);
-            float c = 0.0f;
-            if (a.dneg) {  // uniform
-                c = a.dneg[bb[q] * (int64_t)N + k];
-                if constexpr (P == 2) {
-                    const float sc = a.sneg[bb[q] * (int64_t)N + k];
-                    c = sc > 0.0f ? c / sc : 0.0f;
+    for (int q = 0; q < kNegSeg; ++q) s_ga[q][tid] = 0.0f;
+    __syncthreads();
+    if (a.dneg) {  // uniform
+        for (int k0 = 0; k0 < N; k0 += KN) {
+            const int kn = N - k0 < KN ? N - k0 : KN;
+            for (int i = tid; i < kNegSeg * KN; i += 256) {
+                const int q = i / KN, k = i % KN;
+                float c = 0.0f;
+                if (q < cnt && k < kn) {
+                    const int64_t o = s_b[q] * (int64_t)N + k0 + k;
+                    c = a.dneg[o];
+                    if constexpr (P == 2) {
+                        const float s = a.sneg[o];
+                        c = s > 0.0f ? c / s : 0.0f;
+                    }
                 }
+                s_c[q][k] = c;
             }
-            coef[u] = -c;
-        }
+            __syncthreads();
+            float pr[KN], sum[KN];
+            int g = -1;
+            auto flush = [&] {
+                if (!colok) return;
+                float *dst;
+                int64_t stride = d;
+                if (g == g_before) dst = partial + ((j * N + k0) * 2 + 0) * (int64_t)d, stride = 2 * d;
+                else if (g == g_after) dst = partial + ((j * N + k0) * 2 + 1) * (int64_t)d, stride = 2 * d;
+                else dst = a.ql + ((int64_t)x.rowp[g] + k0) * d;
 #pragma unroll
-        for (int u = 0; u < kFly; ++u) {
-            const int q = q0 + u;
-            if (q < cnt) {
-                if (q > 0 && gg[q] != gg[q - 1]) {
-                    flush(gg[q - 1]);
+                for (int k = 0; k < KN; ++k)
+                    if (k < kn) dst[k * stride + col] = sum[k];
+            };
+            float ya = a.y[(int64_t)s_pa[0] * d + cc];
+#pragma unroll 1
+            for (int q = 0; q < cnt; ++q) {
+                if (s_g[q] != g) {  // uniform
+                    if (g >= 0) flush();
+                    g = s_g[q];
+                    const float *src = a.y + ((int64_t)s_pp[q] + k0) * d + cc;
 #pragma unroll
-                    for (int e = 0; e < NQ; ++e) acc.v[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    for (int k = 0; k < KN; ++k) pr[k] = src[(k < kn ? k : kn - 1) * (int64_t)d], sum[k] = 0.0f;
                 }
-                neg_accumulate<P, NQ>(acc, ya[u], pr[u], coef[u]);
+                const float next = a.y[(int64_t)s_pa[q + 1 < cnt ? q + 1 : q] * d + cc];
+                const float cv = s_c[q][lane & (KN - 1)];
+                float ga = 0.0f;
+#pragma unroll
+                for (int k = 0; k < KN; ++k) {
+                    const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(cv), k));
+                    const float u = ya - pr[k], ph = P == 1 ? sgn(u) : u;
+                    ga = fmaf(c, ph, ga);
+                    sum[k] = fmaf(-c, ph, sum[k]);
+                }
+                s_ga[q][tid] += ga;
+                ya = next;
             }
+            flush();
+            __syncthreads();  // the next turn's coefficients
         }
+    } else {
+        // no upstream gradient for the pairs: zero rows, by the blocks in which a group starts
+        for (int q = 0; q < cnt && colok; ++q)
+            if (p0 + q == x.k_seg[s_g[q]])
+                for (int k = 0; k < N; ++k) a.ql[((int64_t)s_pp[q] + k) * d + col] = 0.0f;
+        for (int k = 0; k < N && colok; ++k) partial[((j * N + k) * 2 + 0) * (int64_t)d + col] = 0.0f, partial[((j * N + k) * 2 + 1) * (int64_t)d + col] = 0.0f;
     }
-    flush(gg[cnt - 1]);
+    if (!colok) return;  // (no barrier below)
+    const float sg = x.head ? -1.0f : 1.0f;
+#pragma unroll 2
+    for (int q = 0; q < cnt; ++q) {
+        const int b = s_b[q], ra = s_pa[q], rp = x.rowpos[b];
+        const float yp = a.y[(int64_t)rp * d + col], eh = a.ent[x.h[b] * (int64_t)d + col], et = a.ent[x.t[b] * (int64_t)d + col];
+        float gs = a.dpos ? a.dpos[b] : 0.0f;
+        if constexpr (P == 2) {
+            const float s = a.spos[b];
+            gs = s > 0.0f ? gs / s : 0.0f;
+        }
+        const float qp = gs * (P == 1 ? sgn(yp) : yp), ga = s_ga[q][tid];
+        a.ql[(int64_t)rp * d + col] = qp;
+        a.xl[(int64_t)rp * d + col] = eh - et;
+        a.ql[(int64_t)ra * d + col] = ga;
+        a.xl[(int64_t)ra * d + col] = x.head ? et : eh;
+        a.qr[b * (int64_t)d + col] = fmaf(sg, ga, qp);
+    }
 }
 
 template <int NQ>
@@ -584,10 +550,10 @@ __global__ __launch_bounds__(256) void tneg_occ_kernel(NegIdx x, const float *dx
             stmt;                          \
         }                                  \
     } while (0)
-#define TNEG_BY_NORM(p_, kern, grid_, ...)                                                          \
+#define TNEG_BY_NORM(p_, kern, W_, grid_, ...)                                                          \
     do {                                                                                            \
-        if ((p_) == 1) hipLaunchKernelGGL((kern<1, NQ_>), grid_, dim3(256), 0, st, __VA_ARGS__);    \
-        else hipLaunchKernelGGL((kern<2, NQ_>), grid_, dim3(256), 0, st, __VA_ARGS__);              \
+        if ((p_) == 1) hipLaunchKernelGGL((kern<1, W_>), grid_, dim3(256), 0, st, __VA_ARGS__);    \
+        else hipLaunchKernelGGL((kern<2, W_>), grid_, dim3(256), 0, st, __VA_ARGS__);              \
     } while (0)
 // The workspaces are sized for the worst case G = min(B, n_rel * n_chunks) groups (the count is only known on
 // the device): about four arrays of (2 B + G N) * dim floats, with many relations about four times the
@@ -687,7 +653,7 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
     NegPairArgs pa{};
     pa.ent = tab->ent, pa.y = y, pa.pos = pos, pa.neg = neg, pa.resid = resid;
     const dim3 pgrid((unsigned)ceil_div(s.B, 4));
-    TNEG_BY_WIDTH(d, TNEG_BY_NORM(tab->norm_p, tneg_pair_fwd_kernel, pgrid, x, pa));
+    TNEG_BY_WIDTH(d, TNEG_BY_NORM(tab->norm_p, tneg_pair_fwd_kernel, NQ_, pgrid, x, pa));
     timeline_mark(bat->timeline, st, "tneg_pair_fwd_kernel");
     KGE_CHECK_LAUNCH();
     return KGE_OK;
@@ -723,12 +689,14 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     NegPairArgs pa{};
     pa.ent = tab->ent, pa.y = y, pa.dpos = dpos, pa.dneg = dneg, pa.spos = saved->pos, pa.sneg = saved->neg;
     pa.xl = xl, pa.ql = ql, pa.qr = qr;
-    const dim3 agrid((unsigned)ceil_div(s.B, 4)), pgrid((unsigned)ceil_div(s.G_cap * s.N, 4));
-    TNEG_BY_WIDTH(d, TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_a_kernel, agrid, x, pa));
+    const dim3 pgrid((unsigned)ceil_div(s.G_cap * s.N, 4));
     float *ppart = reinterpret_cast<float *>(ws + l.ppart);
     const int32_t *k_sseg = reinterpret_cast<const int32_t *>(fws + fl.ksseg);
+    const dim3 bgrid((unsigned)ceil_div(s.B, kNegSeg), (unsigned)ceil_div(d, 256));
+    if (s.N <= 16) TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 16, bgrid, x, pa, k_sseg, ppart);
+    else if (s.N <= 32) TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 32, bgrid, x, pa, k_sseg, ppart);
+    else TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 64, bgrid, x, pa, k_sseg, ppart);
     const dim3 sgrid((unsigned)ceil_div(ceil_div(s.B, kNegSeg) * s.N, 4));
-    TNEG_BY_WIDTH(d, TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_p1_kernel, sgrid, x, pa, k_sseg, ppart));
     TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_pair_bwd_p2_kernel<NQ_>, sgrid, dim3(256), 0, st, x, k_sseg, ppart, ql));
     TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_prow_operands_kernel<NQ_>, pgrid, dim3(256), 0, st, x, tab->ent, xl));
     hipLaunchKernelGGL(tneg_chunk_groups_kernel, dim3((unsigned)s.n_chunks), dim3(64), 0, st, x, glist, gcount);

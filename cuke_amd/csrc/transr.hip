@@ -1101,6 +1101,12 @@ struct DmArgs {
     // their outer products.  fx null: every group dense.
     float *fx, *fq;
     int factor_max;
+    // Listed rows (TransR against shared negatives; with qs, xs null): row p is E[lh[p]] - E[lt[p]], lt[p] = -1 subtracts zero_row.
+    const float *lent;
+    const int64_t *lh, *lt;
+    const float *zero_row;  // d zeros
+    __device__ __forceinline__ bool derived() const { return xs == nullptr && lh == nullptr; }
+    __device__ __forceinline__ const float *list_t(int64_t p) const { return lt[p] >= 0 ? lent + lt[p] * d : zero_row; }
 };
 
 // dM of a group of at most kThin triples: four outer products written as one contiguous stream.
@@ -1114,7 +1120,7 @@ __device__ __forceinline__ void transr_thin_dm_body(const DmArgs &a, float *lds,
     if (rows > kThin) return;
     const int d = a.d, nq4 = d >> 2, tid = threadIdx.x;
     const int P = 256 / nq4;
-    const bool derived = a.xs == nullptr;
+    const bool derived = a.derived(), listed = a.lh != nullptr;
     // (the same addresses in every lane: scalar loads)
     const float *xh[4], *xt[4], *qrow[4];
     float qcoef[4];
@@ -1125,11 +1131,13 @@ __device__ __forceinline__ void transr_thin_dm_body(const DmArgs &a, float *lds,
             const RowMeta m = bwd_row_meta(a.src, p, d);
             xh[r] = a.src.ent + m.xh * d, xt[r] = a.src.ent + m.xt * d;
             qrow[r] = bwd_qbase(a.src) + m.qoff, qcoef[r] = m.coef;
+        } else if (listed) {
+            xh[r] = a.lent + a.lh[p] * d, xt[r] = a.list_t(p), qrow[r] = a.qs + (int64_t)p * d, qcoef[r] = 1.0f;
         } else {
             xh[r] = a.xs + (int64_t)p * d, xt[r] = xh[r], qrow[r] = a.qs + (int64_t)p * d, qcoef[r] = 1.0f;
         }
     }
-    const bool sub_t = derived && !a.src.rescal, sign_rows = derived && !a.src.rescal && a.src.norm_p == 1;
+    const bool sub_t = (derived && !a.src.rescal) || listed, sign_rows = derived && !a.src.rescal && a.src.norm_p == 1;
     const bool factored = a.fx && rows <= a.factor_max;
     float4 *sXT = reinterpret_cast<float4 *>(lds);  // [d] x[0..3][k]
     for (int f = tid; f < 4 * nq4; f += 256) {
@@ -1241,24 +1249,26 @@ __device__ __forceinline__ void transr_dm_small_body(const DmArgs &a, float *lds
     const int d = a.d, pitch = d + 4, nq4 = d >> 2;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kk = lane >> 4;
     const int nq = (n + 15) / 16;  // 1 or 2
-    const bool derived = a.xs == nullptr;
+    const bool derived = a.derived(), listed = a.lh != nullptr;
     float *sX = lds;                                                      // [kDmSmall][pitch]
     int64_t *sOff = reinterpret_cast<int64_t *>(lds + kDmSmallLdsFloats);  // [kDmSmall]
-    __shared__ int64_t s_xh[kDmSmall], s_xt[kDmSmall];
+    __shared__ const float *s_xh[kDmSmall], *s_xt[kDmSmall];
     __shared__ float s_c[kDmSmall];
     if (tid < kDmSmall) {
         const int p = s0 + (tid < n ? tid : n - 1);
         if (derived) {
             const RowMeta m = bwd_row_meta(a.src, p, d);
-            s_xh[tid] = m.xh * d, s_xt[tid] = m.xt * d, s_c[tid] = m.coef, sOff[tid] = m.qoff;
+            s_xh[tid] = a.src.ent + m.xh * d, s_xt[tid] = a.src.ent + m.xt * d, s_c[tid] = m.coef, sOff[tid] = m.qoff;
         } else {
-            s_xh[tid] = (int64_t)p * d, s_xt[tid] = s_xh[tid], s_c[tid] = 1.0f, sOff[tid] = (int64_t)p * d;
+            s_xh[tid] = listed ? a.lent + a.lh[p] * d : a.xs + (int64_t)p * d, s_xt[tid] = listed ? a.list_t(p) : s_xh[tid];
+            s_c[tid] = 1.0f, sOff[tid] = (int64_t)p * d;
         }
     }
     __syncthreads();
-    const float *xbase = derived ? a.src.ent : a.xs;
-    const bool sub_t = derived && !a.src.rescal;
+    const bool sub_t = (derived && !a.src.rescal) || listed;
     {
+        typedef const float __attribute__((address_space(1))) *global_row;  // (read back from LDS: not followed with flat loads)
+        typedef const floatx4 __attribute__((address_space(1))) *global_quad;
         constexpr int kBatch = 4;
         const int total = 16 * nq * nq4;
         for (int f0 = tid; f0 < total; f0 += 256 * kBatch) {
@@ -1268,8 +1278,8 @@ __device__ __forceinline__ void transr_dm_small_body(const DmArgs &a, float *lds
                 const int f = f0 + 256 * q < total ? f0 + 256 * q : 0;  // clamped: unconditional loads
                 const int row = f / nq4, k4 = (f % nq4) * 4;
                 const int rc = row < n ? row : n - 1;
-                v[q] = *reinterpret_cast<const float4 *>(xbase + s_xh[rc] + k4);
-                u[q] = *reinterpret_cast<const float4 *>(xbase + s_xt[rc] + k4);
+                const floatx4 xv = *(global_quad)((global_row)s_xh[rc] + k4), xu = *(global_quad)((global_row)s_xt[rc] + k4);
+                v[q] = make_float4(xv[0], xv[1], xv[2], xv[3]), u[q] = make_float4(xu[0], xu[1], xu[2], xu[3]);
             }
 #pragma unroll
             for (int q = 0; q < kBatch; ++q) {
@@ -1360,7 +1370,7 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
     const int seg_end = a.seg_offsets[g + 1];
     if (blk < 0) {  // a small group, whole, by this workgroup
         float *whole = a.dm + (int64_t)g * d * d;
-        if (a.xs == nullptr && !a.src.rescal && a.src.norm_p == 1) transr_dm_small_body<true>(a, lds, s0, seg_end - s0, whole);
+        if (a.derived() && !a.src.rescal && a.src.norm_p == 1) transr_dm_small_body<true>(a, lds, s0, seg_end - s0, whole);
         else transr_dm_small_body<false>(a, lds, s0, seg_end - s0, whole);
         return;
     }
@@ -1371,7 +1381,7 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
     const int li = lane & 15, kk = lane >> 4;
     const bool two_blocks = i0 + 16 < d;
     const int n = s1 - s0, nq = (n + 15) / 16;
-    const bool derived = a.xs == nullptr;
+    const bool derived = a.derived();
 
     // stage: thread i owns position s0 + i: the row's offset for the right operand, and the 32 columns
     // i0 .. i0 + 31 of its left operand (eight 128-bit loads, sixteen for TransR's two entity rows, all in
@@ -1387,6 +1397,9 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
             const RowMeta m = bwd_row_meta(a.src, p, d);
             ph = a.src.ent + m.xh * d, pt = a.src.ent + m.xt * d;
             sOff[tid] = m.qoff, coef = m.coef, sub_t = !a.src.rescal;
+        } else if (a.lh) {
+            ph = a.lent + a.lh[p] * d, pt = a.list_t(p), sub_t = true;
+            sOff[tid] = (int64_t)p * d;
         } else {
             ph = a.xs + (int64_t)p * d, pt = ph;
             sOff[tid] = (int64_t)p * d;

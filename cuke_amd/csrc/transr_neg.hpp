@@ -83,7 +83,7 @@ static NegFwdLayout neg_fwd_layout(const kge_tables *tab, const NegShape &s)
 }
 
 struct NegBwdLayout {
-    size_t xl, ql, dxl, occ, qr, glist, gcount, ppart, part_e, part_r, dpart, total;
+    size_t zero, ql, dxl, occ, qr, glist, gcount, ppart, part_e, part_r, dpart, total;
 };
 
 static NegBwdLayout neg_bwd_layout(const NegShape &s)
@@ -96,7 +96,7 @@ static NegBwdLayout neg_bwd_layout(const NegShape &s)
         return at;
     };
     const size_t rows = sizeof(float) * (size_t)(s.L_cap * s.d);
-    l.xl = take(rows), l.ql = take(rows), l.dxl = take(rows);
+    l.zero = take(sizeof(float) * (size_t)s.d), l.ql = take(rows), l.dxl = take(rows);
     l.occ = take(sizeof(float) * (size_t)((2 * s.B + s.NN) * s.d));
     l.qr = take(sizeof(float) * (size_t)(s.B * s.d));
     l.glist = take(sizeof(int32_t) * s.B);
@@ -189,11 +189,14 @@ __global__ void tneg_list_kernel(NegIdx x)
 }
 
 // One wave per chunk: the first list row of every group that has a positive in the chunk, in the
-// order of the groups' first positives (glist[c * C + i], i < gcount[c]).
-__global__ __launch_bounds__(64) void tneg_chunk_groups_kernel(NegIdx x, int32_t *glist, int32_t *gcount)
+// order of the groups' first positives (glist[c * C + i], i < gcount[c]).  The first one also clears the row that dM subtracts
+// from list rows without a second entity.
+__global__ __launch_bounds__(64) void tneg_chunk_groups_kernel(NegIdx x, int32_t *glist, int32_t *gcount, float *zero_row)
 {
     const int64_t c = blockIdx.x;
     const int lane = threadIdx.x;
+    if (c == 0)
+        for (int i = lane; i < x.d; i += kWave) zero_row[i] = 0.0f;
     int count = 0;
     for (int64_t i0 = 0; i0 < x.C; i0 += kWave) {
         const int64_t i = i0 + lane;
@@ -256,7 +259,7 @@ struct NegPairArgs {
     float *pos, *neg;       // forward outputs (pos nullable)
     float *resid;           // forward: positives' residual rows [B, d] (nullable)
     const float *dpos, *dneg, *spos, *sneg;  // backward inputs (dpos / dneg nullable)
-    float *xl, *ql, *qr;    // backward: left operands / upstream rows of the list, per-positive relation rows
+    float *ql, *qr;         // backward: upstream rows of the list, per-positive relation rows
 };
 
 // One wave per positive: pos[b] = ||y_pos||, neg[b][k] = ||a_b - P_(g(b),k)||.
@@ -304,8 +307,8 @@ __global__ __launch_bounds__(256) void tneg_pair_fwd_kernel(NegIdx x, NegPairArg
 //   the P row's                     Q_k  = - sum over the group's b of the same.
 // A group that lies wholly inside the block leaves its Q rows final, one that began in an earlier block goes to partial slot 0 of the
 // block, one that continues past it to slot 1 (the scheme of seg_reduce.hip); tneg_pair_bwd_p2_kernel adds those up.  The order of
-// every sum is fixed by the sorted order.  The positives' own rows (upstream rows of both list rows, left operands, the row that goes
-// to the relation table) are finished here as well.
+// every sum is fixed by the sorted order.  The positives' own rows (upstream rows of both list rows, the row that goes to the
+// relation table) are finished here as well.
 //   Bound by the rows it reads (P rows once per block and group, 90 MB at 4096 x 64 x 200) and the stores behind them.  As two kernels, a wave
 //   per positive over its group's P rows and a wave per (eight positions, negative) over both rows of every pair, it was 600 MB out of the
 //   L2 and 144 us; now 55 us (4096 positives x 64 negatives x 200, 1270 groups).
@@ -398,7 +401,7 @@ __global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArg
 #pragma unroll 2
     for (int q = 0; q < cnt; ++q) {
         const int b = s_b[q], ra = s_pa[q], rp = x.rowpos[b];
-        const float yp = a.y[(int64_t)rp * d + col], eh = a.ent[x.h[b] * (int64_t)d + col], et = a.ent[x.t[b] * (int64_t)d + col];
+        const float yp = a.y[(int64_t)rp * d + col];
         float gs = a.dpos ? a.dpos[b] : 0.0f;
         if constexpr (P == 2) {
             const float s = a.spos[b];
@@ -406,9 +409,7 @@ __global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArg
         }
         const float qp = gs * (P == 1 ? sgn(yp) : yp), ga = s_ga[q][tid];
         a.ql[(int64_t)rp * d + col] = qp;
-        a.xl[(int64_t)rp * d + col] = eh - et;
         a.ql[(int64_t)ra * d + col] = ga;
-        a.xl[(int64_t)ra * d + col] = x.head ? et : eh;
         a.qr[b * (int64_t)d + col] = fmaf(sg, ga, qp);
     }
 }
@@ -444,18 +445,6 @@ __global__ __launch_bounds__(256) void tneg_pair_bwd_p2_kernel(NegIdx x, const i
             }
     }
     neg_store_row(ql + (int64_t)(x.rowp[g] + k) * d, d, lane, acc);
-}
-
-// Left operands of the P rows for dM: the negatives' entity rows in list order (one wave per row).
-template <int NQ>
-__global__ __launch_bounds__(256) void tneg_prow_operands_kernel(NegIdx x, const float *ent, float *xl)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t g = w / x.N;
-    if (g >= x.k_num[0]) return;
-    const int row = x.rowp[g] + (int)(w % x.N);
-    neg_store_row(xl + (int64_t)row * x.d, x.d, lane, neg_load_row<NQ>(ent + x.hl[row] * (int64_t)x.d, x.d, lane));
 }
 
 // Occurrence rows in the order of the entity inspection, concat(h, t, neg): the list's dX rows are
@@ -680,7 +669,7 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     const kge_inspection *ri = bat->rel_insp;
     const int d = (int)tab->dim;
     float *y = reinterpret_cast<float *>(fws + fl.y);
-    float *xl = reinterpret_cast<float *>(ws + l.xl), *ql = reinterpret_cast<float *>(ws + l.ql);
+    float *zero_row = reinterpret_cast<float *>(ws + l.zero), *ql = reinterpret_cast<float *>(ws + l.ql);
     float *dxl = reinterpret_cast<float *>(ws + l.dxl), *occ = reinterpret_cast<float *>(ws + l.occ);
     float *qr = reinterpret_cast<float *>(ws + l.qr);
     int32_t *glist = reinterpret_cast<int32_t *>(ws + l.glist), *gcount = reinterpret_cast<int32_t *>(ws + l.gcount);
@@ -688,8 +677,7 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
 
     NegPairArgs pa{};
     pa.ent = tab->ent, pa.y = y, pa.dpos = dpos, pa.dneg = dneg, pa.spos = saved->pos, pa.sneg = saved->neg;
-    pa.xl = xl, pa.ql = ql, pa.qr = qr;
-    const dim3 pgrid((unsigned)ceil_div(s.G_cap * s.N, 4));
+    pa.ql = ql, pa.qr = qr;
     float *ppart = reinterpret_cast<float *>(ws + l.ppart);
     const int32_t *k_sseg = reinterpret_cast<const int32_t *>(fws + fl.ksseg);
     const dim3 bgrid((unsigned)ceil_div(s.B, kNegSeg), (unsigned)ceil_div(d, 256));
@@ -698,8 +686,7 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     else TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 64, bgrid, x, pa, k_sseg, ppart);
     const dim3 sgrid((unsigned)ceil_div(ceil_div(s.B, kNegSeg) * s.N, 4));
     TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_pair_bwd_p2_kernel<NQ_>, sgrid, dim3(256), 0, st, x, k_sseg, ppart, ql));
-    TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_prow_operands_kernel<NQ_>, pgrid, dim3(256), 0, st, x, tab->ent, xl));
-    hipLaunchKernelGGL(tneg_chunk_groups_kernel, dim3((unsigned)s.n_chunks), dim3(64), 0, st, x, glist, gcount);
+    hipLaunchKernelGGL(tneg_chunk_groups_kernel, dim3((unsigned)s.n_chunks), dim3(64), 0, st, x, glist, gcount, zero_row);
     timeline_mark(bat->timeline, st, "tneg_pair_bwd kernels");
 
     // dX = Q M^T over the list (rows stay in list order), dM = X^T Q per relation
@@ -707,8 +694,8 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
                 TilePlan{}, ql, nullptr, nullptr, nullptr, dxl, nullptr, d, tab->norm_p, 0, 0, BwdSrc{}};
     if (const int rc = launch_product(2, ga, plans, s.plans, s.U_cap, nullptr, s.B, FusedInsp{}, st)) return rc;
     timeline_mark(bat->timeline, st, s.plans.tall ? "transr_tall_kernel<dX>" : "transr_gemm_kernel<dX>");
-    DmArgs da{xl, ql, x.segl, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + l.dpart), d, ri->num_unique,
-              BwdSrc{}, nullptr, nullptr, 0};
+    DmArgs da{nullptr, ql, x.segl, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + l.dpart), d, ri->num_unique,
+              BwdSrc{}, nullptr, nullptr, 0, tab->ent, x.hl, x.tl, zero_row};
     hipLaunchKernelGGL(transr_dm_kernel, dim3((unsigned)kDmWgs), dim3(256), dm_lds_bytes(d), st, da, FusedInsp{}, SegL1Rider{});
     timeline_mark(bat->timeline, st, "transr_dm_kernel");
     TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_occ_kernel<NQ_>, dim3((unsigned)(ceil_div(s.B, 4) + s.NN)), dim3(256), 0, st, x, dxl,

@@ -448,19 +448,23 @@ __global__ __launch_bounds__(256) void tneg_pair_bwd_p2_kernel(NegIdx x, const i
 }
 
 // Occurrence rows in the order of the entity inspection, concat(h, t, neg): the list's dX rows are
-// added up per positive (own row and a row: one wave each, workgroups [0, ceil(B / 4))) and per
-// (chunk, negative) over the chunk's groups (one workgroup each: its four waves take the groups
-// i = wave, wave + 4, ... and their sums are added in wave order through LDS).
+// added up per positive (own row and a row: one wave each, the first workgroups) and per
+// (chunk, negative) over the chunk's groups (one workgroup each: its waves take the groups i = wave, wave + occ_waves(), ... and
+// their sums are added in wave order through LDS).  Bound by the chain of round trips per wave: 159 groups a chunk in four waves 34 us,
+// in sixteen 21 us (65 MB).
 template <int NQ>
-__global__ __launch_bounds__(256) void tneg_occ_kernel(NegIdx x, const float *dxl, const int32_t *glist,
+constexpr int occ_waves() { return NQ == 1 ? 16 : 8; }  // (wider rows: registers for eight rows in flight)
+template <int NQ>
+__global__ __launch_bounds__(kWave * occ_waves<NQ>()) void tneg_occ_kernel(NegIdx x, const float *dxl, const int32_t *glist,
                                                        const int32_t *gcount, float *occ)
 {
-    __shared__ float4 s_part[3][NQ * kWave];
+    constexpr int kOccWaves = occ_waves<NQ>();
+    __shared__ float4 s_part[kOccWaves - 1][NQ * kWave];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int d = x.d;
-    const int64_t pos_blocks = ceil_div(x.B, 4);
+    const int64_t pos_blocks = ceil_div(x.B, kOccWaves);
     if ((int64_t)blockIdx.x < pos_blocks) {
-        const int64_t w = (int64_t)blockIdx.x * 4 + wave;
+        const int64_t w = (int64_t)blockIdx.x * kOccWaves + wave;
         if (w >= x.B) return;
         const NegRow<NQ> dp = neg_load_row<NQ>(dxl + (int64_t)x.rowpos[w] * d, d, lane), da = neg_load_row<NQ>(dxl + (int64_t)x.rowa[w] * d, d, lane);
         NegRow<NQ> oh, ot;
@@ -488,16 +492,16 @@ __global__ __launch_bounds__(256) void tneg_occ_kernel(NegIdx x, const float *dx
 #pragma unroll
     for (int e = 0; e < NQ; ++e) acc.v[e] = make_float4(0.f, 0.f, 0.f, 0.f);
     constexpr int kFly = NQ == 1 ? 8 : (NQ == 2 ? 4 : 2);  // groups in flight per wave
-    for (int i = wave; i < cnt; i += 4 * kFly) {
+    for (int i = wave; i < cnt; i += kOccWaves * kFly) {
         NegRow<NQ> r[kFly];
 #pragma unroll
         for (int u = 0; u < kFly; ++u) {
-            const int iu = i + 4 * u;
+            const int iu = i + kOccWaves * u;
             r[u] = neg_load_row<NQ>(dxl + (int64_t)(glist[c * x.C + (iu < cnt ? iu : i)] + k) * d, d, lane);
         }
 #pragma unroll
         for (int u = 0; u < kFly; ++u)
-            if (i + 4 * u < cnt) {
+            if (i + kOccWaves * u < cnt) {
 #pragma unroll
                 for (int e = 0; e < NQ; ++e)
                     acc.v[e] = make_float4(acc.v[e].x + r[u].v[e].x, acc.v[e].y + r[u].v[e].y, acc.v[e].z + r[u].v[e].z,
@@ -511,11 +515,11 @@ __global__ __launch_bounds__(256) void tneg_occ_kernel(NegIdx x, const float *dx
     __syncthreads();
     if (wave == 0) {
 #pragma unroll
-        for (int e = 0; e < NQ; ++e) {
-            const float4 p1 = s_part[0][e * kWave + lane], p2 = s_part[1][e * kWave + lane], p3 = s_part[2][e * kWave + lane];
-            acc.v[e] = make_float4((acc.v[e].x + p1.x) + (p2.x + p3.x), (acc.v[e].y + p1.y) + (p2.y + p3.y),
-                                   (acc.v[e].z + p1.z) + (p2.z + p3.z), (acc.v[e].w + p1.w) + (p2.w + p3.w));
-        }
+        for (int e = 0; e < NQ; ++e)
+            for (int w = 0; w + 1 < kOccWaves; ++w) {
+                const float4 p = s_part[w][e * kWave + lane];
+                acc.v[e] = make_float4(acc.v[e].x + p.x, acc.v[e].y + p.y, acc.v[e].z + p.z, acc.v[e].w + p.w);
+            }
         neg_store_row(occ + (2 * x.B + q) * (int64_t)d, d, lane, acc);
     }
 }
@@ -698,7 +702,7 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
               BwdSrc{}, nullptr, nullptr, 0, tab->ent, x.hl, x.tl, zero_row};
     hipLaunchKernelGGL(transr_dm_kernel, dim3((unsigned)kDmWgs), dim3(256), dm_lds_bytes(d), st, da, FusedInsp{}, SegL1Rider{});
     timeline_mark(bat->timeline, st, "transr_dm_kernel");
-    TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_occ_kernel<NQ_>, dim3((unsigned)(ceil_div(s.B, 4) + s.NN)), dim3(256), 0, st, x, dxl,
+    TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_occ_kernel<NQ_>, dim3((unsigned)(ceil_div(s.B, occ_waves<NQ_>()) + s.NN)), dim3(kWave * occ_waves<NQ_>()), 0, st, x, dxl,
                                         glist, gcount, occ));
     timeline_mark(bat->timeline, st, "tneg_occ_kernel");
     KGE_CHECK_LAUNCH();

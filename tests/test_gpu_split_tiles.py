@@ -130,3 +130,26 @@ def test_grouped_infinities_and_nans_as_fp32_has_them():
     fine = want.isfinite()
     # both sides round: 2 (4 + sqrt(128)) half ulps of the terms' total
     assert bool(((got.double() - want.double()).abs() <= 2.0 ** -23 * (4 + 128 ** 0.5) * size)[fine].all())
+
+
+@pytest.mark.parametrize("model", ["DistMult", "ComplEx", "TransF"])
+def test_a_step_whose_split_tiles_host_the_inspection(model):
+    """(65536 ids beside 384 tiles: the riding form gives the bits of the inspection beside the step, and of a call without workspace's
+    general tiles within rounding)"""
+    import ctypes as C
+    from cuke_amd import _lib
+    from cuke_amd.kge import TrainStep
+    E, R, h, r, t, neg = _case(model, 5000, 96, 8192, 768, 64, 7)
+    st = TrainStep(KGEModel(model, E, R), h, r, t, neg, 128, loss="margin", sign=1.0)
+    assert st.fusable
+    outs = []
+    for fused in (True, False):
+        st.run(fused=fused)
+        g = st.sparse_grads()
+        outs.append([x.clone() for x in (st.pos, st.neg, st.loss, g.ent_ids, g.ent_rows, g.rel_rows)])
+    assert all(torch.equal(x, y) for x, y in zip(*outs))
+    neg2, side = torch.empty_like(st.neg), torch.empty(8192, device="cuda")
+    p = lambda x: C.c_void_p(x.data_ptr())
+    assert _lib.lib().kge_score_fwd(C.byref(st.m._tab), C.byref(st.bat), p(st.pos), p(neg2), p(side) if model == "TransF" else None, None, None, None, 0,
+                                    C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert not torch.equal(neg2, st.neg) and torch.allclose(neg2, st.neg, rtol=1e-5, atol=1e-5 * float(st.neg.std()))

@@ -87,7 +87,7 @@ def measured_traffic(workload, label, matrix_core_tiles=False, dense=False):
         for name, by in rows.items():
             base = name.replace("kge::", "")
             if base == key or base.startswith(key + "<") or (key.endswith(">") and base.replace(" ", "") == key.replace(" ", "")):
-                if matrix_core_tiles and ((key == "score_neg_kernel") or (key == "bwd_tile_kernel" and not base.endswith("true>"))):
+                if matrix_core_tiles and ((key == "score_neg_kernel") or (key == "bwd_tile_kernel" and base[:-1].split(", ")[3] != "true")):
                     continue  # the vector-ALU form of a tile kernel
                 total += by
                 names.append(name)

@@ -279,7 +279,8 @@ int kge_residual_fwd(const kge_tables *tab, const kge_batch *bat, float *out, vo
  * TransE / RotatE with shared negatives on small batches (the 32 x 32 pair tiles would leave one or
  * two workgroups per CU): given kge_score_fwd_workspace() bytes of workspace the reduction axis of
  * every tile is split over up to four workgroups (partial score planes in the workspace, a finishing
- * kernel); without the workspace the same call runs one workgroup per tile.
+ * kernel); without the workspace the same call runs one workgroup per tile.  DistMult / ComplEx / TransF with large batches
+ * (hundreds of 128 x 128 tiles) put their query rows there and score on the bf16 matrix cores; without it, on the fp32 ones.
  * TransE, and DistMult / ComplEx on the matrix-core tiles: when pos and neg are both requested, no
  * side output is and no inspection rides along, the positives are scored by extra workgroups of the
  * shared-negative launch (one launch instead of two; a timeline then has no "score_pos_kernel"

@@ -1087,6 +1087,17 @@ bool transr_grouped_path_ok(const kge_tables *tab, const kge_batch *bat)
 constexpr int kDmChunk = KGE_TR_DM_CHUNK;  // triples of one relation group per dM work item (at most 256: one per thread when staging)
 constexpr int kDmXP = 36;      // LDS pitch of a staged left-operand row (32 columns + 4: the four lane groups of an MFMA step read distinct banks)
 
+// (global, not generic: a pointer that went through LDS would otherwise be followed with flat loads, which also count as LDS
+// operations and are waited for as such)
+typedef const float __attribute__((address_space(1))) *global_f32;
+
+__device__ __forceinline__ float4 load4g(global_f32 p)
+{
+    typedef const floatx4 __attribute__((address_space(1))) *global_f32x4;
+    const floatx4 v = *(global_f32x4)p;
+    return make_float4(v[0], v[1], v[2], v[3]);
+}
+
 struct DmArgs {
     const float *xs, *qs;  // operand rows in sorted order [B, d]; null: formed from `src` (BwdSrc)
     const int32_t *seg_offsets;
@@ -1105,6 +1116,7 @@ struct DmArgs {
     const float *lent;
     const int64_t *lh, *lt;
     const float *zero_row;  // d zeros
+    int32_t *ticket;        // transr_dm_split_kernel: kDmTickets zeros
     __device__ __forceinline__ bool derived() const { return xs == nullptr && lh == nullptr; }
     __device__ __forceinline__ const float *list_t(int64_t p) const { return lt[p] >= 0 ? lent + lt[p] * d : zero_row; }
 };
@@ -1462,6 +1474,160 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
     }
 }
 
+// The same sums over listed rows (TransR against shared negatives), for the items of larger groups: 128 x 128 of the result on the
+// bf16 matrix cores (mfma_split.hpp).  By fp32 instructions and 32 rows of the result each item reads the chunk's whole q rows for 32
+// columns of x (152 us for the 87 000 listed rows of 4096 triples x 200 with 549 relations; now 123, matrix cores busy for 30 % of it,
+// VALUs for 34: the splits and the index chain in front of each of 2740 items, most of five slices or fewer).  Here both operands' columns pass
+// through LDS once per 128 of the other's, transposed on the way (positions are the product's inner dimension), in slices of 32
+// positions; wave w stages the 32 columns w of both and forms the blocks (w % 2 + {0, 2}) x (w / 2 + {0, 2}) of 32 x 32, so tiles of
+// fewer blocks spread over the waves.  A position past the end repeats the last one against an x that is zero, a column past the end
+// repeats the last quad and is stored nowhere.  Sums that are NaN are formed again in fp32.
+constexpr int kDmTile = 128;
+__host__ __device__ inline int dm_split_tiles(int d) { return (d + kDmTile - 1) / kDmTile; }
+struct DmSplitRows {  // the chunk's entity rows, x = h - t
+    global_f32 h[kDmChunk], t[kDmChunk];
+    uint32_t any_t[kDmChunk / kSplitK];  // per slice: positions that have a t
+};
+constexpr size_t kDmSplitStage = sizeof(__bf16) * kSplitPitch * 2 * kDmTile;
+
+__device__ __forceinline__ void transr_dm_split_item(const DmArgs &a, float *lds, int tile, int blk)
+{
+    const int d = a.d, nt = dm_split_tiles(d);
+    const int g = __builtin_amdgcn_readfirstlane(a.plan.tile_seg[tile]), s0 = __builtin_amdgcn_readfirstlane(a.plan.tile_p0[tile]);
+    const int slot = __builtin_amdgcn_readfirstlane(a.plan.tile_part[tile]), seg_end = __builtin_amdgcn_readfirstlane(a.seg_offsets[g + 1]);
+    const int n = seg_end - s0 < kDmChunk ? seg_end - s0 : kDmChunk;
+    float *dst = slot >= 0 ? a.part + (int64_t)slot * d * d : a.dm + (int64_t)g * d * d;
+    const int i0 = blk / nt * kDmTile, j0 = blk % nt * kDmTile;
+    const int ni = d - i0 < kDmTile ? d - i0 : kDmTile, nj = d - j0 < kDmTile ? d - j0 : kDmTile;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 31, fg = lane >> 5;
+    const int wi = wave & 1, wj = wave >> 1;
+
+    __bf16(*sX)[kSplitPitch] = reinterpret_cast<__bf16(*)[kSplitPitch]>(lds);  // by column
+    __bf16(*sQ)[kSplitPitch] = sX + kDmTile;
+    DmSplitRows &R = *reinterpret_cast<DmSplitRows *>(reinterpret_cast<char *>(lds) + kDmSplitStage);
+    bool sub = false;
+    if (tid < n) {
+        const int64_t t = a.lt[s0 + tid];
+        R.h[tid] = (global_f32)(a.lent + a.lh[s0 + tid] * d);
+        R.t[tid] = (global_f32)(t >= 0 ? a.lent + t * d : a.zero_row);
+        sub = t >= 0;
+    }
+    const uint64_t subs = __ballot(sub);
+    if ((lane & 31) == 0) R.any_t[tid / kSplitK] = (uint32_t)(subs >> lane);
+
+    const int kb = tid & 7, nb = tid >> 3;  // this thread's four positions of a slice, its four columns
+    const bool has_x = 32 * wave < ni, has_q = 32 * wave < nj;
+    const int xc = i0 + 4 * nb < d ? i0 + 4 * nb : d - 4, qc = j0 + 4 * nb < d ? j0 + 4 * nb : d - 4;
+    const float *qs = a.qs + (int64_t)s0 * d + qc;
+    float4 v[4], w[4], q[4];
+    auto load_q = [&](int k0) {
+        if (!has_q) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = load_quad(qs + (int64_t)min(k0 + 4 * kb + e, n - 1) * d);
+    };
+    auto load_x = [&](int k0) {
+        if (!has_x) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = load4g(R.h[min(k0 + 4 * kb + e, n - 1)] + xc), w[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (__builtin_amdgcn_readfirstlane(R.any_t[k0 / kSplitK])) {  // (a relation's list begins with the few rows that have one)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = load4g(R.t[min(k0 + 4 * kb + e, n - 1)] + xc);
+        }
+    };
+    auto put3 = [](__bf16 *at, float x0, float x1, float x2, float x3) {
+        bf16x4 p[kSplitParts];
+        split_quad(make_float4(x0, x1, x2, x3), p);
+#pragma unroll
+        for (int c = 0; c < kSplitParts; ++c) *reinterpret_cast<bf16x4 *>(at + c * kSplitK) = p[c];
+    };
+    auto put = [&](int k0) {
+        if (has_x) {
+            float4 x[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool ok = k0 + 4 * kb + e < n;
+                x[e] = make_float4(ok ? v[e].x - w[e].x : 0.0f, ok ? v[e].y - w[e].y : 0.0f, ok ? v[e].z - w[e].z : 0.0f, ok ? v[e].w - w[e].w : 0.0f);
+            }
+            put3(&sX[4 * nb + 0][4 * kb], x[0].x, x[1].x, x[2].x, x[3].x);
+            put3(&sX[4 * nb + 1][4 * kb], x[0].y, x[1].y, x[2].y, x[3].y);
+            put3(&sX[4 * nb + 2][4 * kb], x[0].z, x[1].z, x[2].z, x[3].z);
+            put3(&sX[4 * nb + 3][4 * kb], x[0].w, x[1].w, x[2].w, x[3].w);
+        }
+        if (has_q) {
+            put3(&sQ[4 * nb + 0][4 * kb], q[0].x, q[1].x, q[2].x, q[3].x);
+            put3(&sQ[4 * nb + 1][4 * kb], q[0].y, q[1].y, q[2].y, q[3].y);
+            put3(&sQ[4 * nb + 2][4 * kb], q[0].z, q[1].z, q[2].z, q[3].z);
+            put3(&sQ[4 * nb + 3][4 * kb], q[0].w, q[1].w, q[2].w, q[3].w);
+        }
+    };
+
+    load_q(0);  // (flies across the barrier)
+    __syncthreads();
+    load_x(0);
+    floatx16 lead[2][2], rest[2][2];  // sums of the leading products / of the corrections
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) lead[i][j][e] = 0.0f, rest[i][j][e] = 0.0f;
+    const bool active = 32 * wi < ni && 32 * wj < nj;
+#pragma unroll 1
+    for (int k0 = 0; k0 < n; k0 += kSplitK) {
+        put(k0);
+        __syncthreads();
+        if (k0 + kSplitK < n) load_x(k0 + kSplitK), load_q(k0 + kSplitK);
+        __builtin_amdgcn_sched_barrier(0);  // (the requests go out before the products, not after them)
+        if (active) {  // (blocks past the result's edge are formed as well and stored nowhere)
+#pragma unroll 1
+            for (int k = 8 * fg; k < kSplitK && k0 + k - 8 * fg < n; k += 16) {
+                bf16x8 xv[2][kSplitParts];
+#pragma unroll
+                for (int c = 0; c < kSplitParts; ++c)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) xv[i][c] = *reinterpret_cast<const bf16x8 *>(&sX[32 * wi + 64 * i + fr][c * kSplitK + k]);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    bf16x8 qv[kSplitParts];
+#pragma unroll
+                    for (int c = 0; c < kSplitParts; ++c) qv[c] = *reinterpret_cast<const bf16x8 *>(&sQ[32 * wj + 64 * j + fr][c * kSplitK + k]);
+#pragma unroll
+                    for (int c = 0; c < kSplitTerms; ++c)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            floatx16 &acc = c + 1 < kSplitTerms ? rest[i][j] : lead[i][j];
+                            acc = mfma_bf16(xv[i][kTermA[c]], qv[kTermB[c]], acc);
+                        }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!active) return;
+
+    // Lane (fr, fg) holds of block (i, j) the rows 8 (e / 4) + 4 fg + e % 4 of column fr.
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int rb = 32 * wi + 64 * i + 4 * fg, cb = 32 * wj + 64 * j + fr;
+            if (cb >= nj) continue;
+            float *out = dst + (int64_t)(i0 + rb) * d + j0 + cb;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = 8 * (e / 4) + e % 4;
+                if (rb + row >= ni) continue;
+                float s = lead[i][j][e] + rest[i][j][e];
+                if (s != s) {
+                    s = 0.0f;
+                    for (int p = 0; p < n; ++p)
+                        s = fmaf(R.h[p][i0 + rb + row] - R.t[p][i0 + rb + row], a.qs[(int64_t)(s0 + p) * d + j0 + cb], s);
+                }
+                out[(int64_t)row * d] = s;
+            }
+        }
+}
+
 static size_t dm_lds_bytes(int d)  // the staged left operand and its row offsets, or the thin groups' transposed rows
 {
     const size_t item = sizeof(float) * kDmChunk * kDmXP + sizeof(int64_t) * kDmChunk, thin = sizeof(float) * 4 * (size_t)d;
@@ -1471,10 +1637,20 @@ static size_t dm_lds_bytes(int d)  // the staged left operand and its row offset
 
 // Item `it` of a dM pass: the (chunk, row block) items of the larger groups first (the long chains), then the
 // small groups, then the thin ones.  False: past the end of the lists.
+template <bool SPLIT>
 __device__ __forceinline__ bool transr_dm_work(const DmArgs &a, float *lds, int it, int n_long, int n_small, int n_thin)
 {
-    if (it < n_long) transr_dm_item(a, lds, a.plan.item_tile[it], a.plan.item_blk[it]);
-    else if (it < n_long + n_small) transr_dm_item(a, lds, a.plan.item_tile[a.plan.max_items - 1 - (it - n_long)], -1);
+    if (it < n_long) {
+        if constexpr (SPLIT) {
+            // A chunk's items go to workgroups of one XCD (consecutive workgroups go to XCDs in turn): they share its rows.
+            const int nib = dm_split_tiles(a.d) * dm_split_tiles(a.d), turn = 8 * nib;
+            const int m = it / turn * turn, r = it - m;
+            if (m + turn <= n_long) it = m + (r & 7) * nib + (r >> 3);
+            transr_dm_split_item(a, lds, a.plan.item_tile[it], a.plan.item_blk[it]);
+        } else {
+            transr_dm_item(a, lds, a.plan.item_tile[it], a.plan.item_blk[it]);
+        }
+    } else if (it < n_long + n_small) transr_dm_item(a, lds, a.plan.item_tile[a.plan.max_items - 1 - (it - n_long)], -1);
     else if (it < n_long + n_small + n_thin) transr_thin_dm_body(a, lds, a.plan.thin_g[it - n_long - n_small]);
     else return false;
     return true;
@@ -1493,8 +1669,34 @@ __global__ __launch_bounds__(256, KGE_TR_OCC) void transr_dm_kernel(DmArgs a, Fu
         return;
     }
     const int n_long = a.plan.num_items[0], n_small = a.plan.num_items[1], n_thin = a.plan.num_thin[0];
-    for (int it = bid; transr_dm_work(a, lds, it, n_long, n_small, n_thin); it += kDmWgs)
+    for (int it = bid; transr_dm_work<false>(a, lds, it, n_long, n_small, n_thin); it += kDmWgs)
         __syncthreads();  // the next item reuses the staging buffers
+}
+
+// Listed rows: a plan of 128 x 128 items (launch_plans), two workgroups a CU.  Chunks run from a few rows to 256, so the items are
+// handed out as workgroups come free: one counter per XCD, the first item by the workgroup's number.
+constexpr int kDmSplitWgs = 2 * 256, kDmTickets = 8 * 32;  // (the counters in cache lines of their own)
+__global__ __launch_bounds__(256, 2) void transr_dm_split_kernel(DmArgs a)
+{
+    extern __shared__ __align__(16) float lds[];  // dm_split_lds_bytes()
+    __shared__ int s_next;
+    const int n_long = a.plan.num_items[0], n_small = a.plan.num_items[1], n_thin = a.plan.num_thin[0];
+    const int xcd = blockIdx.x & 7;
+    for (int it = blockIdx.x;;) {
+        int next = 0;
+        if (threadIdx.x == 0) next = kDmSplitWgs + xcd + 8 * atomicAdd(&a.ticket[32 * xcd], 1);  // (on its way during the item)
+        if (!transr_dm_work<true>(a, lds, it, n_long, n_small, n_thin)) break;
+        if (threadIdx.x == 0) s_next = next;
+        __syncthreads();  // (the next item reuses the staging buffers as well)
+        it = s_next;
+        __syncthreads();
+    }
+}
+
+static size_t dm_split_lds_bytes(int d)
+{
+    const size_t split = kDmSplitStage + sizeof(DmSplitRows), other = dm_lds_bytes(d);
+    return split > other ? split : other;
 }
 
 // An inspector step that rides with nothing: the fused entity inspection of a TransR / RESCAL step has
@@ -1532,9 +1734,9 @@ static size_t plan_ints(int64_t tiles, int64_t split, int64_t items = 0)
 {
     return (size_t)(64 + 5 * tiles + 3 * split + (items > 0 ? tiles + 2 * items : 0) + 8);
 }
-static int dm_nib(int64_t d) { return (int)ceil_div(d, 32); }
+static int dm_nib(int64_t d, bool split) { return split ? dm_split_tiles((int)d) * dm_split_tiles((int)d) : (int)ceil_div(d, 32); }
 static int dm_small_max(int64_t d) { return dm_small_fits((int)d) ? kDmSmall : kThin; }
-static int64_t dm_item_cap(int64_t dtiles, int64_t d) { return dtiles * ceil_div(d, 32); }
+static int64_t dm_item_cap(int64_t dtiles, int64_t d) { return dtiles * (dm_nib(d, false) > dm_nib(d, true) ? dm_nib(d, false) : dm_nib(d, true)); }
 static size_t dplan_ints(int64_t dtiles, int64_t dsplit, int64_t d) { return plan_ints(dtiles, dsplit, dm_item_cap(dtiles, d)); }
 
 static TilePlan plan_at(void *base, int64_t tiles, int64_t split, int64_t items = 0)
@@ -1586,10 +1788,10 @@ static Plans plans_at(void *base, const PlanSizes &z)
     return r;
 }
 
-static void launch_plans(const kge_inspection *ri, const int32_t *seg_offsets, const Plans &p, int64_t d, hipStream_t st)
+static void launch_plans(const kge_inspection *ri, const int32_t *seg_offsets, const Plans &p, int64_t d, bool split, hipStream_t st)
 {
     hipLaunchKernelGGL(transr_plan_kernel, dim3(3), dim3(1024), 0, st, ri->num_unique, seg_offsets, ri->unique_ids, p.dm, kDmChunk,
-                       dm_nib(d), dm_small_max(d), p.tiles, kTM, p.tall, kTallRows);
+                       dm_nib(d, split), dm_small_max(d), p.tiles, kTM, p.tall, kTallRows);
 }
 
 static PlanSizes plan_sizes(const kge_tables *tab, const kge_batch *bat)
@@ -1698,7 +1900,7 @@ int launch_transr_fwd(const kge_tables *tab, const kge_batch *bat, float *pos, f
     const kge_inspection *ri = bat->rel_insp;
     const PlanSizes z = plan_sizes(tab, bat);
     const Plans plans = plans_at(workspace, z);
-    if (!bat->plans_ready) launch_plans(ri, ri->seg_offsets, plans, tab->dim, st);
+    if (!bat->plans_ready) launch_plans(ri, ri->seg_offsets, plans, tab->dim, false, st);
     GemmArgs a{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
                plans.tiles, nullptr, nullptr, pos, resid, nullptr, nullptr, (int)tab->dim, tab->norm_p,
                thin_groups(tab, bat), (int)z.tiles, BwdSrc{}, bat->back_rows};
@@ -1750,7 +1952,7 @@ int launch_transr_plan(const kge_tables *tab, const kge_batch *bat, void *worksp
     if (!mfma_path_ok(tab, bat) || gemm_lds_bytes((int)tab->dim) > kMaxGemmLds) return KGE_EUNSUPPORTED;
     if (!workspace || workspace_bytes < transr_fwd_workspace(tab, bat)) return KGE_EWORKSPACE;
     const kge_inspection *ri = bat->rel_insp;
-    launch_plans(ri, ri->seg_offsets, plans_at(workspace, plan_sizes(tab, bat)), tab->dim, st);
+    launch_plans(ri, ri->seg_offsets, plans_at(workspace, plan_sizes(tab, bat)), tab->dim, false, st);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }
@@ -1862,7 +2064,7 @@ int launch_rescal_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
                        dneg ? g0 : nullptr, saved->residual, xs, qs, head ? occ : occ + B * d, B, d, head ? 1 : 0);
     const PlanSizes z = plan_sizes(tab, bat);
     const Plans plans = plans_at(ws + p.off_plans, z);
-    launch_plans(ri, ri->seg_offsets, plans, d, st);
+    launch_plans(ri, ri->seg_offsets, plans, d, false, st);
     // head: the tails' rows (g E[h] + G) Proj[r], the forward product on rows given as an array, written per triple
     GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
                 TilePlan{}, head ? xs : qs, nullptr, nullptr, head ? occ + B * d : nullptr, head ? nullptr : occ, nullptr, d, tab->norm_p, 0, 0,
@@ -1923,7 +2125,7 @@ int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_sav
         hipLaunchKernelGGL(transr_insp_step_kernel, dim3((unsigned)f1.blocks), dim3(256), lds_with(f1, 0), st, f1);
         timeline_mark(bat->timeline, st, "inspector step");
     }
-    if (!have_plans) launch_plans(ri, ri->seg_offsets, plans, d, st);
+    if (!have_plans) launch_plans(ri, ri->seg_offsets, plans, d, false, st);
     // Upstream rows q and left operands x are formed inside the two kernels from the forward pass's rows
     // (BwdSrc); RESCAL's tail occurrence rows g * v come out of the dX kernel's staging.
     const BwdSrc src{tab->ent, saved->residual, dpos, saved->pos, bat->h, bat->t, ri->perm, tab->norm_p, rescal ? 1 : 0,

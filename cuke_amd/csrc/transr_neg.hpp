@@ -24,6 +24,7 @@ struct NegShape {
     int64_t B, N, C, n_chunks, NN, d, U_cap, G_cap, L_cap;
     int64_t dslots;
     PlanSizes plans;
+    bool dm_split;
 };
 
 static NegShape neg_shape(const kge_tables *tab, const kge_batch *bat)
@@ -40,6 +41,14 @@ static NegShape neg_shape(const kge_tables *tab, const kge_batch *bat)
     if (want_tall(s.d, s.L_cap, tab->n_rel)) s.plans.tall = tall_tiles(s.U_cap, s.L_cap);
     else s.plans.tiles = s.U_cap + s.L_cap / kTM + 1;
     s.dslots = 2 * (s.L_cap / kDmChunk) + 2;
+    // dM by items of 128 x 128 where there can be one for each resident workgroup: below that the fp32 items, four to seven times as many,
+    // spread a chunk's walk over more of the chip (1024 triples x 128, 50 relations, N = 16: 17.5 us against 28.7; 4096 x 152, 10
+    // relations, N = 64: 28.4 against 28.5).  Groups of fewer negatives are a slice or two, all index chain and epilogue (1024 x 200, 500
+    // relations, N = 40: 55 against 60), and those of at most kDmSmall rows one workgroup's work in both, three a CU with the fp32 kernel
+    // (2048 x 100, 1345 relations, N = 20: 27 against 32).  Above: 4096 x 200, 1345 relations, N = 64 151 -> 123; x 256, 200 relations
+    // 262 -> 166; x 48, 2000 relations 98 -> 68; 2048 x 128, 300 relations, N = 48 48 -> 32; 512 x 64, 2000 relations, N = 64 21 -> 17.
+    const int64_t nt = dm_split_tiles((int)s.d);
+    s.dm_split = s.N >= 48 && s.plans.dtiles * nt * nt >= kDmSplitWgs;
     return s;
 }
 
@@ -96,7 +105,7 @@ static NegBwdLayout neg_bwd_layout(const NegShape &s)
         return at;
     };
     const size_t rows = sizeof(float) * (size_t)(s.L_cap * s.d);
-    l.zero = take(sizeof(float) * (size_t)s.d), l.ql = take(rows), l.dxl = take(rows);
+    l.zero = take(sizeof(float) * ((size_t)s.d + kDmTickets)), l.ql = take(rows), l.dxl = take(rows);
     l.occ = take(sizeof(float) * (size_t)((2 * s.B + s.NN) * s.d));
     l.qr = take(sizeof(float) * (size_t)(s.B * s.d));
     l.glist = take(sizeof(int32_t) * s.B);
@@ -196,7 +205,7 @@ __global__ __launch_bounds__(64) void tneg_chunk_groups_kernel(NegIdx x, int32_t
     const int64_t c = blockIdx.x;
     const int lane = threadIdx.x;
     if (c == 0)
-        for (int i = lane; i < x.d; i += kWave) zero_row[i] = 0.0f;
+        for (int i = lane; i < x.d + kDmTickets; i += kWave) zero_row[i] = 0.0f;  // (and the counters behind it)
     int count = 0;
     for (int64_t i0 = 0; i0 < x.C; i0 += kWave) {
         const int64_t i = i0 + lane;
@@ -633,7 +642,7 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
     const int64_t list_blocks = ceil_div(list_threads, 256);
     hipLaunchKernelGGL(tneg_list_kernel, dim3((unsigned)(list_blocks < 8192 ? list_blocks : 8192)), dim3(256), 0, st, x);
     const Plans plans = plans_at(ws + l.plans, s.plans);
-    launch_plans(ri, x.segl, plans, d, st);
+    launch_plans(ri, x.segl, plans, d, s.dm_split, st);
     timeline_mark(bat->timeline, st, "row list + transr_plan_kernel");
 
     // one grouped pass projects every list row
@@ -699,9 +708,10 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     if (const int rc = launch_product(2, ga, plans, s.plans, s.U_cap, nullptr, s.B, FusedInsp{}, st)) return rc;
     timeline_mark(bat->timeline, st, s.plans.tall ? "transr_tall_kernel<dX>" : "transr_gemm_kernel<dX>");
     DmArgs da{nullptr, ql, x.segl, plans.dm, grads->aux_rows, reinterpret_cast<float *>(ws + l.dpart), d, ri->num_unique,
-              BwdSrc{}, nullptr, nullptr, 0, tab->ent, x.hl, x.tl, zero_row};
-    hipLaunchKernelGGL(transr_dm_kernel, dim3((unsigned)kDmWgs), dim3(256), dm_lds_bytes(d), st, da, FusedInsp{}, SegL1Rider{});
-    timeline_mark(bat->timeline, st, "transr_dm_kernel");
+              BwdSrc{}, nullptr, nullptr, 0, tab->ent, x.hl, x.tl, zero_row, reinterpret_cast<int32_t *>(zero_row + d)};
+    if (s.dm_split) hipLaunchKernelGGL(transr_dm_split_kernel, dim3((unsigned)kDmSplitWgs), dim3(256), dm_split_lds_bytes(d), st, da);
+    else hipLaunchKernelGGL(transr_dm_kernel, dim3((unsigned)kDmWgs), dim3(256), dm_lds_bytes(d), st, da, FusedInsp{}, SegL1Rider{});
+    timeline_mark(bat->timeline, st, s.dm_split ? "transr_dm_split_kernel" : "transr_dm_kernel");
     TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_occ_kernel<NQ_>, dim3((unsigned)(ceil_div(s.B, occ_waves<NQ_>()) + s.NN)), dim3(kWave * occ_waves<NQ_>()), 0, st, x, dxl,
                                         glist, gcount, occ));
     timeline_mark(bat->timeline, st, "tneg_occ_kernel");

@@ -22,9 +22,6 @@ constexpr int kTallRing = 4;    // supersteps (16 rows of k) of the projection i
 constexpr int kSplitRows = 16;    // tiles of more rows go by the bf16 matrix cores ...
 constexpr int kSplitItems = 256;  // ... where a launch has more items than that
 constexpr int kTallWgs = 4096;  // workgroups of a launch at most; they stride over the tiles
-// (global, not generic: a pointer that went through LDS would otherwise be followed with flat loads, which also count as LDS
-// operations and are waited for as such)
-typedef const float __attribute__((address_space(1))) *global_f32;
 
 struct TallRows {  // what a tile knows about its rows (LDS, behind the staging buffers)
     global_f32 v[kTallRows], w[kTallRows];     // the rows the left operand is formed from
@@ -37,13 +34,6 @@ struct TallRows {  // what a tile knows about its rows (LDS, behind the staging 
 constexpr size_t kTallStage = sizeof(__bf16) * kSplitPitch * (kTallRows + kTallCols);
 static_assert(kTallStage >= sizeof(float) * 2 * kTallRows * kTallPitch && kTallStage % 16 == 0, "the row table stands behind both forms");
 constexpr size_t kTallLds = kTallStage + sizeof(TallRows);
-
-__device__ __forceinline__ float4 load4g(global_f32 p)
-{
-    typedef const floatx4 __attribute__((address_space(1))) *global_f32x4;
-    const floatx4 v = *(global_f32x4)p;
-    return make_float4(v[0], v[1], v[2], v[3]);
-}
 
 __host__ __device__ inline int tall_col_blocks(int d) { return (d + kTallCols - 1) / kTallCols; }
 // columns of a block / of a wave: an even split, multiples of four / two

@@ -20,6 +20,7 @@
 namespace kge {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef double v4d __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------------------
 // 1 + 2: tile kernel.  "Owners" keep their slice of the row in registers and accumulate
@@ -127,10 +128,15 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     constexpr bool kDot = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF ||
                           MODEL == KGE_RESCAL;  // score = query . t' (+ const)
     // TransE, L2: sum_l g_l (o - x_l) = o sum_l g_l - sum_l g_l x_l, the owner's row times its coefficients' sum and the dot models'
-    // product, folded once per step like the differences' sum it replaces.  2-norm of the entity rows' error against 64 bits,
-    // differences -> product: margin loss 8.2e-8 -> 7.3e-8 (3000 x 600 x 200 negatives x 150), 9.5e-8 -> 8.5e-8 (1024 x 1024 x 400), gradients of
-    // both signs 1.63e-7 -> 1.54e-7 and 2.17e-7 -> 2.09e-7; unfolded 9.9e-8 / 1.3e-7 / 3.2e-7 / 4.8e-7.
-    // The two orientations at 30000 x 200 x 150: 204 -> 113 us.
+    // product.  The two sides are of the size of the ROWS, their difference of the size of the rows' distances, and training
+    // draws rows together: in fp32 the product form loses what the rows have in common.  So it is formed in 64 bits
+    // (v_mfma_f64_16x16x4_f64): products of fp32 values are exact there, and what the sums round away is 2^-29 of what one fp32
+    // rounding of a difference does to rows that differ at all.
+    //   2-norm of the gradient rows' error against 64 bits, 1024 x 200 negatives x 150, spread 0.05, differences -> product in fp32 -> in 64
+    //   bits: centred rows 5.9e-8 -> 4.7e-8 -> 2.5e-8; offset 0.25 in every column 5.9e-8 -> 3.2e-7 -> 2.5e-8, offset 5 5.9e-8 -> 6.9e-6 ->
+    //   2.5e-8; a negative within 1e-4 of every h + r 5.9e-8 -> 7.2e-7 -> 2.5e-8, within 1e-5 5.9e-8 -> 7.1e-6 -> 2.5e-8.
+    //   Bound by the 64-bit matrix instructions (43 TFLOP/s measured; fp32's 120): the two orientations at 30000 x 200 x 150 206 us by
+    //   differences, 113 by fp32 products, 181 now.
     constexpr bool kDiff = MODEL == KGE_TRANSE && P == 2 && MF;
     constexpr bool kMf = (kDot || kDiff) && MF;  // the sum over loopers on the matrix cores (else on the vector ALUs)
     constexpr bool kL2 = (MODEL == KGE_TRANSE || kTH) && P == 2;
@@ -238,10 +244,14 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     constexpr int EW = 4;  // MFMAs (columns per lane) per wave
     static_assert(!kMf || TO == 64, "a wave per 16 of 64 owners");
     const int mlane = tid & 63, ob = tid >> 6, fj = mlane & 15, fg = mlane >> 4;
-    float csum = 0.0f;  // kDiff: this lane's share of the coefficients of owner 16 ob + fj
     v4f macc[EW];
 #pragma unroll
     for (int e = 0; e < EW; ++e) macc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    // kDiff: the same in 64 bits, where a lane receives D[i = l / 16 + 4 v][j]
+    double csum = 0.0;  // this lane's share of the coefficients of owner 16 ob + fj
+    v4d dacc[EW];
+#pragma unroll
+    for (int e = 0; e < EW; ++e) dacc[e] = v4d{0.0, 0.0, 0.0, 0.0};
 
     // ---- staging: a three-deep software pipeline --------------------------------------------
     // While step st is computed, the rows and coefficients of step st+1 are in flight and so are
@@ -408,32 +418,21 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
         // into the running one per step, so rounding grows with sqrt(steps) of the large partial
         // sums instead of sqrt(loopers)
         if constexpr (kMf) {
-            v4f mstep[EW];
-            float cstep = 0.0f;
-            if constexpr (kDiff) {
-#pragma unroll
-                for (int e = 0; e < EW; ++e) mstep[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-            }
 #pragma unroll
             for (int q = 0; q < kKL / 16; ++q)
 #pragma unroll
                 for (int ms = 0; ms < 4; ++ms) {
                     const int l = 16 * q + 4 * fg + ms;
                     const float av = sG[0][l][ob * 16 + fj];
-                    if constexpr (kDiff) cstep += av;
                     const float4 b4 = *reinterpret_cast<const float4 *>(&sL[0][l][4 * fj]);
                     const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
+                    if constexpr (kDiff) csum += (double)av;
 #pragma unroll
                     for (int e = 0; e < EW; ++e) {
-                        v4f &acc = kDiff ? mstep[e] : macc[e];
-                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], acc, 0, 0, 0);
+                        if constexpr (kDiff) dacc[e] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av, (double)bv[e], dacc[e], 0, 0, 0);
+                        else macc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], macc[e], 0, 0, 0);
                     }
                 }
-            if constexpr (kDiff) {
-                csum += cstep;
-#pragma unroll
-                for (int e = 0; e < EW; ++e) macc[e] += mstep[e];
-            }
         }
         float4 sacc[NOUT][RO_];
 #pragma unroll
@@ -589,11 +588,14 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
         if constexpr (kDiff) {
             csum += __shfl_xor(csum, 16, kWave);
             csum += __shfl_xor(csum, 32, kWave);
+            double cs[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) cs[v] = __shfl(csum, fg + 4 * v, kWave);
             const int c0 = gcol(4 * fj);
             float4 mine[4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) {  // (rows past the tile's edge: its last row again, not stored)
-                const int oc = min(ot0 + ob * 16 + 4 * fg + v, n_own - 1);
+                const int oc = min(ot0 + ob * 16 + fg + 4 * v, n_own - 1);
                 if constexpr (OWNER_POS) {
                     const int64_t b = (int64_t)c * a.C + oc;
                     float4 none;
@@ -605,10 +607,12 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             }
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const float cs = __shfl(csum, 4 * fg + v, kWave);
-                macc[0][v] = fmaf(mine[v].x, cs, -macc[0][v]), macc[1][v] = fmaf(mine[v].y, cs, -macc[1][v]);
-                macc[2][v] = fmaf(mine[v].z, cs, -macc[2][v]), macc[3][v] = fmaf(mine[v].w, cs, -macc[3][v]);
+                const int ol = ot0 + ob * 16 + fg + 4 * v;
+                if (ol >= n_own) continue;
+                auto diff = [&](float own, int e) { return (float)fma((double)own, cs[v], -dacc[e][v]); };
+                put(a.out0 + ((int64_t)c * n_own + ol) * (int64_t)d, 4 * fj, make_float4(diff(mine[v].x, 0), diff(mine[v].y, 1), diff(mine[v].z, 2), diff(mine[v].w, 3)));
             }
+            return;
         }
 #pragma unroll
         for (int v = 0; v < 4; ++v) {

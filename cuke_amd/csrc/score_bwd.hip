@@ -715,9 +715,16 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
     // the size rule follows launch_neg_mp (see there)
     constexpr bool kDotModel = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL;
     if constexpr (kDotModel || (MODEL == KGE_TRANSE && P == 2)) {
-        // matrix-core inner loop (KGE_PAIR_SUMS_VALU keeps the vector-ALU loop): a wave gets all 64
-        // columns of its 16 owners with 64-owner tiles, which win at every size
-        if (!dot_valu) {
+        // matrix-core inner loop (KGE_PAIR_SUMS_VALU keeps the vector-ALU loop): a wave gets all 64 columns of its 16 owners with
+        // 64-owner tiles, which win at every size for the dot products.  TransE L2's 64-bit products are slow enough for the walk of one
+        // tile to show: smaller differences' tiles are faster until the owners of the longer walk (min(C, N) of them a chunk) fill
+        // about a hundred 64-owner tiles, or until the differences take 64-owner tiles themselves.  us, matrix / differences, by
+        // columns of tiles x chunks x min(C, N):  900 41 / 33 (1500 x 500 x 100 x 150)   2400 92 / 89 (5000 x 1000 x 48 x 600)
+        //   3000 56 / 52 (3000 x 600 x 200 x 150)   4096 25 / 22 (1024 x 256 x 256 x 256)   6000 65 / 73 (6000 x 600 x 200 x 150), but 21 / 18
+        //   (2000 x 100 x 100 x 130)   6144 26 / 32 (1536 x 256 x 256 x 256)   7168 42 / 48 (1024 x 512 x 512 x 400)   12000 22 / 26 (4000 x 100 x
+        //   100 x 130)   28672 192 / 217 (4096 x 1024 x 1024 x 400); from 1024 tiles on 112 / 165 (4096 x 1024 x 50 x 1000), 40 / 41 (16384 x 16 x 16 x 100).
+        const bool fill = kDotModel || big >= 1024 || gx * n_chunks * (a.C < a.N ? a.C : a.N) >= 6144;
+        if (!dot_valu && fill) {
             // (ComplEx by quads: column tiles pair 32 real with the matching 32 imaginary columns)
             const int64_t gxm = (MODEL == KGE_COMPLEX && a.vec) ? ceil_div(a.d / 2, 32) : gx;
             const unsigned gh = xcd_grid(gxm, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxm, ceil_div(a.N, 64), n_chunks);

@@ -8,13 +8,13 @@ from cuke_amd.kge import KGEModel
 
 pytestmark = pytest.mark.gpu
 
-# (batch, chunk, n_neg, dim): the 64-bit products and the differences' 16-, 32- and 64-owner tiles, with and without a narrow last column
-# tile; odd widths and counts
+# (batch, chunk, n_neg, dim): the 64-bit products' side of the rule and the differences' 16-, 32- and 64-owner tiles, with and without
+# a narrow last column tile; odd widths and counts
 SHAPES = [
-    (1536, 256, 200, 150, "matrix_cores"), 
-    (1024, 256, 256, 400, "matrix_cores"), 
-    (2000, 500, 130, 801, "matrix_cores"),   # odd rows and a last tile of 33 columns
-    (8192, 128, 1, 130, "matrix_cores"),     # single owners
+    (1536, 256, 200, 150, "matrix_cores"),   # 3 x 6 x 200 owners are too few: 16-owner differences
+    (1024, 256, 256, 400, "matrix_cores"),   # 7 x 4 x 256: products
+    (2000, 500, 130, 801, "matrix_cores"),   # products, odd rows and a last tile of 33 columns
+    (8192, 128, 1, 130, "matrix_cores"),     # 576 tiles of single owners: 32-owner differences
     (1100, 100, 77, 200, "vector_alus"),     # 16 owners
     (2048, 128, 128, 550, "vector_alus"),    # 32 owners
     (4096, 256, 256, 523, "vector_alus"),    # 64 owners, 11 columns in narrow tiles

@@ -9,8 +9,9 @@
 //   1.9e-7; one sign 1.6e-7 -> 1.2e-7 at 416; spread exponents 1.2e-7 -> 1.2e-7 at 416.  (One accumulator for all six: 3.0e-7 at 416, worse
 //   than fp32; the three products of two-part sums: 4e-6.)  No bias.
 //   Rate: 2.1 PFLOP/s of bf16 measured, 350 TFLOP/s of such products, against 156 of v_mfma_f32_16x16x4_f32.
-// An operand that is infinite (or rounds to infinity, above 3.39e38) makes NaN of v1, so every sum it enters comes out NaN; callers form
-// sums that are NaN again in plain fp32 (pair_dot below), which gives infinities and NaNs the meaning they have there.
+// An operand that is infinite (or rounds to infinity, above 3.39e38) makes NaN of v1, so every sum it enters comes out NaN; and leading
+// parts that were rounded up can overflow where the product of the values does not.  Callers form sums that are not finite again in
+// plain fp32 (pair_dot below), which gives overflow, infinities and NaNs the meaning they have there.
 #pragma once
 
 #include "common.hpp"
@@ -54,6 +55,9 @@ __device__ __forceinline__ floatx16 mfma_bf16(bf16x8 a, bf16x8 b, floatx16 c) { 
 // the products of the two operands' parts, smallest first: (part of a, part of b) of step t; the last one is the leading product
 constexpr int kSplitTerms = 6;
 __device__ constexpr int kTermA[kSplitTerms] = {0, 2, 1, 0, 1, 0}, kTermB[kSplitTerms] = {2, 0, 1, 1, 0, 0};
+
+// Whether a sum says nothing about its fp32 value.
+__device__ __forceinline__ bool not_finite(float s) { return !(fabsf(s) <= 3.402823466e38f); }
 
 // a . b in plain fp32
 __device__ inline float pair_dot(const float *a, const float *b, int n)

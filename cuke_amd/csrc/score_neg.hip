@@ -647,7 +647,7 @@ __global__ __launch_bounds__(256, 2) void score_neg_split_kernel(SplitArgs a, Fu
                 const int kl = kt0 + wcol + 32 * n + fr;
                 if (kl >= a.N) continue;
                 float s = lead[m][n][v] + rest[m][n][v];
-                if (s != s) s = pair_dot(a.query + b * d, a.ent + a.neg[(int64_t)c * a.N + kl] * (int64_t)d, d);
+                if (not_finite(s)) s = pair_dot(a.query + b * d, a.ent + a.neg[(int64_t)c * a.N + kl] * (int64_t)d, d);
                 a.out[b * a.N + kl] = s + shift;
             }
         }

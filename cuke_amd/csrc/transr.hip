@@ -1481,7 +1481,7 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
 // through LDS once per 128 of the other's, transposed on the way (positions are the product's inner dimension), in slices of 32
 // positions; wave w stages the 32 columns w of both and forms the blocks (w % 2 + {0, 2}) x (w / 2 + {0, 2}) of 32 x 32, so tiles of
 // fewer blocks spread over the waves.  A position past the end repeats the last one against an x that is zero, a column past the end
-// repeats the last quad and is stored nowhere.  Sums that are NaN are formed again in fp32.
+// repeats the last quad and is stored nowhere.  Sums that are not finite are formed again in fp32.
 constexpr int kDmTile = 128;
 __host__ __device__ inline int dm_split_tiles(int d) { return (d + kDmTile - 1) / kDmTile; }
 struct DmSplitRows {  // the chunk's entity rows, x = h - t
@@ -1618,7 +1618,7 @@ __device__ __forceinline__ void transr_dm_split_item(const DmArgs &a, float *lds
                 const int row = 8 * (e / 4) + e % 4;
                 if (rb + row >= ni) continue;
                 float s = lead[i][j][e] + rest[i][j][e];
-                if (s != s) {
+                if (not_finite(s)) {
                     s = 0.0f;
                     for (int p = 0; p < n; ++p)
                         s = fmaf(R.h[p][i0 + rb + row] - R.t[p][i0 + rb + row], a.qs[(int64_t)(s0 + p) * d + j0 + cb], s);

@@ -464,13 +464,13 @@ __device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int ti
         __syncthreads();
     }
 
-    // A sum that came out NaN (mfma_split.hpp): the caller forms the tile again in fp32.
+    // A sum that is not finite (mfma_split.hpp): the caller forms the tile again in fp32.
     const bool colok = 32 * wave + fr < span;
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) lead[i][e] += rest[i][e], bad = bad || (colok && lead[i][e] != lead[i][e]);
+        for (int e = 0; e < 16; ++e) lead[i][e] += rest[i][e], bad = bad || (colok && not_finite(lead[i][e]));
     if (__syncthreads_or(bad)) return true;
 
     // Lane (fr, fg) holds rows 32 i + 8 (e / 4) + 4 fg + e % 4, column c0 + 32 wave + fr.
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256, 3) void transr_tall_kernel(TallArgs t, FusedIn
     if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(lds))) return;
     const int ncb = tall_col_blocks(t.g.d), n = t.g.plan.num_tiles[0] * ncb, step = (int)gridDim.x - fi.blocks, first = (int)blockIdx.x - fi.blocks;
     const int split_rows = n > kSplitItems ? kSplitRows : kTallRows;  // tiles of more rows are split
-    uint64_t again = 0;  // items (by turn; launch_tall gives a workgroup at most 64) whose sums were not all numbers
+    uint64_t again = 0;  // items (by turn; launch_tall gives a workgroup at most 64) whose sums were not all finite
     auto rows_of = [&](int it) { return t.g.plan.tile_end[it / ncb] - t.g.plan.tile_p0[it / ncb]; };
     for (int it = first, turn = 0; it < n; it += step, ++turn)
         if (rows_of(it) > split_rows) {

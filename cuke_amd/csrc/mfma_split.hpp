@@ -10,8 +10,8 @@
 //   than fp32; the three products of two-part sums: 4e-6.)  No bias.
 //   Rate: 2.1 PFLOP/s of bf16 measured, 350 TFLOP/s of such products, against 156 of v_mfma_f32_16x16x4_f32.
 // An operand that is infinite (or rounds to infinity, above 3.39e38) makes NaN of v1, so every sum it enters comes out NaN; and leading
-// parts that were rounded up can overflow where the product of the values does not.  Callers form sums that are not finite again in
-// plain fp32 (pair_dot below), which gives overflow, infinities and NaNs the meaning they have there.
+// parts that were rounded up can overflow where the product of the values does not.  So a tile that holds a sum that is not finite is
+// formed again with fp32 instructions (mfma_fp32 below), which gives overflow, infinities and NaNs the meaning they have there.
 #pragma once
 
 #include "common.hpp"
@@ -56,15 +56,29 @@ __device__ __forceinline__ floatx16 mfma_bf16(bf16x8 a, bf16x8 b, floatx16 c) { 
 constexpr int kSplitTerms = 6;
 __device__ constexpr int kTermA[kSplitTerms] = {0, 2, 1, 0, 1, 0}, kTermB[kSplitTerms] = {2, 0, 1, 1, 0, 0};
 
+// ---- the same blocks by fp32 instructions ----
 // Whether a sum says nothing about its fp32 value.
 __device__ __forceinline__ bool not_finite(float s) { return !(fabsf(s) <= 3.402823466e38f); }
 
-// a . b in plain fp32
-__device__ inline float pair_dot(const float *a, const float *b, int n)
+// A K = 2 step of a 32 x 32 block: lane l holds row l % 32 of its operand, k = l / 32; receives what mfma_bf16 gives it.
+__device__ __forceinline__ floatx16 mfma_fp32(float a, float b, floatx16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
+
+// Staged rows: 32 columns of a row and 16 bytes of padding (shorter than the three parts').  Eight columns of an A x B block: lane group
+// l / 32 takes four of them from 128-bit reads of its rows.
+constexpr int kPlainPitch = kSplitK + 4;
+static_assert(sizeof(float) * kPlainPitch <= sizeof(__bf16) * kSplitPitch, "fits where the parts stood");
+template <int A, int B>
+__device__ __forceinline__ void plain_step(const float4 (&av)[A], const float4 (&bv)[B], floatx16 (&acc)[A][B])
 {
-    float s = 0.0f;
-    for (int i = 0; i < n; ++i) s = fmaf(a[i], b[i], s);
-    return s;
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            acc[i][j] = mfma_fp32(av[i].x, bv[j].x, acc[i][j]);
+            acc[i][j] = mfma_fp32(av[i].y, bv[j].y, acc[i][j]);
+            acc[i][j] = mfma_fp32(av[i].z, bv[j].z, acc[i][j]);
+            acc[i][j] = mfma_fp32(av[i].w, bv[j].w, acc[i][j]);
+        }
 }
 
 }  // namespace kge

@@ -634,6 +634,43 @@ __global__ __launch_bounds__(256, 2) void score_neg_split_kernel(SplitArgs a, Fu
         __syncthreads();
     }
 
+    bool bad = false;  // (rows past the tile's edge repeat one of its own)
+#pragma unroll
+    for (int m = 0; m < MB; ++m)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) lead[m][n][v] += rest[m][n][v], bad = bad || not_finite(lead[m][n][v]);
+    if (__syncthreads_or(bad)) {  // the tile again by fp32 instructions (mfma_split.hpp)
+        float(*fA)[kPlainPitch] = reinterpret_cast<float(*)[kPlainPitch]>(dyn_smem);
+        float(*fT)[kPlainPitch] = fA + TB;
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) lead[m][n][v] = 0.0f;
+#pragma unroll 1
+        for (int j0 = 0; j0 < d; j0 += kSplitK) {
+            load_slice(j0);
+#pragma unroll
+            for (int s = 0; s < SB; ++s) *reinterpret_cast<float4 *>(&fA[srow + 32 * s][scol]) = mask4<true>(ra[s], j0 + scol, d);
+#pragma unroll
+            for (int s = 0; s < SN; ++s) *reinterpret_cast<float4 *>(&fT[srow + 32 * s][scol]) = mask4<true>(rt[s], j0 + scol, d);
+            __syncthreads();
+#pragma unroll 1
+            for (int k = 4 * fg; k < kSplitK; k += 8) {
+                float4 av[MB], tv[NB];
+#pragma unroll
+                for (int m = 0; m < MB; ++m) av[m] = *reinterpret_cast<const float4 *>(&fA[wrow + 32 * m + fr][k]);
+#pragma unroll
+                for (int n = 0; n < NB; ++n) tv[n] = *reinterpret_cast<const float4 *>(&fT[wcol + 32 * n + fr][k]);
+                plain_step(av, tv, lead);
+            }
+            __syncthreads();
+        }
+    }
+
 #pragma unroll
     for (int m = 0; m < MB; ++m)
 #pragma unroll
@@ -645,10 +682,7 @@ __global__ __launch_bounds__(256, 2) void score_neg_split_kernel(SplitArgs a, Fu
 #pragma unroll
             for (int n = 0; n < NB; ++n) {
                 const int kl = kt0 + wcol + 32 * n + fr;
-                if (kl >= a.N) continue;
-                float s = lead[m][n][v] + rest[m][n][v];
-                if (not_finite(s)) s = pair_dot(a.query + b * d, a.ent + a.neg[(int64_t)c * a.N + kl] * (int64_t)d, d);
-                a.out[b * a.N + kl] = s + shift;
+                if (kl < a.N) a.out[b * a.N + kl] = lead[m][n][v] + shift;
             }
         }
 }

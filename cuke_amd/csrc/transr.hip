@@ -1481,7 +1481,7 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
 // through LDS once per 128 of the other's, transposed on the way (positions are the product's inner dimension), in slices of 32
 // positions; wave w stages the 32 columns w of both and forms the blocks (w % 2 + {0, 2}) x (w / 2 + {0, 2}) of 32 x 32, so tiles of
 // fewer blocks spread over the waves.  A position past the end repeats the last one against an x that is zero, a column past the end
-// repeats the last quad and is stored nowhere.  Sums that are not finite are formed again in fp32.
+// repeats the last quad and is stored nowhere.  An item with sums that are not finite is formed again in fp32.
 constexpr int kDmTile = 128;
 __host__ __device__ inline int dm_split_tiles(int d) { return (d + kDmTile - 1) / kDmTile; }
 struct DmSplitRows {  // the chunk's entity rows, x = h - t
@@ -1603,29 +1603,72 @@ __device__ __forceinline__ void transr_dm_split_item(const DmArgs &a, float *lds
         }
         __syncthreads();
     }
-    if (!active) return;
-
     // Lane (fr, fg) holds of block (i, j) the rows 8 (e / 4) + 4 fg + e % 4 of column fr.
+    auto store = [&] {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int rb = 32 * wi + 64 * i + 4 * fg, cb = 32 * wj + 64 * j + fr;
+                if (cb >= nj) continue;
+                float *out = dst + (int64_t)(i0 + rb) * d + j0 + cb;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int row = 8 * (e / 4) + e % 4;
+                    if (rb + row >= ni) continue;
+                    const float s = lead[i][j][e] + rest[i][j][e];
+                    bad = bad || not_finite(s);
+                    out[(int64_t)row * d] = s;
+                }
+            }
+        return bad;
+    };
+    if (!__syncthreads_or(store())) return;
+
+    // The item again by fp32 instructions (mfma_split.hpp); a position past the end is zero on both sides.
+    float(*fX)[kPlainPitch] = reinterpret_cast<float(*)[kPlainPitch]>(lds);
+    float(*fQ)[kPlainPitch] = fX + kDmTile;
+    auto put_plain = [&](float(*at)[kPlainPitch], const float4 (&x)[4]) {
+        *reinterpret_cast<float4 *>(&at[4 * nb + 0][4 * kb]) = make_float4(x[0].x, x[1].x, x[2].x, x[3].x);
+        *reinterpret_cast<float4 *>(&at[4 * nb + 1][4 * kb]) = make_float4(x[0].y, x[1].y, x[2].y, x[3].y);
+        *reinterpret_cast<float4 *>(&at[4 * nb + 2][4 * kb]) = make_float4(x[0].z, x[1].z, x[2].z, x[3].z);
+        *reinterpret_cast<float4 *>(&at[4 * nb + 3][4 * kb]) = make_float4(x[0].w, x[1].w, x[2].w, x[3].w);
+    };
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int rb = 32 * wi + 64 * i + 4 * fg, cb = 32 * wj + 64 * j + fr;
-            if (cb >= nj) continue;
-            float *out = dst + (int64_t)(i0 + rb) * d + j0 + cb;
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = 8 * (e / 4) + e % 4;
-                if (rb + row >= ni) continue;
-                float s = lead[i][j][e] + rest[i][j][e];
-                if (not_finite(s)) {
-                    s = 0.0f;
-                    for (int p = 0; p < n; ++p)
-                        s = fmaf(R.h[p][i0 + rb + row] - R.t[p][i0 + rb + row], a.qs[(int64_t)(s0 + p) * d + j0 + cb], s);
+            for (int e = 0; e < 16; ++e) lead[i][j][e] = 0.0f, rest[i][j][e] = 0.0f;
+#pragma unroll 1
+    for (int k0 = 0; k0 < n; k0 += kSplitK) {
+        load_x(k0), load_q(k0);
+        float4 x[4], y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool ok = k0 + 4 * kb + e < n;
+            x[e] = make_float4(ok ? v[e].x - w[e].x : 0.0f, ok ? v[e].y - w[e].y : 0.0f, ok ? v[e].z - w[e].z : 0.0f, ok ? v[e].w - w[e].w : 0.0f);
+            y[e] = make_float4(ok ? q[e].x : 0.0f, ok ? q[e].y : 0.0f, ok ? q[e].z : 0.0f, ok ? q[e].w : 0.0f);
+        }
+        if (has_x) put_plain(fX, x);
+        if (has_q) put_plain(fQ, y);
+        __syncthreads();
+        if (active) {
+#pragma unroll 1
+            for (int k = 4 * fg; k < kSplitK; k += 8) {
+                float4 xv[2], qv[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    xv[i] = *reinterpret_cast<const float4 *>(&fX[32 * wi + 64 * i + fr][k]);
+                    qv[i] = *reinterpret_cast<const float4 *>(&fQ[32 * wj + 64 * i + fr][k]);
                 }
-                out[(int64_t)row * d] = s;
+                plain_step(xv, qv, lead);
             }
         }
+        __syncthreads();
+    }
+    store();
 }
 
 static size_t dm_lds_bytes(int d)  // the staged left operand and its row offsets, or the thin groups' transposed rows

@@ -142,6 +142,14 @@ __device__ __forceinline__ void tall_sweep(const TallLoader<MODE> &bl, int d, Ta
     }
 }
 
+// threadIdx.x, opaque: what follows from it is formed anew per tile and not held across the forms of a tile that share a kernel
+__device__ __forceinline__ int tile_tid()
+{
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+
 // fills the row table of the tile's `rows` rows from position p0 on (one thread per row; later rows repeat the first)
 template <int MODE>
 __device__ __forceinline__ void tall_rows(const GemmArgs &a, TallRows &R, int p0, int rows, bool array, bool derived)
@@ -178,7 +186,7 @@ __device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int til
 {
     const GemmArgs &a = t.g;
     const int d = a.d, ncb = tall_col_blocks(d);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kk = lane >> 4;
+    const int tid = tile_tid(), lane = tid & 63, wave = tid >> 6, li = lane & 15, kk = lane >> 4;
     // (uniform, but the compiler cannot know: the kernel also stores)
     const int p0 = __builtin_amdgcn_readfirstlane(a.plan.tile_p0[tile]), seg_end = __builtin_amdgcn_readfirstlane(a.plan.tile_end[tile]);
     const int64_t rid = __builtin_amdgcn_readfirstlane(a.plan.tile_rid[tile]);
@@ -335,7 +343,7 @@ __device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int ti
 {
     const GemmArgs &a = t.g;
     const int d = a.d, ncb = tall_col_blocks(d);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 31, fg = lane >> 5;
+    const int tid = tile_tid(), lane = tid & 63, wave = tid >> 6, fr = lane & 31, fg = lane >> 5;
     const int p0 = __builtin_amdgcn_readfirstlane(a.plan.tile_p0[tile]), seg_end = __builtin_amdgcn_readfirstlane(a.plan.tile_end[tile]);
     const int64_t rid = __builtin_amdgcn_readfirstlane(a.plan.tile_rid[tile]);
     const int rows = seg_end - p0 < kTallRows ? seg_end - p0 : kTallRows;

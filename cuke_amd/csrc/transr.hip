@@ -1813,6 +1813,7 @@ struct Plans {
 };
 struct PlanSizes {
     int64_t tiles, dtiles, dsplit, tall, d;
+    bool tall_split;
 };
 
 static size_t plans_bytes(const PlanSizes &z)
@@ -1841,7 +1842,7 @@ static PlanSizes plan_sizes(const kge_tables *tab, const kge_batch *bat)
 {
     const int64_t B = bat->batch, groups = B < tab->n_rel ? B : tab->n_rel;
     return PlanSizes{max_tiles(tab, bat), groups + B / kDmChunk + 1, B / kDmChunk + 1 /* a split group has more than kDmChunk triples */,
-                     want_tall(tab->dim, B, tab->n_rel) ? tall_tiles(groups, B) : 0, tab->dim};
+                     want_tall(tab->dim, B, tab->n_rel) ? tall_tiles(groups, B) : 0, tab->dim, tall_may_split(tab->dim, B, groups)};
 }
 
 static size_t lds_with(const FusedInsp &fi, size_t own)
@@ -1868,7 +1869,7 @@ static int launch_product(int mode, GemmArgs a, const Plans &p, const PlanSizes 
 {
     if (z.tall) {
         a.plan = p.tall;
-        return launch_tall(mode, a, z.tall, part, B, fi, st);
+        return launch_tall(mode, a, z.tall, z.tall_split, part, B, fi, st);
     }
     a.plan = p.tiles, a.max_tiles = (int)z.tiles, a.thin_groups = (int)groups;
     switch (mode) {

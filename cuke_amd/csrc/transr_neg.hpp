@@ -37,7 +37,7 @@ static NegShape neg_shape(const kge_tables *tab, const kge_batch *bat)
     const int64_t pairs = tab->n_rel * s.n_chunks;
     s.G_cap = s.B < pairs ? s.B : pairs;
     s.L_cap = 2 * s.B + s.G_cap * s.N;
-    s.plans = PlanSizes{0, s.U_cap + s.L_cap / kDmChunk + 1, s.L_cap / kDmChunk + 1, 0, s.d};
+    s.plans = PlanSizes{0, s.U_cap + s.L_cap / kDmChunk + 1, s.L_cap / kDmChunk + 1, 0, s.d, tall_may_split(s.d, s.L_cap, s.U_cap)};
     if (want_tall(s.d, s.L_cap, tab->n_rel)) s.plans.tall = tall_tiles(s.U_cap, s.L_cap);
     else s.plans.tiles = s.U_cap + s.L_cap / kTM + 1;
     s.dslots = 2 * (s.L_cap / kDmChunk) + 2;

@@ -487,12 +487,22 @@ __device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int ti
     float rv = 0.0f;  // the relation's row
     if constexpr (MODE == 0 || MODE == 3) rv = a.rel[rid * (int64_t)d + col];
     float *const out = MODE == 2 ? a.occ_h : a.resid;
+    float tail[RB][16];  // RESCAL: the tails' rows, all requested before the first of them is waited for
+    if (MODE == 1 && want_pos) {  // uniform
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int row = 32 * i + 8 * (e / 4) + 4 * fg + e % 4;
+                tail[i][e] = a.ent[R.t[row < rows ? row : 0] * (int64_t)d + col];
+            }
+    }
 #pragma unroll
     for (int i = 0; i < RB; ++i)
 #pragma unroll
         for (int e0 = 0; e0 < 16; e0 += 4) {
             const int row0 = 32 * i + 2 * e0 + 4 * fg;
-            float y[4], tv[4];
+            float y[4];
             int rb[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -500,16 +510,13 @@ __device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int ti
                 y[e] = lead[i][e0 + e], rb[e] = R.b[row];
                 if constexpr (MODE == 0) y[e] += rv;
                 if constexpr (MODE == 3) y[e] += R.f[row] * rv;  // +-1 or 0: exact products
-                tv[e] = 0.0f;
-                if constexpr (MODE == 1)
-                    if (want_pos) tv[e] = a.ent[R.t[row < rows ? row : 0] * (int64_t)d + col];
             }
             if constexpr (MODE < 2) {
                 if (want_pos) {  // uniform
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         float s;
-                        if constexpr (MODE == 1) s = y[e] * tv[e];
+                        if constexpr (MODE == 1) s = y[e] * tail[i][e0 + e];
                         else s = a.norm_p == 1 ? fabsf(y[e]) : y[e] * y[e];
                         s = row16_sum(colok ? s : 0.0f);
                         if ((fr & 15) == 0) R.sum[2 * wave + (fr >> 4)][row0 + e] = s;
@@ -542,25 +549,27 @@ __device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int ti
     return false;
 }
 
-// Two loops over the workgroup's items, not two branches in one: side by side in a loop the two forms' invariants are held at once and 17 to 80
-// registers per lane spill.
-template <int MODE>
+// SPLIT: launches that may hold more than kSplitItems items (tall_may_split); the others leave the split tiles' code out.
+// Two loops over the workgroup's items, not two branches in one: side by side in a loop the two forms' invariants are held at once.
+template <int MODE, bool SPLIT>
 __global__ __launch_bounds__(256, 3) void transr_tall_kernel(TallArgs t, FusedInsp fi)
 {
     extern __shared__ __align__(16) float lds[];
     if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(lds))) return;
     const int ncb = tall_col_blocks(t.g.d), n = t.g.plan.num_tiles[0] * ncb, step = (int)gridDim.x - fi.blocks, first = (int)blockIdx.x - fi.blocks;
-    const int split_rows = n > kSplitItems ? kSplitRows : kTallRows;  // tiles of more rows are split
+    const int split_rows = SPLIT && n > kSplitItems ? kSplitRows : kTallRows;  // tiles of more rows are split
     uint64_t again = 0;  // items (by turn; launch_tall gives a workgroup at most 64) whose sums were not all finite
     auto rows_of = [&](int it) { return t.g.plan.tile_end[it / ncb] - t.g.plan.tile_p0[it / ncb]; };
-    for (int it = first, turn = 0; it < n; it += step, ++turn)
-        if (rows_of(it) > split_rows) {
-            if (split_tile<MODE, 2>(t, lds, it / ncb, it % ncb)) again |= uint64_t(1) << turn;
-            __syncthreads();  // the next tile reuses the staging buffers
-        }
+    if constexpr (SPLIT) {
+        for (int it = first, turn = 0; it < n; it += step, ++turn)
+            if (rows_of(it) > split_rows) {
+                if (split_tile<MODE, 2>(t, lds, it / ncb, it % ncb)) again |= uint64_t(1) << turn;
+                __syncthreads();  // the next tile reuses the staging buffers
+            }
+    }
     for (int it = first, turn = 0; it < n; it += step, ++turn) {
         const int tile = it / ncb, cb = it % ncb, rows = rows_of(it);
-        if (rows > split_rows && !((again >> turn) & 1)) continue;
+        if (SPLIT && rows > split_rows && !((again >> turn) & 1)) continue;
         if (rows > 48) tall_tile<MODE, 4>(t, lds, tile, cb);
         else if (rows > 32) tall_tile<MODE, 3>(t, lds, tile, cb);
         else if (rows > 16) tall_tile<MODE, 2>(t, lds, tile, cb);
@@ -604,10 +613,17 @@ static bool want_tall(int64_t d, int64_t rows, int64_t n_rel)
 }
 
 static int64_t tall_tiles(int64_t groups, int64_t rows) { return groups + rows / kTallRows + 1; }
+// Whether a launch may hold more than kSplitItems items: by the tiles that groups make on average, the last of each half full.  (A
+// kernel with the split tiles' code is slower even where none is split: RESCAL score calls of 6400 triples over 20 relations, width 64
+// 8.7 -> 12.0 us, width 200 16.2 -> 21.0.)
+static bool tall_may_split(int64_t d, int64_t rows, int64_t groups)
+{
+    return (rows / kTallRows + groups / 2) * tall_col_blocks((int)d) > kSplitItems;
+}
 static size_t tall_part_floats(int64_t d, int64_t B) { return tall_col_blocks((int)d) > 1 ? (size_t)tall_col_blocks((int)d) * (size_t)B : 0; }
 
 // max_tiles: upper bound of the plan's tiles (a.plan holds tiles of kTallRows).  part: tall_part_floats() where a.pos is set.
-static int launch_tall(int mode, const GemmArgs &a, int64_t max_tiles, float *part, int64_t B, const FusedInsp &fi, hipStream_t st)
+static int launch_tall(int mode, const GemmArgs &a, int64_t max_tiles, bool split, float *part, int64_t B, const FusedInsp &fi, hipStream_t st)
 {
     const int ncb = tall_col_blocks(a.d);
     if (a.pos && ncb > 1 && !part) return KGE_EWORKSPACE;
@@ -616,11 +632,12 @@ static int launch_tall(int mode, const GemmArgs &a, int64_t max_tiles, float *pa
     const int64_t wgs = items / 64 + 1 > kTallWgs ? items / 64 + 1 : kTallWgs;  // (at most 64 items each: transr_tall_kernel)
     const dim3 grid((unsigned)((items < wgs ? items : wgs) + fi.blocks)), block(256);
     const size_t lds = fi.blocks > 0 && (size_t)fi.lds_bytes > kTallLds ? (size_t)fi.lds_bytes : kTallLds;
+    auto launch = [&](auto plain_kernel, auto split_kernel) { hipLaunchKernelGGL(split ? split_kernel : plain_kernel, grid, block, lds, st, t, fi); };
     switch (mode) {
-    case 0: hipLaunchKernelGGL(transr_tall_kernel<0>, grid, block, lds, st, t, fi); break;
-    case 1: hipLaunchKernelGGL(transr_tall_kernel<1>, grid, block, lds, st, t, fi); break;
-    case 2: hipLaunchKernelGGL(transr_tall_kernel<2>, grid, block, lds, st, t, fi); break;
-    default: hipLaunchKernelGGL(transr_tall_kernel<3>, grid, block, lds, st, t, fi);
+    case 0: launch(transr_tall_kernel<0, false>, transr_tall_kernel<0, true>); break;
+    case 1: launch(transr_tall_kernel<1, false>, transr_tall_kernel<1, true>); break;
+    case 2: launch(transr_tall_kernel<2, false>, transr_tall_kernel<2, true>); break;
+    default: launch(transr_tall_kernel<3, false>, transr_tall_kernel<3, true>);
     }
     if (a.pos && ncb > 1)
         hipLaunchKernelGGL(tall_finish_kernel, dim3((unsigned)ceil_div(B, 256)), dim3(256), 0, st, part, ncb, B,

@@ -19,7 +19,7 @@ constexpr int kTallCols = 128;  // columns per workgroup at most: 32 per wave, t
 constexpr int kTallKC = 64;     // columns of the left operand staged at a time
 constexpr int kTallPitch = kTallKC + 4;
 constexpr int kTallRing = 4;    // supersteps (16 rows of k) of the projection in flight per wave, one of them in use
-constexpr int kSplitRows = 16;    // tiles of more rows go by the bf16 matrix cores ...
+constexpr int kSplitRows = 32;    // tiles of more rows go by the bf16 matrix cores ...
 constexpr int kSplitItems = 256;  // ... where a launch has more items than that
 constexpr int kTallWgs = 4096;  // workgroups of a launch at most; they stride over the tiles
 
@@ -335,9 +335,11 @@ __device__ __forceinline__ void tall_tile(const TallArgs &t, float *lds, int til
 // (a thread takes 4 x 4 elements: four rows of it are loaded, four columns written, 64 bytes of a row and 16 banks apart per two lanes).
 //   What bounds it: the matrix cores and the slices' barriers where groups are large, else the projections' bytes.  Whole calls, fp32 tiles
 //   -> these: RESCAL 8192 x 1024 over 51 relations (Zipf) 230 -> 184 us, 8192 x 512 over 11 82 -> 64; TransR 4096 x 512 over 60 64 -> 50,
-//   over 237 91 -> 88 (bytes); the row list and dX of TransR against shared negatives, 4096 x 200 over 1345, 126 + 145 -> 122 + 107 us.
+//   over 237 91 -> 86 (bytes); the row list and dX of TransR against shared negatives, 4096 x 200 over 1345, 126 + 145 -> 122 + 107 us.
 //   A launch of at most one item per CU runs every slice at its full latency and keeps the fp32 tiles' four supersteps in flight
-//   (4096 x 128 over 20: 25 against 27 us); tiles of at most 16 rows do half of the matrix work in fp32's 16-row blocks.
+//   (4096 x 128 over 20: 25 against 27 us).  Tiles of at most 32 rows do half of the work or less in fp32's 16-row blocks and keep more of the
+//   projection in flight: score calls of 17 to 30 rows a relation (4096 to 7000 triples over 237, widths 400 and 512) TransR 80 to 100 us
+//   split, 66 to 82 in fp32, RESCAL 82 to 97 and 67 to 79; split as one block of 32 rows 75 to 95.
 template <int MODE, int RB>
 __device__ __forceinline__ bool split_tile(const TallArgs &t, float *lds, int tile, int cb)
 {

@@ -1842,7 +1842,7 @@ static PlanSizes plan_sizes(const kge_tables *tab, const kge_batch *bat)
 {
     const int64_t B = bat->batch, groups = B < tab->n_rel ? B : tab->n_rel;
     return PlanSizes{max_tiles(tab, bat), groups + B / kDmChunk + 1, B / kDmChunk + 1 /* a split group has more than kDmChunk triples */,
-                     want_tall(tab->dim, B, tab->n_rel) ? tall_tiles(groups, B) : 0, tab->dim, tall_may_split(tab->dim, B, groups)};
+                     want_tall(tab->model, tab->dim, B, tab->n_rel) ? tall_tiles(groups, B) : 0, tab->dim, tall_may_split(tab->dim, B, groups)};
 }
 
 static size_t lds_with(const FusedInsp &fi, size_t own)

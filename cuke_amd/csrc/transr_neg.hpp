@@ -38,7 +38,7 @@ static NegShape neg_shape(const kge_tables *tab, const kge_batch *bat)
     s.G_cap = s.B < pairs ? s.B : pairs;
     s.L_cap = 2 * s.B + s.G_cap * s.N;
     s.plans = PlanSizes{0, s.U_cap + s.L_cap / kDmChunk + 1, s.L_cap / kDmChunk + 1, 0, s.d, tall_may_split(s.d, s.L_cap, s.U_cap)};
-    if (want_tall(s.d, s.L_cap, tab->n_rel)) s.plans.tall = tall_tiles(s.U_cap, s.L_cap);
+    if (want_tall(tab->model, s.d, s.L_cap, tab->n_rel)) s.plans.tall = tall_tiles(s.U_cap, s.L_cap);
     else s.plans.tiles = s.U_cap + s.L_cap / kTM + 1;
     s.dslots = 2 * (s.L_cap / kDmChunk) + 2;
     // dM by items of 128 x 128 where there can be one for each resident workgroup: below that the fp32 items, four to seven times as many,

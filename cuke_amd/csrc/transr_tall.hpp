@@ -590,6 +590,13 @@ __global__ __launch_bounds__(256) void tall_finish_kernel(const float *part, int
     pos[b] = root ? sqrtf(s) : s;
 }
 
+// Whether a launch may hold more than kSplitItems items: by the tiles that groups make on average, the last of each half full.  (A
+// kernel with the split tiles' code is slower even where none is split: RESCAL score calls of 6400 triples over 20 relations, width 64
+// 8.7 -> 12.0 us, width 200 16.2 -> 21.0.)
+static bool tall_may_split(int64_t d, int64_t rows, int64_t groups)
+{
+    return (rows / kTallRows + groups / 2) * tall_col_blocks((int)d) > kSplitItems;
+}
 
 // Whether a batch of `rows` rows in at most n_rel groups goes by these tiles rather than by 32-row tiles and streamed
 // small groups (transr_gemm_kernel).  The rule sees the counts, not the distribution.  Both sides measured over 64 to
@@ -600,28 +607,23 @@ __global__ __launch_bounds__(256) void tall_finish_kernel(const float *part, int
 //   up to 256           two column blocks stage every row twice: only where the 32-row tiles leave compute units idle.
 //                       Up to 200 tiles 1.00 (0.79 to 1.17) and 0.94; 201 to 256 tiles 1.17 (1.00 to 1.41) and 0.97;
 //                       above 1.17 (0.84 to 1.56) and 0.95.  Groups that fill their tiles' 64 rows on average (from 32 rows per
-//                       relation on) go by the bf16 matrix cores there: score calls 0.79 to 0.96 (8192 triples over 20 to 237
-//                       relations, width 132 / 200 / 256), TransR's row list of 90000 rows over 588 relations below; at 8 rows
-//                       per relation 0.95 to 1.14, at 2 1.1 to 1.3
+//                       relation on) go by the bf16 matrix cores there, if the launch has the items for it: score calls 0.73 to 0.98
+//                       (8192 triples over 3 to 237 relations, width 132 / 200 / 256), RESCAL's at width 132 1.00 to 1.09; TransR's row
+//                       list of 90000 rows over 588 relations below; at 8 rows per relation 0.95 to 1.14, at 2 1.1 to 1.3.  With
+//                       fewer items (4000 to 7400 triples over 3 to 100 relations, fp32 tiles) TransR 0.86 to 1.04, mean 0.96, from width
+//                       160 on and 1.00 below; RESCAL, whose scores of two column blocks take a kernel more, 0.92 to 1.12, mean 1.03
 //   above               a 32-row tile is one workgroup however wide its rows are: few groups leave the chip idle.
 //                       0.76 (0.24 to 1.33) and 0.78; where streaming is taken (many groups of a few rows, bound by
 //                       reading the projections) 0.95 (0.70 to 1.28) and 0.89
-static bool want_tall(int64_t d, int64_t rows, int64_t n_rel)
+static bool want_tall(int model, int64_t d, int64_t rows, int64_t n_rel)
 {
     const int64_t groups = rows < n_rel ? rows : n_rel, short_tiles = groups + rows / 32;
     if (d <= kTallCols) return short_tiles <= 256 || rows >= 4 * n_rel;
-    if (d <= 2 * kTallCols) return short_tiles <= 200 || rows >= 32 * n_rel;
+    if (d <= 2 * kTallCols) return short_tiles <= 200 || (rows >= 32 * n_rel && (tall_may_split(d, rows, groups) || (model == KGE_TRANSR && d >= 160)));
     return groups <= 256 || rows >= 16 * n_rel;
 }
 
 static int64_t tall_tiles(int64_t groups, int64_t rows) { return groups + rows / kTallRows + 1; }
-// Whether a launch may hold more than kSplitItems items: by the tiles that groups make on average, the last of each half full.  (A
-// kernel with the split tiles' code is slower even where none is split: RESCAL score calls of 6400 triples over 20 relations, width 64
-// 8.7 -> 12.0 us, width 200 16.2 -> 21.0.)
-static bool tall_may_split(int64_t d, int64_t rows, int64_t groups)
-{
-    return (rows / kTallRows + groups / 2) * tall_col_blocks((int)d) > kSplitItems;
-}
 static size_t tall_part_floats(int64_t d, int64_t B) { return tall_col_blocks((int)d) > 1 ? (size_t)tall_col_blocks((int)d) * (size_t)B : 0; }
 
 // max_tiles: upper bound of the plan's tiles (a.plan holds tiles of kTallRows).  part: tall_part_floats() where a.pos is set.

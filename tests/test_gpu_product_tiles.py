@@ -81,3 +81,27 @@ def test_the_timeline_names_the_form_that_ran(n_rel, dim, kw, form):
     names = [name for name, _ in st.kernel_times(2)]
     first = "list>" if kw else "fwd>"
     assert any(n.endswith(f"transr_{form}_kernel<{first}") for n in names) and f"transr_{form}_kernel<dX>" in names, names
+
+
+@pytest.mark.parametrize("dim,n_rel,batch,tiles", [
+    (200, 20, 5600, "tall"),    # at most 200 short tiles
+    (132, 20, 6400, "gemm"),    # more, and too few 64-row tiles for the bf16 matrix cores
+    (200, 100, 4500, "gemm"),
+    (200, 20, 8192, "tall"),    # 276 items of 64 rows x 128 columns on average
+    (256, 237, 7500, "gemm"),   # fewer than 32 rows a relation
+])
+def test_the_rule_between_the_tiles(dim, n_rel, batch, tiles):
+    from cuke_amd.kge import KGEModel, TrainStep
+    g = torch.Generator(device="cuda")
+    g.manual_seed(dim)
+    E, A = (torch.randn(*s, generator=g, device="cuda") * 0.05 for s in ((3000, dim), (n_rel, dim, dim)))
+    h, t = (torch.randint(0, 3000, (batch,), generator=g, device="cuda") for _ in range(2))
+    r = torch.arange(batch, device="cuda") % n_rel
+    st = TrainStep(KGEModel("RESCAL", E, None, A), h, r, t, dpos=torch.randn(batch, generator=g, device="cuda"))
+    names = [k for k, _ in st.kernel_times(steps=1)]
+    assert any(f"transr_{tiles}_kernel<fwd>" in k for k in names), names
+    want = torch.empty(batch, dtype=torch.float64, device="cuda")
+    for u in range(n_rel):
+        m = r == u
+        want[m] = ((E[h[m]].double() @ A[u].double()) * E[t[m]].double()).sum(1)
+    assert_close(st.pos.cpu().numpy(), want.cpu().numpy(), what="scores")

@@ -214,7 +214,7 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
     // run-time value it put a branch around every pair of the micro-tile.
     auto sweep = [&](auto pass_tag) {
         constexpr int pass = decltype(pass_tag)::value;
-        constexpr int kInnerUnroll = (MODEL == KGE_TRANSH || (MODEL == KGE_ROTATE && RB == 4)) ? 2 : kKD / 4;
+        constexpr int kInnerUnroll = MODEL == KGE_TRANSH ? 2 : kKD / 4;
         if (slice0 < slice1) load_slice(slice0 * kKD, pass);
 #pragma unroll 1
         for (int s = slice0; s < slice1; ++s) {
@@ -222,9 +222,8 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void score_neg_kernel(NegArgs a,
             __syncthreads();
             if (s + 1 < slice1) load_slice((s + 1) * kKD, pass);
             __builtin_amdgcn_sched_barrier(0);  // (the requests go out before the compute, not after it)
-            // (TransH keeps three sums per pair, RotatE two row planes: unrolled all the way, the hoisted LDS reads push the
-            // 4 x 4 micro-tile over the register budget and twenty to fifty registers per lane go through
-            // scratch memory every step)
+            // (TransH keeps three sums per pair: unrolled all the way, the hoisted LDS reads push the 4 x 4 micro-tile over the register
+            // budget and twenty to fifty registers per lane go through scratch memory every step)
 #pragma unroll kInnerUnroll
             for (int i4 = 0; i4 < kKD / 4; ++i4) {
                 float4 av[NPA][RB], tv[NPT][RK];
@@ -779,8 +778,10 @@ static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, c
     // inspector workgroups that share the machine with these launches raise their wave priority.
     constexpr bool kDotModel = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL;
     // Rows of fewer than four floats take the 32x32 tile whatever the size: only that tile is compiled in
-    // the scalar-load form.
-    const int tile = !a.vec ? 2 : big_tiles >= 1024 ? 4 : (kDotModel && !dot_valu ? 3 : 2);  // 2: 32x32, 3: 32x64, 4: 64x64
+    // the scalar-load form.  RotatE takes it too: its pairs are bound by the vector ALUs (a square root each), five waves per SIMD instead of
+    // three keep them busier, and its launches end more evenly (64 x 64 -> 32 x 32, us: 30000 x 200 negatives x 150 187 -> 153, x 400 409 ->
+    // 328; 739 x 6351 x 196 132 -> 119; 16384 x 1024 x 48 119 -> 121, x 1000 1569 -> 1488).
+    const int tile = !a.vec || MODEL == KGE_ROTATE ? 2 : big_tiles >= 1024 ? 4 : (kDotModel && !dot_valu ? 3 : 2);  // 2: 32x32, 3: 32x64, 4: 64x64
     const int TB = tile == 4 ? 64 : 32, TN = tile == 2 ? 32 : 64;
     // (workgroups that score the positives, if the launch carries them, follow the tiles')
     const unsigned tile_blocks = xcd_grid(ceil_div(a.N, TN), ceil_div(a.C, TB), n_chunks) * (unsigned)(a.ksplit > 1 ? a.ksplit : 1);
@@ -808,12 +809,11 @@ static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, c
         }
         return KGE_EINVAL;
     }
-    if (tile == 3) {  // 32 positives x 64 negatives
-        if (save) NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 2, 4, true);
-        else NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 2, 4, false);
-    } else if (tile == 4) {
-        if (save) NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, true);
-        else NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, false);
+    if (tile == 4) {
+        if constexpr (MODEL != KGE_ROTATE) {
+            if (save) NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, true);
+            else NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, false);
+        }
     } else {
         if (save) NEG_LAUNCH(score_neg_kernel, MODEL, P, 2, 2, true);
         else NEG_LAUNCH(score_neg_kernel, MODEL, P, 2, 2, false);

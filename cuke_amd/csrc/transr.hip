@@ -1482,6 +1482,8 @@ __device__ __forceinline__ void transr_dm_item(const DmArgs &a, float *lds, int 
 // positions; wave w stages the 32 columns w of both and forms the blocks (w % 2 + {0, 2}) x (w / 2 + {0, 2}) of 32 x 32, so tiles of
 // fewer blocks spread over the waves.  A position past the end repeats the last one against an x that is zero, a column past the end
 // repeats the last quad and is stored nowhere.  An item with sums that are not finite is formed again in fp32.
+//   2-norm of the error against 64 bits (1024 triples, half of them of one relation, 64 negatives), fp32 items -> these: width 128 2.8e-7 ->
+//   1.05e-7, width 60 2.0e-7 -> 7.2e-8, width 200 2.8e-7 -> 1.07e-7.
 constexpr int kDmTile = 128;
 __host__ __device__ inline int dm_split_tiles(int d) { return (d + kDmTile - 1) / kDmTile; }
 struct DmSplitRows {  // the chunk's entity rows, x = h - t

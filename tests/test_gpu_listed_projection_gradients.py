@@ -46,3 +46,47 @@ def test_listed_projection_gradients_beyond_bf16(oracle):
     assert np.isfinite(want).all() and np.isfinite(got).all() and np.abs(want[:, 7]).max() > 1e30
     rows = np.abs(want[:, 7]).max(1) > 1e30  # the relations that meet the value
     assert_close(got[rows, 7], want[rows, 7], what="the column with the value", rows=True)
+
+
+@pytest.mark.parametrize("dim,batch,n_rel,chunk,n_neg", [(128, 1024, 1100, 128, 64), (60, 1024, 1100, 512, 48), (200, 512, 300, 64, 64)])
+def test_listed_projection_gradients_against_64_bits(dim, batch, n_rel, chunk, n_neg):
+    """L1, upstream gradients that are multiples of 2^-12: every upstream row is an exact sum of signs, so what differs from 64 bits
+    is the product of the rows alone.  Half of the triples share a relation (items of 256 positions and their partial sums)."""
+    from cuke_amd.kge import KGEModel
+    g = torch.Generator(device="cuda")
+    g.manual_seed(dim)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda") * 0.05
+    E, R, A = rand(3000, dim), rand(n_rel, dim), rand(n_rel, dim, dim)
+    ids = lambda n, k: torch.randint(0, n, (k,), generator=g, device="cuda")
+    h, t, neg, r = ids(3000, batch), ids(3000, batch), ids(3000, batch // chunk * n_neg), ids(n_rel, batch)
+    r[torch.rand(batch, generator=g, device="cuda") < 0.5] = 0
+    dpos, dneg = (ids(2048, k).float().add_(1).div_(4096) for k in (batch, batch * n_neg))
+    dneg = dneg.view(batch, n_neg)
+    m = KGEModel("TransR", E, R, A, norm_p=1)
+    fw = m.score(h, r, t, neg, chunk)
+    grads = m.backward(fw, dpos, dneg)
+    rows = {int(u): i for i, u in enumerate(grads.rel_ids.tolist())}
+    D = lambda x: x.double()
+    for u in [0] + r.unique()[1:8].tolist():
+        M, want, size, n = D(A[u]), torch.zeros(dim, dim, dtype=torch.float64, device="cuda"), 0.0, 0
+        sure = torch.ones(dim, dtype=torch.bool, device="cuda")  # columns in which no residual is within rounding of zero
+        for c in range(batch // chunk):
+            b = torch.arange(c * chunk, (c + 1) * chunk, device="cuda")
+            b = b[r[b] == u]
+            if b.numel() == 0:
+                continue
+            hx, tx, nx = D(E[h[b]]), D(E[t[b]]), D(E[neg.view(-1, n_neg)[c]])
+            yp = (hx - tx) @ M + D(R[u])
+            a = hx @ M + D(R[u])
+            pair = a[:, None, :] - (nx @ M)[None]
+            sure &= (pair.abs().amin((0, 1)) > 1e-6) & (yp.abs().amin(0) > 1e-6)
+            cs = D(dneg[b])[:, :, None] * pair.sign()
+            for x, q in (((D(E[h[b]] - E[t[b]])), D(dpos[b])[:, None] * yp.sign()), (hx, cs.sum(1)), (nx, -cs.sum(0))):
+                want += x.t().contiguous() @ q
+                size = size + x.abs().t().contiguous() @ q.abs()
+                n += x.shape[0]
+        got = D(grads.aux_rows.view(-1, dim, dim)[rows[u]])
+        err = ((got - want).abs() / size)[:, sure] * 2 ** 24
+        assert sure.float().mean() > 0.5
+        # each product and each addition rounds once: sqrt(n) half ulps of the terms' total, at most
+        assert float(err.max()) <= 4 + n ** 0.5, (u, n, float(err.max()))

@@ -693,14 +693,19 @@ static size_t tile_lds_bytes(const FusedInsp &fi)
 }
 
 // the form of the kernel that the widths allow
-#define LAUNCH_TILE(RO_, MF_, GRID, ...)                                                                                         \
+#define LAUNCH_TILE_VEC(RO_, MF_, GRID, ...)                                                                                     \
     do {                                                                                                                         \
-        if (a.vec && a.vecn)                                                                                                     \
+        if (a.vecn)                                                                                                              \
             hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, true, true>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi);   \
-        else if (a.vec)                                                                                                          \
-            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, true, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi);  \
         else                                                                                                                     \
-            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, false, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi); \
+            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, true, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi);  \
+    } while (0)
+#define LAUNCH_TILE(RO_, GRID, ...)                                                                                              \
+    do {                                                                                                                         \
+        if (a.vec)                                                                                                               \
+            LAUNCH_TILE_VEC(RO_, false, GRID, __VA_ARGS__);                                                                      \
+        else                                                                                                                     \
+            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, false, false, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi); \
     } while (0)
 
 template <int MODEL, int P>
@@ -724,13 +729,13 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
         //   (2000 x 100 x 100 x 130)   6144 26 / 32 (1536 x 256 x 256 x 256)   7168 42 / 48 (1024 x 512 x 512 x 400)   12000 22 / 26 (4000 x 100 x
         //   100 x 130)   28672 192 / 217 (4096 x 1024 x 1024 x 400); from 1024 tiles on 112 / 165 (4096 x 1024 x 50 x 1000), 40 / 41 (16384 x 16 x 16 x 100).
         const bool fill = kDotModel || big >= 1024 || gx * n_chunks * (a.C < a.N ? a.C : a.N) >= 6144;
-        if (!dot_valu && fill) {
+        if (!dot_valu && fill && a.vec) {  // (rows of fewer than four floats: vector ALUs)
             // (ComplEx by quads: column tiles pair 32 real with the matching 32 imaginary columns)
-            const int64_t gxm = (MODEL == KGE_COMPLEX && a.vec) ? ceil_div(a.d / 2, 32) : gx;
+            const int64_t gxm = MODEL == KGE_COMPLEX ? ceil_div(a.d / 2, 32) : gx;
             const unsigned gh = xcd_grid(gxm, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxm, ceil_div(a.N, 64), n_chunks);
             const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
             const TileGrid tg{(int)gh, (int)gn, 0, 0};
-            LAUNCH_TILE(4, true, dim3(gh + gn + fi.blocks), tg);
+            LAUNCH_TILE_VEC(4, true, dim3(gh + gn + fi.blocks), tg);
             KGE_CHECK_LAUNCH();
             return KGE_OK;
         }
@@ -741,19 +746,19 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
         const unsigned nn = narrow ? xcd_grid(1, ceil_div(a.N, 64), n_chunks) : 0;
         const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
         const TileGrid tg{(int)gh, (int)gn, (int)nh, (int)nn};
-        LAUNCH_TILE(4, false, dim3(gh + gn + nh + nn + fi.blocks), tg);
+        LAUNCH_TILE(4, dim3(gh + gn + nh + nn + fi.blocks), tg);
     } else if (big >= 512) {
         const unsigned gh = xcd_grid(gx, ceil_div(a.C, 32), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 32), n_chunks);
         const size_t lds = tile_lds_bytes<MODEL, 2>(fi);
         const TileGrid tg{(int)gh, (int)gn, 0, 0};
-        LAUNCH_TILE(2, false, dim3(gh + gn + fi.blocks), tg);
+        LAUNCH_TILE(2, dim3(gh + gn + fi.blocks), tg);
     } else {
         // a batch this small leaves one or two 32-owner workgroups per CU: 16-owner tiles double the
         // waves that hide each other's latency
         const unsigned gh = xcd_grid(gx, ceil_div(a.C, 16), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 16), n_chunks);
         const size_t lds = tile_lds_bytes<MODEL, 1>(fi);
         const TileGrid tg{(int)gh, (int)gn, 0, 0};
-        LAUNCH_TILE(1, false, dim3(gh + gn + fi.blocks), tg);
+        LAUNCH_TILE(1, dim3(gh + gn + fi.blocks), tg);
     }
     KGE_CHECK_LAUNCH();
     return KGE_OK;

@@ -806,7 +806,6 @@ static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, c
         }
     }
     const size_t lds = neg_lds(NPA, TB, TN, NPT, fi);
-    const bool save = MODEL == KGE_TRANSH && a.side_neg;
     if (a.ksplit > 1) {  // (neg_ksplit: 32 x 32 tiles of TransE / RotatE)
         if constexpr (MODEL == KGE_TRANSE || MODEL == KGE_ROTATE) {
             NEG_LAUNCH(score_neg_kernel, MODEL, P, 2, 2, false);
@@ -817,14 +816,16 @@ static int launch_neg_mp(const NegArgs &a_in, int64_t n_chunks, bool dot_valu, c
         }
         return KGE_EINVAL;
     }
-    if (tile == 4) {
-        if constexpr (MODEL != KGE_ROTATE) {
-            if (save) NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, true);
-            else NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, false);
-        }
+    auto launch = [&](auto save) {  // (TransH alone has something to save)
+        constexpr bool SAVE = decltype(save)::value;
+        if (tile == 2) NEG_LAUNCH(score_neg_kernel, MODEL, P, 2, 2, SAVE);
+        else if constexpr (MODEL != KGE_ROTATE) NEG_LAUNCH_VEC(score_neg_kernel, MODEL, P, 4, 4, SAVE);
+    };
+    if constexpr (MODEL == KGE_TRANSH) {
+        if (a.side_neg) launch(std::true_type{});
+        else launch(std::false_type{});
     } else {
-        if (save) NEG_LAUNCH(score_neg_kernel, MODEL, P, 2, 2, true);
-        else NEG_LAUNCH(score_neg_kernel, MODEL, P, 2, 2, false);
+        launch(std::false_type{});
     }
     KGE_CHECK_LAUNCH();
     return KGE_OK;

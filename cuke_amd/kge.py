@@ -258,8 +258,9 @@ class KGEModel:
     Remb   [n_rel, dim] float32 (RotatE: [n_rel, dim/2] phases; RESCAL: None)
     aux    TransH: hyperplane normals [n_rel, dim] (the reference's Pemb);
            TransR / RESCAL: projections [n_rel, dim, dim] (the reference's Proj)
-    pair_sums  "matrix_cores" (default) or "vector_alus": where the shared-negative tile kernels of
-           DistMult / ComplEx sum their pair products (``pair_sums`` can be reassigned between calls)
+    pair_sums  "matrix_cores" (default) or "vector_alus": where the shared-negative tile kernels of the
+           dot-product models and of TransE's L2 gradients sum their pair products (``pair_sums`` can be reassigned
+           between calls; the projections of TransR / RESCAL run on the matrix cores either way)
     """
 
     def __init__(self, model: str, Eemb, Remb=None, aux=None, norm_p: int = 2, gamma: float = 0.0,

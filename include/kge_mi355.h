@@ -67,10 +67,13 @@ typedef struct kge_tables {
                           projections [n_rel, dim, dim] (Proj); else NULL */
 } kge_tables;
 
-/* kge_tables.flags.  The shared-negative tile kernels of DistMult / ComplEx sum their pair
-   products on the matrix cores (fp32 MFMA, fp32 accumulate) unless this bit asks for the vector
-   ALUs; both forms meet the same tolerance.  The choice travels with the call, so concurrent
-   callers cannot disturb each other.  No counterpart in the reference. */
+/* kge_tables.flags.  The shared-negative tile kernels sum pair products on the matrix cores unless this
+   bit asks for the vector ALUs: the scores and gradients of the dot-product pairs (DistMult, ComplEx, TransF, RESCAL)
+   by fp32 instructions, scores of large batches as three-part bf16 products with fp32 sums (no larger an error against 64
+   bits), and TransE's L2 gradients in 64 bits where the batch is large enough for it.  Both forms meet the same tolerance.  The
+   bit does not reach the projections of TransR and RESCAL: their grouped products and the projection gradients against shared
+   negatives run on the matrix cores, in fp32 or as three-part bf16 products, whatever it says.  The choice travels with the
+   call, so concurrent callers cannot disturb each other.  No counterpart in the reference. */
 enum { KGE_PAIR_SUMS_VALU = 1 };
 
 /*
@@ -281,8 +284,8 @@ int kge_residual_fwd(const kge_tables *tab, const kge_batch *bat, float *out, vo
  * every tile is split over up to four workgroups (partial score planes in the workspace, a finishing
  * kernel); without the workspace the same call runs one workgroup per tile.  DistMult / ComplEx / TransF with large batches
  * (hundreds of 128 x 128 tiles) put their query rows there and score on the bf16 matrix cores; without it, on the fp32 ones.
- * TransE, and DistMult / ComplEx on the matrix-core tiles: when pos and neg are both requested, no
- * side output is and no inspection rides along, the positives are scored by extra workgroups of the
+ * TransE, and DistMult / ComplEx on the fp32 matrix-core tiles (not the bf16 ones of the batches above): when pos and neg are
+ * both requested, no side output is and no inspection rides along, the positives are scored by extra workgroups of the
  * shared-negative launch (one launch instead of two; a timeline then has no "score_pos_kernel"
  * entry and its "score_neg_kernel" entry includes the positives).  Results are the same bits.
  * RotatE: `residual` [B, dim] receives the rotated heads h e^{i theta}; the shared-negative

@@ -291,13 +291,15 @@ __global__ __launch_bounds__(kMidThreads) void inspect_mid_dedup_kernel(MidJobs 
 // Up to kSmallN ids are sorted, deduplicated and finished by one workgroup of sixteen waves, keys in registers and LDS: the sets of an
 // eager training loop or of a projection model's call.  Bound by its own chain: a round of 64 keys per wave is ranked with db ballots, and
 // every digit pass has four barriers.  Digits of at most seven bits keep the counters of all waves in 8 KB.
-//   Against the mid path's launches (histogram, digit passes, dedup, each a trip to memory and back), us:
-//     table rows        1024 ids       2048          3072          4096          8192
-//           50        9.9 ->  5.4   10.0 ->  6.8  10.2 ->  9.5  10.3 -> 10.9  11.0 -> 22
-//          237       10.4 ->  6.5   10.8 ->  8.4  11.3 -> 11.7  11.0 -> 13.4  11.8 -> 26
-//         1345       16.2 ->  7.0   17.1 ->  9.1  17.4 -> 13.0  17.5 -> 15.0  18.1 -> 29
-//        14951       18.6 ->  7.5   21.5 ->  9.9  22.6 -> 14.2  22.7 -> 16.4  24.2 -> 33
-//          1e6       22.4 ->  9.4   25.5 -> 12.5  26.3 -> 18.1  26.7 -> 20.8  28.0 -> 43
+//   Against the mid path's launches (histogram, digit passes, dedup, each a trip to memory and back), random ids, us:
+//     table rows         500 ids       1024          2048          3000          4096
+//           50        9.3 ->  6.3   10.2 ->  6.2  11.2 ->  6.8
+//          237       10.1 ->  6.3   10.8 ->  6.6  11.4 ->  8.2
+//         1345       15.9 ->  6.5   16.4 ->  6.8  17.5 ->  8.8  17.4 -> 12.2  17.7 -> 13.7
+//        14951       17.6 ->  7.0   18.8 ->  7.2  21.9 ->  9.2  22.8 -> 13.1  23.0 -> 14.7
+//          1e6       21.3 ->  8.2   22.5 ->  8.6  25.6 -> 11.4  26.3 -> 16.5  26.6 -> 18.7
+//   (8192 ids took 1.5 to 2 times the launches' time, 4096 ids of 50 or 237 rows 1.1 to 1.2 times.)  Ids that follow each other, 4096 of 1345
+//   rows: 19.5 us before the counters and places were skewed, by launches 16.9, now 13.4.
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / kWave;
 constexpr int kSmallDigitBits = 7;
 constexpr int64_t kSmallN = 4096;  // four keys per thread; half of it where one digit pass of few bins competes
@@ -307,9 +309,13 @@ template <int R>
 __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jobs)
 {
     constexpr int kPer = (kSmallWaves << kSmallDigitBits) / kSmallThreads;  // counters a thread scans, at most
-    __shared__ uint32_t s_key[kSmallThreads * R];
-    __shared__ uint16_t s_val[kSmallThreads * R];
-    __shared__ uint32_t s_cnt[kSmallWaves << kSmallDigitBits];  // [digit][wave]: the order that a stable sort takes them in
+    // (places are skewed: ids that follow each other scatter a power of two apart, sixteen lanes to a bank without it)
+    auto key_at = [](int i) { return i + (i >> 6); };
+    auto cnt_at = [](int q) { return q + (q >> 4); };
+    __shared__ uint32_t s_key[kSmallThreads * R + (kSmallThreads * R >> 6)];
+    __shared__ uint16_t s_val[kSmallThreads * R + (kSmallThreads * R >> 6)];
+    // [digit][wave]: the order that a stable sort takes them in
+    __shared__ uint32_t s_cnt[(kSmallWaves << kSmallDigitBits) + (kSmallWaves << kSmallDigitBits >> 4)];
     __shared__ uint32_t s_tot[kSmallWaves];
     __builtin_amdgcn_s_setprio(3);  // see mid_scatter_body
     const MidJob &J = jobs.j[blockIdx.x];
@@ -354,7 +360,7 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
     const uint64_t lt_mask = lane ? (~0ull >> (kWave - lane)) : 0ull;
     for (int pass = 0; pass < J.npass; ++pass) {
         const int shift = pass * db;
-        for (int i = tid; i < counters; i += kSmallThreads) s_cnt[i] = 0;
+        for (int i = tid; i < cnt_at(counters); i += kSmallThreads) s_cnt[i] = 0;
         __syncthreads();
         uint32_t rank[R];
 #pragma unroll
@@ -370,8 +376,9 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
             const int leader = __ffsll((unsigned long long)peers) - 1;
             uint32_t old = 0;
             if (ok && lane == leader) {
-                old = s_cnt[dg * kSmallWaves + wave];
-                s_cnt[dg * kSmallWaves + wave] = old + __popcll(peers);
+                uint32_t &count = s_cnt[cnt_at(dg * kSmallWaves + wave)];
+                old = count;
+                count = old + __popcll(peers);
             }
             old = __shfl(old, leader < 0 ? 0 : leader, kWave);
             rank[j] = old + __popcll(peers & lt_mask);
@@ -382,21 +389,21 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int q = tid * per + i;
-            c[i] = i < per && q < counters ? s_cnt[q] : 0;
+            c[i] = i < per && q < counters ? s_cnt[cnt_at(q)] : 0;
             sum += c[i];
         }
         uint32_t run = scan(sum, total);
 #pragma unroll
         for (int i = 0; i < kPer; ++i) {
             const int q = tid * per + i;
-            if (i < per && q < counters) s_cnt[q] = run;
+            if (i < per && q < counters) s_cnt[cnt_at(q)] = run;
             run += c[i];
         }
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < R; ++j)
             if (at[j] < n) {
-                const uint32_t to = s_cnt[((key[j] >> shift) & mask) * kSmallWaves + wave] + rank[j];
+                const int to = key_at(s_cnt[cnt_at(((key[j] >> shift) & mask) * kSmallWaves + wave)] + rank[j]);
                 s_key[to] = key[j], s_val[to] = (uint16_t)val[j];
             }
         __syncthreads();
@@ -404,19 +411,19 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
 #pragma unroll
             for (int j = 0; j < R; ++j) {
                 const int i = at[j] < n ? at[j] : n - 1;
-                key[j] = s_key[i], val[j] = s_val[i];
+                key[j] = s_key[key_at(i)], val[j] = s_val[key_at(i)];
             }
         }
     }
 
     // runs of equal keys: a thread takes R consecutive sorted positions
     const int lo = tid * R;
-    uint32_t prev = lo > 0 && lo < n ? s_key[lo - 1] : 0, heads = 0;
+    uint32_t prev = lo > 0 && lo < n ? s_key[key_at(lo - 1)] : 0, heads = 0;
     bool head[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         const int i = lo + j;
-        key[j] = i < n ? s_key[i] : 0;
+        key[j] = i < n ? s_key[key_at(i)] : 0;
         head[j] = i < n && (i == 0 || key[j] != prev);
         prev = key[j];
         heads += head[j] ? 1 : 0;
@@ -433,7 +440,7 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
                 J.out.seg_offsets[run] = i;
                 ++run;
             }
-            const int32_t seg = (int32_t)run - 1, p = s_val[i];
+            const int32_t seg = (int32_t)run - 1, p = s_val[key_at(i)];
             J.out.perm[i] = p;
             J.out.sorted_seg[i] = seg;
             J.out.inverse[p] = seg;

@@ -64,3 +64,12 @@ def test_inspect_in_one_workgroup_and_past_it(oracle, n, n_rows):
     check(oracle, [ids], n_rows)
     check(oracle, [ids[:n // 3], np.minimum(ids[n // 3:], n_rows // 5)], n_rows)
     check(oracle, [np.full(n, n_rows - 1, np.int64)], n_rows)
+
+
+@pytest.mark.parametrize("n,n_rows", [(1024, 1 << 20), (2048, 40), (2047, 1345), (4096, 1345), (4095, 14951)])
+def test_inspect_ids_that_follow_each_other(oracle, n, n_rows):
+    """(the one-workgroup kernel scatters them a power of two apart)"""
+    ids = np.arange(n, dtype=np.int64)
+    check(oracle, [ids % n_rows], n_rows)
+    check(oracle, [(n_rows - 1 - ids % n_rows)], n_rows)
+    check(oracle, [(ids * 64) % n_rows, (ids * 2048) % n_rows], n_rows)

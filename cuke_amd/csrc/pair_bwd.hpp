@@ -1,0 +1,351 @@
+// Gradient tiles that evaluate every pair once (TransE, RotatE): included by score_bwd.hip.
+//
+// A workgroup owns TO negatives x 32 columns of one chunk and walks the chunk's positives (a range of them, `splits` workgroups
+// share them), staged kKL at a time with their coefficients.  A thread holds four columns of RO negatives; per positive it adds
+// the pair's gradient element to the negative's sum (registers) AND to the positive's, which the eight lane groups of a wave add up by
+// lane exchanges and the waves through LDS.  bwd_tile_kernel's two orientations form the same element twice, and with it
+// what the element costs: a sign or a reciprocal square root.
+// The positives' sums are complete over the TO negatives of the workgroup only: one plane of [B, d] rows per tile of negatives,
+// added up by bwd_pos_kernel; the negatives' rows likewise have one plane per range of positives, added up as the
+// segmented reduction loads them.
+#pragma once
+
+#include "inspector_mid.hpp"
+#include "tile_common.hpp"
+
+namespace kge {
+
+constexpr int kPairCols = 32;   // columns of the row per workgroup
+constexpr int kPairKL = 16;     // positives staged per step
+constexpr int kPairPitch = kPairCols + 4;
+constexpr int kPairRO = 4, kPairWaves = 4;
+constexpr int kPairOwners = kPairWaves * 8 * kPairRO;  // negatives of a workgroup whose waves all hold different ones
+
+template <int MODEL>
+struct PairShape {
+    static constexpr int NPL = MODEL == KGE_ROTATE ? 2 : 1;  // planes of a row and of its sums
+    static constexpr int PG = kPairOwners + 4;
+    static constexpr int kRowFloats = NPL * kPairKL * kPairPitch, kCoefFloats = kPairKL * PG;
+    static constexpr int kLdsFloats = kRowFloats + kCoefFloats + kPairKL * kPairWaves * NPL * kPairCols;
+};
+
+struct PairPlan {
+    int phases;   // 1, 2 or 4: waves of a workgroup that share its negatives and take turns at the positives
+    int tiles;    // tiles of negatives: planes of the positives' sums
+    int splits;   // ranges of positives: planes of the negatives' rows
+    int per;      // positives of a range, a multiple of the step
+};
+
+struct PairArgs {
+    PairPlan plan;
+    float *g0;                 // [tiles][B, d]
+    int64_t gplane;            // B * d
+    float *occ_neg, *more_neg; // plane 0 of the negatives' rows [n_chunks * N, d]; planes 1 ... splits - 1
+    int64_t nplane;            // n_chunks * N * d
+};
+
+__device__ __forceinline__ void swap_halves(float &a, float &b)  // upper 32 lanes of a <-> lower 32 lanes of b
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_rows(float &a, float &b)  // odd rows of 16 lanes of a <-> even rows of b
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float add_ror8(float v)  // v + the value eight lanes on within the row of 16
+{
+    return v + __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x128, 0xf, 0xf, true));
+}
+
+// Bound by vector-ALU issue (per wave instruction 2 clocks for subtractions and multiply-adds, 4 for the sign's v_med3, 8 for
+// v_rsq): a RotatE element 26 clocks where two orientations took 52, a TransE L1 element 10 for 16, and two to four for the exchanges.
+//   Gradient tiles, us, both orientations -> every pair once:  RotatE 1024 x 256 negatives x 1000 72 -> 55, 8192 x 256 x 500 in chunks of 1024
+//   295 -> 184, 4278 x 300 x 426 in chunks of 31 245 -> 128;  TransE L1 30000 x 200 x 150 230 -> 158, 4096 x 1024 x 150 136 -> 87.
+template <int MODEL, int P, int PH>
+__global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) void bwd_pair_kernel(TileArgs a, PairArgs pa, FusedInsp fi)
+{
+    using S = PairShape<MODEL>;
+    constexpr bool kRot = MODEL == KGE_ROTATE, kSc = !kRot && P == 1, kL2 = !kRot && P == 2;
+    constexpr int RO = kPairRO, WAVES = kPairWaves, NPL = S::NPL, PG = S::PG, KL = kPairKL, TH = WAVES * kWave;
+    constexpr int wo = WAVES / PH, TO = wo * 8 * RO;   // waves of different negatives; negatives of the tile
+    constexpr int CPT = (KL * TO / 4 + TH - 1) / TH;   // coefficient quads per thread
+    constexpr int NRAW = 2;
+    extern __shared__ __align__(16) char dyn_smem[];
+    if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
+    float(*sL)[KL][kPairPitch] = reinterpret_cast<float(*)[KL][kPairPitch]>(dyn_smem);
+    float(*sG)[PG] = reinterpret_cast<float(*)[PG]>(dyn_smem + sizeof(float) * S::kRowFloats);
+    float *sR = reinterpret_cast<float *>(dyn_smem) + S::kRowFloats + S::kCoefFloats;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), own_wave = wave % wo, phase = wave / wo;
+    const int tx = lane & 7, ty = own_wave * 8 + (lane >> 3);
+    const int d = a.d, half = d >> 1, klen = pair_len<MODEL>(d);
+    int c, tile_y, tile_x;
+    if (!xcd_tile((int)blockIdx.x - fi.blocks, (klen + kPairCols - 1) / kPairCols, pa.plan.tiles * pa.plan.splits, a.n_chunks, c, tile_y, tile_x)) return;
+    const int tile = tile_y / pa.plan.splits, split = tile_y - tile * pa.plan.splits;
+    const int k0 = tile * TO;                                             // first negative
+    const int b0 = split * pa.plan.per, b1 = min(a.C, b0 + pa.plan.per);  // positives of the chunk
+    // (a quad of columns that would run past the row's end is moved back to end with it: see bwd_tile_body)
+    const int lcol = tile_x * kPairCols + tx * 4, col = min(lcol, klen - 4), skip = lcol - col;
+
+    // ---- negatives: registers ------------------------------------------------------------
+    float4 own[NPL][RO], acc[NPL][RO];
+#pragma unroll
+    for (int o = 0; o < RO; ++o) {
+        const float *pt = a.ent + a.neg[(int64_t)c * a.N + min(k0 + ty * RO + o, a.N - 1)] * (int64_t)d;
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) {
+            own[q][o] = load_quad(pt + q * half + col);
+            acc[q][o] = zero4();
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < RO; ++o)
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) {
+            if (k0 + ty * RO + o >= a.N) own[q][o] = zero4();
+            if constexpr (kSc) own[q][o] = scale4(own[q][o], kSgnScale);
+        }
+
+    // ---- staging: rows by the first 8 KL threads, coefficients by all; requested a step ahead, ids two ------------
+    const int srow = tid >> 3;
+    const bool stager = tid < KL * 8;
+    int64_t ih = 0, ir = 0;
+    float4 rraw[NRAW], craw[CPT], sraw[kL2 ? CPT : 1];
+    auto load_idx = [&](int l0) {
+        if (kRot || !stager) return;
+        const int64_t b = (int64_t)c * a.C + min(l0 + srow, a.C - 1);
+        ih = a.h[b], ir = a.r[b];
+    };
+    auto load_step = [&](auto stag, int l0) {
+        constexpr int kEdge = decltype(stag)::value;  // 1: a quad of coefficients may straddle its row's end (see bwd_tile_body); 2: rows of fewer than four
+        if (stager) {
+            const float *pq = kRot ? a.query + ((int64_t)c * a.C + min(l0 + srow, a.C - 1)) * d : nullptr;
+            load_query_raw<MODEL, true>(a.ent + ih * (int64_t)d, a.rel + ir * (int64_t)a.rel_dim, nullptr, pq, col, klen, half, rraw);
+        }
+        auto ld = [](const float *p, int kl, int lim) {
+            if constexpr (kEdge == 1) return shift_quad(ld4_raw<true>(p, kl, lim), kl + 4 - lim);
+            else return ld4_whole<kEdge == 0>(p, kl, lim);
+        };
+#pragma unroll
+        for (int s = 0; s < CPT; ++s) {
+            const int f = tid + TH * s, lrow = f / (TO / 4), kl = k0 + (f % (TO / 4)) * 4, bl = l0 + lrow;
+            const bool inside = lrow < KL && bl < b1;
+            const int64_t off = ((int64_t)c * a.C + (inside ? bl : 0)) * a.N;
+            craw[s] = ld(a.dneg + off, kl, inside ? a.N : 0);
+            if constexpr (kL2) sraw[s] = ld(a.sneg + off, kl, inside ? a.N : 0);
+        }
+    };
+    auto load_rows = [&](int l0) {
+        if (a.N < 4) return load_step(std::integral_constant<int, 2>{}, l0);  // uniform
+        if ((a.N & 3) && k0 + TO > a.N) return load_step(std::integral_constant<int, 1>{}, l0);
+        load_step(std::integral_constant<int, 0>{}, l0);
+    };
+    auto store_step = [&](int l0) {
+        if (stager) {
+            float4 q0, q1;
+            combine_query<MODEL, true>(rraw, 0.0f, col, l0 + srow < b1 ? klen : 0, half, a.rsign, q0, q1);
+            *reinterpret_cast<float4 *>(&sL[0][srow][tx * 4]) = kSc ? scale4(q0, kSgnScale) : q0;
+            if constexpr (NPL == 2) *reinterpret_cast<float4 *>(&sL[1][srow][tx * 4]) = q1;
+        }
+#pragma unroll
+        for (int s = 0; s < CPT; ++s) {
+            const int f = tid + TH * s, lrow = f / (TO / 4);
+            if (lrow >= KL) continue;
+            float4 g = craw[s];
+            if constexpr (kL2) {
+                const float4 sc = sraw[s];
+                g.x = sc.x > 0.0f ? g.x / sc.x : 0.0f;
+                g.y = sc.y > 0.0f ? g.y / sc.y : 0.0f;
+                g.z = sc.z > 0.0f ? g.z / sc.z : 0.0f;
+                g.w = sc.w > 0.0f ? g.w / sc.w : 0.0f;
+            }
+            *reinterpret_cast<float4 *>(&sG[lrow][(f % (TO / 4)) * 4]) = g;
+        }
+    };
+
+    load_idx(b0);
+    load_rows(b0);
+    load_idx(b0 + KL);
+#pragma unroll 1
+    for (int l0 = b0; l0 < b1; l0 += KL) {
+        store_step(l0);
+        __syncthreads();
+        if (l0 + KL < b1) {
+            load_rows(l0 + KL);
+            load_idx(l0 + 2 * KL);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        float4 sacc[NPL][RO];  // (a step's sums of their own: rounding grows with the steps, not the positives)
+#pragma unroll
+        for (int q = 0; q < NPL; ++q)
+#pragma unroll
+            for (int o = 0; o < RO; ++o) sacc[q][o] = zero4();
+        // (unrolled, the exchanges' registers and the next positive's operands spill)
+#pragma unroll 1
+        for (int l = phase; l < KL; l += PH) {
+            float lv[NPL][4], sum[NPL][4];
+#pragma unroll
+            for (int q = 0; q < NPL; ++q) {
+                const float4 v = *reinterpret_cast<const float4 *>(&sL[q][l][tx * 4]);
+                lv[q][0] = v.x, lv[q][1] = v.y, lv[q][2] = v.z, lv[q][3] = v.w;
+                sum[q][0] = sum[q][1] = sum[q][2] = sum[q][3] = 0.0f;
+            }
+            const float4 cf = *reinterpret_cast<const float4 *>(&sG[l][ty * RO]);
+#pragma unroll
+            for (int o = 0; o < RO; ++o) {
+                const float g = reinterpret_cast<const float *>(&cf)[o];
+                const float *t0 = reinterpret_cast<const float *>(&own[0][o]), *t1 = reinterpret_cast<const float *>(&own[NPL - 1][o]);
+                float *n0 = reinterpret_cast<float *>(&sacc[0][o]), *n1 = reinterpret_cast<float *>(&sacc[NPL - 1][o]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (kRot) {
+                        const float ur = lv[0][e] - t0[e], ui = lv[1][e] - t1[e];
+                        // (the 1e-37: see bwd_tile_body)
+                        const float k = g * __builtin_amdgcn_rsqf(fmaf(ur, ur, fmaf(ui, ui, 1e-37f)));
+                        n0[e] = fmaf(k, ur, n0[e]), n1[e] = fmaf(k, ui, n1[e]);
+                        sum[0][e] = fmaf(-k, ur, sum[0][e]), sum[1][e] = fmaf(-k, ui, sum[1][e]);
+                    } else {
+                        const float u = lv[0][e] - t0[e];  // (P == 1: times 2^100)
+                        const float s = P == 1 ? sgn_of_scaled(u) : u;
+                        sum[0][e] = fmaf(g, s, sum[0][e]);
+                        n0[e] = fmaf(-g, s, n0[e]);
+                    }
+                }
+            }
+            // The wave's eight lane groups: the values leave pairwise, so that each exchange halves what is carried.  A lane ends with column
+            // 4 tx + i of one plane.
+            float *red = sR + (l * WAVES + own_wave) * (NPL * kPairCols);
+            const int rho = (lane >> 4) & 1, beta = (lane >> 3) & 1, hi = lane >> 5;
+            if constexpr (NPL == 2) {
+                float w[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    swap_halves(sum[0][i], sum[1][i]);
+                    w[i] = sum[0][i] + sum[1][i];
+                }
+                swap_rows(w[0], w[2]);
+                swap_rows(w[1], w[3]);
+                const float y0 = add_ror8(w[0] + w[2]), y1 = add_ror8(w[1] + w[3]);
+                red[hi * kPairCols + tx * 4 + 2 * rho + beta] = beta ? y1 : y0;
+            } else {
+                swap_halves(sum[0][0], sum[0][2]);
+                swap_halves(sum[0][1], sum[0][3]);
+                float z0 = sum[0][0] + sum[0][2], z1 = sum[0][1] + sum[0][3];
+                swap_rows(z0, z1);
+                const float y = add_ror8(z0 + z1);
+                if (beta == 0) red[tx * 4 + 2 * hi + rho] = y;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < NPL; ++q)
+#pragma unroll
+            for (int o = 0; o < RO; ++o) acc[q][o] = add4(acc[q][o], sacc[q][o]);
+        __syncthreads();
+        // the waves' sums of this step's positives
+#pragma unroll
+        for (int s = 0; s < KL * NPL * kPairCols / TH; ++s) {
+            const int v = tid + TH * s, l = v / (NPL * kPairCols), pc = v % (NPL * kPairCols), lc = pc % kPairCols;
+            float x = sR[l * WAVES * (NPL * kPairCols) + pc];
+#pragma unroll
+            for (int w = 1; w < wo; ++w) x += sR[(l * WAVES + w) * (NPL * kPairCols) + pc];
+            const int jl = tile_x * kPairCols + (lc & ~3), j = min(jl, klen - 4);
+            if (l0 + l < b1 && (lc & 3) >= jl - j)
+                pa.g0[tile * pa.gplane + ((int64_t)c * a.C + l0 + l) * d + (pc >= kPairCols ? half : 0) + j + (lc & 3)] = x;
+        }
+    }
+
+    if constexpr (PH > 1) {  // the phases' sums of the same negatives
+        __syncthreads();
+        float4 *sS = reinterpret_cast<float4 *>(dyn_smem);
+        static_assert(sizeof(float4) * NPL * RO * TH * 3 / 4 <= sizeof(float) * S::kLdsFloats, "three of four phases pass through LDS");
+        constexpr int slots = wo * kWave;
+        const int slot = own_wave * kWave + lane;
+        if (phase > 0) {
+#pragma unroll
+            for (int q = 0; q < NPL; ++q)
+#pragma unroll
+                for (int o = 0; o < RO; ++o) sS[((phase - 1) * NPL * RO + q * RO + o) * slots + slot] = acc[q][o];
+        }
+        __syncthreads();
+        if (phase > 0) return;
+        for (int p = 1; p < PH; ++p)
+#pragma unroll
+            for (int q = 0; q < NPL; ++q)
+#pragma unroll
+                for (int o = 0; o < RO; ++o) acc[q][o] = add4(acc[q][o], sS[((p - 1) * NPL * RO + q * RO + o) * slots + slot]);
+    }
+#pragma unroll
+    for (int o = 0; o < RO; ++o) {
+        const int kl = k0 + ty * RO + o;
+        if (kl >= a.N) continue;
+        float *dst = (split ? pa.more_neg + (split - 1) * pa.nplane : pa.occ_neg) + ((int64_t)c * a.N + kl) * d;
+#pragma unroll
+        for (int q = 0; q < NPL; ++q) {
+            float *p = dst + q * half + col;
+            const float4 v = acc[q][o];
+            if (skip == 0) {
+                store_quad(p, v);
+            } else {
+                if (skip <= 1) p[1] = v.y;
+                if (skip <= 2) p[2] = v.z;
+                if (skip <= 3) p[3] = v.w;
+            }
+        }
+    }
+}
+
+// Whether a batch's gradient tiles evaluate every pair once, and how they are cut.  Both ways timed over 200 random shapes (256 ... 16384
+// positives, chunks and negatives 16 ... 1024, widths 48 ... 1000; tiles, per-positive kernel and reductions together).
+//   RotatE: always; 0.73 of the time in the mean, 1.06 at worst (874 x 77 negatives x 322 in chunks of 38).
+//   TransE L1: 0.87 in the mean by the rule below.  A thread of the other tiles walks the longer side of a chunk; from 160 on that walk costs a
+//   small batch more than the extra planes do.  A batch that fills the chip goes by the padded pairs of both forms.
+//   TransE L2, where differences are summed (launch_tiles): no sign to save, so only the walk counts: 0.83 from 280 on, 1.0 below.
+inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *out)
+{
+    if (!bat->neg || bat->chunk <= 0 || bat->n_neg <= 0 || !rows_by_quads(tab)) return false;  // (rows by quads)
+    if (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE) return false;
+    const int64_t n_chunks = bat->batch / bat->chunk, C = bat->chunk, N = bat->n_neg, klen = tab->model == KGE_ROTATE ? tab->dim / 2 : tab->dim;
+    const int64_t cols = ceil_div(klen, kPairCols) * n_chunks, steps = ceil_div(C, kPairKL), longer = C > N ? C : N;
+    // Negatives of a workgroup: 128, or 64 / 32 by waves in two / four phases (5 / 20 % slower per pair), by what the last tile wastes and
+    // what the planes cost (a plane of a batch beyond the caches as much as 17 negatives, else 6).  A launch that cannot fill the chip takes smaller ones.
+    const int64_t plane = bat->batch * tab->dim >= 4000000 ? 17 : 6;
+    auto cost = [&](int ph) { return ceil_div(N, kPairOwners / ph) * (kPairOwners / ph * (ph == 1 ? 100 : ph == 2 ? 105 : 120) + plane * 100); };
+    int ph = cost(1) <= cost(2) && cost(1) <= cost(4) ? 1 : (cost(2) <= cost(4) ? 2 : 4);
+    while (ph < 4 && cols * ceil_div(N, kPairOwners / ph) * steps < 384) ph *= 2;
+    const int64_t tiles = ceil_div(N, kPairOwners / ph);
+    // Ranges of positives: 640 workgroups, and of long chunks at most 192 positives each (up to eight ranges).  RotatE 1024 x 256 x 1000, 128
+    // workgroups a range: 2 / 4 / 6 / 8 ranges 71 / 57 / 60 / 55 us, and the reduction 2 us a plane.
+    int64_t splits = ceil_div(640, cols * tiles);
+    const int64_t by_length = ceil_div(C, 192) < 8 ? ceil_div(C, 192) : 8;
+    splits = splits > by_length ? splits : by_length;
+    splits = splits < steps ? splits : steps;
+    out->phases = ph, out->tiles = (int)tiles;
+    out->per = (int)(ceil_div(steps, splits) * kPairKL);
+    out->splits = (int)ceil_div(C, out->per);
+    if (tab->model == KGE_ROTATE) return true;
+    if (tab->norm_p == 2) return longer >= 280 && !transe_by_products(tab->dim, C, N, n_chunks);
+    // clocks per wave: a padded pair of the other tiles 9.5 per orientation, one here 16
+    const int64_t gx = ceil_div(klen, kTI), big = gx * (ceil_div(C, 64) + ceil_div(N, 64)) * n_chunks, to = big >= 1024 ? 64 : (big >= 512 ? 32 : 16);
+    const double padded = (double)(ceil_div(C, to) * to * ceil_div(N, 32) * 32 + ceil_div(N, to) * to * ceil_div(C, 32) * 32);
+    const double both = 9.5 * (double)(gx * kTI * n_chunks) * padded;
+    const double once = 16.0 * (double)(cols * kPairCols) * (double)(steps * kPairKL * (tiles * kPairOwners / ph) + plane * tiles * C);
+    const bool fills = both > 1.5e10;  // (about 100 us)
+    return once < both * (longer < 160 ? 0.8 : (fills ? 0.95 : 1.2));
+}
+
+template <int MODEL, int P>
+static int launch_pairs(const TileArgs &a, const PairArgs &pa, const FusedInsp &fi, hipStream_t st)
+{
+    size_t lds = sizeof(float) * PairShape<MODEL>::kLdsFloats;
+    if (fi.blocks > 0 && (size_t)fi.lds_bytes > lds) lds = (size_t)fi.lds_bytes;
+    const int klen = MODEL == KGE_ROTATE ? a.d / 2 : a.d;
+    const unsigned grid = xcd_grid(ceil_div(klen, kPairCols), (int64_t)pa.plan.tiles * pa.plan.splits, a.n_chunks) + (unsigned)fi.blocks;
+    const auto kernel = pa.plan.phases == 1 ? bwd_pair_kernel<MODEL, P, 1> : (pa.plan.phases == 2 ? bwd_pair_kernel<MODEL, P, 2> : bwd_pair_kernel<MODEL, P, 4>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kPairWaves * kWave), lds, st, a, pa, fi);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+}  // namespace kge

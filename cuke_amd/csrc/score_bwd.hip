@@ -692,6 +692,18 @@ static size_t tile_lds_bytes(const FusedInsp &fi)
     return fi.blocks > 0 && (size_t)fi.lds_bytes > own ? (size_t)fi.lds_bytes : own;
 }
 
+
+// TransE L2 as 64-bit products (kDiff of bwd_tile_body) or as differences: the rule's figures are in launch_tiles.
+static bool transe_by_products(int64_t d, int64_t C, int64_t N, int64_t n_chunks)
+{
+    const int64_t gx = ceil_div(d, kTI);
+    return gx * (ceil_div(C, 64) + ceil_div(N, 64)) * n_chunks >= 1024 || gx * n_chunks * (C < N ? C : N) >= 6144;
+}
+
+}  // namespace kge
+#include "pair_bwd.hpp"
+namespace kge {
+
 // the form of the kernel that the widths allow
 #define LAUNCH_TILE_VEC(RO_, MF_, GRID, ...)                                                                                     \
     do {                                                                                                                         \
@@ -714,9 +726,9 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
 {
     const int klen = MODEL == KGE_ROTATE ? a.d / 2 : a.d;
     const int64_t gx = ceil_div(klen, kTI);
-    const bool narrow = narrow_cols(klen) > 0;       // the last 1..16 columns go to narrow tiles (64-owner VALU launches)
-    const int64_t gxw = narrow ? klen / kTI : gx;    // wide column tiles of such a launch
-    const int64_t big = gx * (ceil_div(a.C, 64) + ceil_div(a.N, 64)) * n_chunks;
+    [[maybe_unused]] const bool narrow = narrow_cols(klen) > 0;       // the last 1..16 columns go to narrow tiles (64-owner VALU launches)
+    [[maybe_unused]] const int64_t gxw = narrow ? klen / kTI : gx;    // wide column tiles of such a launch
+    [[maybe_unused]] const int64_t big = gx * (ceil_div(a.C, 64) + ceil_div(a.N, 64)) * n_chunks;
     // the size rule follows launch_neg_mp (see there)
     constexpr bool kDotModel = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL;
     if constexpr (kDotModel || (MODEL == KGE_TRANSE && P == 2)) {
@@ -728,7 +740,7 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
         //   3000 56 / 52 (3000 x 600 x 200 x 150)   4096 25 / 22 (1024 x 256 x 256 x 256)   6000 65 / 73 (6000 x 600 x 200 x 150), but 21 / 18
         //   (2000 x 100 x 100 x 130)   6144 26 / 32 (1536 x 256 x 256 x 256)   7168 42 / 48 (1024 x 512 x 512 x 400)   12000 22 / 26 (4000 x 100 x
         //   100 x 130)   28672 192 / 217 (4096 x 1024 x 1024 x 400); from 1024 tiles on 112 / 165 (4096 x 1024 x 50 x 1000), 40 / 41 (16384 x 16 x 16 x 100).
-        const bool fill = kDotModel || big >= 1024 || gx * n_chunks * (a.C < a.N ? a.C : a.N) >= 6144;
+        const bool fill = kDotModel || transe_by_products(a.d, a.C, a.N, n_chunks);
         if (!dot_valu && fill && a.vec) {  // (rows of fewer than four floats: vector ALUs)
             // (ComplEx by quads: column tiles pair 32 real with the matching 32 imaginary columns)
             const int64_t gxm = MODEL == KGE_COMPLEX ? ceil_div(a.d / 2, 32) : gx;
@@ -740,26 +752,35 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
             return KGE_OK;
         }
     }
-    if (big >= 1024) {
-        const unsigned gh = xcd_grid(gxw, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxw, ceil_div(a.N, 64), n_chunks);
-        const unsigned nh = narrow ? xcd_grid(1, ceil_div(a.C, 64), n_chunks) : 0;
-        const unsigned nn = narrow ? xcd_grid(1, ceil_div(a.N, 64), n_chunks) : 0;
-        const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
-        const TileGrid tg{(int)gh, (int)gn, (int)nh, (int)nn};
-        LAUNCH_TILE(4, dim3(gh + gn + nh + nn + fi.blocks), tg);
-    } else if (big >= 512) {
-        const unsigned gh = xcd_grid(gx, ceil_div(a.C, 32), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 32), n_chunks);
-        const size_t lds = tile_lds_bytes<MODEL, 2>(fi);
-        const TileGrid tg{(int)gh, (int)gn, 0, 0};
-        LAUNCH_TILE(2, dim3(gh + gn + fi.blocks), tg);
-    } else {
-        // a batch this small leaves one or two 32-owner workgroups per CU: 16-owner tiles double the
-        // waves that hide each other's latency
-        const unsigned gh = xcd_grid(gx, ceil_div(a.C, 16), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 16), n_chunks);
-        const size_t lds = tile_lds_bytes<MODEL, 1>(fi);
-        const TileGrid tg{(int)gh, (int)gn, 0, 0};
-        LAUNCH_TILE(1, dim3(gh + gn + fi.blocks), tg);
+    if constexpr (MODEL != KGE_ROTATE) {  // (RotatE's rows by quads go by pairs, see pair_bwd.hpp)
+        if (big >= 1024) {
+            const unsigned gh = xcd_grid(gxw, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxw, ceil_div(a.N, 64), n_chunks);
+            const unsigned nh = narrow ? xcd_grid(1, ceil_div(a.C, 64), n_chunks) : 0;
+            const unsigned nn = narrow ? xcd_grid(1, ceil_div(a.N, 64), n_chunks) : 0;
+            const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
+            const TileGrid tg{(int)gh, (int)gn, (int)nh, (int)nn};
+            LAUNCH_TILE(4, dim3(gh + gn + nh + nn + fi.blocks), tg);
+            KGE_CHECK_LAUNCH();
+            return KGE_OK;
+        }
+        if (big >= 512) {
+            const unsigned gh = xcd_grid(gx, ceil_div(a.C, 32), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 32), n_chunks);
+            const size_t lds = tile_lds_bytes<MODEL, 2>(fi);
+            const TileGrid tg{(int)gh, (int)gn, 0, 0};
+            LAUNCH_TILE(2, dim3(gh + gn + fi.blocks), tg);
+            KGE_CHECK_LAUNCH();
+            return KGE_OK;
+        }
     }
+    // a batch this small leaves one or two 32-owner workgroups per CU: 16-owner tiles double the
+    // waves that hide each other's latency
+    const unsigned gh = xcd_grid(gx, ceil_div(a.C, 16), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 16), n_chunks);
+    const size_t lds = tile_lds_bytes<MODEL, 1>(fi);
+    const TileGrid tg{(int)gh, (int)gn, 0, 0};
+    if constexpr (MODEL == KGE_ROTATE)
+        hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, 1, false, false, false>), dim3(gh + gn + fi.blocks), dim3(256), lds, st, a, g0, g1, occ_neg, tg, fi);
+    else
+        LAUNCH_TILE(1, dim3(gh + gn + fi.blocks), tg);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }
@@ -779,12 +800,21 @@ struct PosBwdArgs {
     float *occ_w;          // [B, d] TransH
     int64_t B;
     int d, rel_dim;
+    int planes;            // g0, g1: planes of [B, d] rows to be added up
 };
 
 template <int V>
-__device__ __forceinline__ Vec<V> ldz(const float *p, int j)
+__device__ __forceinline__ Vec<V> ldz(const float *p, int j, int planes = 1, int64_t stride = 0)
 {
-    if (p) return Vec<V>::load(p + j);
+    if (p) {
+        Vec<V> s = Vec<V>::load(p + j);
+        for (int q = 1; q < planes; ++q) {
+            const Vec<V> m = Vec<V>::load(p + q * stride + j);
+#pragma unroll
+            for (int e = 0; e < V; ++e) s.v[e] += m.v[e];
+        }
+        return s;
+    }
     Vec<V> z;
 #pragma unroll
     for (int e = 0; e < V; ++e) z.v[e] = 0.0f;
@@ -821,11 +851,12 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
         gs = s > 0.0f ? g / s : 0.0f;
     }
 
+    const int64_t gplane = a.B * d;
     if constexpr (MODEL == KGE_TRANSE) {
         for (int j0 = lane * V; j0 < d; j0 += kWave * V) {
             const int j = RowPiece<V, RAG>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j);
-            const Vec<V> G = ldz<V>(g0, j);
+            const Vec<V> G = ldz<V>(g0, j, a.planes, gplane);
             Vec<V> dh, dt;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
@@ -913,7 +944,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             const Vec<V> hr = Vec<V>::load(eh + j), hi = Vec<V>::load(eh + half + j);
             const Vec<V> tr = Vec<V>::load(et + j), ti = Vec<V>::load(et + half + j);
             const Vec<V> th = Vec<V>::load(rr + j);
-            const Vec<V> Gr = ldz<V>(g0, j), Gi = ldz<V>(g0, half + j);
+            const Vec<V> Gr = ldz<V>(g0, j, a.planes, gplane), Gi = ldz<V>(g0, half + j, a.planes, gplane);
             Vec<V> dhr, dhi, dth, dtr, dti;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
@@ -1030,7 +1061,9 @@ __global__ void fill_zero_kernel(float *p, int64_t n)
 // ---------------------------------------------------------------------------------------
 struct BwdPlan {
     int64_t n_occ, nn;
-    size_t off_occ_e, off_occ_r, off_occ_w, off_g0, off_g1, off_part_e, off_part_r, off_part_w, total;
+    bool by_pairs;   // the gradient tiles evaluate every pair once (pair_bwd.hpp)
+    PairPlan pairs;
+    size_t off_more, off_occ_e, off_occ_r, off_occ_w, off_g0, off_g1, off_part_e, off_part_r, off_part_w, total;
 };
 
 static size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
@@ -1050,8 +1083,11 @@ static BwdPlan make_bwd_plan(const kge_tables *tab, const kge_batch *bat)
     p.off_occ_e = take(p.n_occ * d);
     p.off_occ_r = take(B * rd);
     p.off_occ_w = take(tab->model == KGE_TRANSH ? B * d : 0);
-    p.off_g0 = take(bat->neg ? B * d : 0);
+    p.by_pairs = plan_pairs(tab, bat, &p.pairs);
+    if (!p.by_pairs) p.pairs = PairPlan{1, 1, 1, 0};
+    p.off_g0 = take(bat->neg ? p.pairs.tiles * B * d : 0);
     p.off_g1 = take(bat->neg && tab->model == KGE_TRANSH ? B * d : 0);
+    p.off_more = take((p.pairs.splits - 1) * p.nn * d);
     p.off_part_e = take(seg_partial_floats(p.n_occ, d));
     p.off_part_r = take(seg_partial_floats(B, rd));
     p.off_part_w = take(tab->model == KGE_TRANSH ? seg_partial_floats(B, d) : 0);
@@ -1169,6 +1205,11 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
                    vecn ? 1 : 0, (int)n_chunks, head ? -1.0f : 1.0f,
                    chained ? 1 : 0, head ? bat->h : bat->t, dpos, head ? occ_e + B * d : occ_e, head ? occ_e : occ_e + B * d, occ_r};
         float *occ_neg = occ_e + 2 * B * d;
+        if (p.by_pairs) {
+            const PairArgs pr{p.pairs, g0, B * d, occ_neg, reinterpret_cast<float *>(ws + p.off_more), p.nn * d};
+            if (model == KGE_ROTATE) rc = launch_pairs<KGE_ROTATE, 2>(a, pr, fi_pass, st);
+            else rc = P == 1 ? launch_pairs<KGE_TRANSE, 1>(a, pr, fi_pass, st) : launch_pairs<KGE_TRANSE, 2>(a, pr, fi_pass, st);
+        } else
         switch (model) {
         case KGE_TRANSE:
             rc = P == 1 ? launch_tiles<KGE_TRANSE, 1>(a, g0, g1, occ_neg, n_chunks, dv, fi_pass, st)
@@ -1193,7 +1234,7 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
     if (!chained) {
     PosBwdArgs pa{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, dpos, saved->pos, saved->side_pos,
                   g0, g1, have_neg ? dneg : nullptr, bat->n_neg, occ_e, occ_e + B * d, occ_r, occ_w, B, (int)d,
-                  (int)tab->rel_dim};
+                  (int)tab->rel_dim, p.pairs.tiles};
     switch (model) {
     case KGE_TRANSE:
         rc = P == 1 ? launch_pos_bwd<KGE_TRANSE, 1>(pa, vec, head, fi_dedup, st) : launch_pos_bwd<KGE_TRANSE, 2>(pa, vec, head, fi_dedup, st);
@@ -1213,10 +1254,14 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
 
     if (bat->insp_ready && hipStreamWaitEvent(st, reinterpret_cast<hipEvent_t>(bat->insp_ready), 0) != hipSuccess)
         return KGE_ELAUNCH;
-    const SegJob jobs[3] = {
+    SegJob jobs[3] = {
         {occ_e, bat->ent_insp, (int)d, grads->ent_rows, reinterpret_cast<float *>(ws + p.off_part_e), false},
         {occ_r, bat->rel_insp, (int)tab->rel_dim, grads->rel_rows, reinterpret_cast<float *>(ws + p.off_part_r), false},
         {occ_w, bat->rel_insp, (int)d, grads->aux_rows, reinterpret_cast<float *>(ws + p.off_part_w), false}};
+    if (have_neg && p.pairs.splits > 1) {
+        jobs[0].more = reinterpret_cast<const float *>(ws + p.off_more), jobs[0].more_planes = p.pairs.splits - 1;
+        jobs[0].more_from = 2 * B, jobs[0].more_stride = p.nn * d;
+    }
     return launch_seg_reduce_jobs(jobs, model == KGE_TRANSH ? 3 : 2, st, bat->timeline);
 }
 

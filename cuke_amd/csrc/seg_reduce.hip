@@ -124,7 +124,8 @@ static int plan_jobs(const SegJob *jobs, int n_jobs, SegL1Rider *out, int64_t *m
         if (!jb.ins || jb.ins->n == 0 || jb.d == 0) continue;
         r.jobs.j[m] = SegArgs{jb.occ, jb.identity_perm ? nullptr : jb.ins->perm, jb.ins->sorted_seg,
                               jb.ins->seg_offsets, jb.ins->n, jb.d, jb.out, jb.partial,
-                              jb.scale_num, jb.scale_den, (jb.scaled ? 1 : 0) | (jb.sign_rows ? 2 : 0), (int)jb.wrap};
+                              jb.scale_num, jb.scale_den, (jb.scaled ? 1 : 0) | (jb.sign_rows ? 2 : 0), (int)jb.wrap,
+                              jb.more, jb.more_planes, (int)jb.more_from, jb.more_stride};
         v4 = v4 && quad_row(jb.d);
         ++m;
     }

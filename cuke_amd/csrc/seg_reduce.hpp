@@ -23,6 +23,11 @@ struct SegJob {
     // wrap > 0: occurrence i >= wrap takes row i - wrap (and its scale) with the opposite sign: the head and tail
     // occurrences of a translation model's triple share one row, +row for the head and -row for the tail.
     int64_t wrap = 0;
+    // Rows from `more_from` on are sums of 1 + more_planes rows: plane p's row for occurrence i is row i - more_from of
+    // more + p * more_stride.
+    const float *more = nullptr;
+    int more_planes = 0;
+    int64_t more_from = 0, more_stride = 0;
 };
 
 inline int64_t seg_partial_floats(int64_t n, int64_t d) { return ceil_div(n > 0 ? n : 1, kSegL) * 2 * d; }
@@ -48,6 +53,9 @@ struct SegArgs {
     const float *scale_num, *scale_den;   // row transform (SegJob), transform bit 0 = scaled, bit 1 = sign
     int transform;
     int wrap;                             // SegJob::wrap (0: none)
+    const float *more;                    // SegJob::more
+    int more_planes, more_from;
+    int64_t more_stride;
 };
 struct SegArgs3 {
     SegArgs j[3];
@@ -114,6 +122,15 @@ __device__ __forceinline__ void seg_l1_wave(const SegArgs &a, int64_t w)
     Vec<V> v[kSegL];
 #pragma unroll
     for (int q = 0; q < kSegL; ++q) v[q] = Vec<V>::load(a.occ + (int64_t)src[q] * d + cc);
+    for (int z = 0; z < a.more_planes; ++z) {  // uniform
+        Vec<V> m[kSegL];
+#pragma unroll
+        for (int q = 0; q < kSegL; ++q) m[q] = Vec<V>::load(a.more + z * a.more_stride + (int64_t)(src[q] < a.more_from ? 0 : src[q] - a.more_from) * d + cc);
+#pragma unroll
+        for (int q = 0; q < kSegL; ++q)
+#pragma unroll
+            for (int e = 0; e < V; ++e) v[q].v[e] += src[q] < a.more_from ? 0.0f : m[q].v[e];
+    }
     if (a.transform) {  // uniform: the rows count as scale * phi(row)
         float sc[kSegL];
 #pragma unroll

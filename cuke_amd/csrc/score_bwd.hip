@@ -118,7 +118,7 @@ __host__ __device__ inline int narrow_cols(int klen)
 // over the 64-column tiles.  A 64-column tile there would keep 12 of its 16 column lanes idle;
 // instead the column lanes are regrouped as 4 column groups x 4 owner sub-tiles and every thread
 // owns one row (RO_ = 1) of its sub-tile, so all 256 threads work on the 64 owners x 16 columns.
-template <int MODEL, int P, bool OWNER_POS, int RO, bool MF, bool VEC, bool VECN, bool NARROW = false>
+template <int MODEL, int P, bool OWNER_POS, int RO, bool MF, bool VEC, bool VECN, bool NARROW = false, bool HALF = false>
 __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float *smem, int col_base = 0)
 {
     static_assert(!(NARROW && MF), "the matrix-core loop has no narrow form");
@@ -241,7 +241,10 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     // g = l / 16 with looper 4 g + s; a lane's 128-bit read of four consecutive columns of that
     // looper's row feeds four MFMAs, so MFMA e owns the columns 4 j + e.  A wave owns 16 owners and
     // all 64 columns.
-    constexpr int EW = 4;  // MFMAs (columns per lane) per wave
+    // HALF: the last column tile, at most 32 columns, of the 64-bit products, whose matrix instructions bound them: a lane has two columns
+    // (30000 x 200 x 150, 22 of 64 columns in the last of three tiles: 178 -> 164 us)
+    static_assert(!HALF || kDiff, "a form of the 64-bit products");
+    constexpr int EW = HALF ? 2 : 4;  // MFMAs (columns per lane) per wave
     static_assert(!kMf || TO == 64, "a wave per 16 of 64 owners");
     const int mlane = tid & 63, ob = tid >> 6, fj = mlane & 15, fg = mlane >> 4;
     v4f macc[EW];
@@ -249,9 +252,9 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
     for (int e = 0; e < EW; ++e) macc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     // kDiff: the same in 64 bits, where a lane receives D[i = l / 16 + 4 v][j]
     double csum = 0.0;  // this lane's share of the coefficients of owner 16 ob + fj
-    v4d dacc[EW];
+    v4d dacc[4];
 #pragma unroll
-    for (int e = 0; e < EW; ++e) dacc[e] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (int e = 0; e < 4; ++e) dacc[e] = v4d{0.0, 0.0, 0.0, 0.0};
 
     // ---- staging: a three-deep software pipeline --------------------------------------------
     // While step st is computed, the rows and coefficients of step st+1 are in flight and so are
@@ -417,7 +420,28 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
         // two-level sum: the kKL loopers of a step go into a fresh accumulator that is folded
         // into the running one per step, so rounding grows with sqrt(steps) of the large partial
         // sums instead of sqrt(loopers)
-        if constexpr (kMf) {
+        if constexpr (kDiff) {
+            {
+#pragma unroll
+                for (int q = 0; q < kKL / 16; ++q)
+#pragma unroll
+                    for (int ms = 0; ms < 4; ++ms) {
+                        const int l = 16 * q + 4 * fg + ms;
+                        const float av = sG[0][l][ob * 16 + fj];
+                        csum += (double)av;
+                        float bv[EW];
+                        if constexpr (EW == 2) {
+                            const float2 b2 = *reinterpret_cast<const float2 *>(&sL[0][l][2 * fj]);
+                            bv[0] = b2.x, bv[1] = b2.y;
+                        } else {
+                            const float4 b4 = *reinterpret_cast<const float4 *>(&sL[0][l][4 * fj]);
+                            bv[0] = b4.x, bv[1] = b4.y, bv[2] = b4.z, bv[3] = b4.w;
+                        }
+#pragma unroll
+                        for (int e = 0; e < EW; ++e) dacc[e] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av, (double)bv[e], dacc[e], 0, 0, 0);
+                    }
+            }
+        } else if constexpr (kMf) {
 #pragma unroll
             for (int q = 0; q < kKL / 16; ++q)
 #pragma unroll
@@ -426,12 +450,8 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
                     const float av = sG[0][l][ob * 16 + fj];
                     const float4 b4 = *reinterpret_cast<const float4 *>(&sL[0][l][4 * fj]);
                     const float bv[4] = {b4.x, b4.y, b4.z, b4.w};
-                    if constexpr (kDiff) csum += (double)av;
 #pragma unroll
-                    for (int e = 0; e < EW; ++e) {
-                        if constexpr (kDiff) dacc[e] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)av, (double)bv[e], dacc[e], 0, 0, 0);
-                        else macc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], macc[e], 0, 0, 0);
-                    }
+                    for (int e = 0; e < EW; ++e) macc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv[e], macc[e], 0, 0, 0);
                 }
         }
         float4 sacc[NOUT][RO_];
@@ -591,7 +611,14 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
             double cs[4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) cs[v] = __shfl(csum, fg + 4 * v, kWave);
-            const int c0 = gcol(4 * fj);
+            if constexpr (HALF) {  // even lanes take the odd ones' two columns and leave them nothing to store
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) dacc[2 + e][v] = __shfl_xor(dacc[e][v], 1, kWave);
+            }
+            const int lc = HALF ? 2 * (fj & ~1) : 4 * fj, c0 = gcol(lc);
+
             float4 mine[4];
 #pragma unroll
             for (int v = 0; v < 4; ++v) {  // (rows past the tile's edge: its last row again, not stored)
@@ -608,9 +635,9 @@ __device__ __forceinline__ void bwd_tile_body(const TileArgs &a, int lid, float 
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int ol = ot0 + ob * 16 + fg + 4 * v;
-                if (ol >= n_own) continue;
+                if ((HALF && (fj & 1)) || ol >= n_own) continue;
                 auto diff = [&](float own, int e) { return (float)fma((double)own, cs[v], -dacc[e][v]); };
-                put(a.out0 + ((int64_t)c * n_own + ol) * (int64_t)d, 4 * fj, make_float4(diff(mine[v].x, 0), diff(mine[v].y, 1), diff(mine[v].z, 2), diff(mine[v].w, 3)));
+                put(a.out0 + ((int64_t)c * n_own + ol) * (int64_t)d, lc, make_float4(diff(mine[v].x, 0), diff(mine[v].y, 1), diff(mine[v].z, 2), diff(mine[v].w, 3)));
             }
             return;
         }
@@ -657,17 +684,26 @@ __global__ __launch_bounds__(256, KGE_TILE_OCC) void bwd_tile_kernel(TileArgs a,
     if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
     float *smem = reinterpret_cast<float *>(dyn_smem);
     int lid = (int)blockIdx.x - fi.blocks;
-    if (lid < grid.head) {
-        a.out0 = g0, a.out1 = g1;
-        bwd_tile_body<MODEL, P, true, RO, MF, VEC, VECN>(a, lid, smem);
+    const bool head = lid < grid.head;
+    if (head || lid < grid.head + grid.neg) {
+        if (!head) lid -= grid.head;
+        a.out0 = head ? g0 : occ_neg, a.out1 = head ? g1 : nullptr;
+        if constexpr (MODEL == KGE_TRANSE && P == 2 && MF) {
+            // the last column tile of rows that fill half of it (separate bodies: as a branch between the products the variants spill)
+            const int tiles_x = (a.d + kTI - 1) / kTI, rows = head ? a.C : a.N;
+            int c, ty, tx;
+            if (!xcd_tile(lid, tiles_x, (rows + 63) / 64, a.n_chunks, c, ty, tx)) return;
+            if (a.d - tx * kTI <= 32) {
+                if (head) bwd_tile_body<MODEL, P, true, RO, MF, VEC, VECN, false, true>(a, lid, smem);
+                else bwd_tile_body<MODEL, P, false, RO, MF, VEC, VECN, false, true>(a, lid, smem);
+                return;
+            }
+        }
+        if (head) bwd_tile_body<MODEL, P, true, RO, MF, VEC, VECN>(a, lid, smem);
+        else bwd_tile_body<MODEL, P, false, RO, MF, VEC, VECN>(a, lid, smem);
         return;
     }
     lid -= grid.head;
-    if (lid < grid.neg) {
-        a.out0 = occ_neg, a.out1 = nullptr;
-        bwd_tile_body<MODEL, P, false, RO, MF, VEC, VECN>(a, lid, smem);
-        return;
-    }
     if constexpr (RO == 4 && !MF) {
         lid -= grid.neg;
         const int klen = pair_len<MODEL>(a.d);

@@ -3,6 +3,8 @@ positives, their ragged edges, widths that end inside a quad, rows of one to thr
 both sides of the rule."""
 import pytest
 
+import test_gpu_transe_distances
+
 from cuke_amd import synth
 from test_gpu_backward import compare, run_both
 
@@ -29,3 +31,10 @@ def test_gradients(oracle, model, p, batch, chunk, n_neg, dim, mode):
     # RotatE: unit vectors of residuals a thousand times smaller than their operands, where the 32-bit oracle itself leaves the bar: one
     # complex element of the 32500 of 4096 x 257 x 130 head lies 2.3 bars from 64 bits there, the kernel's 0.25
     compare(g, ref, f"{model} L{p} {batch}x{n_neg}x{dim} {mode}", outliers=(4e-5, 4.0) if model == "RotatE" else None)
+
+
+@pytest.mark.parametrize("dim", [5, 34, 65, 96, 97, 150])
+@pytest.mark.parametrize("mode", ["tail", "head"])
+def test_last_column_tile_of_the_64_bit_products(dim, mode):
+    """One to 32 columns left over (and 33, where the whole tile takes them)."""
+    test_gpu_transe_distances.test_gradients_of_close_rows(8192, 256, 200, dim, "matrix_cores", "offset 0.25", mode)

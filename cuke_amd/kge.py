@@ -1015,7 +1015,7 @@ class TrainStep:
     def run(self, backward=True, overlap=True, pipeline=False, inputs_ready=None, fused=None):
         """Enqueue one step.
 
-        fused (default whenever the batch qualifies: index sets of at most 65536 ids; shared
+        fused (default where the batch qualifies and it is the faster form: index sets of at most 65536 ids; shared
         negatives, or TransR / RESCAL on their grouped path): the inspector's workgroups ride in
         front of the score kernels' own workgroups in the same launches, so the whole step is one
         chain of kernels on one stream with the inspection off its critical path.  TransR /
@@ -1047,7 +1047,15 @@ class TrainStep:
         if not pipeline:
             self.bat.plans_ready = 0  # the forward call plans for itself
         if fused is None:
-            fused = backward and not pipeline and self.fusable
+            # The projection models' explicit triples: with back rows two launches carry an inspection's four steps and the other two
+            # took launches of their own between forward and backward; up to 4096 ids are one launch for both sets.  Both index sets
+            # inspected in one batch up front are the faster chain then (with the optimizer steps: TransR 8192 triples x 200 of 1345
+            # relations 221 -> 209 us, 4096 x 256 of 500 185 -> 176, 512 x 128 of 237 91 -> 74; RESCAL 512 x 128 80 -> 71; TransR 2048 x 201,
+            # which cannot ride, 310 -> 295; RESCAL 4096 x 200, 8192 ids and no back rows, 159 -> 161).
+            up_front = backward and not pipeline and self.needs_rel_groups and self.neg is None and \
+                (self.back_rows is not None or 2 * self.B <= 4096)
+            fused = backward and not pipeline and self.fusable and not up_front
+            overlap = overlap and not up_front
         if fused:
             if not (backward and self.fusable) or pipeline or self._staged:
                 raise KgeError("fused inspection needs a backward step over a batch that qualifies "

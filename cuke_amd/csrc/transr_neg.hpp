@@ -55,11 +55,11 @@ static NegShape neg_shape(const kge_tables *tab, const kge_batch *bat)
 // forward workspace: the group inspection, the row list, both tile plans and the projected rows;
 // kge_score_bwd finds them through kge_saved.fwd_workspace
 struct NegFwdLayout {
-    size_t keys, knum, kuniq, kseg, kperm, kinv, ksseg, kws, kws_bytes;
+    size_t knum, kseg, kinv, ksseg;
     size_t gstart, segl, rowpos, rowa, rowp, hl, tl, rsl, plans, y, total;
 };
 
-static NegFwdLayout neg_fwd_layout(const kge_tables *tab, const NegShape &s)
+static NegFwdLayout neg_fwd_layout(const NegShape &s)
 {
     NegFwdLayout l{};
     size_t o = 0;
@@ -68,15 +68,10 @@ static NegFwdLayout neg_fwd_layout(const kge_tables *tab, const NegShape &s)
         o += up256(bytes > 0 ? bytes : 1);
         return at;
     };
-    l.keys = take(sizeof(int64_t) * s.B);
     l.knum = take(sizeof(int32_t));
-    l.kuniq = take(sizeof(int64_t) * s.B);
     l.kseg = take(sizeof(int32_t) * (s.B + 1));
-    l.kperm = take(sizeof(int32_t) * s.B);
     l.kinv = take(sizeof(int32_t) * s.B);
     l.ksseg = take(sizeof(int32_t) * s.B);
-    l.kws_bytes = kge_inspect_workspace(s.B, tab->n_rel * s.n_chunks);
-    l.kws = take(l.kws_bytes);
     l.gstart = take(sizeof(int32_t) * (s.U_cap + 1));
     l.segl = take(sizeof(int32_t) * (s.U_cap + 1));
     l.rowpos = take(sizeof(int32_t) * s.B);
@@ -123,11 +118,8 @@ struct NegIdx {
     const int64_t *h, *r, *t, *neg;
     // inspection of the relation ids (the caller's rel_insp)
     const int32_t *r_num, *r_seg, *r_perm, *r_inv, *r_sseg;
-    const int64_t *r_uniq;
-    // inspection of the group keys r * n_chunks + chunk
-    int64_t *keys;
-    const int32_t *k_num, *k_seg, *k_perm, *k_inv;
-    const int64_t *k_uniq;
+    // the groups (relation, chunk), in relation order: their number, segments of the positions, group of a positive / of a position
+    int32_t *k_num, *k_seg, *k_inv, *k_sseg;
     int32_t *gstart, *segl, *rowpos, *rowa, *rowp;
     int64_t *hl, *tl;
     float *rsl;
@@ -135,33 +127,67 @@ struct NegIdx {
     int d, head;
 };
 
-__global__ void tneg_keys_kernel(NegIdx x)
+// The groups of positives that share relation and chunk.  The relation inspection's order is stable, so within a relation the positives, and
+// with them their chunks, ascend: a group begins where either changes, and its first position holds its smallest positive.  A workgroup
+// owns kGroupPos positions and counts the groups that begin before them itself (8 bytes a position), so it waits for no other.
+//   gstart[u]: relation u's first group; segl[u]: its first list row = 2 per positive of the smaller relations + N per group
+// (The groups as an inspection of keys relation * n_chunks + chunk, with a kernel for the keys and one for the starts, took 26 us of
+// launches at 4096 positives; this one 8.)
+constexpr int kGroupThreads = 1024, kGroupPos = 4 * kGroupThreads;
+__global__ __launch_bounds__(kGroupThreads) void tneg_groups_kernel(NegIdx x)
 {
-    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < x.B) x.keys[b] = x.r[b] * x.n_chunks + b / x.C;
-}
-
-// gstart[u]: index of relation u's first group in the (relation-major) key order; segl[u]: first
-// list row of relation u = 2 positions per positive of the smaller relations + N per group
-__global__ void tneg_gstart_kernel(NegIdx x)
-{
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    const int U = x.r_num[0], G = x.k_num[0];
-    if (u > U) return;
-    if (u == U) {
-        x.gstart[U] = G;
-        x.segl[U] = (int32_t)(2 * x.B + x.N * G);
-        return;
+    __shared__ int s_wave[kGroupThreads / kWave], s_before[kGroupThreads / kWave];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, B = (int)x.B;
+    const uint32_t C = (uint32_t)x.C;
+    int b[4], u[4];
+    int heads, rel_heads;  // bit i: position p + i begins a group / a relation
+    auto look = [&](int p) {  // (unconditional loads: positions past the end read the last one)
+        const int pp = min(max(p - 1, 0), B - 1);
+        int b0 = x.r_perm[pp], u0 = x.r_sseg[pp];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) b[i] = x.r_perm[min(p + i, B - 1)], u[i] = x.r_sseg[min(p + i, B - 1)];
+        uint32_t c0 = (uint32_t)b0 / C;
+        heads = rel_heads = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t c = (uint32_t)b[i] / C;
+            const bool first = p + i == 0, rel = first || u[i] != u0;
+            if (p + i < B && rel) rel_heads |= 1 << i;
+            if (p + i < B && (rel || c != c0)) heads |= 1 << i;
+            c0 = c, u0 = u[i];
+        }
+    };
+    const int start = (int)blockIdx.x * kGroupPos;
+    int before = 0;
+    for (int q = 0; q < start; q += kGroupPos) {
+        look(q + 4 * tid);
+        before += __popc(heads);
     }
-    const int64_t target = x.r_uniq[u] * x.n_chunks;
-    int lo = 0, hi = G;  // first group whose key is >= target
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (x.k_uniq[mid] < target) lo = mid + 1;
-        else hi = mid;
+    before = wave_sum_i(before);
+    const int p = start + 4 * tid;
+    look(p);
+    int scan = __popc(heads);  // inclusive over the wave
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int v = __shfl_up(scan, o, kWave);
+        if (lane >= o) scan += v;
     }
-    x.gstart[u] = lo;
-    x.segl[u] = (int32_t)(2 * x.r_seg[u] + x.N * lo);
+    if (lane == kWave - 1) s_wave[wave] = scan;
+    if (lane == 0) s_before[wave] = before;
+    __syncthreads();
+    int g = scan - __popc(heads) - 1;  // the group of the position in front of this thread's
+    for (int w = 0; w < kGroupThreads / kWave; ++w) g += s_before[w] + (w < wave ? s_wave[w] : 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (p + i >= B) break;
+        if (heads >> i & 1) x.k_seg[++g] = p + i;
+        x.k_sseg[p + i] = g, x.k_inv[b[i]] = g;
+        if (rel_heads >> i & 1) x.gstart[u[i]] = g, x.segl[u[i]] = (int32_t)(2 * (int64_t)(p + i) + x.N * g);
+        if (p + i == B - 1) {
+            x.k_num[0] = g + 1, x.k_seg[g + 1] = B;
+            x.gstart[u[i] + 1] = g + 1, x.segl[u[i] + 1] = (int32_t)(2 * x.B + x.N * (g + 1));
+        }
+    }
 }
 
 // The list rows (entity to project, entity to subtract or -1, factor of the relation row) and where
@@ -186,7 +212,7 @@ __global__ void tneg_list_kernel(NegIdx x)
             const int64_t q = i - x.B;
             const int g = (int)(q / x.N), k = (int)(q % x.N);
             if (g >= G) continue;
-            const int brep = x.k_perm[x.k_seg[g]];  // any positive of the group names its relation and chunk
+            const int brep = x.r_perm[x.k_seg[g]];  // any positive of the group names its relation and chunk
             const int u = x.r_inv[brep];
             const int64_t c = brep / x.C;
             const int n_u = x.r_seg[u + 1] - x.r_seg[u];
@@ -197,26 +223,36 @@ __global__ void tneg_list_kernel(NegIdx x)
     }
 }
 
-// One wave per chunk: the first list row of every group that has a positive in the chunk, in the
-// order of the groups' first positives (glist[c * C + i], i < gcount[c]).  The first one also clears the row that dM subtracts
-// from list rows without a second entity.
-__global__ __launch_bounds__(64) void tneg_chunk_groups_kernel(NegIdx x, int32_t *glist, int32_t *gcount, float *zero_row)
+// For chunk c: the first list row of every group that has a positive in the chunk, in the order of the groups' first positives
+// (glist[c * C + i], i < gcount[c]).  The first one also clears the row that dM subtracts from list rows without a second
+// entity.  A workgroup of 256 threads of tneg_pair_bwd_p2_kernel's launch, which needs none of it (as a launch of its own, a wave a chunk, 11 us).
+struct ChunkGroups {
+    int32_t *glist, *gcount;
+    float *zero_row;
+};
+__device__ __forceinline__ void tneg_chunk_groups(const NegIdx &x, const ChunkGroups &o, int64_t c)
 {
-    const int64_t c = blockIdx.x;
-    const int lane = threadIdx.x;
+    __shared__ int s_cnt[2][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (c == 0)
-        for (int i = lane; i < x.d + kDmTickets; i += kWave) zero_row[i] = 0.0f;  // (and the counters behind it)
-    int count = 0;
-    for (int64_t i0 = 0; i0 < x.C; i0 += kWave) {
-        const int64_t i = i0 + lane;
+        for (int i = tid; i < x.d + kDmTickets; i += 256) o.zero_row[i] = 0.0f;  // (and the counters behind it)
+    int count = 0, turn = 0;
+    for (int64_t i0 = 0; i0 < x.C; i0 += 256, turn ^= 1) {
+        const int64_t i = i0 + tid;
         const int64_t b = c * x.C + (i < x.C ? i : x.C - 1);
         const int g = x.k_inv[b];
-        const bool rep = i < x.C && x.k_perm[x.k_seg[g]] == (int32_t)b;  // the stable sort puts the smallest b first
+        const bool rep = i < x.C && x.r_perm[x.k_seg[g]] == (int32_t)b;
         const uint64_t m = __ballot(rep);
-        if (rep) glist[c * x.C + count + __popcll(m & ((1ull << lane) - 1))] = x.rowp[g];
-        count += __popcll(m);
+        if (lane == 0) s_cnt[turn][wave] = __popcll(m);
+        __syncthreads();  // (one a turn: the counts alternate between two places)
+        int at = count;
+        for (int w = 0; w < 4; ++w) {
+            if (w < wave) at += s_cnt[turn][w];
+            count += s_cnt[turn][w];
+        }
+        if (rep) o.glist[c * x.C + at + __popcll(m & ((1ull << lane) - 1))] = x.rowp[g];
     }
-    if (lane == 0) gcount[c] = count;
+    if (tid == 0) o.gcount[c] = count;
 }
 
 // A row held by a wave: NQ float4 per lane (NQ = ceil(dim / 256) <= 4, a template parameter of
@@ -322,7 +358,7 @@ __global__ __launch_bounds__(256) void tneg_pair_fwd_kernel(NegIdx x, NegPairArg
 //   per positive over its group's P rows and a wave per (eight positions, negative) over both rows of every pair, it was 600 MB out of the
 //   L2 and 144 us; now 55 us (4096 positives x 64 negatives x 200, 1270 groups).
 template <int P, int KN>
-__global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArgs a, const int32_t *k_sseg, float *partial)
+__global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArgs a, float *partial)
 {
     __shared__ float s_c[kNegSeg][kWave];   // the pairs' coefficients, KN negatives at a time
     __shared__ float s_ga[kNegSeg][256];
@@ -335,10 +371,10 @@ __global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArg
     const int cc = colok ? col : d - 1;  // clamped: unconditional loads
     if (tid < kNegSeg) {
         const int64_t pc = p0 + (tid < cnt ? tid : cnt - 1);
-        const int b = x.k_perm[pc], g = k_sseg[pc];
+        const int b = x.r_perm[pc], g = x.k_sseg[pc];
         s_b[tid] = b, s_g[tid] = g, s_pa[tid] = x.rowa[b], s_pp[tid] = x.rowp[g];
     }
-    const int g_before = p0 > 0 ? k_sseg[p0 - 1] : -1, g_after = p0 + cnt < x.B ? k_sseg[p0 + cnt] : -1;
+    const int g_before = p0 > 0 ? x.k_sseg[p0 - 1] : -1, g_after = p0 + cnt < x.B ? x.k_sseg[p0 + cnt] : -1;
 #pragma unroll
     for (int q = 0; q < kNegSeg; ++q) s_ga[q][tid] = 0.0f;
     __syncthreads();
@@ -424,17 +460,18 @@ __global__ __launch_bounds__(256) void tneg_pair_bwd_kernel(NegIdx x, NegPairArg
 }
 
 template <int NQ>
-__global__ __launch_bounds__(256) void tneg_pair_bwd_p2_kernel(NegIdx x, const int32_t *k_sseg, const float *partial, float *ql)
+__global__ __launch_bounds__(256) void tneg_pair_bwd_p2_kernel(NegIdx x, const float *partial, float *ql, ChunkGroups chunks)
 {
+    if ((int64_t)blockIdx.x < x.n_chunks) return tneg_chunk_groups(x, chunks, blockIdx.x);
     const int lane = threadIdx.x & 63;
-    const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t w = ((int64_t)blockIdx.x - x.n_chunks) * 4 + (threadIdx.x >> 6);
     const int N = (int)x.N, d = x.d;
     const int64_t j = w / N;
     const int k = (int)(w % N);
     const int64_t p0 = j * kNegSeg;
     if (p0 >= x.B) return;
     const int64_t p1 = p0 + kNegSeg < x.B ? p0 + kNegSeg : x.B;
-    const int g = k_sseg[p1 - 1];
+    const int g = x.k_sseg[p1 - 1];
     const int s0 = x.k_seg[g], s1 = x.k_seg[g + 1];
     if (s1 <= p0 + kNegSeg || s0 < p0) return;  // no group starts here and continues
     const int64_t je = (s1 - 1) / kNegSeg;
@@ -571,13 +608,13 @@ static bool transr_neg_path_ok(const kge_tables *tab, const kge_batch *bat)
     if (!(s.n_chunks > 0 && tab->n_rel * s.n_chunks < (int64_t(1) << 31) && s.L_cap < (int64_t(1) << 31) &&
           s.L_cap * s.d < (int64_t(1) << 36)))
         return false;
-    return neg_fwd_layout(tab, s).total + neg_bwd_layout(s).total <= kNegWorkspaceCap;
+    return neg_fwd_layout(s).total + neg_bwd_layout(s).total <= kNegWorkspaceCap;
 }
 
 size_t transr_neg_fwd_workspace(const kge_tables *tab, const kge_batch *bat)
 {
     if (!transr_neg_path_ok(tab, bat)) return 0;
-    return neg_fwd_layout(tab, neg_shape(tab, bat)).total;
+    return neg_fwd_layout(neg_shape(tab, bat)).total;
 }
 
 size_t transr_neg_bwd_workspace(const kge_tables *tab, const kge_batch *bat)
@@ -592,13 +629,10 @@ static NegIdx neg_idx(const kge_tables *tab, const kge_batch *bat, const NegShap
     NegIdx x{};
     x.h = bat->h, x.r = bat->r, x.t = bat->t, x.neg = bat->neg;
     x.r_num = ri->num_unique, x.r_seg = ri->seg_offsets, x.r_perm = ri->perm, x.r_inv = ri->inverse, x.r_sseg = ri->sorted_seg;
-    x.r_uniq = ri->unique_ids;
-    x.keys = reinterpret_cast<int64_t *>(ws + l.keys);
     x.k_num = reinterpret_cast<int32_t *>(ws + l.knum);
-    x.k_uniq = reinterpret_cast<int64_t *>(ws + l.kuniq);
     x.k_seg = reinterpret_cast<int32_t *>(ws + l.kseg);
-    x.k_perm = reinterpret_cast<int32_t *>(ws + l.kperm);
     x.k_inv = reinterpret_cast<int32_t *>(ws + l.kinv);
+    x.k_sseg = reinterpret_cast<int32_t *>(ws + l.ksseg);
     x.gstart = reinterpret_cast<int32_t *>(ws + l.gstart);
     x.segl = reinterpret_cast<int32_t *>(ws + l.segl);
     x.rowpos = reinterpret_cast<int32_t *>(ws + l.rowpos);
@@ -619,31 +653,21 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
     if (bat->fuse_inspection) return KGE_EINVAL;  // this path runs its own group inspection
     if (!neg) return KGE_EINVAL;
     const NegShape s = neg_shape(tab, bat);
-    const NegFwdLayout l = neg_fwd_layout(tab, s);
+    const NegFwdLayout l = neg_fwd_layout(s);
     if (!workspace || workspace_bytes < l.total || !aligned16(workspace)) return KGE_EWORKSPACE;
     char *ws = static_cast<char *>(workspace);
     const NegIdx x = neg_idx(tab, bat, s, l, ws);
     const kge_inspection *ri = bat->rel_insp;
     const int d = (int)tab->dim;
 
-    // groups: inspection of the keys relation * n_chunks + chunk
-    hipLaunchKernelGGL(tneg_keys_kernel, dim3((unsigned)ceil_div(s.B, 256)), dim3(256), 0, st, x);
-    const kge_inspection kin{s.B, tab->n_rel * s.n_chunks, const_cast<int32_t *>(x.k_num), const_cast<int64_t *>(x.k_uniq),
-                             const_cast<int32_t *>(x.k_seg), const_cast<int32_t *>(x.k_perm), const_cast<int32_t *>(x.k_inv),
-                             reinterpret_cast<int32_t *>(ws + l.ksseg)};
-    const int64_t *parts[1] = {x.keys};
-    const int64_t lens[1] = {s.B};
-    if (const int rc = kge_inspect(parts, lens, 1, kin.n_rows, &kin, ws + l.kws, l.kws_bytes, st)) return rc;
-    timeline_mark(bat->timeline, st, "inspect(relation, chunk)");
-
-    // the list and its tile plans
-    hipLaunchKernelGGL(tneg_gstart_kernel, dim3((unsigned)ceil_div(s.U_cap + 1, 256)), dim3(256), 0, st, x);
+    // the groups, the list and its tile plans
+    hipLaunchKernelGGL(tneg_groups_kernel, dim3((unsigned)ceil_div(s.B, kGroupPos)), dim3(kGroupThreads), 0, st, x);
     const int64_t list_threads = s.B + s.G_cap * s.N;
     const int64_t list_blocks = ceil_div(list_threads, 256);
     hipLaunchKernelGGL(tneg_list_kernel, dim3((unsigned)(list_blocks < 8192 ? list_blocks : 8192)), dim3(256), 0, st, x);
     const Plans plans = plans_at(ws + l.plans, s.plans);
     launch_plans(ri, x.segl, plans, d, s.dm_split, st);
-    timeline_mark(bat->timeline, st, "row list + transr_plan_kernel");
+    timeline_mark(bat->timeline, st, "groups + row list + transr_plan_kernel");
 
     // one grouped pass projects every list row
     float *y = reinterpret_cast<float *>(ws + l.y);
@@ -667,7 +691,7 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     if (!transr_neg_path_ok(tab, bat)) return KGE_EUNSUPPORTED;
     if (bat->fuse_inspection) return KGE_EINVAL;
     const NegShape s = neg_shape(tab, bat);
-    const NegFwdLayout fl = neg_fwd_layout(tab, s);
+    const NegFwdLayout fl = neg_fwd_layout(s);
     const NegBwdLayout l = neg_bwd_layout(s);
     // the forward call's workspace holds the groups, the list, the plans and the projected rows
     if (!saved->fwd_workspace || saved->fwd_workspace_bytes < fl.total) return KGE_EINVAL;
@@ -692,14 +716,13 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     pa.ent = tab->ent, pa.y = y, pa.dpos = dpos, pa.dneg = dneg, pa.spos = saved->pos, pa.sneg = saved->neg;
     pa.ql = ql, pa.qr = qr;
     float *ppart = reinterpret_cast<float *>(ws + l.ppart);
-    const int32_t *k_sseg = reinterpret_cast<const int32_t *>(fws + fl.ksseg);
     const dim3 bgrid((unsigned)ceil_div(s.B, kNegSeg), (unsigned)ceil_div(d, 256));
-    if (s.N <= 16) TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 16, bgrid, x, pa, k_sseg, ppart);
-    else if (s.N <= 32) TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 32, bgrid, x, pa, k_sseg, ppart);
-    else TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 64, bgrid, x, pa, k_sseg, ppart);
-    const dim3 sgrid((unsigned)ceil_div(ceil_div(s.B, kNegSeg) * s.N, 4));
-    TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_pair_bwd_p2_kernel<NQ_>, sgrid, dim3(256), 0, st, x, k_sseg, ppart, ql));
-    hipLaunchKernelGGL(tneg_chunk_groups_kernel, dim3((unsigned)s.n_chunks), dim3(64), 0, st, x, glist, gcount, zero_row);
+    if (s.N <= 16) TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 16, bgrid, x, pa, ppart);
+    else if (s.N <= 32) TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 32, bgrid, x, pa, ppart);
+    else TNEG_BY_NORM(tab->norm_p, tneg_pair_bwd_kernel, 64, bgrid, x, pa, ppart);
+    const dim3 sgrid((unsigned)(ceil_div(ceil_div(s.B, kNegSeg) * s.N, 4) + s.n_chunks));
+    const ChunkGroups chunks{glist, gcount, zero_row};
+    TNEG_BY_WIDTH(d, hipLaunchKernelGGL(tneg_pair_bwd_p2_kernel<NQ_>, sgrid, dim3(256), 0, st, x, ppart, ql, chunks));
     timeline_mark(bat->timeline, st, "tneg_pair_bwd kernels");
 
     // dX = Q M^T over the list (rows stay in list order), dM = X^T Q per relation

@@ -165,9 +165,12 @@ int launch_seg_reduce_jobs(const SegJob *jobs, int n_jobs, hipStream_t st, kge_t
     const bool v4 = pl.v4 != 0;
     const SumRider none{};
     int64_t g1x = pl.blocks_x;
-    if (rd.max_sums > 0 && g1x < 256) g1x = 256;  // (a small reduction still gives the rider a grid's worth of workgroups)
+    // (a small reduction still gives the rider a grid of its own: 8704 rows beside 60 sums of 40 items each, TransR 4096 x 64 negatives x 200, whole
+    // step with 256 / 1024 / 2560 workgroups 629 / 620 / 622 us)
+    constexpr int64_t kRiderBlocks = 1024;
+    if (rd.max_sums > 0 && g1x < kRiderBlocks) g1x = kRiderBlocks;
     int64_t g2x = max_blocks * max_nch;
-    if (level1_rode && rd.max_sums > 0 && g2x < 256) g2x = 256;
+    if (level1_rode && rd.max_sums > 0 && g2x < kRiderBlocks) g2x = kRiderBlocks;
     const bool r1 = !level1_rode && rd.max_sums > 0, r2 = level1_rode && rd.max_sums > 0;
     const dim3 g1((unsigned)g1x, (unsigned)(m + (r1 ? 1 : 0))), g2((unsigned)g2x, (unsigned)(m + (r2 ? 1 : 0))), block(256);
     const bool level2 = m > 0 || r2;

@@ -1834,10 +1834,10 @@ static Plans plans_at(void *base, const PlanSizes &z)
     return r;
 }
 
-static void launch_plans(const kge_inspection *ri, const int32_t *seg_offsets, const Plans &p, int64_t d, bool split, hipStream_t st)
+static void launch_plans(const kge_inspection *ri, const int32_t *seg_offsets, const Plans &p, int64_t d, hipStream_t st)
 {
     hipLaunchKernelGGL(transr_plan_kernel, dim3(3), dim3(1024), 0, st, ri->num_unique, seg_offsets, ri->unique_ids, p.dm, kDmChunk,
-                       dm_nib(d, split), dm_small_max(d), p.tiles, kTM, p.tall, kTallRows);
+                       dm_nib(d, false), dm_small_max(d), p.tiles, kTM, p.tall, kTallRows);
 }
 
 static PlanSizes plan_sizes(const kge_tables *tab, const kge_batch *bat)
@@ -1946,7 +1946,7 @@ int launch_transr_fwd(const kge_tables *tab, const kge_batch *bat, float *pos, f
     const kge_inspection *ri = bat->rel_insp;
     const PlanSizes z = plan_sizes(tab, bat);
     const Plans plans = plans_at(workspace, z);
-    if (!bat->plans_ready) launch_plans(ri, ri->seg_offsets, plans, tab->dim, false, st);
+    if (!bat->plans_ready) launch_plans(ri, ri->seg_offsets, plans, tab->dim, st);
     GemmArgs a{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
                plans.tiles, nullptr, nullptr, pos, resid, nullptr, nullptr, (int)tab->dim, tab->norm_p,
                thin_groups(tab, bat), (int)z.tiles, BwdSrc{}, bat->back_rows};
@@ -1998,7 +1998,7 @@ int launch_transr_plan(const kge_tables *tab, const kge_batch *bat, void *worksp
     if (!mfma_path_ok(tab, bat) || gemm_lds_bytes((int)tab->dim) > kMaxGemmLds) return KGE_EUNSUPPORTED;
     if (!workspace || workspace_bytes < transr_fwd_workspace(tab, bat)) return KGE_EWORKSPACE;
     const kge_inspection *ri = bat->rel_insp;
-    launch_plans(ri, ri->seg_offsets, plans_at(workspace, plan_sizes(tab, bat)), tab->dim, false, st);
+    launch_plans(ri, ri->seg_offsets, plans_at(workspace, plan_sizes(tab, bat)), tab->dim, st);
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }
@@ -2110,7 +2110,7 @@ int launch_rescal_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
                        dneg ? g0 : nullptr, saved->residual, xs, qs, head ? occ : occ + B * d, B, d, head ? 1 : 0);
     const PlanSizes z = plan_sizes(tab, bat);
     const Plans plans = plans_at(ws + p.off_plans, z);
-    launch_plans(ri, ri->seg_offsets, plans, d, false, st);
+    launch_plans(ri, ri->seg_offsets, plans, d, st);
     // head: the tails' rows (g E[h] + G) Proj[r], the forward product on rows given as an array, written per triple
     GemmArgs ga{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, ri->perm, ri->seg_offsets, ri->num_unique, ri->unique_ids,
                 TilePlan{}, head ? xs : qs, nullptr, nullptr, head ? occ + B * d : nullptr, head ? nullptr : occ, nullptr, d, tab->norm_p, 0, 0,
@@ -2171,7 +2171,7 @@ int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_sav
         hipLaunchKernelGGL(transr_insp_step_kernel, dim3((unsigned)f1.blocks), dim3(256), lds_with(f1, 0), st, f1);
         timeline_mark(bat->timeline, st, "inspector step");
     }
-    if (!have_plans) launch_plans(ri, ri->seg_offsets, plans, d, false, st);
+    if (!have_plans) launch_plans(ri, ri->seg_offsets, plans, d, st);
     // Upstream rows q and left operands x are formed inside the two kernels from the forward pass's rows
     // (BwdSrc); RESCAL's tail occurrence rows g * v come out of the dX kernel's staging.
     const BwdSrc src{tab->ent, saved->residual, dpos, saved->pos, bat->h, bat->t, ri->perm, tab->norm_p, rescal ? 1 : 0,

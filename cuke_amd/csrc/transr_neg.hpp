@@ -118,6 +118,7 @@ struct NegIdx {
     const int64_t *h, *r, *t, *neg;
     // inspection of the relation ids (the caller's rel_insp)
     const int32_t *r_num, *r_seg, *r_perm, *r_inv, *r_sseg;
+    const int64_t *r_uniq;
     // the groups (relation, chunk), in relation order: their number, segments of the positions, group of a positive / of a position
     int32_t *k_num, *k_seg, *k_inv, *k_sseg;
     int32_t *gstart, *segl, *rowpos, *rowa, *rowp;
@@ -190,13 +191,17 @@ __global__ __launch_bounds__(kGroupThreads) void tneg_groups_kernel(NegIdx x)
     }
 }
 
-// The list rows (entity to project, entity to subtract or -1, factor of the relation row) and where
-// each positive's and each group's rows sit.
-__global__ void tneg_list_kernel(NegIdx x)
+// The tile plan of the list product, which needs of the list no more than where the relations' rows start (the first workgroup), beside
+// the list rows (entity to project, entity to subtract or -1, factor of the relation row) and where
+// each positive's and each group's rows sit.  (The list, then both plans: 5 + 19 us at 90000 rows; the plan of dM, the longer one,
+// rides with tneg_pair_fwd_kernel.)
+__global__ __launch_bounds__(1024) void tneg_list_kernel(NegIdx x, TilePlan plan, int tile)
 {
+    __shared__ int s_tot[2][96];
+    if (blockIdx.x == 0) return plan_body<false>(x.r_num, x.segl, x.r_uniq, plan, tile, 0, 0, s_tot);
     const int64_t total = x.B + x.G_cap * x.N;
     const int G = x.k_num[0];
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t i = ((int64_t)blockIdx.x - 1) * blockDim.x + threadIdx.x; i < total; i += ((int64_t)gridDim.x - 1) * blockDim.x) {
         if (i < x.B) {
             const int p = (int)i;  // position in relation order
             const int u = x.r_sseg[p], s0 = x.r_seg[u], n_u = x.r_seg[u + 1] - s0, j = p - s0;
@@ -307,12 +312,19 @@ struct NegPairArgs {
     float *ql, *qr;         // backward: upstream rows of the list, per-positive relation rows
 };
 
-// One wave per positive: pos[b] = ||y_pos||, neg[b][k] = ||a_b - P_(g(b),k)||.
+// One wave per positive: pos[b] = ||y_pos||, neg[b][k] = ||a_b - P_(g(b),k)||.  The first workgroup makes the plan of the backward pass's dM.
+struct DmPlanArgs {
+    TilePlan plan;
+    int chunk, nib, small_max;
+};
+constexpr int kPairFwdWaves = 16;
 template <int P, int NQ>
-__global__ __launch_bounds__(256) void tneg_pair_fwd_kernel(NegIdx x, NegPairArgs a)
+__global__ __launch_bounds__(kWave *kPairFwdWaves) void tneg_pair_fwd_kernel(NegIdx x, NegPairArgs a, DmPlanArgs dm)
 {
+    __shared__ int s_tot[2][96];
+    if (blockIdx.x == 0) return plan_body<true>(x.r_num, x.segl, x.r_uniq, dm.plan, dm.chunk, dm.nib, dm.small_max, s_tot);
     const int lane = threadIdx.x & 63;
-    const int64_t b = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t b = ((int64_t)blockIdx.x - 1) * kPairFwdWaves + (threadIdx.x >> 6);
     if (b >= x.B) return;
     const int d = x.d;
     const int N = (int)x.N;
@@ -629,6 +641,7 @@ static NegIdx neg_idx(const kge_tables *tab, const kge_batch *bat, const NegShap
     NegIdx x{};
     x.h = bat->h, x.r = bat->r, x.t = bat->t, x.neg = bat->neg;
     x.r_num = ri->num_unique, x.r_seg = ri->seg_offsets, x.r_perm = ri->perm, x.r_inv = ri->inverse, x.r_sseg = ri->sorted_seg;
+    x.r_uniq = ri->unique_ids;
     x.k_num = reinterpret_cast<int32_t *>(ws + l.knum);
     x.k_seg = reinterpret_cast<int32_t *>(ws + l.kseg);
     x.k_inv = reinterpret_cast<int32_t *>(ws + l.kinv);
@@ -663,11 +676,11 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
     // the groups, the list and its tile plans
     hipLaunchKernelGGL(tneg_groups_kernel, dim3((unsigned)ceil_div(s.B, kGroupPos)), dim3(kGroupThreads), 0, st, x);
     const int64_t list_threads = s.B + s.G_cap * s.N;
-    const int64_t list_blocks = ceil_div(list_threads, 256);
-    hipLaunchKernelGGL(tneg_list_kernel, dim3((unsigned)(list_blocks < 8192 ? list_blocks : 8192)), dim3(256), 0, st, x);
+    const int64_t list_blocks = ceil_div(list_threads, 1024);
     const Plans plans = plans_at(ws + l.plans, s.plans);
-    launch_plans(ri, x.segl, plans, d, s.dm_split, st);
-    timeline_mark(bat->timeline, st, "groups + row list + transr_plan_kernel");
+    hipLaunchKernelGGL(tneg_list_kernel, dim3((unsigned)(list_blocks < 2048 ? list_blocks : 2048) + 1), dim3(1024), 0, st, x,
+                       s.plans.tall ? plans.tall : plans.tiles, s.plans.tall ? kTallRows : kTM);
+    timeline_mark(bat->timeline, st, "groups + row list + plan");
 
     // one grouped pass projects every list row
     float *y = reinterpret_cast<float *>(ws + l.y);
@@ -678,8 +691,9 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
 
     NegPairArgs pa{};
     pa.ent = tab->ent, pa.y = y, pa.pos = pos, pa.neg = neg, pa.resid = resid;
-    const dim3 pgrid((unsigned)ceil_div(s.B, 4));
-    TNEG_BY_WIDTH(d, TNEG_BY_NORM(tab->norm_p, tneg_pair_fwd_kernel, NQ_, pgrid, x, pa));
+    const DmPlanArgs dm{plans.dm, kDmChunk, dm_nib(d, s.dm_split), dm_small_max(d)};
+    const dim3 pgrid((unsigned)ceil_div(s.B, kPairFwdWaves) + 1), pblock(kWave * kPairFwdWaves);
+    TNEG_BY_WIDTH(d, hipLaunchKernelGGL((tab->norm_p == 1 ? tneg_pair_fwd_kernel<1, NQ_> : tneg_pair_fwd_kernel<2, NQ_>), pgrid, pblock, 0, st, x, pa, dm));
     timeline_mark(bat->timeline, st, "tneg_pair_fwd_kernel");
     KGE_CHECK_LAUNCH();
     return KGE_OK;

@@ -114,9 +114,12 @@ __device__ __forceinline__ void block_exclusive_scans(const int (&v)[N], int *s_
 // dM kernel (`nib` row blocks per chunk, groups of at most `small_max` triples as one item).  Groups of more than two
 // entries are written by their whole wave (one thread writing its entries in turn made the kernel as long as the
 // largest group: 190 us for groups of thousands).  What is left is the launch and two round trips to memory.
+// share < kPlanShares: this workgroup is one of kPlanShares that make the plan together: all of them place every group, and
+// each writes an equal part of the larger groups.
+constexpr int kPlanShares = 8;
 template <bool CHUNKED>
 __device__ __forceinline__ void plan_body(const int32_t *num_unique, const int32_t *seg_offsets, const int64_t *unique_ids, const TilePlan &plan,
-                                          int tile, int nib, int small_max, int (*s_tot)[96])
+                                          int tile, int nib, int small_max, int (*s_tot)[96], int share = kPlanShares)
 {
     constexpr int N = CHUNKED ? 6 : 1;  // tiles; then split slots, splits, thin groups, long items, small items
     const int U = num_unique[0], tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -164,7 +167,7 @@ __device__ __forceinline__ void plan_body(const int32_t *num_unique, const int32
             if (v[0] > 0) entry(at[0], 0, g, s0, s1, rid, part);
             if (v[0] > 1) entry(at[0] + 1, 1, g, s0, s1, rid, part);
         }
-        for (uint64_t m = __ballot(many); m; m &= m - 1) {
+        for (uint64_t m = __ballot(many && (share == kPlanShares || lane % kPlanShares == share)); m; m &= m - 1) {
             const int l = __ffsll((unsigned long long)m) - 1;  // (uniform: the ballot is)
             const int cnt = __builtin_amdgcn_readlane(v[0], l), to = __builtin_amdgcn_readlane(at[0], l);
             const int p0 = __builtin_amdgcn_readlane(s0, l), end = __builtin_amdgcn_readlane(s1, l), r = __builtin_amdgcn_readlane(rid, l);

@@ -312,7 +312,8 @@ struct NegPairArgs {
     float *ql, *qr;         // backward: upstream rows of the list, per-positive relation rows
 };
 
-// One wave per positive: pos[b] = ||y_pos||, neg[b][k] = ||a_b - P_(g(b),k)||.  The first workgroup makes the plan of the backward pass's dM.
+// One wave per positive: pos[b] = ||y_pos||, neg[b][k] = ||a_b - P_(g(b),k)||.  The first workgroups make the plan of the backward pass's dM (one alone
+// took longer than all the pairs: 36 us against 25).
 struct DmPlanArgs {
     TilePlan plan;
     int chunk, nib, small_max;
@@ -322,9 +323,9 @@ template <int P, int NQ>
 __global__ __launch_bounds__(kWave *kPairFwdWaves) void tneg_pair_fwd_kernel(NegIdx x, NegPairArgs a, DmPlanArgs dm)
 {
     __shared__ int s_tot[2][96];
-    if (blockIdx.x == 0) return plan_body<true>(x.r_num, x.segl, x.r_uniq, dm.plan, dm.chunk, dm.nib, dm.small_max, s_tot);
+    if (blockIdx.x < kPlanShares) return plan_body<true>(x.r_num, x.segl, x.r_uniq, dm.plan, dm.chunk, dm.nib, dm.small_max, s_tot, (int)blockIdx.x);
     const int lane = threadIdx.x & 63;
-    const int64_t b = ((int64_t)blockIdx.x - 1) * kPairFwdWaves + (threadIdx.x >> 6);
+    const int64_t b = ((int64_t)blockIdx.x - kPlanShares) * kPairFwdWaves + (threadIdx.x >> 6);
     if (b >= x.B) return;
     const int d = x.d;
     const int N = (int)x.N;
@@ -692,7 +693,7 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
     NegPairArgs pa{};
     pa.ent = tab->ent, pa.y = y, pa.pos = pos, pa.neg = neg, pa.resid = resid;
     const DmPlanArgs dm{plans.dm, kDmChunk, dm_nib(d, s.dm_split), dm_small_max(d)};
-    const dim3 pgrid((unsigned)ceil_div(s.B, kPairFwdWaves) + 1), pblock(kWave * kPairFwdWaves);
+    const dim3 pgrid((unsigned)ceil_div(s.B, kPairFwdWaves) + kPlanShares), pblock(kWave * kPairFwdWaves);
     TNEG_BY_WIDTH(d, hipLaunchKernelGGL((tab->norm_p == 1 ? tneg_pair_fwd_kernel<1, NQ_> : tneg_pair_fwd_kernel<2, NQ_>), pgrid, pblock, 0, st, x, pa, dm));
     timeline_mark(bat->timeline, st, "tneg_pair_fwd_kernel");
     KGE_CHECK_LAUNCH();

@@ -47,13 +47,18 @@ class Timeline(C.Structure):
 PAIR_SUMS_VALU = 1  # kge_tables.flags
 
 
+class LossTotal(C.Structure):
+    _fields_ = [("parts", C.c_void_p), ("n", C.c_int64), ("scale", C.c_double), ("loss", C.c_void_p)]
+
+
 class Batch(C.Structure):
     _fields_ = [("batch", C.c_int64), ("h", C.c_void_p), ("r", C.c_void_p), ("t", C.c_void_p),
                 ("neg", C.c_void_p), ("chunk", C.c_int64), ("n_neg", C.c_int64),
                 ("ent_insp", C.POINTER(Inspection)), ("rel_insp", C.POINTER(Inspection)),
                 ("insp_ready", C.c_void_p), ("neg_mode", C.c_int32), ("fuse_inspection", C.c_int32),
                 ("insp_jobs", C.c_void_p), ("timeline", C.POINTER(Timeline)),
-                ("plans_ready", C.c_int32), ("reserved", C.c_int32), ("back_rows", C.c_void_p)]
+                ("plans_ready", C.c_int32), ("reserved", C.c_int32), ("back_rows", C.c_void_p),
+                ("loss_total", C.c_void_p)]
 
 
 class Saved(C.Structure):
@@ -106,6 +111,9 @@ EXPORTS = {
     "kge_margin_loss": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_float,
                                   C.c_float, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
                                   C.c_size_t, C.c_void_p]),
+    "kge_margin_loss_parts": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_float,
+                                        C.c_float, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p,
+                                        C.c_size_t, C.POINTER(LossTotal), C.c_void_p]),
     "kge_margin_loss_static": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_float,
                                          C.c_float, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "kge_score_bwd_workspace": (C.c_size_t, [C.POINTER(Tables), C.POINTER(Batch)]),

@@ -4,6 +4,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "loss_total.hpp"
 
 namespace kge {
 
@@ -11,8 +12,8 @@ constexpr int kLossWaves = 4;
 
 // Bound by its two passes over the [B, N] scores (read, gradient written), 128 bits per lane from four scores a row on.
 // A workgroup strides over the rows and leaves ONE partial loss: with one per row the single workgroup that adds them
-// up walked 16384 to 30000 doubles, 18 to 30 us; over at most kLossBlocks partials it is 2 us.
-constexpr int kLossBlocks = 1024;
+// up walked 16384 to 30000 doubles, 18 to 30 us; over at most kLossBlocks partials it is 2 us, which a training step gives to
+// the last launch of its backward pass (kge_margin_loss_parts).
 
 template <int V, bool RAG>
 __global__ __launch_bounds__(kLossWaves *kWave) void margin_rows_kernel(
@@ -56,29 +57,10 @@ __global__ __launch_bounds__(kLossWaves *kWave) void margin_rows_kernel(
     }
 }
 
-__global__ __launch_bounds__(256) void margin_total_kernel(const double *block_loss, int n, double scale,
-                                                           float *loss)
+__global__ __launch_bounds__(256) void margin_total_kernel(kge_loss_total total)
 {
     __shared__ double s[256];
-    double acc = 0.0;
-    if (n > 0) {  // uniform; an empty batch has no partial, and may have no workspace, to read
-        double v[kLossBlocks / 256];  // all loads of a thread in flight together
-#pragma unroll
-        for (int q = 0; q < kLossBlocks / 256; ++q) {
-            const int i = threadIdx.x + 256 * q;
-            v[q] = block_loss[i < n ? i : 0];
-            if (i >= n) v[q] = 0.0;
-        }
-#pragma unroll
-        for (int q = 0; q < kLossBlocks / 256; ++q) acc += v[q];
-    }
-    s[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) loss[0] = (float)(s[0] * scale);
+    loss_total_block(total, s);
 }
 
 // Scratch of kge_margin_loss_static: the partial losses, at most one double per positive.  Every
@@ -117,14 +99,13 @@ size_t kge_margin_loss_workspace(int64_t batch, int64_t n_neg)
     return batch > 0 ? sizeof(double) * (size_t)batch : 0;
 }
 
-int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n_neg, float margin,
-                    float sign, float *loss, float *dpos, float *dneg, void *workspace,
-                    size_t workspace_bytes, void *stream)
+// The row kernel, and what is left to add up behind it.
+static int launch_rows(const float *pos, const float *neg, int64_t batch, int64_t n_neg, float margin, float sign, float *loss, float *dpos,
+                       float *dneg, void *workspace, size_t workspace_bytes, kge_loss_total *total, hipStream_t st)
 {
     if (batch < 0 || n_neg < 0 || !loss) return KGE_EINVAL;
     if (batch > 0 && n_neg > 0 && (!pos || !neg)) return KGE_EINVAL;
     if (batch > 0 && (!workspace || workspace_bytes < sizeof(double) * (size_t)batch)) return KGE_EWORKSPACE;
-    hipStream_t st = as_stream(stream);
     const double count = (double)batch * (double)n_neg;
     const float inv = count > 0 ? (float)(1.0 / count) : 0.0f;
     double *rows = static_cast<double *>(workspace);
@@ -135,7 +116,28 @@ int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n
         const auto kernel = n_neg % 4 == 0 ? margin_rows_kernel<4, false> : (quad_row(n_neg) ? margin_rows_kernel<4, true> : margin_rows_kernel<1, false>);
         hipLaunchKernelGGL(kernel, grid, block, 0, st, pos, neg, batch, n_neg, margin, sign, inv, dpos, dneg, rows);
     }
-    hipLaunchKernelGGL(margin_total_kernel, dim3(1), dim3(256), 0, st, rows, blocks, count > 0 ? 1.0 / count : 0.0, loss);
+    *total = kge_loss_total{rows, blocks, count > 0 ? 1.0 / count : 0.0, loss};
+    return KGE_OK;
+}
+
+int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n_neg, float margin,
+                    float sign, float *loss, float *dpos, float *dneg, void *workspace,
+                    size_t workspace_bytes, void *stream)
+{
+    kge_loss_total total;
+    hipStream_t st = as_stream(stream);
+    if (const int rc = launch_rows(pos, neg, batch, n_neg, margin, sign, loss, dpos, dneg, workspace, workspace_bytes, &total, st)) return rc;
+    hipLaunchKernelGGL(margin_total_kernel, dim3(1), dim3(256), 0, st, total);
+    KGE_CHECK_LAUNCH();
+    return KGE_OK;
+}
+
+int kge_margin_loss_parts(const float *pos, const float *neg, int64_t batch, int64_t n_neg, float margin,
+                          float sign, float *loss, float *dpos, float *dneg, void *workspace,
+                          size_t workspace_bytes, kge_loss_total *total, void *stream)
+{
+    if (!total || batch < 1) return KGE_EINVAL;
+    if (const int rc = launch_rows(pos, neg, batch, n_neg, margin, sign, loss, dpos, dneg, workspace, workspace_bytes, total, as_stream(stream))) return rc;
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

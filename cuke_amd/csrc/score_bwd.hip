@@ -1298,7 +1298,7 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
         jobs[0].more = reinterpret_cast<const float *>(ws + p.off_more), jobs[0].more_planes = p.pairs.splits - 1;
         jobs[0].more_from = 2 * B, jobs[0].more_stride = p.nn * d;
     }
-    return launch_seg_reduce_jobs(jobs, model == KGE_TRANSH ? 3 : 2, st, bat->timeline);
+    return launch_seg_reduce_jobs(jobs, model == KGE_TRANSH ? 3 : 2, st, bat->timeline, nullptr, false, bat->loss_total);
 }
 
 }  // extern "C"

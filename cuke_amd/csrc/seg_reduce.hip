@@ -9,6 +9,7 @@
 // Level 2: the block in which a long run STARTS adds that run's slot-1 partial and the slot-0
 // partials of the following blocks (four waves share the blocks, combined through LDS).
 // The summation order is fixed by the sorted order, so results are deterministic.
+#include "loss_total.hpp"
 #include "seg_reduce.hpp"
 
 namespace kge {
@@ -52,9 +53,13 @@ __global__ __launch_bounds__(256) void seg_reduce_l1(SegArgs3 jobs, SumRider rid
 // One workgroup per (block, chunk of 64 V columns): the column chunks of a wide row are independent
 // chains of round trips and run side by side (nch = chunks of the widest job of the launch).
 template <int V>
-__global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, SumRider rider)
+__global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, SumRider rider, kge_loss_total loss)
 {
-    __shared__ float s_part[4][kWave * 4];
+    __shared__ __align__(8) float s_part[4][kWave * 4];
+    if (loss.loss && blockIdx.x == gridDim.x - 1) {  // (past every job's last block; beside them it takes no time: a launch of its own 2 us)
+        if (blockIdx.y == 0) loss_total_block(loss, reinterpret_cast<double *>(&s_part[0][0]));
+        return;
+    }
     if (rider.max_sums > 0 && blockIdx.y == gridDim.y - 1) {  // (when level 1 rode in the launch the sums depend on)
         sum_rider_body(rider);
         return;
@@ -153,14 +158,16 @@ SegL1Rider plan_seg_l1_rider(const SegJob *jobs, int n_jobs)
 }
 
 int launch_seg_reduce_jobs(const SegJob *jobs, int n_jobs, hipStream_t st, kge_timeline *timeline, const SumRider *rider,
-                           bool level1_rode)
+                           bool level1_rode, const kge_loss_total *loss)
 {
+    if (loss && (!loss->loss || loss->n < 1 || loss->n > kLossBlocks || !loss->parts)) return KGE_EINVAL;
+    const kge_loss_total total = loss ? *loss : kge_loss_total{};
     const SumRider rd = rider && rider->max_sums > 0 ? *rider : SumRider{};
     if (rd.max_sums > 0 && (rd.row_floats % 4 != 0 || !aligned16(rd.part) || !aligned16(rd.out))) return KGE_EINVAL;
     SegL1Rider pl{};
     int64_t max_blocks = 0, max_nch = 1;
     const int m = plan_jobs(jobs, n_jobs, &pl, &max_blocks, &max_nch);
-    if (m == 0 && rd.max_sums == 0) return KGE_OK;
+    if (m == 0 && rd.max_sums == 0 && !loss) return KGE_OK;
     const SegArgs3 &args = pl.jobs;
     const bool v4 = pl.v4 != 0;
     const SumRider none{};
@@ -172,20 +179,20 @@ int launch_seg_reduce_jobs(const SegJob *jobs, int n_jobs, hipStream_t st, kge_t
     int64_t g2x = max_blocks * max_nch;
     if (level1_rode && rd.max_sums > 0 && g2x < kRiderBlocks) g2x = kRiderBlocks;
     const bool r1 = !level1_rode && rd.max_sums > 0, r2 = level1_rode && rd.max_sums > 0;
-    const dim3 g1((unsigned)g1x, (unsigned)(m + (r1 ? 1 : 0))), g2((unsigned)g2x, (unsigned)(m + (r2 ? 1 : 0))), block(256);
-    const bool level2 = m > 0 || r2;
+    const dim3 g1((unsigned)g1x, (unsigned)(m + (r1 ? 1 : 0))), g2((unsigned)(g2x + (loss ? 1 : 0)), (unsigned)(m + (r2 ? 1 : 0) > 0 ? m + (r2 ? 1 : 0) : 1)), block(256);
+    const bool level1 = !level1_rode && (m > 0 || r1), level2 = m > 0 || r2 || loss;
     if (v4) {
-        if (!level1_rode) {
+        if (level1) {
             hipLaunchKernelGGL(seg_reduce_l1<4>, g1, block, 0, st, args, r1 ? rd : none);
             timeline_mark(timeline, st, "seg_reduce_l1");
         }
-        if (level2) hipLaunchKernelGGL(seg_reduce_l2<4>, g2, block, 0, st, args, (int)max_nch, r2 ? rd : none);
+        if (level2) hipLaunchKernelGGL(seg_reduce_l2<4>, g2, block, 0, st, args, (int)max_nch, r2 ? rd : none, total);
     } else {
-        if (!level1_rode) {
+        if (level1) {
             hipLaunchKernelGGL(seg_reduce_l1<1>, g1, block, 0, st, args, r1 ? rd : none);
             timeline_mark(timeline, st, "seg_reduce_l1");
         }
-        if (level2) hipLaunchKernelGGL(seg_reduce_l2<1>, g2, block, 0, st, args, (int)max_nch, r2 ? rd : none);
+        if (level2) hipLaunchKernelGGL(seg_reduce_l2<1>, g2, block, 0, st, args, (int)max_nch, r2 ? rd : none, total);
     }
     if (level2) timeline_mark(timeline, st, "seg_reduce_l2");
     KGE_CHECK_LAUNCH();

@@ -74,9 +74,10 @@ struct SegL1Rider {
 SegL1Rider plan_seg_l1_rider(const SegJob *jobs, int n_jobs);
 
 // Up to three jobs share the same two launches.  level1_rode: the level-1 pass of exactly these jobs has run as a
-// SegL1Rider; only level 2 is launched, and it carries the rider's sums.
+// SegL1Rider; only level 2 is launched, and it carries the rider's sums.  loss (optional): a batch's loss, added up by one more
+// workgroup of level 2.
 int launch_seg_reduce_jobs(const SegJob *jobs, int n_jobs, hipStream_t st, kge_timeline *timeline = nullptr,
-                           const SumRider *rider = nullptr, bool level1_rode = false);
+                           const SumRider *rider = nullptr, bool level1_rode = false, const kge_loss_total *loss = nullptr);
 
 #ifdef __HIPCC__
 // Level 1 for wave `w` of job `a` (a wave owns kSegL consecutive sorted positions and one chunk of 64 V columns).

@@ -17,14 +17,21 @@ static int step_body(const kge_tables *tab, kge_batch *bat, const kge_step_buffe
 {
     int rc = kge_score_fwd(tab, bat, buf->pos, buf->neg, buf->side_pos, buf->side_neg, buf->residual, fws, fws_bytes, stream);
     if (rc) return rc;
-    if (buf->loss) {
+    kge_loss_total total;
+    kge_batch own = *bat;  // (its loss is added up behind the backward pass)
+    if (buf->loss && own.batch < 1) {
         if ((rc = kge_margin_loss(buf->pos, buf->neg, bat->batch, bat->n_neg, buf->margin, buf->sign, buf->loss, buf->dpos, buf->dneg,
                                   buf->loss_workspace, buf->loss_workspace_bytes, stream)))
             return rc;
+    } else if (buf->loss) {
+        if ((rc = kge_margin_loss_parts(buf->pos, buf->neg, bat->batch, bat->n_neg, buf->margin, buf->sign, buf->loss, buf->dpos, buf->dneg,
+                                        buf->loss_workspace, buf->loss_workspace_bytes, &total, stream)))
+            return rc;
+        own.loss_total = &total;
     }
     kge_saved saved{buf->pos, buf->neg, buf->side_pos, buf->side_neg, buf->residual, nullptr, 0, bat->back_rows};
     if (tab->model == KGE_TRANSR || tab->model == KGE_RESCAL) saved.fwd_workspace = fws, saved.fwd_workspace_bytes = fws_bytes;
-    return kge_score_bwd(tab, bat, &saved, buf->dpos, buf->dneg, &buf->grads, buf->bwd_workspace, buf->bwd_workspace_bytes, stream);
+    return kge_score_bwd(tab, &own, &saved, buf->dpos, buf->dneg, &buf->grads, buf->bwd_workspace, buf->bwd_workspace_bytes, stream);
 }
 
 extern "C" int kge_train_step(const kge_tables *tab, kge_step_batch *cur, const kge_step_buffers *buf, int fused, void *stream,

@@ -2130,7 +2130,7 @@ int launch_rescal_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
         return KGE_ELAUNCH;
     const SegJob jobs[1] = {{occ, bat->ent_insp, d, grads->ent_rows, reinterpret_cast<float *>(ws + p.off_part_e), false}};
     const SumRider finish = dm_finish_rider(da, p.dsplit);
-    return launch_seg_reduce_jobs(jobs, 1, st, bat->timeline, &finish);
+    return launch_seg_reduce_jobs(jobs, 1, st, bat->timeline, &finish, false, bat->loss_total);
 }
 
 int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *saved, const float *dpos,
@@ -2218,7 +2218,7 @@ int launch_transr_bwd(const kge_tables *tab, const kge_batch *bat, const kge_sav
     timeline_mark(bat->timeline, st, "transr_dm_kernel");
     KGE_CHECK_LAUNCH();
     const SumRider finish = dm_finish_rider(da, p.dsplit);
-    return launch_seg_reduce_jobs(jobs, n_jobs, st, bat->timeline, &finish, ride);
+    return launch_seg_reduce_jobs(jobs, n_jobs, st, bat->timeline, &finish, ride, bat->loss_total);
 }
 
 #include "transr_neg.hpp"

@@ -759,5 +759,5 @@ int launch_transr_neg_bwd(const kge_tables *tab, const kge_batch *bat, const kge
     const SegJob jobs[2] = {{occ, bat->ent_insp, d, grads->ent_rows, reinterpret_cast<float *>(ws + l.part_e), false},
                             {qr, ri, d, grads->rel_rows, reinterpret_cast<float *>(ws + l.part_r), false}};
     const SumRider finish = dm_finish_rider(da, s.plans.dsplit);  // the split groups' partial matrices
-    return launch_seg_reduce_jobs(jobs, 2, st, bat->timeline, &finish);
+    return launch_seg_reduce_jobs(jobs, 2, st, bat->timeline, &finish, false, bat->loss_total);
 }

@@ -931,6 +931,26 @@ class TrainStep:
                                               _ptr(self._ws_l), self._ws_l.numel(), st), "kge_margin_loss")
             self._mark("margin_loss", st)
 
+    def _loss_and_backward(self, st):
+        """loss_grad() and backward().  Where neither is replaced, the loss's last sum rides in backward's last launch: one launch
+        less on the chain (DistMult 4096 x 256, step with the optimizer: 74.6 -> 72.6 us)."""
+        cls, own = type(self), self.__dict__
+        if self.loss_kind != "margin" or self.B < 1 or cls.loss_grad is not TrainStep.loss_grad or \
+                cls.backward is not TrainStep.backward or "loss_grad" in own or "backward" in own:
+            self.loss_grad(st)
+            self.backward(st)
+            return
+        total = _lib.LossTotal()
+        _lib.check(self.L.kge_margin_loss_parts(_ptr(self.pos), _ptr(self.neg), self.B, self.N, self.margin, self.sign,
+                                                _ptr(self.loss), _ptr(self.dpos), _ptr(self.dneg), _ptr(self._ws_l),
+                                                self._ws_l.numel(), C.byref(total), st), "kge_margin_loss_parts")
+        self._mark("margin_loss", st)
+        self.bat.loss_total = C.addressof(total)
+        try:
+            self.backward(st)
+        finally:
+            self.bat.loss_total = None
+
     def backward(self, st):
         _lib.check(self.L.kge_score_bwd(C.byref(self.m._tab), C.byref(self.bat), C.byref(self.saved),
                                         _ptr(self.dpos), _ptr(self.dneg), C.byref(self.grads), _ptr(self._ws_b),
@@ -1067,8 +1087,7 @@ class TrainStep:
                     _lib.check(self.L.kge_inspect_batch(C.byref(self._jobs[1]), 1, st), "kge_inspect_batch(relations)")
                     self._mark("inspect(relations)", st)
                 self.forward(st)
-                self.loss_grad(st)
-                self.backward(st)
+                self._loss_and_backward(st)
             finally:
                 bat.fuse_inspection = 0
             self._record_done(main)
@@ -1080,8 +1099,7 @@ class TrainStep:
                 self._mark("inspect", st)
             self.forward(st, backward)
             if backward:
-                self.loss_grad(st)
-                self.backward(st)
+                self._loss_and_backward(st)
             return
         if pipeline:
             if not self._staged:
@@ -1098,8 +1116,7 @@ class TrainStep:
                 main.wait_event(cur.insp_event)
                 cur.bat.insp_ready = None
                 self.forward(st)
-                self.loss_grad(st)
-                self.backward(st)
+                self._loss_and_backward(st)
                 self._record_done(main, pipeline)
                 return
             elif self.needs_rel_groups:
@@ -1118,8 +1135,7 @@ class TrainStep:
             cur.insp_event.record(side)
         cur.bat.insp_ready = cur.insp_event.cuda_event
         self.forward(st)
-        self.loss_grad(st)
-        self.backward(st)
+        self._loss_and_backward(st)
         self._record_done(main, pipeline)
 
     def _record_done(self, main, force=False):
@@ -1210,8 +1226,7 @@ class TrainStep:
             _lib.check(self.L.kge_inspect_batch(C.byref(self._jobs[1]), 1, st), "kge_inspect_batch(relations)")
         self.forward(st, backward)
         if backward:
-            self.loss_grad(st)
-            self.backward(st)
+            self._loss_and_backward(st)
         main.wait_stream(side)                                   # join
 
     # ---- the staged issue from native code: one library call per step ----

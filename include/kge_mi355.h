@@ -130,6 +130,15 @@ typedef struct kge_inspection {
 
 enum { KGE_NEG_TAIL = 0, KGE_NEG_HEAD = 1 };
 
+/* A margin loss whose partial sums are still to be added up: *loss = scale * sum of parts[0..n), n at most 1024.  Filled by
+   kge_margin_loss_parts, finished by the kge_score_bwd call whose kge_batch.loss_total points to it. */
+typedef struct kge_loss_total {
+    const double *parts; /* in the loss call's workspace */
+    int64_t n;
+    double scale;
+    float *loss;
+} kge_loss_total;
+
 /* One batch of triples.  neg == NULL: positives only. */
 typedef struct kge_batch {
     int64_t batch;       /* B positives */
@@ -190,6 +199,9 @@ typedef struct kge_batch {
        residual rows must be requested in the same call.  No counterpart in the reference, which has no
        executed backward pass (apps/kge/kge.py:393-515). */
     float *back_rows;
+    /* Optional, read by kge_score_bwd alone: the loss of this batch that kge_margin_loss_parts left in parts, on the same
+       stream.  The last launch of kge_score_bwd adds it up, which takes a launch of its own off the chain of a step. */
+    const kge_loss_total *loss_total;
 } kge_batch;
 
 /* Forward outputs that backward consumes. */
@@ -351,6 +363,11 @@ size_t kge_margin_loss_workspace(int64_t batch, int64_t n_neg);
 int kge_margin_loss(const float *pos, const float *neg, int64_t batch, int64_t n_neg,
                     float margin, float sign, float *loss, float *dpos, float *dneg,
                     void *workspace, size_t workspace_bytes, void *stream);
+/* kge_margin_loss without its last sum: *total says what is left to do, and the workspace holds it until that is done.  loss[1] is
+ * written by the kge_score_bwd call that is handed total (kge_batch.loss_total).  batch >= 1. */
+int kge_margin_loss_parts(const float *pos, const float *neg, int64_t batch, int64_t n_neg,
+                          float margin, float sign, float *loss, float *dpos, float *dneg,
+                          void *workspace, size_t workspace_bytes, kge_loss_total *total, void *stream);
 
 /*
  * kge_margin_loss for callers that cannot allocate device memory (code under HIP graph capture,

@@ -73,3 +73,32 @@ def test_inspect_ids_that_follow_each_other(oracle, n, n_rows):
     check(oracle, [ids % n_rows], n_rows)
     check(oracle, [(n_rows - 1 - ids % n_rows)], n_rows)
     check(oracle, [(ids * 64) % n_rows, (ids * 2048) % n_rows], n_rows)
+
+
+@pytest.mark.parametrize("n,n_rows", [((5000, 5001), (3000, 64)), ((8192, 16384), (65, 14951)), ((4097, 60000), (2048, 5000)),
+                                      ((0, 9000), (1345, 4000)), ((6000, 6000), (2047, 1 << 23))])
+def test_a_narrow_set_beside_a_wide_one(oracle, n, n_rows):
+    """Two sets in one batch of launches: a set of one digit pass takes two beside a set of two or three (from 65 rows on)."""
+    import ctypes as C
+
+    from cuke_amd import _lib
+    from cuke_amd.kge import inspect
+    rng = np.random.default_rng(n[0] + n_rows[0])
+    ids = [rng.integers(0, r, k, dtype=np.int64) for k, r in zip(n, n_rows)]
+    dev = [torch.from_numpy(x).cuda() for x in ids]
+    got = [inspect([x], r) for x, r in zip(dev, n_rows)]
+    L, jobs, ws = _lib.lib(), (_lib.InspectJob * 2)(), []
+    for j, g, x, r in zip(jobs, got, dev, n_rows):
+        for a in (g.num_unique_dev, g.unique_ids, g.seg_offsets, g.perm, g.inverse, g.sorted_seg):
+            a.fill_(-1)
+        size = int(L.kge_inspect_workspace(x.numel(), r))
+        ws.append(torch.empty(max(size, 1), dtype=torch.uint8, device="cuda"))
+        j.parts[0], j.part_len[0], j.n_parts, j.n_rows, j.out = x.data_ptr(), x.numel(), 1, r, g._c
+        j.workspace, j.workspace_bytes = ws[-1].data_ptr(), size
+    assert L.kge_inspect_batch(jobs, 2, C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    for g, x in zip(got, ids):
+        ref, k, u = oracle.inspect(x), x.size, int(g.num_unique_dev.item())
+        assert u == ref.unique_ids.shape[0]
+        for a, want in ((g.unique_ids[:u], ref.unique_ids), (g.seg_offsets[:u + 1], ref.seg_offsets), (g.perm[:k], ref.perm),
+                        (g.inverse[:k], ref.inverse), (g.sorted_seg[:k], ref.inverse[ref.perm])):
+            assert np.array_equal(a.cpu().numpy().astype(np.int64), want)

@@ -133,27 +133,24 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
             }
         }
     }
+    uint32_t dg[kKeysPerThread];
+    bool ok[kKeysPerThread];
+    uint64_t peers[kKeysPerThread];
+#pragma unroll
+    for (int j = 0; j < kKeysPerThread; ++j) ok[j] = wbase + j * kWave + lane < n, dg[j] = (key[j] >> shift) & mask;
+    same_digit(dg, ok, digit_bits, peers);
 #pragma unroll
     for (int j = 0; j < kKeysPerThread; ++j) {
-        const int64_t i = wbase + j * kWave + lane;
-        const bool ok = i < n;
-        const uint32_t dg = (key[j] >> shift) & mask;
-        uint64_t peers = __ballot(ok);
-        for (int bit = 0; bit < digit_bits; ++bit) {
-            const bool one = (dg >> bit) & 1u;
-            const uint64_t m = __ballot(one);
-            peers &= one ? m : ~m;
-        }
         // lanes with !ok fall out: their `peers` may be anything but they never write
-        const int leader = __ffsll((unsigned long long)peers) - 1;
-        const uint32_t cnt = __popcll(peers);
+        const int leader = __ffsll((unsigned long long)peers[j]) - 1;
+        const uint32_t cnt = __popcll(peers[j]);
         uint32_t old = 0;
-        if (ok && lane == leader) {
-            old = s_cnt[wave][dg];
-            s_cnt[wave][dg] = old + cnt;
+        if (ok[j] && lane == leader) {
+            old = s_cnt[wave][dg[j]];
+            s_cnt[wave][dg[j]] = old + cnt;
         }
         old = __shfl(old, leader < 0 ? 0 : leader, kWave);
-        lrank[j] = old + __popcll(peers & lt_mask);
+        lrank[j] = old + __popcll(peers[j] & lt_mask);
         __builtin_amdgcn_wave_barrier();  // keep the rounds' LDS counter updates in order
     }
     __syncthreads();
@@ -172,8 +169,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
     for (int j = 0; j < kKeysPerThread; ++j) {
         const int64_t i = wbase + j * kWave + lane;
         if (i < n) {
-            const uint32_t dg = (key[j] >> shift) & mask;
-            const uint32_t pos = s_cnt[wave][dg] + lrank[j];
+            const uint32_t pos = s_cnt[wave][dg[j]] + lrank[j];
             keys_out[pos] = key[j];
             vals_out[pos] = val[j];
         }
@@ -362,26 +358,23 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
         const int shift = pass * db;
         for (int i = tid; i < cnt_at(counters); i += kSmallThreads) s_cnt[i] = 0;
         __syncthreads();
-        uint32_t rank[R];
+        uint32_t rank[R], dg[R];
+        bool ok[R];
+        uint64_t peers[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) ok[j] = at[j] < n, dg[j] = (key[j] >> shift) & mask;
+        same_digit(dg, ok, db, peers);
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            const bool ok = at[j] < n;
-            const uint32_t dg = (key[j] >> shift) & mask;
-            uint64_t peers = __ballot(ok);
-            for (int bit = 0; bit < db; ++bit) {
-                const bool one = (dg >> bit) & 1u;
-                const uint64_t mm = __ballot(one);
-                peers &= one ? mm : ~mm;
-            }
-            const int leader = __ffsll((unsigned long long)peers) - 1;
+            const int leader = __ffsll((unsigned long long)peers[j]) - 1;
             uint32_t old = 0;
-            if (ok && lane == leader) {
-                uint32_t &count = s_cnt[cnt_at(dg * kSmallWaves + wave)];
+            if (ok[j] && lane == leader) {
+                uint32_t &count = s_cnt[cnt_at(dg[j] * kSmallWaves + wave)];
                 old = count;
-                count = old + __popcll(peers);
+                count = old + __popcll(peers[j]);
             }
             old = __shfl(old, leader < 0 ? 0 : leader, kWave);
-            rank[j] = old + __popcll(peers & lt_mask);
+            rank[j] = old + __popcll(peers[j] & lt_mask);
             __builtin_amdgcn_wave_barrier();
         }
         __syncthreads();
@@ -403,7 +396,7 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
 #pragma unroll
         for (int j = 0; j < R; ++j)
             if (at[j] < n) {
-                const int to = key_at(s_cnt[cnt_at(((key[j] >> shift) & mask) * kSmallWaves + wave)] + rank[j]);
+                const int to = key_at(s_cnt[cnt_at(dg[j] * kSmallWaves + wave)] + rank[j]);
                 s_key[to] = key[j], s_val[to] = (uint16_t)val[j];
             }
         __syncthreads();
@@ -417,6 +410,8 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
     }
 
     // runs of equal keys: a thread takes R consecutive sorted positions
+    uint16_t *s_seg = reinterpret_cast<uint16_t *>(s_cnt);  // the counters are done with, and no fewer
+    static_assert(sizeof(s_cnt) >= sizeof(uint16_t) * kSmallThreads * R, "a run number per key");
     const int lo = tid * R;
     uint32_t prev = lo > 0 && lo < n ? s_key[key_at(lo - 1)] : 0, heads = 0;
     bool head[R];
@@ -440,12 +435,18 @@ __global__ __launch_bounds__(kSmallThreads) void inspect_small_kernel(MidJobs jo
                 J.out.seg_offsets[run] = i;
                 ++run;
             }
-            const int32_t seg = (int32_t)run - 1, p = s_val[key_at(i)];
-            J.out.perm[i] = p;
-            J.out.sorted_seg[i] = seg;
-            J.out.inverse[p] = seg;
+            s_key[s_val[key_at(i)]] = run - 1;  // (every thread has its keys: a scan's barriers lie between)
+            s_seg[i] = (uint16_t)(run - 1);
         }
     }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; ++j)  // (by way of LDS: stores of whole lines)
+        if (at[j] < n) {
+            J.out.perm[at[j]] = s_val[key_at(at[j])];
+            J.out.sorted_seg[at[j]] = s_seg[at[j]];
+            J.out.inverse[at[j]] = (int32_t)s_key[at[j]];
+        }
 }
 
 static void launch_small(const MidJobs &jobs, int n_jobs, int64_t max_n, hipStream_t st)

@@ -45,6 +45,30 @@ struct KeySrc {
     }
 };
 
+// The lanes of the wave whose digit is this lane's, for R digits at a time: of every bit the mask of the lanes that agree with this one.
+// Bits outside, digits inside: R chains side by side, each bit one ballot, the bit spread over a word and two three-operand
+// instructions per half.  ok: lanes that take part.
+template <int R>
+__device__ __forceinline__ void same_digit(const uint32_t (&dg)[R], const bool (&ok)[R], int bits, uint64_t (&peers)[R])
+{
+    uint32_t lo[R], hi[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const uint64_t m = __ballot(ok[j]);
+        lo[j] = (uint32_t)m, hi[j] = (uint32_t)(m >> 32);
+    }
+    for (int bit = 0; bit < bits; ++bit) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const uint32_t spread = (uint32_t)__builtin_amdgcn_sbfe((int)dg[j], bit, 1);  // all ones or none
+            const uint64_t m = __ballot(spread != 0);
+            lo[j] &= ~((uint32_t)m ^ spread), hi[j] &= ~((uint32_t)(m >> 32) ^ spread);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) peers[j] = (uint64_t)hi[j] << 32 | lo[j];
+}
+
 // exclusive scan of s[0..bins) in place (bins <= 2048, 256 threads)
 __device__ inline void block_exclusive_scan(uint32_t *s, int bins, uint32_t *wave_tot)
 {
@@ -296,26 +320,25 @@ __device__ __forceinline__ void mid_scatter_body(const MidJob &J, int pass, int 
     }
 
     const uint64_t lt_mask = lane ? (~0ull >> (kWave - lane)) : 0ull;
-    uint32_t lrank[kMidRounds];
+    uint32_t lrank[kMidRounds], dg[kMidRounds];
+    bool ok[kMidRounds];
+    uint64_t peers[kMidRounds];
 #pragma unroll
     for (int j = 0; j < kMidRounds; ++j) {
-        const int i = my0 + wave * (kMidRounds * kWave) + j * kWave + lane;
-        const bool ok = i < n;
-        const uint32_t dg = (key[j] >> shift) & mask;
-        uint64_t peers = __ballot(ok);
-        for (int bit = 0; bit < J.db; ++bit) {
-            const bool one = (dg >> bit) & 1u;
-            const uint64_t mm = __ballot(one);
-            peers &= one ? mm : ~mm;
-        }
-        const int leader = __ffsll((unsigned long long)peers) - 1;
+        ok[j] = my0 + wave * (kMidRounds * kWave) + j * kWave + lane < n;
+        dg[j] = (key[j] >> shift) & mask;
+    }
+    same_digit(dg, ok, J.db, peers);
+#pragma unroll
+    for (int j = 0; j < kMidRounds; ++j) {
+        const int leader = __ffsll((unsigned long long)peers[j]) - 1;
         uint32_t old = 0;
-        if (ok && lane == leader) {
-            old = s_cnt[wave * bins + dg];
-            s_cnt[wave * bins + dg] = old + __popcll(peers);
+        if (ok[j] && lane == leader) {
+            old = s_cnt[wave * bins + dg[j]];
+            s_cnt[wave * bins + dg[j]] = old + __popcll(peers[j]);
         }
         old = __shfl(old, leader < 0 ? 0 : leader, kWave);
-        lrank[j] = old + __popcll(peers & lt_mask);
+        lrank[j] = old + __popcll(peers[j] & lt_mask);
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
@@ -333,13 +356,12 @@ __device__ __forceinline__ void mid_scatter_body(const MidJob &J, int pass, int 
     for (int j = 0; j < kMidRounds; ++j) {
         const int i = my0 + wave * (kMidRounds * kWave) + j * kWave + lane;
         if (i < n) {
-            const uint32_t dg = (key[j] >> shift) & mask;
-            const uint32_t pos = s_cnt[wave * bins + dg] + lrank[j];
+            const uint32_t pos = s_cnt[wave * bins + dg[j]] + lrank[j];
             kout[pos] = key[j];
             vout[pos] = val[j];
             if (finish) {
-                J.out.sorted_seg[pos] = (int32_t)s_u[dg];
-                J.out.inverse[val[j]] = (int32_t)s_u[dg];
+                J.out.sorted_seg[pos] = (int32_t)s_u[dg[j]];
+                J.out.inverse[val[j]] = (int32_t)s_u[dg[j]];
             }
         }
     }
@@ -382,16 +404,22 @@ __device__ __forceinline__ void mid_dedup_body(const MidJob &J, int bx, uint32_t
     }
     before = (uint32_t)wave_sum_i((int)before);
     if (lane == 0) s_red[wave] = before;
-    // thread owns 4 consecutive sorted positions
+    // thread owns 4 consecutive sorted positions: their keys with one 128-bit load (the buffer is a whole number of quads)
+    static_assert(kMidRounds == 4, "a quad of positions per thread");
     const int lo = my0 + tid * kMidRounds;
-    uint32_t k[kMidRounds];
+    const bool whole = lo + kMidRounds <= n;
+    const uint4 kq = reinterpret_cast<const uint4 *>(keys)[lo < n ? lo >> 2 : 0];
+    const uint32_t k[kMidRounds] = {kq.x, kq.y, kq.z, kq.w};
+    typedef int32_t i4u __attribute__((ext_vector_type(4), aligned(4)));  // (the caller's arrays: dword aligned)
+    i4u pq;
+    if (whole) pq = *reinterpret_cast<const i4u *>(J.out.perm + lo);
+    else pq = i4u{J.out.perm[lo < n ? lo : 0], J.out.perm[lo + 1 < n ? lo + 1 : 0], J.out.perm[lo + 2 < n ? lo + 2 : 0], 0};
     bool head[kMidRounds];
     uint32_t mine = 0;
-    uint32_t prev = (lo > 0 && lo < n) ? keys[lo - 1] : 0;
+    uint32_t prev = keys[lo > 0 && lo < n ? lo - 1 : 0];
 #pragma unroll
     for (int j = 0; j < kMidRounds; ++j) {
         const int i = lo + j;
-        k[j] = i < n ? keys[i] : 0;
         head[j] = i < n && (i == 0 || k[j] != prev);
         prev = k[j];
         mine += head[j] ? 1 : 0;
@@ -413,6 +441,7 @@ __device__ __forceinline__ void mid_dedup_body(const MidJob &J, int bx, uint32_t
         J.out.num_unique[0] = (int32_t)(before + here);
         J.out.seg_offsets[before + here] = n;
     }
+    i4u seg{0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < kMidRounds; ++j) {
         const int i = lo + j;
@@ -422,11 +451,12 @@ __device__ __forceinline__ void mid_dedup_body(const MidJob &J, int bx, uint32_t
                 J.out.seg_offsets[run] = i;
                 ++run;
             }
-            const int32_t seg = (int32_t)run - 1;
-            J.out.sorted_seg[i] = seg;
-            J.out.inverse[J.out.perm[i]] = seg;
+            seg[j] = (int32_t)run - 1;
+            if (!whole) J.out.sorted_seg[i] = seg[j];
+            J.out.inverse[pq[j]] = seg[j];
         }
     }
+    if (whole) *reinterpret_cast<i4u *>(J.out.sorted_seg + lo) = seg;
 }
 
 

@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kSortThreads) void finalize_kernel(const uint32_t *
 // ---- small and medium inputs: the mid-path bodies as kernels of their own -------------------
 __global__ __launch_bounds__(kMidThreads) void inspect_mid_hist_kernel(MidJobs jobs)
 {
-    __shared__ uint32_t smem[mid_hist_lds_words(kMaxBins, kMidMaxPass)];
+    __shared__ uint32_t smem[mid_hist_lds_words(kMaxBins)];
     mid_hist_body(jobs.j[blockIdx.y], blockIdx.x, smem);
 }
 
@@ -294,6 +294,7 @@ __global__ __launch_bounds__(kMidThreads) void inspect_mid_dedup_kernel(MidJobs 
 //         1345       15.9 ->  6.5   16.4 ->  6.8  17.5 ->  8.8  17.4 -> 12.2  17.7 -> 13.7
 //        14951       17.6 ->  7.0   18.8 ->  7.2  21.9 ->  9.2  22.8 -> 13.1  23.0 -> 14.7
 //          1e6       21.3 ->  8.2   22.5 ->  8.6  25.6 -> 11.4  26.3 -> 16.5  26.6 -> 18.7
+//   (Both sides have become faster since: 2048 ids of 1345 rows 7.7 us, 4096 of 1345 10.4, 4096 of 14951 11.2; 8192 of 1345 by launches 16.7.)
 //   (8192 ids took 1.5 to 2 times the launches' time, 4096 ids of 50 or 237 rows 1.1 to 1.2 times.)  Ids that follow each other, 4096 of 1345
 //   rows: 19.5 us before the counters and places were skewed, by launches 16.9, now 13.4.
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / kWave;
@@ -553,7 +554,7 @@ int plan_fused_inspection(const kge_inspect_job *jobs, int n_jobs, int slot, Fus
         J.hist = reinterpret_cast<uint32_t *>(ws + p.off_hist);
         blocks[q] = (int)ceil_div(n, kMidKeys);
         const int step = slot - (kFusedSlots - 2 - J.npass);
-        const int w = step == 0 ? mid_hist_lds_words(1 << J.db, J.npass)
+        const int w = step == 0 ? mid_hist_lds_words(1 << J.db)
                                 : (step >= 1 && step <= J.npass ? mid_pass_lds_words(1 << J.db, J.npass) : 0);
         words = w > words ? w : words;
     }

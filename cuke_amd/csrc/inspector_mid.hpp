@@ -49,14 +49,11 @@ struct KeySrc {
 // Bits outside, digits inside: R chains side by side, each bit one ballot, the bit spread over a word and two three-operand
 // instructions per half.  ok: lanes that take part.
 template <int R>
-__device__ __forceinline__ void same_digit(const uint32_t (&dg)[R], const bool (&ok)[R], int bits, uint64_t (&peers)[R])
+__device__ __forceinline__ void narrow_peers(const uint32_t (&dg)[R], int bits, uint64_t (&peers)[R])
 {
     uint32_t lo[R], hi[R];
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-        const uint64_t m = __ballot(ok[j]);
-        lo[j] = (uint32_t)m, hi[j] = (uint32_t)(m >> 32);
-    }
+    for (int j = 0; j < R; ++j) lo[j] = (uint32_t)peers[j], hi[j] = (uint32_t)(peers[j] >> 32);
     for (int bit = 0; bit < bits; ++bit) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
@@ -67,6 +64,13 @@ __device__ __forceinline__ void same_digit(const uint32_t (&dg)[R], const bool (
     }
 #pragma unroll
     for (int j = 0; j < R; ++j) peers[j] = (uint64_t)hi[j] << 32 | lo[j];
+}
+template <int R>
+__device__ __forceinline__ void same_digit(const uint32_t (&dg)[R], const bool (&ok)[R], int bits, uint64_t (&peers)[R])
+{
+#pragma unroll
+    for (int j = 0; j < R; ++j) peers[j] = __ballot(ok[j]);
+    narrow_peers(dg, bits, peers);
 }
 
 // exclusive scan of s[0..bins) in place (bins <= 2048, 256 threads)
@@ -101,14 +105,11 @@ __device__ inline void block_exclusive_scan(uint32_t *s, int bins, uint32_t *wav
 
 // ---- small and medium inputs (up to 65536 ids) ---------------------------------------------------
 // A workgroup owns 1024 consecutive keys.  The steps of a job are
-//   histogram: every workgroup writes the digit histograms of its own keys, one per pass, to the
-//              job's workspace (a histogram does not depend on key order, so all passes' bin totals
-//              are known before anything is sorted);
-//   scatter p: bin starts = column sums of pass p's histograms; the same-digit keys in front of the
-//              workgroup come from those histograms too in the first pass, and from a recount of
-//              the sorted keys in front of it in a later pass; the workgroup's own keys are ranked
-//              stably with wave ballots and scattered.  A job with a single pass is finished here
-//              (every non-empty bin is one distinct id);
+//   histogram: every workgroup writes the first digit's histogram of its own keys to the job's workspace and clears its rows of the later
+//              digits' tables;
+//   scatter p: bin starts = column sums of pass p's histograms, and the same-digit keys in front of the workgroup come from those too; the
+//              workgroup's own keys are ranked stably with wave ballots and scattered, and counted into the next digit's histograms by
+//              the block that they move to.  A job with a single pass is finished here (every non-empty bin is one distinct id);
 //   dedup:     run detection over the sorted keys.
 // No step depends on another workgroup of the same launch, only on the launch before, so the steps
 // run as launches of their own (several index sets sharing them) or as extra workgroups in front
@@ -163,9 +164,8 @@ __device__ __forceinline__ uint32_t *mid_hist(const MidJob &J, int pass)
     return J.hist + (size_t)pass * mid_blocks(J.n) * (1u << J.db);
 }
 
-// Step 0 of a job: the digit histograms of this workgroup's own keys, one per pass (a histogram
-// does not depend on the order of the keys, so all passes' totals are known before any sorting).
-__host__ __device__ constexpr int mid_hist_lds_words(int bins, int npass) { return bins * npass; }
+// Step 0 of a job: the first digit's histogram of this workgroup's own keys.
+__host__ __device__ constexpr int mid_hist_lds_words(int bins) { return bins; }
 
 __device__ __forceinline__ void mid_hist_body(const MidJob &J, int bx, uint32_t *smem)
 {
@@ -183,24 +183,23 @@ __device__ __forceinline__ void mid_hist_body(const MidJob &J, int bx, uint32_t 
         const int i = my0 + j * kMidThreads + tid;
         key[j] = src(i < n ? i : n - 1);
     }
-    for (int i = tid; i < bins * J.npass; i += kMidThreads) smem[i] = 0;
+    for (int i = tid; i < bins; i += kMidThreads) smem[i] = 0;
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kMidRounds; ++j)
-        if (my0 + j * kMidThreads + tid < n)
-            for (int p = 0; p < J.npass; ++p) atomicAdd(&smem[p * bins + ((key[j] >> (p * J.db)) & mask)], 1u);
+        if (my0 + j * kMidThreads + tid < n) atomicAdd(&smem[key[j] & mask], 1u);
     __syncthreads();
     const size_t row = (size_t)bx * bins;
-    for (int p = 0; p < J.npass; ++p)
-        for (int i = tid; i < bins; i += kMidThreads) mid_hist(J, p)[row + i] = smem[p * bins + i];
+    for (int i = tid; i < bins; i += kMidThreads) mid_hist(J, 0)[row + i] = smem[i];
+    for (int p = 1; p < J.npass; ++p)
+        for (int i = tid; i < bins; i += kMidThreads) mid_hist(J, p)[row + i] = 0;
 }
 
-// One digit pass of job J for the keys [bx * kMidKeys, (bx + 1) * kMidKeys).  Bin starts come from
-// the column sums of the per-workgroup histograms (a few coalesced loads per thread).  The number
-// of same-digit keys in front of this workgroup comes from the same histograms in the first pass
-// (the keys are still in input order, workgroup by workgroup); in a later pass the workgroup counts
-// the digits of the sorted keys in front of it itself (batched loads, LDS atomics).  Its own keys
-// are ranked stably with wave ballots and scattered.
+// One digit pass of job J for the keys [bx * kMidKeys, (bx + 1) * kMidKeys).  Bin starts and the number of same-digit keys in front of
+// this workgroup come from the column sums of the per-workgroup histograms (a few coalesced loads per thread), which the step before
+// has left for the order that the keys are in now.  Its own keys are ranked stably with wave ballots and scattered.  (A later pass used
+// to count the digits of all the keys in front of it: 65000 ids of 14951 rows 42.9 -> 37.5 us, one id 65000 times 88.7 -> 34.2, 16384
+// ids 24.0 -> 23.7, one id 16384 times 34.6 -> 21.0.)
 template <bool FIRST>
 __device__ __forceinline__ void mid_scatter_body(const MidJob &J, int pass, int bx, uint32_t *smem)
 {
@@ -265,32 +264,6 @@ __device__ __forceinline__ void mid_scatter_body(const MidJob &J, int pass, int 
         for (int w = 0; w < kMidWaves; ++w) reinterpret_cast<uint4 *>(s_cnt + w * bins)[q] = make_uint4(0, 0, 0, 0);
     }
     __syncthreads();
-    if (pass > 0) {  // s_bef held the histogram-order count, which only the first pass can use
-        for (int i = tid; i < bins; i += kMidThreads) s_bef[i] = 0;
-        __syncthreads();
-        // (my0 is a multiple of 1024 and the key buffers are 256-byte aligned: whole groups of four
-        // keys per 128-bit load, sixteen groups per thread in flight)
-        constexpr int kBatch = 16;
-        const uint4 *kin4 = reinterpret_cast<const uint4 *>(kin);
-        const int groups = my0 >> 2;
-        for (int g0 = 0; g0 < groups; g0 += kBatch * kMidThreads) {
-            uint4 kb[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                const int g = g0 + u * kMidThreads + tid;
-                kb[u] = kin4[g < groups ? g : groups - 1];  // clamped: unconditional loads, masked below
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                if (g0 + u * kMidThreads + tid < groups) {
-                    atomicAdd(&s_bef[(kb[u].x >> shift) & mask], 1u);
-                    atomicAdd(&s_bef[(kb[u].y >> shift) & mask], 1u);
-                    atomicAdd(&s_bef[(kb[u].z >> shift) & mask], 1u);
-                    atomicAdd(&s_bef[(kb[u].w >> shift) & mask], 1u);
-                }
-        }
-        __syncthreads();
-    }
     // A job with a single pass sorts by the whole key, so every non-empty bin is one distinct id:
     // the run structure falls out of the histogram and no dedup step is needed.
     const bool finish = J.npass == 1;
@@ -352,18 +325,31 @@ __device__ __forceinline__ void mid_scatter_body(const MidJob &J, int pass, int 
         }
     }
     __syncthreads();
+    uint32_t pos[kMidRounds];
 #pragma unroll
-    for (int j = 0; j < kMidRounds; ++j) {
-        const int i = my0 + wave * (kMidRounds * kWave) + j * kWave + lane;
-        if (i < n) {
-            const uint32_t pos = s_cnt[wave * bins + dg[j]] + lrank[j];
-            kout[pos] = key[j];
-            vout[pos] = val[j];
+    for (int j = 0; j < kMidRounds; ++j) pos[j] = s_cnt[wave * bins + dg[j]] + lrank[j];
+#pragma unroll
+    for (int j = 0; j < kMidRounds; ++j)
+        if (ok[j]) {
+            kout[pos[j]] = key[j];
+            vout[pos[j]] = val[j];
             if (finish) {
-                J.out.sorted_seg[pos] = (int32_t)s_u[dg[j]];
+                J.out.sorted_seg[pos[j]] = (int32_t)s_u[dg[j]];
                 J.out.inverse[val[j]] = (int32_t)s_u[dg[j]];
             }
         }
+    if (pass + 1 < J.npass) {  // uniform
+        // The next pass's histograms, by the block a key has moved to: an atomic per cell and round.  (An atomic per key took 10 us longer on
+        // skewed ids.)  Lanes of one digit move to consecutive places, so to one block or to two that follow each other.
+        uint32_t *next = mid_hist(J, pass + 1);
+        uint32_t nd[kMidRounds], place[kMidRounds];
+#pragma unroll
+        for (int j = 0; j < kMidRounds; ++j) nd[j] = (key[j] >> (shift + J.db)) & mask, place[j] = pos[j] / kMidKeys;
+        narrow_peers(nd, J.db, peers);
+        narrow_peers(place, 1, peers);
+#pragma unroll
+        for (int j = 0; j < kMidRounds; ++j)
+            if (ok[j] && lane == __ffsll((unsigned long long)peers[j]) - 1) atomicAdd(&next[(size_t)place[j] * bins + nd[j]], (uint32_t)__popcll(peers[j]));
     }
 }
 

@@ -1,4 +1,4 @@
-// Gradient tiles that evaluate every pair once (TransE, RotatE): included by score_bwd.hip.
+// Gradient tiles that evaluate every pair once (TransE, RotatE, TransH L1): included by score_bwd.hip.
 //
 // A workgroup owns TO negatives x 32 columns of one chunk and walks the chunk's positives (a range of them, `splits` workgroups
 // share them), staged kKL at a time with their coefficients.  A thread holds four columns of RO negatives; per positive it adds
@@ -23,10 +23,14 @@ constexpr int kPairOwners = kPairWaves * 8 * kPairRO;  // negatives of a workgro
 
 template <int MODEL>
 struct PairShape {
-    static constexpr int NPL = MODEL == KGE_ROTATE ? 2 : 1;  // planes of a row and of its sums
+    static constexpr bool kTH = MODEL == KGE_TRANSH;
+    static constexpr int NPN = MODEL == KGE_ROTATE ? 2 : 1;  // planes of a negative's row and of its sums
+    static constexpr int NPL = kTH ? 2 : NPN;                // planes of a positive's (TransH: the query and w) and of its sums
+    static constexpr int NC = kTH ? 3 : 1;                   // coefficients of a pair
     static constexpr int PG = kPairOwners + 4;
-    static constexpr int kRowFloats = NPL * kPairKL * kPairPitch, kCoefFloats = kPairKL * PG;
-    static constexpr int kLdsFloats = kRowFloats + kCoefFloats + kPairKL * kPairWaves * NPL * kPairCols;
+    static constexpr int kRowFloats = NPL * kPairKL * kPairPitch, kCoefFloats = NC * kPairKL * PG;
+    static constexpr int kSumFloats = kPairKL * kPairWaves * NPL * kPairCols;
+    static constexpr int kLdsFloats = kRowFloats + kCoefFloats + kSumFloats + (kTH ? kPairKL : 0);
 };
 
 struct PairPlan {
@@ -38,7 +42,7 @@ struct PairPlan {
 
 struct PairArgs {
     PairPlan plan;
-    float *g0;                 // [tiles][B, d]
+    float *g0, *g1;            // [tiles][B, d]; g1: TransH, the sums for w
     int64_t gplane;            // B * d
     float *occ_neg, *more_neg; // plane 0 of the negatives' rows [n_chunks * N, d]; planes 1 ... splits - 1
     int64_t nplane;            // n_chunks * N * d
@@ -64,19 +68,20 @@ __device__ __forceinline__ float add_ror8(float v)  // v + the value eight lanes
 //   Gradient tiles, us, both orientations -> every pair once:  RotatE 1024 x 256 negatives x 1000 72 -> 55, 8192 x 256 x 500 in chunks of 1024
 //   295 -> 184, 4278 x 300 x 426 in chunks of 31 245 -> 128;  TransE L1 30000 x 200 x 150 230 -> 158, 4096 x 1024 x 150 136 -> 87.
 template <int MODEL, int P, int PH>
-__global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) void bwd_pair_kernel(TileArgs a, PairArgs pa, FusedInsp fi)
+__global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_TRANSE ? 4 : 3) void bwd_pair_kernel(TileArgs a, PairArgs pa, FusedInsp fi)
 {
     using S = PairShape<MODEL>;
-    constexpr bool kRot = MODEL == KGE_ROTATE, kSc = !kRot && P == 1, kL2 = !kRot && P == 2;
-    constexpr int RO = kPairRO, WAVES = kPairWaves, NPL = S::NPL, PG = S::PG, KL = kPairKL, TH = WAVES * kWave;
+    constexpr bool kRot = MODEL == KGE_ROTATE, kTH = S::kTH, kSc = !kRot && P == 1, kL2 = !kRot && P == 2;
+    static_assert(!kTH || P == 1, "TransH: L1 only");
+    constexpr int RO = kPairRO, WAVES = kPairWaves, NPL = S::NPL, NPN = S::NPN, NC = S::NC, PG = S::PG, KL = kPairKL, TH = WAVES * kWave;
     constexpr int wo = WAVES / PH, TO = wo * 8 * RO;   // waves of different negatives; negatives of the tile
     constexpr int CPT = (KL * TO / 4 + TH - 1) / TH;   // coefficient quads per thread
-    constexpr int NRAW = 2;
+    constexpr int NRAW = query_raw_count<MODEL>();
     extern __shared__ __align__(16) char dyn_smem[];
     if (fused_insp_block(fi, reinterpret_cast<uint32_t *>(dyn_smem))) return;
     float(*sL)[KL][kPairPitch] = reinterpret_cast<float(*)[KL][kPairPitch]>(dyn_smem);
-    float(*sG)[PG] = reinterpret_cast<float(*)[PG]>(dyn_smem + sizeof(float) * S::kRowFloats);
-    float *sR = reinterpret_cast<float *>(dyn_smem) + S::kRowFloats + S::kCoefFloats;
+    float(*sG)[KL][PG] = reinterpret_cast<float(*)[KL][PG]>(dyn_smem + sizeof(float) * S::kRowFloats);
+    float *sR = reinterpret_cast<float *>(dyn_smem) + S::kRowFloats + S::kCoefFloats, *sA = sR + S::kSumFloats;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), own_wave = wave % wo, phase = wave / wo;
     const int tx = lane & 7, ty = own_wave * 8 + (lane >> 3);
@@ -90,12 +95,12 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
     const int lcol = tile_x * kPairCols + tx * 4, col = min(lcol, klen - 4), skip = lcol - col;
 
     // ---- negatives: registers ------------------------------------------------------------
-    float4 own[NPL][RO], acc[NPL][RO];
+    float4 own[NPN][RO], acc[NPN][RO];
 #pragma unroll
     for (int o = 0; o < RO; ++o) {
         const float *pt = a.ent + a.neg[(int64_t)c * a.N + min(k0 + ty * RO + o, a.N - 1)] * (int64_t)d;
 #pragma unroll
-        for (int q = 0; q < NPL; ++q) {
+        for (int q = 0; q < NPN; ++q) {
             own[q][o] = load_quad(pt + q * half + col);
             acc[q][o] = zero4();
         }
@@ -103,7 +108,7 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
 #pragma unroll
     for (int o = 0; o < RO; ++o)
 #pragma unroll
-        for (int q = 0; q < NPL; ++q) {
+        for (int q = 0; q < NPN; ++q) {
             if (k0 + ty * RO + o >= a.N) own[q][o] = zero4();
             if constexpr (kSc) own[q][o] = scale4(own[q][o], kSgnScale);
         }
@@ -112,7 +117,8 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
     const int srow = tid >> 3;
     const bool stager = tid < KL * 8;
     int64_t ih = 0, ir = 0;
-    float4 rraw[NRAW], craw[CPT], sraw[kL2 ? CPT : 1];
+    float4 rraw[NRAW], craw[CPT], sraw[kL2 ? CPT : 1], c1raw[kTH ? CPT : 1], c2raw[kTH ? CPT : 1];
+    float ral = 0.0f;  // TransH: w . x of the staged positive
     auto load_idx = [&](int l0) {
         if (kRot || !stager) return;
         const int64_t b = (int64_t)c * a.C + min(l0 + srow, a.C - 1);
@@ -122,7 +128,8 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
         constexpr int kEdge = decltype(stag)::value;  // 1: a quad of coefficients may straddle its row's end (see bwd_tile_body); 2: rows of fewer than four
         if (stager) {
             const float *pq = kRot ? a.query + ((int64_t)c * a.C + min(l0 + srow, a.C - 1)) * d : nullptr;
-            load_query_raw<MODEL, true>(a.ent + ih * (int64_t)d, a.rel + ir * (int64_t)a.rel_dim, nullptr, pq, col, klen, half, rraw);
+            load_query_raw<MODEL, true>(a.ent + ih * (int64_t)d, a.rel + ir * (int64_t)a.rel_dim, kTH ? a.aux + ir * (int64_t)d : nullptr, pq, col, klen, half, rraw);
+            if constexpr (kTH) ral = a.side_pos[(int64_t)c * a.C + min(l0 + srow, a.C - 1)];
         }
         auto ld = [](const float *p, int kl, int lim) {
             if constexpr (kEdge == 1) return shift_quad(ld4_raw<true>(p, kl, lim), kl + 4 - lim);
@@ -135,6 +142,10 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
             const int64_t off = ((int64_t)c * a.C + (inside ? bl : 0)) * a.N;
             craw[s] = ld(a.dneg + off, kl, inside ? a.N : 0);
             if constexpr (kL2) sraw[s] = ld(a.sneg + off, kl, inside ? a.N : 0);
+            if constexpr (kTH) {
+                c1raw[s] = ld(a.side_neg + off, kl, inside ? a.N : 0);
+                c2raw[s] = ld(a.side_neg + a.plane + off, kl, inside ? a.N : 0);
+            }
         }
     };
     auto load_rows = [&](int l0) {
@@ -145,9 +156,12 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
     auto store_step = [&](int l0) {
         if (stager) {
             float4 q0, q1;
-            combine_query<MODEL, true>(rraw, 0.0f, col, l0 + srow < b1 ? klen : 0, half, a.rsign, q0, q1);
+            combine_query<MODEL, true>(rraw, ral, col, l0 + srow < b1 ? klen : 0, half, a.rsign, q0, q1);
             *reinterpret_cast<float4 *>(&sL[0][srow][tx * 4]) = kSc ? scale4(q0, kSgnScale) : q0;
-            if constexpr (NPL == 2) *reinterpret_cast<float4 *>(&sL[1][srow][tx * 4]) = q1;
+            if constexpr (NPL == 2) *reinterpret_cast<float4 *>(&sL[1][srow][tx * 4]) = kSc ? scale4(q1, kSgnScale) : q1;
+            if constexpr (kTH) {
+                if (tx == 0) sA[srow] = ral;
+            }
         }
 #pragma unroll
         for (int s = 0; s < CPT; ++s) {
@@ -161,7 +175,11 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
                 g.z = sc.z > 0.0f ? g.z / sc.z : 0.0f;
                 g.w = sc.w > 0.0f ? g.w / sc.w : 0.0f;
             }
-            *reinterpret_cast<float4 *>(&sG[lrow][(f % (TO / 4)) * 4]) = g;
+            *reinterpret_cast<float4 *>(&sG[0][lrow][(f % (TO / 4)) * 4]) = g;
+            if constexpr (kTH) {
+                *reinterpret_cast<float4 *>(&sG[1][lrow][(f % (TO / 4)) * 4]) = c1raw[s];
+                *reinterpret_cast<float4 *>(&sG[NC - 1][lrow][(f % (TO / 4)) * 4]) = mul4(scale4(g, -kSgnUnscale), c2raw[s]);  // multiplies scaled rows
+            }
         }
     };
 
@@ -177,11 +195,12 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
             load_idx(l0 + 2 * KL);
         }
         __builtin_amdgcn_sched_barrier(0);
-        float4 sacc[NPL][RO];  // (a step's sums of their own: rounding grows with the steps, not the positives)
+        float4 sacc[NPN][RO];  // (a step's sums of their own: rounding grows with the steps, not the positives)
 #pragma unroll
-        for (int q = 0; q < NPL; ++q)
+        for (int q = 0; q < NPN; ++q)
 #pragma unroll
             for (int o = 0; o < RO; ++o) sacc[q][o] = zero4();
+        // (TransH: the negatives' sums and those for w are formed with the opposite sign, which no operand has to carry, and change it when they leave)
         // (unrolled, the exchanges' registers and the next positive's operands spill)
 #pragma unroll 1
         for (int l = phase; l < KL; l += PH) {
@@ -192,12 +211,20 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
                 lv[q][0] = v.x, lv[q][1] = v.y, lv[q][2] = v.z, lv[q][3] = v.w;
                 sum[q][0] = sum[q][1] = sum[q][2] = sum[q][3] = 0.0f;
             }
-            const float4 cf = *reinterpret_cast<const float4 *>(&sG[l][ty * RO]);
+            const float4 cf = *reinterpret_cast<const float4 *>(&sG[0][l][ty * RO]);
+            float4 cp = zero4(), ep = zero4();
+            float al = 0.0f;
+            if constexpr (kTH) {
+                cp = *reinterpret_cast<const float4 *>(&sG[1][l][ty * RO]), ep = *reinterpret_cast<const float4 *>(&sG[NC - 1][l][ty * RO]);
+                al = sA[l];
+            }
 #pragma unroll
             for (int o = 0; o < RO; ++o) {
                 const float g = reinterpret_cast<const float *>(&cf)[o];
-                const float *t0 = reinterpret_cast<const float *>(&own[0][o]), *t1 = reinterpret_cast<const float *>(&own[NPL - 1][o]);
-                float *n0 = reinterpret_cast<float *>(&sacc[0][o]), *n1 = reinterpret_cast<float *>(&sacc[NPL - 1][o]);
+                const float *t0 = reinterpret_cast<const float *>(&own[0][o]), *t1 = reinterpret_cast<const float *>(&own[NPN - 1][o]);
+                float *n0 = reinterpret_cast<float *>(&sacc[0][o]), *n1 = reinterpret_cast<float *>(&sacc[NPN - 1][o]);
+                const float cc = reinterpret_cast<const float *>(&cp)[o], ee = reinterpret_cast<const float *>(&ep)[o];
+                const float gk = (al - cc) * g;  // times the sign: the pair's w . (x - t') part of minus w's gradient
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     if constexpr (kRot) {
@@ -206,6 +233,11 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
                         const float k = g * __builtin_amdgcn_rsqf(fmaf(ur, ur, fmaf(ui, ui, 1e-37f)));
                         n0[e] = fmaf(k, ur, n0[e]), n1[e] = fmaf(k, ui, n1[e]);
                         sum[0][e] = fmaf(-k, ur, sum[0][e]), sum[1][e] = fmaf(-k, ui, sum[1][e]);
+                    } else if constexpr (kTH) {
+                        const float s = sgn_of_scaled(fmaf(cc, lv[1][e], lv[0][e] - t0[e]));
+                        sum[0][e] = fmaf(g, s, sum[0][e]);
+                        sum[1][e] = fmaf(ee, t0[e], fmaf(gk, s, sum[1][e]));
+                        n0[e] = fmaf(ee, lv[1][e], fmaf(g, s, n0[e]));
                     } else {
                         const float u = lv[0][e] - t0[e];  // (P == 1: times 2^100)
                         const float s = P == 1 ? sgn_of_scaled(u) : u;
@@ -239,7 +271,7 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
             }
         }
 #pragma unroll
-        for (int q = 0; q < NPL; ++q)
+        for (int q = 0; q < NPN; ++q)
 #pragma unroll
             for (int o = 0; o < RO; ++o) acc[q][o] = add4(acc[q][o], sacc[q][o]);
         __syncthreads();
@@ -250,31 +282,32 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
             float x = sR[l * WAVES * (NPL * kPairCols) + pc];
 #pragma unroll
             for (int w = 1; w < wo; ++w) x += sR[(l * WAVES + w) * (NPL * kPairCols) + pc];
+            if (kTH && pc >= kPairCols) x = -x;
             const int jl = tile_x * kPairCols + (lc & ~3), j = min(jl, klen - 4);
             if (l0 + l < b1 && (lc & 3) >= jl - j)
-                pa.g0[tile * pa.gplane + ((int64_t)c * a.C + l0 + l) * d + (pc >= kPairCols ? half : 0) + j + (lc & 3)] = x;
+                (kTH && pc >= kPairCols ? pa.g1 : pa.g0)[tile * pa.gplane + ((int64_t)c * a.C + l0 + l) * d + (kRot && pc >= kPairCols ? half : 0) + j + (lc & 3)] = x;
         }
     }
 
     if constexpr (PH > 1) {  // the phases' sums of the same negatives
         __syncthreads();
         float4 *sS = reinterpret_cast<float4 *>(dyn_smem);
-        static_assert(sizeof(float4) * NPL * RO * TH * 3 / 4 <= sizeof(float) * S::kLdsFloats, "three of four phases pass through LDS");
+        static_assert(sizeof(float4) * NPN * RO * TH * 3 / 4 <= sizeof(float) * S::kLdsFloats, "three of four phases pass through LDS");
         constexpr int slots = wo * kWave;
         const int slot = own_wave * kWave + lane;
         if (phase > 0) {
 #pragma unroll
-            for (int q = 0; q < NPL; ++q)
+            for (int q = 0; q < NPN; ++q)
 #pragma unroll
-                for (int o = 0; o < RO; ++o) sS[((phase - 1) * NPL * RO + q * RO + o) * slots + slot] = acc[q][o];
+                for (int o = 0; o < RO; ++o) sS[((phase - 1) * NPN * RO + q * RO + o) * slots + slot] = acc[q][o];
         }
         __syncthreads();
         if (phase > 0) return;
         for (int p = 1; p < PH; ++p)
 #pragma unroll
-            for (int q = 0; q < NPL; ++q)
+            for (int q = 0; q < NPN; ++q)
 #pragma unroll
-                for (int o = 0; o < RO; ++o) acc[q][o] = add4(acc[q][o], sS[((p - 1) * NPL * RO + q * RO + o) * slots + slot]);
+                for (int o = 0; o < RO; ++o) acc[q][o] = add4(acc[q][o], sS[((p - 1) * NPN * RO + q * RO + o) * slots + slot]);
     }
 #pragma unroll
     for (int o = 0; o < RO; ++o) {
@@ -282,9 +315,9 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
         if (kl >= a.N) continue;
         float *dst = (split ? pa.more_neg + (split - 1) * pa.nplane : pa.occ_neg) + ((int64_t)c * a.N + kl) * d;
 #pragma unroll
-        for (int q = 0; q < NPL; ++q) {
+        for (int q = 0; q < NPN; ++q) {
             float *p = dst + q * half + col;
-            const float4 v = acc[q][o];
+            const float4 v = kTH ? scale4(acc[q][o], -1.0f) : acc[q][o];
             if (skip == 0) {
                 store_quad(p, v);
             } else {
@@ -301,16 +334,22 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_ROTATE ? 3 : 4) voi
 //   RotatE: always; 0.73 of the time in the mean, 1.06 at worst (874 x 77 negatives x 322 in chunks of 38).
 //   TransE L1: 0.87 in the mean by the rule below.  A thread of the other tiles walks the longer side of a chunk; from 160 on that walk costs a
 //   small batch more than the extra planes do.  A batch that fills the chip goes by the padded pairs of both forms.
+//   TransH L1: a pair here is 10.3 vector instructions an element where both orientations take 12.6, and there are two planes a tile, so it pays where the
+//   other tiles walk a long side with few workgroups, or pad.  By the walk times the 768 resident workgroups over the launch's own, and the
+//   padded pairs of both forms, over 220 shapes of the same ranges: 0.87 in the mean, 1.03 at worst (always: 0.855 and 1.22).  Backward pass, us: 969 x 147
+//   negatives x 96 in one chunk 102 -> 53, 1482 x 18 x 840 in chunks of 741 107 -> 54, 8575 x 222 x 280 in chunks of 25 397 -> 304; left as they
+//   are 8192 x 256 x 200 in chunks of 256 (157, here 172) and 16384 x 1024 x 400 (1745, here 1793: 420 MB of planes).
 //   TransE L2, where differences are summed (launch_tiles): no sign to save, so only the walk counts: 0.83 from 280 on, 1.0 below.
 inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *out)
 {
     if (!bat->neg || bat->chunk <= 0 || bat->n_neg <= 0 || !rows_by_quads(tab)) return false;  // (rows by quads)
-    if (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE) return false;
+    if (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE && !(tab->model == KGE_TRANSH && tab->norm_p == 1)) return false;
+    const bool th = tab->model == KGE_TRANSH;
     const int64_t n_chunks = bat->batch / bat->chunk, C = bat->chunk, N = bat->n_neg, klen = tab->model == KGE_ROTATE ? tab->dim / 2 : tab->dim;
     const int64_t cols = ceil_div(klen, kPairCols) * n_chunks, steps = ceil_div(C, kPairKL), longer = C > N ? C : N;
     // Negatives of a workgroup: 128, or 64 / 32 by waves in two / four phases (5 / 20 % slower per pair), by what the last tile wastes and
     // what the planes cost (a plane of a batch beyond the caches as much as 17 negatives, else 6).  A launch that cannot fill the chip takes smaller ones.
-    const int64_t plane = bat->batch * tab->dim >= 4000000 ? 17 : 6;
+    const int64_t plane = (bat->batch * tab->dim >= 4000000 ? 17 : 6) * (th ? 2 : 1);
     auto cost = [&](int ph) { return ceil_div(N, kPairOwners / ph) * (kPairOwners / ph * (ph == 1 ? 100 : ph == 2 ? 105 : 120) + plane * 100); };
     int ph = cost(1) <= cost(2) && cost(1) <= cost(4) ? 1 : (cost(2) <= cost(4) ? 2 : 4);
     while (ph < 4 && cols * ceil_div(N, kPairOwners / ph) * steps < 384) ph *= 2;
@@ -330,6 +369,13 @@ inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *ou
     const int64_t gx = ceil_div(klen, kTI), big = gx * (ceil_div(C, 64) + ceil_div(N, 64)) * n_chunks, to = big >= 1024 ? 64 : (big >= 512 ? 32 : 16);
     const double padded = (double)(ceil_div(C, to) * to * ceil_div(N, 32) * 32 + ceil_div(N, to) * to * ceil_div(C, 32) * 32);
     const double both = 9.5 * (double)(gx * kTI * n_chunks) * padded;
+    if (th) {
+        const int64_t wgs = gx * (ceil_div(C, to) + ceil_div(N, to)) * n_chunks, quarters = to == 64 && narrow_cols((int)klen) ? 4 * (klen / kTI) + 1 : 4 * gx;
+        const double old_pairs = (double)(quarters * (kTI / 4) * n_chunks) * padded;
+        const double pairs = (double)(cols * kPairCols * tiles) * ((double)(steps * kPairKL) * (kPairOwners / ph) * (ph == 1 ? 1.0 : ph == 2 ? 1.05 : 1.2) + 2.0 * (double)(plane * C));
+        const double walk = 768.0 * (double)longer / (double)wgs, ratio = pairs / old_pairs;
+        return walk > 620.0 || ratio < 0.5 || (walk > 100.0 && ratio < 0.6);
+    }
     const double once = 16.0 * (double)(cols * kPairCols) * (double)(steps * kPairKL * (tiles * kPairOwners / ph) + plane * tiles * C);
     const bool fills = both > 1.5e10;  // (about 100 us)
     return once < both * (longer < 160 ? 0.8 : (fills ? 0.95 : 1.2));

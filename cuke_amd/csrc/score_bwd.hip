@@ -1030,7 +1030,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             const int j = at.at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j),
                          vw = Vec<V>::load(w + j);
-            const Vec<V> G = ldz<V>(g0, j);
+            const Vec<V> G = ldz<V>(g0, j, a.planes, gplane);
 #pragma unroll
             for (int e = 0; e < V; ++e) {
                 const float u = ((vh.v[e] - vt.v[e]) + vr.v[e]) - sd * vw.v[e];
@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(256) void bwd_pos_kernel(PosBwdArgs a, FusedInsp fi
             const int j = RowPiece<V, RAG>(j0, d).at;
             const Vec<V> vh = Vec<V>::load(eh + j), vt = Vec<V>::load(et + j), vr = Vec<V>::load(rr + j),
                          vw = Vec<V>::load(w + j);
-            const Vec<V> G = ldz<V>(g0, j), Gw = ldz<V>(g1, j);
+            const Vec<V> G = ldz<V>(g0, j, a.planes, gplane), Gw = ldz<V>(g1, j, a.planes, gplane);
             Vec<V> dh, dt, dr, dw;
 #pragma unroll
             for (int e = 0; e < V; ++e) {
@@ -1122,7 +1122,7 @@ static BwdPlan make_bwd_plan(const kge_tables *tab, const kge_batch *bat)
     p.by_pairs = plan_pairs(tab, bat, &p.pairs);
     if (!p.by_pairs) p.pairs = PairPlan{1, 1, 1, 0};
     p.off_g0 = take(bat->neg ? p.pairs.tiles * B * d : 0);
-    p.off_g1 = take(bat->neg && tab->model == KGE_TRANSH ? B * d : 0);
+    p.off_g1 = take(bat->neg && tab->model == KGE_TRANSH ? p.pairs.tiles * B * d : 0);
     p.off_more = take((p.pairs.splits - 1) * p.nn * d);
     p.off_part_e = take(seg_partial_floats(p.n_occ, d));
     p.off_part_r = take(seg_partial_floats(B, rd));
@@ -1242,8 +1242,9 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
                    chained ? 1 : 0, head ? bat->h : bat->t, dpos, head ? occ_e + B * d : occ_e, head ? occ_e : occ_e + B * d, occ_r};
         float *occ_neg = occ_e + 2 * B * d;
         if (p.by_pairs) {
-            const PairArgs pr{p.pairs, g0, B * d, occ_neg, reinterpret_cast<float *>(ws + p.off_more), p.nn * d};
+            const PairArgs pr{p.pairs, g0, g1, B * d, occ_neg, reinterpret_cast<float *>(ws + p.off_more), p.nn * d};
             if (model == KGE_ROTATE) rc = launch_pairs<KGE_ROTATE, 2>(a, pr, fi_pass, st);
+            else if (model == KGE_TRANSH) rc = launch_pairs<KGE_TRANSH, 1>(a, pr, fi_pass, st);
             else rc = P == 1 ? launch_pairs<KGE_TRANSE, 1>(a, pr, fi_pass, st) : launch_pairs<KGE_TRANSE, 2>(a, pr, fi_pass, st);
         } else
         switch (model) {

@@ -1,4 +1,4 @@
-"""Gradient tiles that evaluate every pair once (TransE, RotatE): one, two and four phases, several tiles of negatives and ranges of
+"""Gradient tiles that evaluate every pair once (TransE, RotatE, TransH L1): one, two and four phases, several tiles of negatives and ranges of
 positives, their ragged edges, widths that end inside a quad, rows of one to three coefficients; head and tail negatives; the forms on
 both sides of the rule."""
 import pytest
@@ -17,11 +17,12 @@ SHAPES = [
     (256, 16, 129, 36), (512, 512, 130, 66),   # a second tile of one negative; ranges of positives that end inside a step
     (2048, 1024, 128, 8), (514, 257, 300, 264),
     (4096, 64, 257, 130),
+    (1000, 25, 250, 98),                       # one phase and two tiles, for each model
 ]
 
 
 @pytest.mark.parametrize("mode", ["tail", "head"])
-@pytest.mark.parametrize("model,p", [("RotatE", 2), ("TransE", 1), ("TransE", 2)])
+@pytest.mark.parametrize("model,p", [("RotatE", 2), ("TransE", 1), ("TransE", 2), ("TransH", 1)])
 @pytest.mark.parametrize("batch,chunk,n_neg,dim", SHAPES)
 def test_gradients(oracle, model, p, batch, chunk, n_neg, dim, mode):
     # (L1: lattice tables, where every residual is exact and no sign is ambiguous)

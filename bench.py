@@ -46,7 +46,7 @@ BOUND = {"cfg1_transe": "hbm", "cfg2_distmult": "fp32", "cfg2_complex": "fp32", 
 PROFILE_KERNELS = {
     "score_pos_kernel": ["score_pos_kernel"],
     "score_neg_kernel": ["score_neg_kernel", "score_neg_mfma_kernel", "score_neg_split_kernel", "score_neg_finish_kernel"],
-    "bwd_tile_kernel": ["bwd_tile_kernel"],
+    "bwd_tile_kernel": ["bwd_tile_kernel", "bwd_pair_kernel"],
     "bwd_pos_kernel": ["bwd_pos_kernel"],
     "seg_reduce_l1": ["seg_reduce_l1"],
     "seg_reduce_l2": ["seg_reduce_l2"],

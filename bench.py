@@ -46,7 +46,7 @@ BOUND = {"cfg1_transe": "hbm", "cfg2_distmult": "fp32", "cfg2_complex": "fp32", 
 PROFILE_KERNELS = {
     "score_pos_kernel": ["score_pos_kernel"],
     "score_neg_kernel": ["score_neg_kernel", "score_neg_mfma_kernel", "score_neg_split_kernel", "score_neg_finish_kernel"],
-    "bwd_tile_kernel": ["bwd_tile_kernel", "bwd_pair_kernel"],
+    "bwd_tile_kernel": ["bwd_tile_kernel"],
     "bwd_pos_kernel": ["bwd_pos_kernel"],
     "seg_reduce_l1": ["seg_reduce_l1"],
     "seg_reduce_l2": ["seg_reduce_l2"],
@@ -85,7 +85,7 @@ def measured_traffic(workload, label, matrix_core_tiles=False, dense=False):
     total, names = 0.0, []
     for key in want:
         for name, by in rows.items():
-            base = name.replace("kge::", "")
+            base = name.replace("kge::", "").replace("bwd_pair_kernel", "bwd_tile_kernel")  # (one label, two forms: a step runs one of them)
             if base == key or base.startswith(key + "<") or (key.endswith(">") and base.replace(" ", "") == key.replace(" ", "")):
                 if matrix_core_tiles and ((key == "score_neg_kernel") or (key == "bwd_tile_kernel" and base[:-1].split(", ")[3] != "true")):
                     continue  # the vector-ALU form of a tile kernel

@@ -14,13 +14,13 @@
 
 namespace kge {
 
-// The rider's sums: a work item is (sum i, 256 float4 of the row); the slice's workgroups stride over the items.
-__device__ __forceinline__ void sum_rider_body(const SumRider &r)
+// The rider's sums: a work item is (sum i, 256 float4 of the row); the slice's first `width` workgroups, all that it has, stride over the items.
+__device__ __forceinline__ void sum_rider_body(const SumRider &r, unsigned width)
 {
     const int nsum = r.num[0] < r.max_sums ? r.num[0] : r.max_sums;
     const int64_t q4 = r.row_floats / 4;
     const int64_t nb = (q4 + 255) / 256;
-    for (int64_t it = blockIdx.x; it < nsum * nb; it += gridDim.x) {
+    for (int64_t it = blockIdx.x; it < nsum * nb; it += width) {
         const int i = (int)(it / nb);
         const int64_t f = (it % nb) * 256 + threadIdx.x;
         if (f >= q4) continue;
@@ -44,7 +44,7 @@ template <int V>
 __global__ __launch_bounds__(256) void seg_reduce_l1(SegArgs3 jobs, SumRider rider)
 {
     if (rider.max_sums > 0 && blockIdx.y == gridDim.y - 1) {  // the last slice of the grid is the rider's
-        sum_rider_body(rider);
+        sum_rider_body(rider, gridDim.x);
         return;
     }
     seg_l1_wave<V>(jobs.j[blockIdx.y], (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
@@ -56,12 +56,15 @@ template <int V>
 __global__ __launch_bounds__(256) void seg_reduce_l2(SegArgs3 jobs, int nch, SumRider rider, kge_loss_total loss)
 {
     __shared__ __align__(8) float s_part[4][kWave * 4];
-    if (loss.loss && blockIdx.x == gridDim.x - 1) {  // (past every job's last block; beside them it takes no time: a launch of its own 2 us)
+    // With a loss the slices are one workgroup wider than their work, the rider's included; slice 0's adds the loss up.  (Beside the jobs' blocks
+    // it takes no time: a launch of its own 2 us.)
+    const unsigned width = gridDim.x - (loss.loss ? 1 : 0);
+    if (blockIdx.x == width) {
         if (blockIdx.y == 0) loss_total_block(loss, reinterpret_cast<double *>(&s_part[0][0]));
         return;
     }
     if (rider.max_sums > 0 && blockIdx.y == gridDim.y - 1) {  // (when level 1 rode in the launch the sums depend on)
-        sum_rider_body(rider);
+        sum_rider_body(rider, width);
         return;
     }
     const SegArgs &a = jobs.j[blockIdx.y];

@@ -1,9 +1,11 @@
 """The margin loss whose last sum rides in the backward pass: the same bits as the loss call, from one partial to all 1024 of them, with one to
-three reduction jobs beside it, in plain, staged and captured steps."""
+three reduction jobs and the sums of split relations beside it, in plain, staged and captured steps."""
+import ctypes as C
+
 import pytest
 import torch
 
-from cuke_amd import synth
+from cuke_amd import _lib, synth
 from cuke_amd.kge import TrainStep, margin_loss
 from helpers import gpu_model
 
@@ -50,3 +52,30 @@ def test_one_call_staged_and_captured_steps():
     st.loss.fill_(float("nan"))
     st.run_native(None, 0), st.run_native(0, None)
     _same(st)
+
+
+@pytest.mark.parametrize("model", ["TransR", "RESCAL"])
+@pytest.mark.parametrize("batch,dim,n_rel", [(1024, 1024, 2), (2048, 1024, 7), (4096, 512, 15), (8192, 200, 20)])
+def test_beside_the_sums_of_split_relations(model, batch, dim, n_rel):
+    """Explicit triples, where level 1 of the reduction rides with dM and level 2 carries the split relations' sums and the loss: more pieces of
+    sums than the grid has workgroups, and (8192 x 200) fewer."""
+    w = synth.custom_workload(model, n_ent=300, n_rel=n_rel, dim=dim, batch=batch, sigma=0.2, seed=batch)
+    m, ix = gpu_model(w)
+    r = torch.arange(batch, device="cuda") % n_rel
+    st = TrainStep(m, ix["h"], r, ix["t"], dpos=torch.randn(batch, device="cuda"))
+    parts, loss = torch.rand(1000, device="cuda", dtype=torch.float64), torch.empty(1, device="cuda")
+    total = _lib.LossTotal(parts.data_ptr(), parts.numel(), 0.25, loss.data_ptr())
+    rows = [x for x in (st.ent_rows, st.rel_rows, st.aux_rows) if x is not None]
+    for fused in (None, False):
+        got = []
+        for p in (None, C.addressof(total)):
+            for x in (*rows, loss):
+                x.fill_(float("nan"))
+            st.bat.loss_total = p
+            st.run(fused=fused)
+            torch.cuda.synchronize()
+            got.append([x.clone() for x in rows])
+        st.bat.loss_total = None
+        assert not torch.isnan(got[1][-1][:n_rel]).any()
+        assert all(torch.equal(x.view(torch.int32), y.view(torch.int32)) for x, y in zip(*got))
+        assert abs(loss.item() - 0.25 * parts.sum().item()) <= 1e-6 * abs(loss.item())

@@ -1066,6 +1066,7 @@ class TrainStep:
             s_.ent_insp._u = s_.rel_insp._u = None
         if not pipeline:
             self.bat.plans_ready = 0  # the forward call plans for itself
+        up_front = False
         if fused is None:
             # The projection models' explicit triples: with back rows two launches carry an inspection's four steps and the other two
             # took launches of their own between forward and backward; up to 4096 ids are one launch for both sets.  Both index sets
@@ -1093,6 +1094,8 @@ class TrainStep:
             self._record_done(main)
             return
         if not (backward and overlap):
+            if up_front and self._staged:
+                raise KgeError("staged batches are waiting: use run(pipeline=True)")
             self.bat.insp_ready = None
             self.inspect(st, backward)
             if backward or self.needs_rel_groups:
@@ -1100,6 +1103,7 @@ class TrainStep:
             self.forward(st, backward)
             if backward:
                 self._loss_and_backward(st)
+            self._record_done(main)
             return
         if pipeline:
             if not self._staged:

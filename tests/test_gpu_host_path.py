@@ -490,3 +490,43 @@ def test_a_staged_set_is_not_rewritten_before_what_follows_its_step(model, kw):
     torch.cuda.synchronize()
     for k, (ids, n) in enumerate(read):
         assert torch.equal(ids[:int(n)], want[k % 2]), k
+
+
+@pytest.mark.parametrize("model,kw", [("DistMult", dict(chunk=32, n_neg=8)), ("TransR", dict()), ("RESCAL", dict())])
+@pytest.mark.parametrize("step", [dict(), dict(overlap=False), dict(backward=False)])
+def test_a_set_is_not_refilled_under_a_plain_step(model, kw, step):
+    """run() between staged steps, in each of its forms, on a device that is still busy in front of it: the stream that refills the set's index
+    tensors waits for that step too.  While a batch is staged a plain step is refused."""
+    from cuke_amd._lib import KgeError
+    m, batches, make = _two_batches(model, **kw)
+    st, copies = make(batches[0]), torch.cuda.Stream()
+    busy = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
+    st.run(**step)
+    torch.cuda.synchronize()
+    want = st.pos.clone()
+
+    def stage(b):
+        tensors = st.next_inputs(copies)
+        with torch.cuda.stream(copies):
+            for x, y in zip(tensors, b):
+                if x is not None:
+                    x.copy_(y)
+            st.stage(copies.record_event())
+        return tensors
+
+    first = stage(batches[0])
+    if step.get("backward", True) and "overlap" not in step:
+        with pytest.raises(KgeError):
+            st.run()
+    st.run(pipeline=True)
+    for _ in range(20):  # (milliseconds)
+        busy.zero_()
+    st.run(**step)
+    got = st.pos.clone()
+    for _ in range(2):
+        stage(batches[0])
+        st.run(pipeline=True)
+    again = stage(batches[1])
+    assert again[0] is first[0]
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)

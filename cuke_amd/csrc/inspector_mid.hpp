@@ -361,8 +361,12 @@ __device__ __forceinline__ void mid_dedup_body(const MidJob &J, int bx, uint32_t
     uint32_t *s_red = smem, *s_scan = smem + kMidWaves;
     __builtin_amdgcn_s_setprio(3);
     const int n = (int)J.n;
-    const int nblk = n > 0 ? (n + kMidKeys - 1) / kMidKeys : 1;
-    if (bx >= nblk || (J.npass == 1 && n > 0)) return;  // single pass: finished by the scatter step
+    if (n == 0) {  // uniform; the arrays of an empty set may be missing
+        if (bx == 0 && threadIdx.x == 0) J.out.num_unique[0] = 0, J.out.seg_offsets[0] = 0;
+        return;
+    }
+    const int nblk = (n + kMidKeys - 1) / kMidKeys;
+    if (bx >= nblk || J.npass == 1) return;  // single pass: finished by the scatter step
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     const uint32_t *keys = J.keys_final;
     const int my0 = bx * kMidKeys;

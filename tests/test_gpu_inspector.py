@@ -102,3 +102,27 @@ def test_a_narrow_set_beside_a_wide_one(oracle, n, n_rows):
         for a, want in ((g.unique_ids[:u], ref.unique_ids), (g.seg_offsets[:u + 1], ref.seg_offsets), (g.perm[:k], ref.perm),
                         (g.inverse[:k], ref.inverse), (g.sorted_seg[:k], ref.inverse[ref.perm])):
             assert np.array_equal(a.cpu().numpy().astype(np.int64), want)
+
+
+def test_an_empty_set_without_arrays_beside_another():
+    """Nothing to inspect beside a set of the mid-size launches: the empty set has no more than its count and its one offset."""
+    import ctypes as C
+
+    from cuke_amd import _lib
+    from cuke_amd.kge import inspect
+    L, ids = _lib.lib(), torch.arange(9000, device="cuda") * 7 % 4000
+    full = inspect([ids], 4000)
+    want = [x.clone() for x in (full.unique_ids[:full.num_unique], full.perm, full.inverse)]
+    full.perm.fill_(-1)
+    count, offset = torch.full((1,), -1, dtype=torch.int32, device="cuda"), torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    for at in (0, 1):
+        jobs, ws = (_lib.InspectJob * 2)(), []
+        for j, n, rows, out in ((jobs[at], 0, 1345, _lib.Inspection(0, 1345, count.data_ptr(), None, offset.data_ptr(), None, None, None)),
+                                (jobs[1 - at], ids.numel(), 4000, full._c)):
+            ws.append(torch.empty(int(L.kge_inspect_workspace(n, rows)), dtype=torch.uint8, device="cuda"))
+            j.parts[0], j.part_len[0], j.n_parts, j.n_rows, j.out = ids.data_ptr() if n else None, n, 1, rows, out
+            j.workspace, j.workspace_bytes = ws[-1].data_ptr(), ws[-1].numel()
+        count.fill_(-1), offset.fill_(-1), full.perm.fill_(-1)
+        assert L.kge_inspect_batch(jobs, 2, C.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        assert int(count) == 0 and int(offset) == 0
+        assert all(torch.equal(x, y) for x, y in zip(want, (full.unique_ids[:full.num_unique], full.perm, full.inverse)))

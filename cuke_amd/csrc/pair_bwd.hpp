@@ -342,7 +342,7 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_TRANSE ? 4 : 3) voi
 //   TransE L2, where differences are summed (launch_tiles): no sign to save, so only the walk counts: 0.83 from 280 on, 1.0 below.
 inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *out)
 {
-    if (!bat->neg || bat->chunk <= 0 || bat->n_neg <= 0 || !rows_by_quads(tab)) return false;  // (rows by quads)
+    if (!bat->neg || bat->chunk <= 0 || bat->n_neg <= 0 || bat->batch < bat->chunk || !rows_by_quads(tab)) return false;  // (rows by quads)
     if (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE && !(tab->model == KGE_TRANSH && tab->norm_p == 1)) return false;
     const bool th = tab->model == KGE_TRANSH;
     const int64_t n_chunks = bat->batch / bat->chunk, C = bat->chunk, N = bat->n_neg, klen = tab->model == KGE_ROTATE ? tab->dim / 2 : tab->dim;

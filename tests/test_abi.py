@@ -238,3 +238,16 @@ def test_back_rows_are_offered_only_where_the_forward_pass_writes_them():
     b2.ent_insp = C.pointer(ent)
     assert L.kge_score_bwd(C.byref(tables("TransR", dim=202)), C.byref(b2), C.byref(saved), fake, None, C.byref(grads),
                            fake, 1 << 30, None) == -1
+
+
+def test_backward_workspace_of_batches_shorter_than_a_chunk():
+    """Nothing to score, or less than one chunk: the query answers (kge_score_bwd takes the first and refuses the second)."""
+    import ctypes as C
+    from cuke_amd import _lib
+    L, fake = _lib.lib(), 0x10000
+    for model, dim in (("TransE", 64), ("RotatE", 64), ("TransH", 64), ("DistMult", 64), ("TransF", 64)):
+        for p in (1, 2):
+            tab = _lib.Tables(_lib.MODELS[model], p, 0.0, 0, dim, dim, 10, 3, fake, fake, fake)
+            for B in (0, 8):
+                bat = _lib.Batch(B, fake, fake, fake, fake, 16, 16, None, None, None, 0, 0)
+                assert 0 < L.kge_score_bwd_workspace(C.byref(tab), C.byref(bat)) < 1 << 20

@@ -737,7 +737,7 @@ __global__ __launch_bounds__(256) void score_neg_finish_kernel(const float *part
 // for the models whose pair score is one plain sum over the row (TransE, RotatE).
 int neg_ksplit(const kge_tables *tab, const kge_batch *bat)
 {
-    if (!bat->neg || bat->chunk <= 0 || (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE)) return 1;
+    if (!bat->neg || bat->chunk <= 0 || bat->n_neg <= 0 || (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE)) return 1;
     const int64_t n_chunks = bat->batch / bat->chunk;
     if (n_chunks <= 0 || ceil_div(bat->chunk, 64) * ceil_div(bat->n_neg, 64) * n_chunks >= 1024) return 1;  // (64 x 64 tiles)
     const int64_t tiles = xcd_grid(ceil_div(bat->n_neg, 32), ceil_div(bat->chunk, 32), n_chunks);

@@ -251,3 +251,14 @@ def test_backward_workspace_of_batches_shorter_than_a_chunk():
             for B in (0, 8):
                 bat = _lib.Batch(B, fake, fake, fake, fake, 16, 16, None, None, None, 0, 0)
                 assert 0 < L.kge_score_bwd_workspace(C.byref(tab), C.byref(bat)) < 1 << 20
+
+
+def test_forward_workspace_of_no_negatives():
+    """kge_score_fwd refuses a batch of shared negatives with none; the query in front of it answers."""
+    import ctypes as C
+    from cuke_amd import _lib
+    L, fake = _lib.lib(), 0x10000
+    for model in ("TransE", "RotatE", "TransH", "DistMult"):
+        tab = _lib.Tables(_lib.MODELS[model], 2, 0.0, 0, 64, 64, 10, 3, fake, fake, fake)
+        bat = _lib.Batch(16, fake, fake, fake, fake, 16, 0, None, None, None, 0, 0)
+        assert L.kge_score_fwd_workspace(C.byref(tab), C.byref(bat)) == 0

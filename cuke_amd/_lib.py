@@ -146,7 +146,7 @@ EXPORTS = {
 _lib = None
 
 
-ABI_VERSION = 7  # layout of the ctypes structures above; must match kge_abi_version()
+ABI_VERSION = 8  # layout of the ctypes structures above; must match kge_abi_version()
 
 
 def lib() -> C.CDLL:

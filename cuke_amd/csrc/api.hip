@@ -168,7 +168,7 @@ const char *kge_strerror(int status)
     }
 }
 
-int kge_abi_version(void) { return 7; }
+int kge_abi_version(void) { return 8; }
 
 int kge_back_rows_ok(const kge_tables *tab, const kge_batch *bat)
 {

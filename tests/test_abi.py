@@ -34,7 +34,7 @@ def test_binding_table_matches_header():
 def test_strerror_and_version_without_gpu():
     from cuke_amd import _lib
     L = _lib.lib()
-    assert L.kge_abi_version() == _lib.ABI_VERSION == 7
+    assert L.kge_abi_version() == _lib.ABI_VERSION == 8
     assert L.kge_strerror(0) == b"ok"
     assert b"workspace" in L.kge_strerror(-4)
 
@@ -262,3 +262,28 @@ def test_forward_workspace_of_no_negatives():
         tab = _lib.Tables(_lib.MODELS[model], 2, 0.0, 0, 64, 64, 10, 3, fake, fake, fake)
         bat = _lib.Batch(16, fake, fake, fake, fake, 16, 0, None, None, None, 0, 0)
         assert L.kge_score_fwd_workspace(C.byref(tab), C.byref(bat)) == 0
+
+
+def test_a_structure_layout_belongs_to_its_version(tmp_path):
+    """The structures as a C compiler lays them out: the binding's are the same, and the sizes are those of this ABI version (a change of
+    either takes a new version, by which bindings of another layout are refused)."""
+    import ctypes as C
+    import subprocess
+    from cuke_amd import _lib
+    names = {"kge_tables": _lib.Tables, "kge_inspection": _lib.Inspection, "kge_inspect_job": _lib.InspectJob,
+             "kge_timeline": _lib.Timeline, "kge_loss_total": _lib.LossTotal, "kge_batch": _lib.Batch, "kge_saved": _lib.Saved,
+             "kge_grads": _lib.Grads, "kge_step_batch": _lib.StepBatch, "kge_step_buffers": _lib.StepBuffers}
+    prints = "".join(f'printf("{n} %zu\\n", sizeof({n}));' for n in names)
+    offsets = [(n, f[0]) for n, t in names.items() for f in t._fields_]
+    prints += "".join(f'printf("{n}.{f} %zu\\n", offsetof({n}, {f}));' for n, f in offsets)
+    src, exe = tmp_path / "layout.c", tmp_path / "layout"
+    src.write_text(f'#include <stdio.h>\n#include "kge_mi355.h"\nint main(void) {{ {prints} return 0; }}\n')
+    subprocess.run(["gcc", "-I" + os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True)
+    got = dict(line.split() for line in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines())
+    for n, t in names.items():
+        assert int(got[n]) == C.sizeof(t), n
+    for n, f in offsets:
+        assert int(got[f"{n}.{f}"]) == getattr(names[n], f).offset, (n, f)
+    sizes = {8: dict(kge_tables=72, kge_inspection=64, kge_inspect_job=160, kge_timeline=40, kge_loss_total=32, kge_batch=128,
+                     kge_saved=64, kge_grads=48, kge_step_batch=176, kge_step_buffers=168)}
+    assert sizes[_lib.lib().kge_abi_version()] == {n: int(got[n]) for n in names}

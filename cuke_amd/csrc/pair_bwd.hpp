@@ -5,10 +5,12 @@
 // the pair's gradient element to the negative's sum (registers) AND to the positive's, which the eight lane groups of a wave add up by
 // lane exchanges and the waves through LDS.  bwd_tile_kernel's two orientations form the same element twice, and with it
 // what the element costs: a sign or a reciprocal square root.
-// The positives' sums are complete over the TO negatives of the workgroup only: one plane of [B, d] rows per tile of negatives,
+// The positives' sums are complete over the TO negatives of the workgroup only: one plane of [B, d] rows per tile of a launch's negatives,
 // added up by bwd_pos_kernel; the negatives' rows likewise have one plane per range of positives, added up as the
-// segmented reduction loads them.
+// segmented reduction loads them.  Batches of many tiles take several launches, the later ones of which add to the planes.
 #pragma once
+
+#include <cmath>
 
 #include "inspector_mid.hpp"
 #include "tile_common.hpp"
@@ -35,14 +37,16 @@ struct PairShape {
 
 struct PairPlan {
     int phases;   // 1, 2 or 4: waves of a workgroup that share its negatives and take turns at the positives
-    int tiles;    // tiles of negatives: planes of the positives' sums
+    int tiles;    // tiles of negatives
+    int planes;   // planes of the positives' sums: tiles of a launch
     int splits;   // ranges of positives: planes of the negatives' rows
     int per;      // positives of a range, a multiple of the step
 };
 
 struct PairArgs {
     PairPlan plan;
-    float *g0, *g1;            // [tiles][B, d]; g1: TransH, the sums for w
+    int tile0;                 // first tile of the launch
+    float *g0, *g1;            // [planes][B, d]; g1: TransH, the sums for w
     int64_t gplane;            // B * d
     float *occ_neg, *more_neg; // plane 0 of the negatives' rows [n_chunks * N, d]; planes 1 ... splits - 1
     int64_t nplane;            // n_chunks * N * d
@@ -87,9 +91,10 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_TRANSE ? 4 : 3) voi
     const int tx = lane & 7, ty = own_wave * 8 + (lane >> 3);
     const int d = a.d, half = d >> 1, klen = pair_len<MODEL>(d);
     int c, tile_y, tile_x;
-    if (!xcd_tile((int)blockIdx.x - fi.blocks, (klen + kPairCols - 1) / kPairCols, pa.plan.tiles * pa.plan.splits, a.n_chunks, c, tile_y, tile_x)) return;
-    const int tile = tile_y / pa.plan.splits, split = tile_y - tile * pa.plan.splits;
-    const int k0 = tile * TO;                                             // first negative
+    if (!xcd_tile((int)blockIdx.x - fi.blocks, (klen + kPairCols - 1) / kPairCols, pa.plan.planes * pa.plan.splits, a.n_chunks, c, tile_y, tile_x)) return;
+    const int plane = tile_y / pa.plan.splits, split = tile_y - plane * pa.plan.splits;
+    if (pa.tile0 + plane >= pa.plan.tiles) return;                        // (the last of several launches)
+    const int k0 = (pa.tile0 + plane) * TO;                               // first negative
     const int b0 = split * pa.plan.per, b1 = min(a.C, b0 + pa.plan.per);  // positives of the chunk
     // (a quad of columns that would run past the row's end is moved back to end with it: see bwd_tile_body)
     const int lcol = tile_x * kPairCols + tx * 4, col = min(lcol, klen - 4), skip = lcol - col;
@@ -284,8 +289,11 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_TRANSE ? 4 : 3) voi
             for (int w = 1; w < wo; ++w) x += sR[(l * WAVES + w) * (NPL * kPairCols) + pc];
             if (kTH && pc >= kPairCols) x = -x;
             const int jl = tile_x * kPairCols + (lc & ~3), j = min(jl, klen - 4);
-            if (l0 + l < b1 && (lc & 3) >= jl - j)
-                (kTH && pc >= kPairCols ? pa.g1 : pa.g0)[tile * pa.gplane + ((int64_t)c * a.C + l0 + l) * d + (kRot && pc >= kPairCols ? half : 0) + j + (lc & 3)] = x;
+            if (l0 + l < b1 && (lc & 3) >= jl - j) {
+                float *to = (kTH && pc >= kPairCols ? pa.g1 : pa.g0) + plane * pa.gplane + ((int64_t)c * a.C + l0 + l) * d + (kRot && pc >= kPairCols ? half : 0) + j + (lc & 3);
+                if (pa.tile0 > 0) x += *to;  // uniform
+                *to = x;
+            }
         }
     }
 
@@ -329,6 +337,42 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_TRANSE ? 4 : 3) voi
     }
 }
 
+// Bytes of planes that a batch may have whatever its size (a larger one: as many again as it takes without them).
+constexpr int64_t kPairRoom = 512 << 20;
+
+inline PairPlan cut_pairs(int ph, int64_t tiles, int64_t planes, int64_t C, int64_t splits)
+{
+    const int64_t per = ceil_div(ceil_div(C, kPairKL), splits) * kPairKL;
+    return PairPlan{ph, (int)tiles, (int)planes, (int)ceil_div(C, per), (int)per};
+}
+
+// A plan whose planes take no more than `room` bytes beyond the first of either side: fewer ranges, and the tiles in launches of `planes`
+// each, by the rounds of workgroups that all launches take together (`resident` at a time; a round that is not full counts as 0.45 of one
+// and the rest by its share, a launch 0.2 of one beside).  Both orientations / every plane at once / at most 512 MB of planes, tiles with the per-positive
+// kernel and the reductions:
+//   RotatE 1024 x 40943 negatives x 1000, one chunk     222 MB 14.20 ms    2347 MB 7.10 ms   734 MB 7.36 ms
+//   RotatE 8192 x 8192 x 1000                           176    13.43       2470   10.18      569   11.99
+//   RotatE 4096 x 14951 x 400                            57     5.73        985    4.19      473    4.60
+//   TransE L1 4096 x 14951 x 400                         61     3.41        989    2.78      478    3.03
+//   TransE L1 8192 x 4096 x 400 in chunks of 1024       128     1.67        796    1.56      639    1.53
+// (256 MB: 7.96, 16.98, 5.05, 3.39 and 1.58 ms.  The planes' tiles taken one after the other by a workgroup: 20 registers more are spilled.)
+inline PairPlan shrink_pairs(const PairPlan &full, int64_t C, int64_t cols, int64_t resident, int64_t plane_bytes, int64_t range_bytes, int64_t room)
+{
+    PairPlan best = cut_pairs(full.phases, full.tiles, 1, C, 1);
+    double least = -1.0;
+    for (int64_t launches = 1; launches <= full.tiles; launches = launches < 16 ? launches + 1 : 2 * launches) {
+        const int64_t planes = ceil_div(full.tiles, launches);
+        for (int64_t splits = 1; splits <= full.splits; splits = splits < 8 ? splits + 1 : splits + splits / 4) {
+            const PairPlan p = cut_pairs(full.phases, full.tiles, planes, C, splits);
+            if ((planes - 1) * plane_bytes + (p.splits - 1) * range_bytes > room) break;
+            const double rounds = (double)(cols * planes * p.splits) / (double)resident, whole = floor(rounds), part = rounds - whole;
+            const double cost = (double)(ceil_div(full.tiles, planes) * p.per) * (0.2 + whole + (whole < 1.0 ? 1.0 : (part > 0.0 ? 0.45 + 0.55 * part : 0.0)));
+            if (least < 0.0 || cost < least) least = cost, best = p;
+        }
+    }
+    return best;
+}
+
 // Whether a batch's gradient tiles evaluate every pair once, and how they are cut.  Both ways timed over 200 random shapes (256 ... 16384
 // positives, chunks and negatives 16 ... 1024, widths 48 ... 1000; tiles, per-positive kernel and reductions together).
 //   RotatE: always; 0.73 of the time in the mean, 1.06 at worst (874 x 77 negatives x 322 in chunks of 38).
@@ -340,7 +384,7 @@ __global__ __launch_bounds__(kPairWaves *kWave, MODEL == KGE_TRANSE ? 4 : 3) voi
 //   negatives x 96 in one chunk 102 -> 53, 1482 x 18 x 840 in chunks of 741 107 -> 54, 8575 x 222 x 280 in chunks of 25 397 -> 304; left as they
 //   are 8192 x 256 x 200 in chunks of 256 (157, here 172) and 16384 x 1024 x 400 (1745, here 1793: 420 MB of planes).
 //   TransE L2, where differences are summed (launch_tiles): no sign to save, so only the walk counts: 0.83 from 280 on, 1.0 below.
-inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *out)
+inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, int64_t room, PairPlan *out)
 {
     if (!bat->neg || bat->chunk <= 0 || bat->n_neg <= 0 || bat->batch < bat->chunk || !rows_by_quads(tab)) return false;  // (rows by quads)
     if (tab->model != KGE_TRANSE && tab->model != KGE_ROTATE && !(tab->model == KGE_TRANSH && tab->norm_p == 1)) return false;
@@ -355,14 +399,19 @@ inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *ou
     while (ph < 4 && cols * ceil_div(N, kPairOwners / ph) * steps < 384) ph *= 2;
     const int64_t tiles = ceil_div(N, kPairOwners / ph);
     // Ranges of positives: 640 workgroups, and of long chunks at most 192 positives each (up to eight ranges).  RotatE 1024 x 256 x 1000, 128
-    // workgroups a range: 2 / 4 / 6 / 8 ranges 71 / 57 / 60 / 55 us, and the reduction 2 us a plane.
+    // workgroups a range: 2 / 4 / 6 / 8 ranges 71 / 57 / 60 / 55 us, and the reduction 2 us a plane.  A wave of the reduction reads its rows'
+    // planes one after the other, 0.4 us each, a step takes 1.8 to 4.5 us: at most 2.5 times the root of the steps (TransE L1 16384 x 16
+    // negatives x 96 in one chunk, 16 / 32 / 64 / 128 / 205 ranges: 149 / 104 / 91 / 105 / 128 us with the reduction).
     int64_t splits = ceil_div(640, cols * tiles);
     const int64_t by_length = ceil_div(C, 192) < 8 ? ceil_div(C, 192) : 8;
     splits = splits > by_length ? splits : by_length;
+    const int64_t most = (int64_t)(2.5 * sqrt((double)steps)) + 1;
+    splits = splits < most ? splits : most;
     splits = splits < steps ? splits : steps;
-    out->phases = ph, out->tiles = (int)tiles;
-    out->per = (int)(ceil_div(steps, splits) * kPairKL);
-    out->splits = (int)ceil_div(C, out->per);
+    *out = cut_pairs(ph, tiles, tiles, C, splits);
+    const int64_t plane_bytes = 4 * bat->batch * tab->dim * (th ? 2 : 1), range_bytes = 4 * n_chunks * N * tab->dim;
+    if ((tiles - 1) * plane_bytes + (out->splits - 1) * range_bytes > room)
+        *out = shrink_pairs(*out, C, cols, tab->model == KGE_TRANSE ? 1024 : 768, plane_bytes, range_bytes, room);
     if (tab->model == KGE_ROTATE) return true;
     if (tab->norm_p == 2) return longer >= 280 && !transe_by_products(tab->dim, C, N, n_chunks);
     // clocks per wave: a padded pair of the other tiles 9.5 per orientation, one here 16
@@ -382,14 +431,17 @@ inline bool plan_pairs(const kge_tables *tab, const kge_batch *bat, PairPlan *ou
 }
 
 template <int MODEL, int P>
-static int launch_pairs(const TileArgs &a, const PairArgs &pa, const FusedInsp &fi, hipStream_t st)
+static int launch_pairs(const TileArgs &a, PairArgs pa, const FusedInsp &fi, hipStream_t st)
 {
-    size_t lds = sizeof(float) * PairShape<MODEL>::kLdsFloats;
-    if (fi.blocks > 0 && (size_t)fi.lds_bytes > lds) lds = (size_t)fi.lds_bytes;
     const int klen = MODEL == KGE_ROTATE ? a.d / 2 : a.d;
-    const unsigned grid = xcd_grid(ceil_div(klen, kPairCols), (int64_t)pa.plan.tiles * pa.plan.splits, a.n_chunks) + (unsigned)fi.blocks;
+    const unsigned tiles = xcd_grid(ceil_div(klen, kPairCols), (int64_t)pa.plan.planes * pa.plan.splits, a.n_chunks);
     const auto kernel = pa.plan.phases == 1 ? bwd_pair_kernel<MODEL, P, 1> : (pa.plan.phases == 2 ? bwd_pair_kernel<MODEL, P, 2> : bwd_pair_kernel<MODEL, P, 4>);
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kPairWaves * kWave), lds, st, a, pa, fi);
+    for (pa.tile0 = 0; pa.tile0 < pa.plan.tiles; pa.tile0 += pa.plan.planes) {
+        const FusedInsp f = pa.tile0 == 0 ? fi : FusedInsp{};  // (the inspector's step rides once)
+        size_t lds = sizeof(float) * PairShape<MODEL>::kLdsFloats;
+        if (f.blocks > 0 && (size_t)f.lds_bytes > lds) lds = (size_t)f.lds_bytes;
+        hipLaunchKernelGGL(kernel, dim3(tiles + (unsigned)f.blocks), dim3(kPairWaves * kWave), lds, st, a, pa, f);
+    }
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

@@ -1110,24 +1110,30 @@ static BwdPlan make_bwd_plan(const kge_tables *tab, const kge_batch *bat)
     const int64_t B = bat->batch, d = tab->dim, rd = tab->rel_dim;
     p.nn = bat->neg ? (B / bat->chunk) * bat->n_neg : 0;
     p.n_occ = 2 * B + p.nn;
-    size_t o = 0;
-    auto take = [&](int64_t floats) {
-        const size_t at = o;
-        o += up256(sizeof(float) * (size_t)(floats > 0 ? floats : 1));
-        return at;
+    auto layout = [&](const PairPlan &pairs) {
+        size_t o = 0;
+        auto take = [&](int64_t floats) {
+            const size_t at = o;
+            o += up256(sizeof(float) * (size_t)(floats > 0 ? floats : 1));
+            return at;
+        };
+        p.pairs = pairs;
+        p.off_occ_e = take(p.n_occ * d);
+        p.off_occ_r = take(B * rd);
+        p.off_occ_w = take(tab->model == KGE_TRANSH ? B * d : 0);
+        p.off_g0 = take(bat->neg ? pairs.planes * B * d : 0);
+        p.off_g1 = take(bat->neg && tab->model == KGE_TRANSH ? pairs.planes * B * d : 0);
+        p.off_more = take((pairs.splits - 1) * p.nn * d);
+        p.off_part_e = take(seg_partial_floats(p.n_occ, d));
+        p.off_part_r = take(seg_partial_floats(B, rd));
+        p.off_part_w = take(tab->model == KGE_TRANSH ? seg_partial_floats(B, d) : 0);
+        p.total = o;
     };
-    p.off_occ_e = take(p.n_occ * d);
-    p.off_occ_r = take(B * rd);
-    p.off_occ_w = take(tab->model == KGE_TRANSH ? B * d : 0);
-    p.by_pairs = plan_pairs(tab, bat, &p.pairs);
-    if (!p.by_pairs) p.pairs = PairPlan{1, 1, 1, 0};
-    p.off_g0 = take(bat->neg ? p.pairs.tiles * B * d : 0);
-    p.off_g1 = take(bat->neg && tab->model == KGE_TRANSH ? p.pairs.tiles * B * d : 0);
-    p.off_more = take((p.pairs.splits - 1) * p.nn * d);
-    p.off_part_e = take(seg_partial_floats(p.n_occ, d));
-    p.off_part_r = take(seg_partial_floats(B, rd));
-    p.off_part_w = take(tab->model == KGE_TRANSH ? seg_partial_floats(B, d) : 0);
-    p.total = o;
+    layout(PairPlan{1, 1, 1, 1, 0});
+    // The planes of the tiles by pairs: as many bytes again as all else, or kPairRoom
+    PairPlan pairs;
+    p.by_pairs = plan_pairs(tab, bat, (int64_t)p.total > kPairRoom ? (int64_t)p.total : kPairRoom, &pairs);
+    if (p.by_pairs) layout(pairs);
     return p;
 }
 
@@ -1242,7 +1248,7 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
                    chained ? 1 : 0, head ? bat->h : bat->t, dpos, head ? occ_e + B * d : occ_e, head ? occ_e : occ_e + B * d, occ_r};
         float *occ_neg = occ_e + 2 * B * d;
         if (p.by_pairs) {
-            const PairArgs pr{p.pairs, g0, g1, B * d, occ_neg, reinterpret_cast<float *>(ws + p.off_more), p.nn * d};
+            const PairArgs pr{p.pairs, 0, g0, g1, B * d, occ_neg, reinterpret_cast<float *>(ws + p.off_more), p.nn * d};
             if (model == KGE_ROTATE) rc = launch_pairs<KGE_ROTATE, 2>(a, pr, fi_pass, st);
             else if (model == KGE_TRANSH) rc = launch_pairs<KGE_TRANSH, 1>(a, pr, fi_pass, st);
             else rc = P == 1 ? launch_pairs<KGE_TRANSE, 1>(a, pr, fi_pass, st) : launch_pairs<KGE_TRANSE, 2>(a, pr, fi_pass, st);
@@ -1271,7 +1277,7 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
     if (!chained) {
     PosBwdArgs pa{tab->ent, tab->rel, tab->aux, bat->h, bat->r, bat->t, dpos, saved->pos, saved->side_pos,
                   g0, g1, have_neg ? dneg : nullptr, bat->n_neg, occ_e, occ_e + B * d, occ_r, occ_w, B, (int)d,
-                  (int)tab->rel_dim, p.pairs.tiles};
+                  (int)tab->rel_dim, p.pairs.planes};
     switch (model) {
     case KGE_TRANSE:
         rc = P == 1 ? launch_pos_bwd<KGE_TRANSE, 1>(pa, vec, head, fi_dedup, st) : launch_pos_bwd<KGE_TRANSE, 2>(pa, vec, head, fi_dedup, st);

@@ -123,7 +123,14 @@ __device__ __forceinline__ void seg_l1_wave(const SegArgs &a, int64_t w)
     Vec<V> v[kSegL];
 #pragma unroll
     for (int q = 0; q < kSegL; ++q) v[q] = Vec<V>::load(a.occ + (int64_t)src[q] * d + cc);
-    for (int z = 0; z < a.more_planes; ++z) {  // uniform
+    // (a wave whose rows all lie below more_from has no planes to read: 16384 positives x 16 negatives x 96 of 205 planes 224 -> 88 us)
+    int last_src = 0;
+    if (a.more_planes > 0) {
+#pragma unroll
+        for (int q = 0; q < kSegL; ++q) last_src = src[q] > last_src ? src[q] : last_src;
+    }
+    const int planes = last_src >= a.more_from ? a.more_planes : 0;
+    for (int z = 0; z < planes; ++z) {  // uniform
         Vec<V> m[kSegL];
 #pragma unroll
         for (int q = 0; q < kSegL; ++q) m[q] = Vec<V>::load(a.more + z * a.more_stride + (int64_t)(src[q] < a.more_from ? 0 : src[q] - a.more_from) * d + cc);

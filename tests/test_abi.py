@@ -287,3 +287,27 @@ def test_a_structure_layout_belongs_to_its_version(tmp_path):
     sizes = {8: dict(kge_tables=72, kge_inspection=64, kge_inspect_job=160, kge_timeline=40, kge_loss_total=32, kge_batch=128,
                      kge_saved=64, kge_grads=48, kge_step_batch=176, kge_step_buffers=168)}
     assert sizes[_lib.lib().kge_abi_version()] == {n: int(got[n]) for n in names}
+
+
+def test_backward_workspace_of_many_negatives_is_bounded():
+    """The gradient tiles that evaluate every pair once keep partial sums per tile of negatives and per range of positives: at most as many bytes
+    again as the batch takes without them (the products' tiles of DistMult, or TransH's L2 tiles, over the same rows), or 512 MB."""
+    import ctypes as C
+    from cuke_amd import _lib
+    L, fake = _lib.lib(), 0x10000
+
+    def query(model, p, B, chunk, N, d, rel_dim):
+        tab = _lib.Tables(_lib.MODELS[model], p, 0.0, 0, d, rel_dim, 10, 3, fake, fake, fake)
+        return L.kge_score_bwd_workspace(C.byref(tab), C.byref(_lib.Batch(B, fake, fake, fake, fake, chunk, N, None, None, None, 0, 0)))
+
+    by_pairs = set()
+    for B, chunk, N, d in [(1024, 1024, 40943, 1000), (8192, 8192, 8192, 1000), (4096, 4096, 14951, 400), (16384, 1024, 1024, 1000),
+                           (512, 512, 1_000_000, 64), (65536, 65536, 65536, 400), (1 << 20, 1 << 20, 16, 100), (1024, 16, 256, 400)]:
+        for model, p in (("RotatE", 2), ("TransE", 1), ("TransE", 2), ("TransH", 1)):
+            rel_dim = d // 2 if model == "RotatE" else d
+            one = query("TransH", 2, B, chunk, N, d, rel_dim) if model == "TransH" else query("DistMult", 2, B, chunk, N, d, rel_dim)
+            got = query(model, p, B, chunk, N, d, rel_dim)
+            assert one <= got <= one + max(one, 512 << 20) + 1024, (model, p, B, chunk, N, d)
+            if got > one:
+                by_pairs.add((model, p))
+    assert {("RotatE", 2), ("TransE", 1), ("TransH", 1)} <= by_pairs

@@ -1,11 +1,13 @@
 """Gradient tiles that evaluate every pair once (TransE, RotatE, TransH L1): one, two and four phases, several tiles of negatives and ranges of
 positives, their ragged edges, widths that end inside a quad, rows of one to three coefficients; head and tail negatives; the forms on
-both sides of the rule."""
+both sides of the rule; batches whose tiles take several launches."""
 import pytest
+import torch
 
 import test_gpu_transe_distances
 
 from cuke_amd import synth
+from helpers import assert_close, gpu_model
 from test_gpu_backward import compare, run_both
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +41,61 @@ def test_gradients(oracle, model, p, batch, chunk, n_neg, dim, mode):
 def test_last_column_tile_of_the_64_bit_products(dim, mode):
     """One to 32 columns left over (and 33, where the whole tile takes them)."""
     test_gpu_transe_distances.test_gradients_of_close_rows(8192, 256, 200, dim, "matrix_cores", "offset 0.25", mode)
+
+
+def in_64_bits(w, rotated, dpos, dneg, mode, block):
+    """Dense gradients of a workload's entity, relation and normal tables: scores in 64 bits on the GPU, a block of negatives of a chunk at a
+    time, differentiated by autograd.  rotated: RotatE's rows h e^{i theta} (t e^{-i theta}) rounded to fp32, as the pair differences take them."""
+    a, dev = w.arrays, torch.device("cuda:0")
+    E, R, A = tabs = [torch.from_numpy(a[k]).to(dev).double().requires_grad_() if a[k] is not None and a[k].size else None for k in ("E", "R", "A")]
+    h, r, t, neg = (torch.from_numpy(a[k]).to(dev) for k in ("h", "r", "t", "neg"))
+    half = E.shape[1] // 2
+
+    def turn(x, theta):
+        c, s = torch.cos(theta), torch.sin(theta)
+        return torch.cat((x[..., :half] * c - x[..., half:] * s, x[..., :half] * s + x[..., half:] * c), -1)
+
+    def score(x, rel, y):
+        if w.model == "RotatE":  # (x: turned)
+            u = x - y
+            return w.gamma - torch.sqrt(u[..., :half] ** 2 + u[..., half:] ** 2).sum(-1)
+        u = x - y + R[rel]
+        if w.model == "TransH":
+            u = u - ((x - y) * A[rel]).sum(-1, keepdim=True) * A[rel]
+        return u.abs().sum(-1) if w.norm_p == 1 else (u * u).sum(-1).sqrt()
+
+    (score(turn(E[h], R[r]) if w.model == "RotatE" else E[h], r, E[t]) * dpos).sum().backward()
+    C, N, tail = w.chunk, w.n_neg, mode == "tail"
+    for c in range(w.batch // C):
+        b = slice(c * C, (c + 1) * C)
+        for k0 in range(0, N, block):
+            other = E[neg[c * N + k0:c * N + min(k0 + block, N)]][None]
+            kept = E[(h if tail else t)[b]]
+            if w.model == "RotatE":
+                kept = turn(kept, R[r[b]] if tail else -R[r[b]])
+                kept = kept + (rotated[b].double() - kept).detach()
+            kept, rel = kept[:, None], r[b][:, None]
+            s = score(kept, rel, other) if tail or w.model == "RotatE" else score(other, rel, kept)
+            (s * dneg[b, k0:k0 + block]).sum().backward()
+    return [x.grad if x is not None else None for x in tabs]
+
+
+def compare_64(w, mode, what, block=1024):
+    m, ix = gpu_model(w)
+    gen = torch.Generator("cuda:0").manual_seed(2)
+    dpos, dneg = (torch.randn(n, device="cuda:0", generator=gen) for n in (w.batch, (w.batch, w.n_neg)))
+    fw = m.score(ix["h"], ix["r"], ix["t"], ix["neg"], w.chunk, neg_mode=mode)
+    g = m.backward(fw, dpos, dneg)
+    want = in_64_bits(w, fw.residual, dpos.double(), dneg.double(), mode, block)
+    for name, ids, rows, ref in (("entity", g.ent_ids, g.ent_rows, want[0]), ("relation", g.rel_ids, g.rel_rows, want[1]),
+                                 ("normal", g.rel_ids, g.aux_rows, want[2])):
+        if rows is not None:
+            assert_close(rows.cpu().numpy(), ref[ids.long()].cpu().numpy(), what=f"{what} {name} rows", rows=True)
+
+
+@pytest.mark.parametrize("model,p", [("RotatE", 2), ("TransE", 1), ("TransH", 1)])
+def test_many_negatives_take_several_launches(model, p):
+    """Planes of the positives' sums, one per tile of negatives, of more bytes than a batch may have: the tiles' launches add to each other's."""
+    w = synth.custom_workload(model, n_ent=30000, n_rel=7, dim=1000, batch=1100, chunk=1100, n_neg=20500, norm_p=p, sigma=0.2, gamma=4.0,
+                              seed=3, lattice=(p == 1))
+    compare_64(w, "tail", f"{model} L{p}", block=128)

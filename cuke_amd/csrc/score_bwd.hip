@@ -1103,8 +1103,10 @@ struct BwdPlan {
 };
 
 static size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
+constexpr int64_t kPlaneSlack = 3 * 256;  // rounding of the arrays that hold planes
 
-static BwdPlan make_bwd_plan(const kge_tables *tab, const kge_batch *bat)
+// given: bytes of workspace to fit into where the batch's own plan does not, -1: as many as it wants.
+static BwdPlan make_bwd_plan(const kge_tables *tab, const kge_batch *bat, int64_t given = -1)
 {
     BwdPlan p{};
     const int64_t B = bat->batch, d = tab->dim, rd = tab->rel_dim;
@@ -1133,7 +1135,16 @@ static BwdPlan make_bwd_plan(const kge_tables *tab, const kge_batch *bat)
     // The planes of the tiles by pairs: as many bytes again as all else, or kPairRoom
     PairPlan pairs;
     p.by_pairs = plan_pairs(tab, bat, (int64_t)p.total > kPairRoom ? (int64_t)p.total : kPairRoom, &pairs);
-    if (p.by_pairs) layout(pairs);
+    if (!p.by_pairs) return p;
+    const int64_t one = (int64_t)p.total;
+    layout(pairs);
+    // A smaller batch can want more planes than a larger one of the same chunks, whose workspace it may have been given: RotatE, which has no
+    // other tiles, takes the planes that fit, the others the tiles without planes.
+    if (given >= 0 && (int64_t)p.total > given) {
+        p.by_pairs = tab->model == KGE_ROTATE;
+        if (p.by_pairs) plan_pairs(tab, bat, given - one > kPlaneSlack ? given - one - kPlaneSlack : 0, &pairs);
+        layout(p.by_pairs ? pairs : PairPlan{1, 1, 1, 1, 0});
+    }
     return p;
 }
 
@@ -1194,7 +1205,7 @@ int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *
     if (tab->model == KGE_TRANSR || tab->model == KGE_RESCAL)
         return launch_transr_bwd(tab, bat, saved, dpos, grads, workspace, workspace_bytes, st);
 
-    const BwdPlan p = make_bwd_plan(tab, bat);
+    const BwdPlan p = make_bwd_plan(tab, bat, workspace_bytes < (size_t)INT64_MAX ? (int64_t)workspace_bytes : INT64_MAX);
     if (!workspace || workspace_bytes < p.total) return KGE_EWORKSPACE;
     if (bat->ent_insp->n != p.n_occ || bat->rel_insp->n != bat->batch) return KGE_ESHAPE;
     const int model = tab->model, P = tab->norm_p;

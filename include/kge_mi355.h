@@ -391,6 +391,8 @@ int kge_margin_loss_static(const float *pos, const float *neg, int64_t batch, in
  * (apps/kge/kge.py:393-515); this entry point is what a training step needs
  * in their place.
  */
+/* The bytes with which the batch runs fastest: they need not grow with the batch, as a small one can share out more of its sums.
+   A workspace queried for a batch of some chunks serves every batch of fewer chunks with the same chunk, n_neg and tables too. */
 size_t kge_score_bwd_workspace(const kge_tables *tab, const kge_batch *bat);
 int kge_score_bwd(const kge_tables *tab, const kge_batch *bat, const kge_saved *saved,
                   const float *dpos, const float *dneg, const kge_grads *grads,

@@ -1,12 +1,15 @@
 """Gradient tiles that evaluate every pair once (TransE, RotatE, TransH L1): one, two and four phases, several tiles of negatives and ranges of
 positives, their ragged edges, widths that end inside a quad, rows of one to three coefficients; head and tail negatives; the forms on
-both sides of the rule; batches whose tiles take several launches."""
+both sides of the rule; batches whose tiles take several launches, by the planes' bytes and by a workspace's."""
+import ctypes as C
+
 import pytest
 import torch
 
 import test_gpu_transe_distances
 
-from cuke_amd import synth
+from cuke_amd import _lib, synth
+from cuke_amd.kge import TrainStep
 from helpers import assert_close, gpu_model
 from test_gpu_backward import compare, run_both
 
@@ -99,3 +102,43 @@ def test_many_negatives_take_several_launches(model, p):
     w = synth.custom_workload(model, n_ent=30000, n_rel=7, dim=1000, batch=1100, chunk=1100, n_neg=20500, norm_p=p, sigma=0.2, gamma=4.0,
                               seed=3, lattice=(p == 1))
     compare_64(w, "tail", f"{model} L{p}", block=128)
+
+
+@pytest.mark.parametrize("mode", ["tail", "head"])
+@pytest.mark.parametrize("model,p", [("RotatE", 2), ("TransE", 1), ("TransE", 2), ("TransH", 1)])
+@pytest.mark.parametrize("batch,chunk,n_neg,dim", [(600, 300, 450, 70), (200, 200, 350, 50), (1600, 400, 700, 264)])  # (two, four and one phase)
+def test_a_smaller_workspace(model, p, batch, chunk, n_neg, dim, mode):
+    """A workspace queried for a larger batch of the same chunks may hold fewer planes than this batch would take, down to one of either side:
+    the gradients are the same sums, and nothing past its end is written.  Less than that is refused."""
+    from cuke_amd._lib import KgeError
+    w = synth.custom_workload(model, n_ent=500, n_rel=7, dim=dim, batch=batch, chunk=chunk, n_neg=n_neg, norm_p=p, sigma=0.2, gamma=4.0,
+                              ent_zipf=0.8, seed=dim, lattice=(p == 1))
+    m, ix = gpu_model(w)
+    st = TrainStep(m, ix["h"], ix["r"], ix["t"], ix["neg"], chunk, neg_mode=mode, dpos=torch.randn(batch, device="cuda:0"),
+                   dneg=torch.randn((batch, n_neg), device="cuda:0"))
+    st.run()
+    want = in_64_bits(w, st.residual, st.dpos.double(), st.dneg.double(), mode, 1024)
+    like = _lib.Tables.from_buffer_copy(m._tab)  # the same rows without planes: dot products, or TransH's L2 tiles
+    like.model, like.norm_p = (m._tab.model, 2) if model == "TransH" else (_lib.MODELS["DistMult"], 2)
+    one, full = int(_lib.lib().kge_score_bwd_workspace(C.byref(like), C.byref(st.bat))), st._ws_b_bytes
+    plane = 4 * batch * dim
+    assert full > one + 3 * plane or model == "TransE" and p == 2
+    for size in sorted({one, one + plane + 1000, one + 2 * plane + 1000, one + 3 * plane + 1000, full - 1, full}):
+        if not one <= size <= full:
+            continue
+        room = torch.full((size + 4096,), 0x7f, dtype=torch.uint8, device="cuda:0")
+        st._ws_b, st._ws_b_bytes = room, size
+        for x in (st.ent_rows, st.rel_rows, st.aux_rows):
+            if x is not None:
+                x.fill_(float("nan"))
+        for fused in (None, False):
+            st.run(fused=fused)
+            g = st.sparse_grads()
+            for name, ids, rows, ref in (("entity", g.ent_ids, g.ent_rows, want[0]), ("relation", g.rel_ids, g.rel_rows, want[1]),
+                                         ("normal", g.rel_ids, g.aux_rows, want[2])):
+                if rows is not None:
+                    assert_close(rows.cpu().numpy(), ref[ids.long()].cpu().numpy(), what=f"{model} {size - one} bytes of planes, {name} rows", rows=True)
+            assert (room[size:] == 0x7f).all()
+    st._ws_b_bytes = one - 1
+    with pytest.raises(KgeError):
+        st.run()

@@ -1042,6 +1042,10 @@ class TrainStep:
         RESCAL inspect the relations first (the forward pass is planned from their groups); only
         the entity inspection rides.
 
+        Explicit TransR / RESCAL triples inspect both index sets in front of the step instead, in one batch of launches on the
+        same stream, where that is the faster form and ``fused`` is not given (``overlap`` says nothing then; fused=False
+        takes the side stream, fused=True the riding form).
+
         Otherwise, with overlap, the inspector runs on a side stream while the main stream
         computes scores and per-occurrence gradients; backward waits for it right before its
         segmented reduction.  TransR / RESCAL need the relation groups in the forward pass, so
@@ -1072,8 +1076,10 @@ class TrainStep:
             # took launches of their own between forward and backward; up to 4096 ids are one launch for both sets.  Both index sets
             # inspected in one batch up front are the faster chain then (with the optimizer steps: TransR 8192 triples x 200 of 1345
             # relations 221 -> 209 us, 4096 x 256 of 500 185 -> 176, 512 x 128 of 237 91 -> 74; RESCAL 512 x 128 80 -> 71; TransR 2048 x 201,
-            # which cannot ride, 310 -> 295; RESCAL 4096 x 200, 8192 ids and no back rows, 159 -> 161).
-            up_front = backward and not pipeline and self.needs_rel_groups and self.neg is None and \
+            # which cannot ride, 310 -> 295; RESCAL 4096 x 200, 8192 ids and no back rows, 159 -> 161).  Beyond 65536 ids each set takes
+            # launches of its own, and the entities' run beside the forward pass: the step alone, on the side stream / up front,
+            # 40000 x 100 of 50 relations 221 / 243 us, 100000 x 64 of 237 356 / 417, 100000 x 200 of 1345 735 / 799 (40000 x 200 448 / 433).
+            up_front = backward and not pipeline and self.needs_rel_groups and self.neg is None and 2 * self.B <= 65536 and \
                 (self.back_rows is not None or 2 * self.B <= 4096)
             fused = backward and not pipeline and self.fusable and not up_front
             overlap = overlap and not up_front

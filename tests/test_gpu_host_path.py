@@ -530,3 +530,19 @@ def test_a_set_is_not_refilled_under_a_plain_step(model, kw, step):
     assert again[0] is first[0]
     torch.cuda.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("batch,up_front", [(2000, True), (32768, True), (32769, False)])
+def test_large_explicit_batches_inspect_on_the_side_stream(batch, up_front):
+    """Explicit TransR triples: up to 65536 entity ids both sets in front of the step in one call, the entities of more beside the forward pass."""
+    from cuke_amd.kge import TrainStep
+    w = synth.custom_workload("TransR", n_ent=500, n_rel=9, dim=16, batch=batch, sigma=0.3, seed=4)
+    m, ix = gpu_model(w)
+    st, calls = TrainStep(m, ix["h"], ix["r"], ix["t"]), []
+    st.inspect = lambda *a: (calls.append(1), TrainStep.inspect(st, *a))
+    st.run()
+    got = _step_outputs(st)
+    assert calls == ([1] if up_front else [])
+    st.run(fused=False)
+    assert all(torch.equal(x, y) for x, y in zip(got, _step_outputs(st)))
+    assert calls == ([1] if up_front else [])

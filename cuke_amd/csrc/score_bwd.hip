@@ -748,12 +748,16 @@ namespace kge {
         else                                                                                                                     \
             hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, MF_, true, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi);  \
     } while (0)
+// (RotatE's rows by quads go by pairs, see pair_bwd.hpp; two to six floats take all three tile sizes: 65536 x 64 x 4 in chunks of 256, whole
+// step 219 us, by the smallest tiles alone 285)
 #define LAUNCH_TILE(RO_, GRID, ...)                                                                                              \
     do {                                                                                                                         \
-        if (a.vec)                                                                                                               \
-            LAUNCH_TILE_VEC(RO_, false, GRID, __VA_ARGS__);                                                                      \
-        else                                                                                                                     \
-            hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, false, false, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi); \
+        if constexpr (MODEL != KGE_ROTATE)                                                                                       \
+            if (a.vec) {                                                                                                         \
+                LAUNCH_TILE_VEC(RO_, false, GRID, __VA_ARGS__);                                                                  \
+                break;                                                                                                           \
+            }                                                                                                                    \
+        hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, RO_, false, false, false>), GRID, dim3(256), lds, st, a, g0, g1, occ_neg, __VA_ARGS__, fi); \
     } while (0)
 
 template <int MODEL, int P>
@@ -762,9 +766,9 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
 {
     const int klen = MODEL == KGE_ROTATE ? a.d / 2 : a.d;
     const int64_t gx = ceil_div(klen, kTI);
-    [[maybe_unused]] const bool narrow = narrow_cols(klen) > 0;       // the last 1..16 columns go to narrow tiles (64-owner VALU launches)
-    [[maybe_unused]] const int64_t gxw = narrow ? klen / kTI : gx;    // wide column tiles of such a launch
-    [[maybe_unused]] const int64_t big = gx * (ceil_div(a.C, 64) + ceil_div(a.N, 64)) * n_chunks;
+    const bool narrow = narrow_cols(klen) > 0;       // the last 1..16 columns go to narrow tiles (64-owner VALU launches)
+    const int64_t gxw = narrow ? klen / kTI : gx;    // wide column tiles of such a launch
+    const int64_t big = gx * (ceil_div(a.C, 64) + ceil_div(a.N, 64)) * n_chunks;
     // the size rule follows launch_neg_mp (see there)
     constexpr bool kDotModel = MODEL == KGE_DISTMULT || MODEL == KGE_COMPLEX || MODEL == KGE_TRANSF || MODEL == KGE_RESCAL;
     if constexpr (kDotModel || (MODEL == KGE_TRANSE && P == 2)) {
@@ -788,35 +792,26 @@ static int launch_tiles(TileArgs a, float *g0, float *g1, float *occ_neg, int64_
             return KGE_OK;
         }
     }
-    if constexpr (MODEL != KGE_ROTATE) {  // (RotatE's rows by quads go by pairs, see pair_bwd.hpp)
-        if (big >= 1024) {
-            const unsigned gh = xcd_grid(gxw, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxw, ceil_div(a.N, 64), n_chunks);
-            const unsigned nh = narrow ? xcd_grid(1, ceil_div(a.C, 64), n_chunks) : 0;
-            const unsigned nn = narrow ? xcd_grid(1, ceil_div(a.N, 64), n_chunks) : 0;
-            const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
-            const TileGrid tg{(int)gh, (int)gn, (int)nh, (int)nn};
-            LAUNCH_TILE(4, dim3(gh + gn + nh + nn + fi.blocks), tg);
-            KGE_CHECK_LAUNCH();
-            return KGE_OK;
-        }
-        if (big >= 512) {
-            const unsigned gh = xcd_grid(gx, ceil_div(a.C, 32), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 32), n_chunks);
-            const size_t lds = tile_lds_bytes<MODEL, 2>(fi);
-            const TileGrid tg{(int)gh, (int)gn, 0, 0};
-            LAUNCH_TILE(2, dim3(gh + gn + fi.blocks), tg);
-            KGE_CHECK_LAUNCH();
-            return KGE_OK;
-        }
-    }
-    // a batch this small leaves one or two 32-owner workgroups per CU: 16-owner tiles double the
-    // waves that hide each other's latency
-    const unsigned gh = xcd_grid(gx, ceil_div(a.C, 16), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 16), n_chunks);
-    const size_t lds = tile_lds_bytes<MODEL, 1>(fi);
-    const TileGrid tg{(int)gh, (int)gn, 0, 0};
-    if constexpr (MODEL == KGE_ROTATE)
-        hipLaunchKernelGGL((bwd_tile_kernel<MODEL, P, 1, false, false, false>), dim3(gh + gn + fi.blocks), dim3(256), lds, st, a, g0, g1, occ_neg, tg, fi);
-    else
+    if (big >= 1024) {
+        const unsigned gh = xcd_grid(gxw, ceil_div(a.C, 64), n_chunks), gn = xcd_grid(gxw, ceil_div(a.N, 64), n_chunks);
+        const unsigned nh = narrow ? xcd_grid(1, ceil_div(a.C, 64), n_chunks) : 0;
+        const unsigned nn = narrow ? xcd_grid(1, ceil_div(a.N, 64), n_chunks) : 0;
+        const size_t lds = tile_lds_bytes<MODEL, 4>(fi);
+        const TileGrid tg{(int)gh, (int)gn, (int)nh, (int)nn};
+        LAUNCH_TILE(4, dim3(gh + gn + nh + nn + fi.blocks), tg);
+    } else if (big >= 512) {
+        const unsigned gh = xcd_grid(gx, ceil_div(a.C, 32), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 32), n_chunks);
+        const size_t lds = tile_lds_bytes<MODEL, 2>(fi);
+        const TileGrid tg{(int)gh, (int)gn, 0, 0};
+        LAUNCH_TILE(2, dim3(gh + gn + fi.blocks), tg);
+    } else {
+        // a batch this small leaves one or two 32-owner workgroups per CU: 16-owner tiles double the
+        // waves that hide each other's latency
+        const unsigned gh = xcd_grid(gx, ceil_div(a.C, 16), n_chunks), gn = xcd_grid(gx, ceil_div(a.N, 16), n_chunks);
+        const size_t lds = tile_lds_bytes<MODEL, 1>(fi);
+        const TileGrid tg{(int)gh, (int)gn, 0, 0};
         LAUNCH_TILE(1, dim3(gh + gn + fi.blocks), tg);
+    }
     KGE_CHECK_LAUNCH();
     return KGE_OK;
 }

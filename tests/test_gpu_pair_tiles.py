@@ -83,7 +83,7 @@ def in_64_bits(w, rotated, dpos, dneg, mode, block):
     return [x.grad if x is not None else None for x in tabs]
 
 
-def compare_64(w, mode, what, block=1024):
+def compare_64(w, mode, what, block=1024, global_floor=0.0):
     m, ix = gpu_model(w)
     gen = torch.Generator("cuda:0").manual_seed(2)
     dpos, dneg = (torch.randn(n, device="cuda:0", generator=gen) for n in (w.batch, (w.batch, w.n_neg)))
@@ -93,7 +93,8 @@ def compare_64(w, mode, what, block=1024):
     for name, ids, rows, ref in (("entity", g.ent_ids, g.ent_rows, want[0]), ("relation", g.rel_ids, g.rel_rows, want[1]),
                                  ("normal", g.rel_ids, g.aux_rows, want[2])):
         if rows is not None:
-            assert_close(rows.cpu().numpy(), ref[ids.long()].cpu().numpy(), what=f"{what} {name} rows", rows=True)
+            assert_close(rows.cpu().numpy(), ref[ids.long()].cpu().numpy(), what=f"{what} {name} rows", rows=True,
+                         global_floor=global_floor)
 
 
 @pytest.mark.parametrize("model,p", [("RotatE", 2), ("TransE", 1), ("TransH", 1)])
@@ -142,3 +143,13 @@ def test_a_smaller_workspace(model, p, batch, chunk, n_neg, dim, mode):
     st._ws_b_bytes = one - 1
     with pytest.raises(KgeError):
         st.run()
+
+
+@pytest.mark.parametrize("mode", ["tail", "head"])
+@pytest.mark.parametrize("dim", [2, 4, 6])
+@pytest.mark.parametrize("batch,chunk,n_neg", [(8192, 16, 5), (2048, 8, 4), (130, 65, 33)])  # 64, 32 and 16 owners
+def test_rotate_rows_of_less_than_a_quad(batch, chunk, n_neg, dim, mode):
+    """These have no pair tiles."""
+    w = synth.custom_workload("RotatE", n_ent=4000, n_rel=7, dim=dim, batch=batch, chunk=chunk, n_neg=n_neg, sigma=0.2, gamma=4.0, seed=dim)
+    # (rows of two to six floats, each the sum of a few unit vectors that may nearly cancel: a tenth of the array's scale)
+    compare_64(w, mode, f"{batch}x{n_neg}x{dim} {mode}", global_floor=0.1)

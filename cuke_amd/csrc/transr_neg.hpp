@@ -130,10 +130,12 @@ struct NegIdx {
 
 // The groups of positives that share relation and chunk.  The relation inspection's order is stable, so within a relation the positives, and
 // with them their chunks, ascend: a group begins where either changes, and its first position holds its smallest positive.  A workgroup
-// owns kGroupPos positions and counts the groups that begin before them itself (8 bytes a position), so it waits for no other.
+// owns kGroupPos positions and counts the groups that begin before them itself (8 bytes a position), so it waits for no other; four workgroups'
+// positions at a time, since the last workgroup of 131072 positions goes through 31.
 //   gstart[u]: relation u's first group; segl[u]: its first list row = 2 per positive of the smaller relations + N per group
 // (The groups as an inspection of keys relation * n_chunks + chunk, with a kernel for the keys and one for the starts, took 26 us of
-// launches at 4096 positives; this one 8.)
+// launches at 4096 positives; this one 8.  With the row list and the plan behind it, us, groups before a workgroup one position range at a time / four:
+// 32768 positives 33 / 25, 65536 50 / 32, 131072 85 / 47; with the inspection 64, 42 and 74.)
 constexpr int kGroupThreads = 1024, kGroupPos = 4 * kGroupThreads;
 __global__ __launch_bounds__(kGroupThreads) void tneg_groups_kernel(NegIdx x)
 {
@@ -160,9 +162,22 @@ __global__ __launch_bounds__(kGroupThreads) void tneg_groups_kernel(NegIdx x)
     };
     const int start = (int)blockIdx.x * kGroupPos;
     int before = 0;
-    for (int q = 0; q < start; q += kGroupPos) {
-        look(q + 4 * tid);
-        before += __popc(heads);
+    constexpr int kFly = 4;
+    for (int q = 0; q < start; q += kFly * kGroupPos) {
+        int eb[kFly][5], eu[kFly][5];
+#pragma unroll
+        for (int v = 0; v < kFly; ++v) {
+            const int at = q + v * kGroupPos < start ? q + v * kGroupPos + 4 * tid : 4 * tid;  // (in front of `start`, or not counted)
+#pragma unroll
+            for (int i = 0; i < 5; ++i) eb[v][i] = x.r_perm[max(at + i - 1, 0)], eu[v][i] = x.r_sseg[max(at + i - 1, 0)];
+        }
+#pragma unroll
+        for (int v = 0; v < kFly; ++v) {
+            int n = q + v * kGroupPos + 4 * tid == 0 ? 1 : 0;  // (position 0 begins a group; its neighbour in front is itself here)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) n += eu[v][i + 1] != eu[v][i] || (uint32_t)eb[v][i + 1] / C != (uint32_t)eb[v][i] / C ? 1 : 0;
+            before += q + v * kGroupPos < start ? n : 0;
+        }
     }
     before = wave_sum_i(before);
     const int p = start + 4 * tid;

@@ -52,7 +52,7 @@ static NegShape neg_shape(const kge_tables *tab, const kge_batch *bat)
     return s;
 }
 
-// forward workspace: the group inspection, the row list, both tile plans and the projected rows;
+// forward workspace: the groups, the row list, both tile plans and the projected rows;
 // kge_score_bwd finds them through kge_saved.fwd_workspace
 struct NegFwdLayout {
     size_t knum, kseg, kinv, ksseg;
@@ -679,7 +679,7 @@ int launch_transr_neg_fwd(const kge_tables *tab, const kge_batch *bat, float *po
                           size_t workspace_bytes, hipStream_t st)
 {
     if (!transr_neg_path_ok(tab, bat)) return KGE_EUNSUPPORTED;
-    if (bat->fuse_inspection) return KGE_EINVAL;  // this path runs its own group inspection
+    if (bat->fuse_inspection) return KGE_EINVAL;  // no kernel of this path hosts the inspector's workgroups
     if (!neg) return KGE_EINVAL;
     const NegShape s = neg_shape(tab, bat);
     const NegFwdLayout l = neg_fwd_layout(s);

@@ -130,7 +130,7 @@ typedef struct kge_inspection {
 
 enum { KGE_NEG_TAIL = 0, KGE_NEG_HEAD = 1 };
 
-/* A margin loss whose partial sums are still to be added up: *loss = scale * sum of parts[0..n), n at most 1024.  Filled by
+/* (Host memory.)  A margin loss whose partial sums are still to be added up: *loss = scale * sum of parts[0..n), n at most 1024.  Filled by
    kge_margin_loss_parts, finished by the kge_score_bwd call whose kge_batch.loss_total points to it. */
 typedef struct kge_loss_total {
     const double *parts; /* in the loss call's workspace */
@@ -200,7 +200,8 @@ typedef struct kge_batch {
        executed backward pass (apps/kge/kge.py:393-515). */
     float *back_rows;
     /* Optional, read by kge_score_bwd alone: the loss of this batch that kge_margin_loss_parts left in parts, on the same
-       stream.  The last launch of kge_score_bwd adds it up, which takes a launch of its own off the chain of a step. */
+       stream (host memory, read by the call).  The last launch of kge_score_bwd adds it up, which takes a launch of its own off the
+       chain of a step. */
     const kge_loss_total *loss_total;
 } kge_batch;
 

@@ -784,6 +784,30 @@ def stream_calibration(torch, dev):
             "sample": "256 MiB device-to-device copy kernel, (bytes read + bytes written) / time, 4 rotating sources"}
 
 
+def summary(results, machine):
+    """The line of a run: the first workload's record with the machine's calibration and one compact row per workload inside
+    `roofline`.  The others' whole records (16 KB together) go to stderr, so that a reader who keeps the last kilobytes of the
+    output has the line whole."""
+    out = dict(results[0], machine=machine)
+    table = []
+    for r in results:
+        rf, cb = r["roofline"], r.get("cpu_baseline") or {}
+        row = {"workload": r["config"]["workload"], "ms_per_step": round(r["ms_per_step"], 5), "issue": r["config"]["issue"],
+               "scores_per_s": float(f"{r['value']:.4g}"), "kernel": rf["kernel"], "kernel_ms": round(rf["kernel_ms"], 5),
+               "bound": rf["bound"], "frac": round(rf["frac"], 4), "step_bound": rf["step"]["bound"],
+               "step_frac": round(rf["step"]["frac"], 4), "traffic": rf["traffic"],
+               "cpu_1_thread": float(f"{cb['value']:.4g}") if cb else None,
+               "cpu_all_cores": float(f"{cb['all_cores']['value']:.4g}") if cb else None,
+               "cpu_cores": cb["all_cores"]["cores"] if cb else None}
+        dn = r["config"].get("dense_projection_gradients")
+        if dn:
+            row["dense_ms_per_step"] = round(dn["ms_per_step"], 5)
+            row["dense_step_frac"] = round(dn["roofline"]["step"]["frac"], 4)
+        table.append(row)
+    out["roofline"] = dict(out["roofline"], per_workload=table)
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -865,28 +889,9 @@ def main():
               + (f"; every projection gradient dense: {dn['ms_per_step']:.4f} ms/step, step "
                  f"{dn['roofline']['step']['frac']:.3f}" if dn else ""),
               file=sys.stderr, flush=True)
-    out = results[0]
-    out["machine"] = machine
-    if len(results) > 1:
-        out["per_workload"] = results[1:]
-    # one compact row per workload inside `roofline` (the full records are in per_workload)
-    table = []
-    for r in results:
-        rf, cb = r["roofline"], r.get("cpu_baseline") or {}
-        row = {"workload": r["config"]["workload"], "ms_per_step": round(r["ms_per_step"], 5), "issue": r["config"]["issue"],
-               "scores_per_s": float(f"{r['value']:.4g}"), "kernel": rf["kernel"], "kernel_ms": round(rf["kernel_ms"], 5),
-               "bound": rf["bound"], "frac": round(rf["frac"], 4), "step_bound": rf["step"]["bound"],
-               "step_frac": round(rf["step"]["frac"], 4), "traffic": rf["traffic"],
-               "cpu_1_thread": float(f"{cb['value']:.4g}") if cb else None,
-               "cpu_all_cores": float(f"{cb['all_cores']['value']:.4g}") if cb else None,
-               "cpu_cores": cb["all_cores"]["cores"] if cb else None}
-        dn = r["config"].get("dense_projection_gradients")
-        if dn:
-            row["dense_ms_per_step"] = round(dn["ms_per_step"], 5)
-            row["dense_step_frac"] = round(dn["roofline"]["step"]["frac"], 4)
-        table.append(row)
-    out["roofline"]["per_workload"] = table
-    print(json.dumps(out))
+    for r in results[1:]:
+        print("[bench] record " + json.dumps(r), file=sys.stderr, flush=True)
+    print(json.dumps(summary(results, machine)))
 
 
 if __name__ == "__main__":

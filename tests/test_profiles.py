@@ -48,3 +48,21 @@ def test_every_profile_states_its_commands_and_calibration():
 
 def bench_workloads():
     return sorted({c[0] for c in CASES})
+
+
+def test_the_line_of_all_workloads_is_short(bench):
+    """Six records as long as the longest of them make a line of less than 8000 bytes that still says every workload's times."""
+    import json
+
+    def record(name, ms):
+        return {"metric": "scores", "value": 16793600 / ms, "ms_per_step": ms, "config": {"workload": name, "issue": "direct", "more": "x" * 1500},
+                "kernels_ms": {"bwd_tile_kernel": ms}, "cpu_baseline": {"value": 1e6, "cores": 1, "all_cores": {"value": 1e7, "cores": 16}},
+                "roofline": {"kernel": "transr_plan_kernel + transr_fwd_back_kernel", "kernel_ms": ms, "bound": "fp32_valu", "frac": 0.325022389,
+                             "traffic": 1247840000, "step": {"bound": "fp32", "frac": 0.307805355}, "more": "x" * 500}}
+
+    results = [record(n, 0.1 * (i + 1)) for i, n in enumerate(bench.ALL_WORKLOADS)]
+    out = bench.summary(results, {"stream_copy_gbs": 5303.594221744644, "peak_gbs": 8000.0, "sample": "x" * 100})
+    assert len(json.dumps(out)) < 8000 and len(json.dumps(results)) > 12000
+    assert out["config"] == results[0]["config"] and out["value"] == results[0]["value"]
+    assert [(r["workload"], r["ms_per_step"]) for r in out["roofline"]["per_workload"]] == [(r["config"]["workload"], round(r["ms_per_step"], 5)) for r in results]
+    assert "per_workload" not in results[0]["roofline"]

@@ -55,10 +55,10 @@ def test_one_call_staged_and_captured_steps():
 
 
 @pytest.mark.parametrize("model", ["TransR", "RESCAL"])
-@pytest.mark.parametrize("batch,dim,n_rel", [(1024, 1024, 2), (2048, 1024, 7), (4096, 512, 15), (8192, 200, 20)])
+@pytest.mark.parametrize("batch,dim,n_rel", [(1024, 1024, 2), (2048, 1024, 7), (4096, 512, 15), (8192, 200, 20), (2048, 1022, 7)])
 def test_beside_the_sums_of_split_relations(model, batch, dim, n_rel):
     """Explicit triples, where level 1 of the reduction rides with dM and level 2 carries the split relations' sums and the loss: more pieces of
-    sums than the grid has workgroups, and (8192 x 200) fewer."""
+    sums than the grid has workgroups, (8192 x 200) fewer, (1022) rows that are padded first."""
     w = synth.custom_workload(model, n_ent=300, n_rel=n_rel, dim=dim, batch=batch, sigma=0.2, seed=batch)
     m, ix = gpu_model(w)
     r = torch.arange(batch, device="cuda") % n_rel
